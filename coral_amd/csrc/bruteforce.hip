@@ -266,15 +266,18 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __
 // id), sorted, into out.  The scheme of row_select_kernel on keys: the k-th smallest of the per-thread minima bounds
 // the k-th smallest key from above, a second pass collects what lies up to it, a sort finishes.  *overflow is raised
 // when a list lost entries (cnt[q] > cap) or the collection outgrows LDS; the caller then takes another path.
-__global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned long long* __restrict__ lists,
-                                                                  int64_t cap, const unsigned int* __restrict__ cnt,
-                                                                  int k, unsigned long long* __restrict__ out,
-                                                                  int64_t out_stride, int* __restrict__ overflow) {
+// SHRINK: the result replaces the list (out = lists, out_stride = cap) and its count, and tau[q] becomes the value
+// of the k-th key.
+template <bool SHRINK>
+__global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned long long* lists, int64_t cap,
+                                                                  unsigned int* cnt, int k, unsigned long long* out,
+                                                                  int64_t out_stride, float* __restrict__ tau,
+                                                                  int* __restrict__ overflow) {
     __shared__ unsigned long long skeys[kSelCap];
     __shared__ unsigned long long smin[kSelThreads];
     __shared__ unsigned int s_count;
     const int tid = threadIdx.x;
-    const unsigned int have = cnt[blockIdx.x];
+    const unsigned int have = cnt[(size_t)blockIdx.x * kCntStride];
     if (have > (unsigned)cap) {
         if (tid == 0) atomicAdd(overflow, 1);
         return;
@@ -326,6 +329,14 @@ __global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned
             __syncthreads();
         }
     unsigned long long* dst = out + (size_t)blockIdx.x * out_stride;
+    if constexpr (SHRINK) {  // every thread has read the list: the barriers of the sort lie in between
+        for (int i = tid; i < kk; i += kSelThreads) dst[i] = skeys[i];
+        if (tid == 0) {
+            cnt[(size_t)blockIdx.x * kCntStride] = (unsigned)kk;
+            tau[blockIdx.x] = kk == k ? bf_unord32((uint32_t)(skeys[k - 1] >> 32)) : __int_as_float(0x7f800000);
+        }
+        return;
+    }
     for (int i = tid; i < k; i += kSelThreads) {
         unsigned long long key = i < kk ? skeys[i] : ~0ull;
         if ((uint32_t)(key >> 32) == bf_ord32(__int_as_float(0x7f800000))) key = ~0ull;  // tombstoned
@@ -524,7 +535,15 @@ hipError_t launch_row_select(const float* D, int64_t ldD, int nq, int64_t n, int
 hipError_t launch_list_select(const unsigned long long* lists, int64_t cap, const unsigned int* cnt, int nq, int k,
                               unsigned long long* out, int64_t out_stride, int* overflow, hipStream_t stream) {
     if (k > kSelThreads) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(list_select_kernel, dim3(nq), dim3(kSelThreads), 0, stream, lists, cap, cnt, k, out, out_stride,
+    hipLaunchKernelGGL(list_select_kernel<false>, dim3(nq), dim3(kSelThreads), 0, stream, lists, cap,
+                       const_cast<unsigned int*>(cnt), k, out, out_stride, (float*)nullptr, overflow);
+    return hipGetLastError();
+}
+
+hipError_t launch_list_shrink(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, float* tau,
+                              int* overflow, hipStream_t stream) {
+    if (k > kSelThreads || k > cap) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(list_select_kernel<true>, dim3(nq), dim3(kSelThreads), 0, stream, lists, cap, cnt, k, lists, cap, tau,
                        overflow);
     return hipGetLastError();
 }

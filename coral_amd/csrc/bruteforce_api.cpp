@@ -33,7 +33,9 @@ int knn_passes(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, i
     float* D = nullptr;
     unsigned long long* part = nullptr;
     int* redo = nullptr;
+    void* d_split = nullptr;
     auto release = [&]() {
+        (void)hipFree(d_split);
         (void)hipFree(D);
         (void)hipFree(part);
         (void)hipFree(redo);
@@ -50,15 +52,18 @@ int knn_passes(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, i
     HIP_TRY_R(hipMalloc(&D, (size_t)qc * ld * sizeof(float)));
     HIP_TRY_R(hipMalloc(&part, (size_t)Q * nseg * k * sizeof(unsigned long long)));
     HIP_TRY_R(hipMalloc(&redo, (size_t)qc * sizeof(int)));
+    if (screen) HIP_TRY_R(hipMalloc(&d_split, coral::split_queries_bytes((int)qc, idx->dim)));
     for (int64_t q0 = 0; q0 < Q; q0 += qc) {
         const int nq = (int)std::min<int64_t>(qc, Q - q0);
+        if (screen)
+            HIP_TRY_R(coral::launch_split_queries(d_queries + (size_t)q0 * idx->dim, nq, idx->dim, d_qn + q0, d_split, stream));
         for (int64_t s = 0; s < nseg; ++s) {
             const int64_t b0 = s * seg, nb = std::min(seg, n - b0);
             const float* qp = d_queries + (size_t)q0 * idx->dim;
             const float* bp = idx->d_vec + (size_t)b0 * idx->dim;
             const uint32_t* del = have_delete ? idx->d_deleted : nullptr;
             if (screen)
-                HIP_TRY_R(coral::launch_approx_tile(qp, bp, nq, nb, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm + b0, del,
+                HIP_TRY_R(coral::launch_approx_tile(d_split, bp, nq, nb, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm + b0, del,
                                                     b0, D, ld, stream));
             else
                 HIP_TRY_R(coral::launch_distance_tile(qp, bp, nq, nb, idx->dim, idx->metric, del, b0, D, ld, stream));
@@ -96,10 +101,12 @@ constexpr int64_t kListCap = 16384;  // keys a query's candidate list holds in t
 // queries: (1) the distances to a sample of the base (every stride-th tile of 128 points) as a small matrix, whose
 // kc-th smallest entry per row is a bound tau[q] that at least kc entries of the whole row do not exceed; (2) one
 // pass over the whole base that appends the entries up to tau[q] to the query's list (about kc * n / sample of
-// them); (3) the kc smallest keys of every list.  The kept candidates are those of knn_passes(screen = true): the
-// same approximate values, the kc smallest under (value, id).  *used = false when the shape does not suit (kc beyond
-// what list_select_kernel takes, a base too small to sample) or a list overflowed (sample unlike the base, rows of
-// equal values, too few live points in the sample): the caller then goes through the matrix.
+// them) -- or two, where the base is many times the sample: first every step-th tile, whose kc smallest entries give
+// a tighter bound for the rest, then the tiles between; (3) the kc smallest keys of every list.  The kept candidates
+// are those of knn_passes(screen = true): the same approximate values, the kc smallest under (value, id).
+// *used = false when the shape does not suit (kc beyond what list_select_kernel takes, a base too small to sample) or
+// a list overflowed (sample unlike the base, rows of equal values, too few live points in the sample): the caller
+// then goes through the matrix.
 int knn_screen_fused(coral_index* idx, const float* d_queries, int32_t Q, int32_t kc, int32_t have_delete,
                      const float* d_qn, int32_t* d_cid, float* d_cd, hipStream_t stream, bool* used) {
     *used = false;
@@ -107,16 +114,26 @@ int knn_screen_fused(coral_index* idx, const float* d_queries, int32_t Q, int32_
     int64_t tiles = (2 * (int64_t)kc * full_tiles + kListCap - 1) / kListCap;
     tiles = std::max<int64_t>(8, (tiles + 7) & ~(int64_t)7);
     if (kc > 1024 || tiles * 8 > full_tiles || n > 0x7fffffff) return CORAL_OK;
+    // A larger sample than the lists need: an entry that passes costs an atomic and a scattered write.  A sixteenth of
+    // the base, up to 16 384 points.
+    tiles = std::max(tiles, std::min<int64_t>(128, (full_tiles / 16) & ~(int64_t)7));
     const int64_t stride = full_tiles / tiles, ns = tiles * 128;
+    // Two passes with bounds from ns and then from n / step points let through kc (n / step / ns + step) entries per
+    // query instead of kc n / ns; step balances the two.  Worth a pass more only where the appending weighs more than
+    // the launches.
+    int step = 1;
+    if (Q >= 1024 && stride >= 16)
+        while ((step + 1) * (step + 1) <= stride) ++step;
     int64_t qc = std::min<int64_t>(kListCap, (kBufferFloats / ns) & ~(int64_t)127);
     qc = std::min<int64_t>(qc, ((int64_t)Q + 127) & ~(int64_t)127);
     float *D = nullptr, *tau = nullptr;
     unsigned long long *keys = nullptr, *lists = nullptr;
     unsigned int* cnt = nullptr;
     int *redo = nullptr, *overflow = nullptr;
+    void* d_split = nullptr;
     auto release = [&]() {
         (void)hipFree(D), (void)hipFree(tau), (void)hipFree(keys), (void)hipFree(lists);
-        (void)hipFree(cnt), (void)hipFree(redo), (void)hipFree(overflow);
+        (void)hipFree(cnt), (void)hipFree(redo), (void)hipFree(overflow), (void)hipFree(d_split);
     };
 #define HIP_TRY_R(expr)                                                                  \
     do {                                                                                 \
@@ -131,7 +148,8 @@ int knn_screen_fused(coral_index* idx, const float* d_queries, int32_t Q, int32_
     HIP_TRY_R(hipMalloc(&tau, (size_t)qc * sizeof(float)));
     HIP_TRY_R(hipMalloc(&keys, (size_t)qc * kc * sizeof(unsigned long long)));
     HIP_TRY_R(hipMalloc(&lists, (size_t)qc * kListCap * sizeof(unsigned long long)));
-    HIP_TRY_R(hipMalloc(&cnt, (size_t)qc * sizeof(unsigned int)));
+    HIP_TRY_R(hipMalloc(&cnt, (size_t)qc * coral::kCntStride * sizeof(unsigned int)));
+    HIP_TRY_R(hipMalloc(&d_split, coral::split_queries_bytes((int)qc, idx->dim)));
     HIP_TRY_R(hipMalloc(&redo, (size_t)qc * sizeof(int)));
     HIP_TRY_R(hipMalloc(&overflow, sizeof(int)));
     HIP_TRY_R(coral::launch_fill_u32(reinterpret_cast<uint32_t*>(overflow), 1, 0u, stream));
@@ -139,13 +157,19 @@ int knn_screen_fused(coral_index* idx, const float* d_queries, int32_t Q, int32_
     for (int64_t q0 = 0; q0 < Q; q0 += qc) {
         const int nq = (int)std::min<int64_t>(qc, Q - q0);
         const float* qp = d_queries + (size_t)q0 * idx->dim;
-        HIP_TRY_R(coral::launch_approx_tile(qp, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm, del, 0, D,
-                                            ns, stream, tiles, stride));
+        HIP_TRY_R(coral::launch_split_queries(qp, nq, idx->dim, d_qn + q0, d_split, stream));
+        HIP_TRY_R(coral::launch_approx_tile(d_split, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm, del,
+                                            0, D, ns, stream, tiles, (int)stride));
         HIP_TRY_R(coral::launch_row_select(D, ns, nq, ns, kc, 0, keys, kc, redo, stream));
         HIP_TRY_R(coral::launch_bound_from_keys(keys, kc, kc - 1, nq, tau, stream));
-        HIP_TRY_R(coral::launch_fill_u32(cnt, (size_t)nq, 0u, stream));
-        HIP_TRY_R(coral::launch_approx_filter(qp, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm, del, tau,
-                                              lists, kListCap, cnt, stream));
+        HIP_TRY_R(coral::launch_fill_u32(cnt, (size_t)nq * coral::kCntStride, 0u, stream));
+        HIP_TRY_R(coral::launch_approx_filter(d_split, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm, del,
+                                              tau, lists, kListCap, cnt, step, stream));
+        if (step > 1) {
+            HIP_TRY_R(coral::launch_list_shrink(lists, kListCap, cnt, nq, kc, tau, overflow, stream));
+            HIP_TRY_R(coral::launch_approx_filter(d_split, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm,
+                                                  del, tau, lists, kListCap, cnt, -step, stream));
+        }
         HIP_TRY_R(coral::launch_list_select(lists, kListCap, cnt, nq, kc, keys, kc, overflow, stream));
         HIP_TRY_R(coral::launch_merge_segments(keys, nq, 1, kc, /*signed distances*/ 0, d_cid + (size_t)q0 * kc,
                                                d_cd + (size_t)q0 * kc, stream));

@@ -3,19 +3,28 @@
 // The exact search (bruteforce.hip) accumulates every (query, base) pair in the reference's order, one fused
 // multiply-add per dimension on the vector units, because ids and distances must be reproducible bit for bit.  Almost
 // all of that work goes into pairs that are nowhere near the k best.  Here the same pairs are first measured
-// approximately, as |q|^2 + |b|^2 - 2 q.b with the inner products on fp32 MFMA (v_mfma_f32_32x32x2_f32: full
-// fp32 operands and accumulation, only the order of the additions differs), k + 32 candidates per query are kept,
-// and rerank_kernel measures just those in the reference's order.  The result is exact, not approximately exact: a
-// query is accepted only if its k-th exact distance lies below the worst kept approximate distance by more than a
-// bound on what the two ways of rounding can differ by; otherwise it is flagged and goes through the exact search.
+// approximately, as |q|^2 + |b|^2 - 2 q.b with the inner products on the matrix cores, k + 32 candidates per query
+// are kept, and rerank_kernel measures just those in the reference's order.  The result is exact, not approximately
+// exact: a query is accepted only if its k-th exact distance lies below the worst kept approximate distance by more
+// than a bound on what the two ways of rounding can differ by; otherwise it is flagged and goes through the exact
+// search.
 //
-// Error bound.  With u = 2^-24 and any order of fp32 fused multiply-adds, a sum of dim products q_i b_i is within
-// dim u |q| |b| of the true value (first order), the two norms within dim u of themselves, the two final additions
-// add 4 u (|q|^2 + |b|^2); the reference-order distance itself is within (dim + 2) u of the true one.  Together the
-// approximate and the reference-order value of a pair differ by less than 4 (dim + 2) u (|q|^2 + |b|^2); the check
-// uses twice that, with the largest |b|^2 of the index.
+// The inner products.  A row x is scaled by a power of two that puts |x| into [2^13, 2^14) and every scaled component
+// is split into two halves, hi = half(x) and lo = half(x - hi); x - hi is exact, so hi + lo is x to 22 bits.  Then
+// q.b = hi.hi + hi.lo + lo.hi on v_mfma_f32_32x32x16_f16 (products exact, fp32 accumulation): three multiplications at
+// sixteen times the rate of the fp32 form.
+//
+// Error bound, with u = 2^-24.  Splitting: each component is off by at most 2^-22 of itself, and lo.lo is left out:
+// 12 u |q| |b| over the sum (components below 2^-28 of their row's norm lose more, but of less: sqrt(dim) 2^-38 |q| |b|
+// in all).  Accumulation: 3 dim additions, within 2 u of the running sum each even if the hardware truncates:
+// 6 dim u |q| |b|.  The inner product enters twice: (6 dim + 12) u (|q|^2 + |b|^2).  The two norms are within dim u of
+// themselves, the final additions add 4 u (|q|^2 + |b|^2), the reference-order distance is within (dim + 2) u of the
+// true one.  Together the approximate and the reference-order value of a pair differ by less than
+// 8 (dim + 4) u (|q|^2 + |b|^2); the check takes the largest |b|^2 of the index.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "bruteforce.h"
 
@@ -24,14 +33,10 @@ namespace coral {
 namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-#ifndef CORAL_MFMA_BK
-#define CORAL_MFMA_BK 8
-#endif
-constexpr int MT = 128, NT = 128, BK = CORAL_MFMA_BK;  // tile of queries x base points per workgroup, dimensions per LDS stage
-constexpr int NS = BK / 8;                              // 16-byte pieces per thread, operand and stage
-constexpr int RS = BK == 8 ? 8 : BK + 4;                // floats from one row to the next in LDS
-
+constexpr int MT = 256, NT = 128, BK = 16;  // tile of queries x base points per workgroup, dimensions per LDS stage
+constexpr int kStageA = 2 * MT * BK, kStageB = 2 * NT * BK;  // halves per stage: the hi plane, then the lo plane
 
 __device__ __forceinline__ uint32_t mf_ord32(float s) {
     const uint32_t u = __float_as_uint(s);
@@ -40,6 +45,25 @@ __device__ __forceinline__ uint32_t mf_ord32(float s) {
 __device__ __forceinline__ float mf_unord32(uint32_t o) {
     const uint32_t u = (o & 0x80000000u) ? (o ^ 0x80000000u) : ~o;
     return __uint_as_float(u);
+}
+
+// e with |x| 2^e in [2^13, 2^14) for a row of squared norm n2; within [-40, 60], which rows of norm 0, of norms whose
+// square leaves the normal range, and of infinite norms meet (the last are never accepted: their error bound is
+// infinite), so that no product of two such powers overflows
+__device__ __forceinline__ int mf_scale_exp(float n2) {
+    const int E = (int)((__float_as_uint(n2) >> 23) & 0xffu) - 127;  // n2 in [2^E, 2^(E+1))
+    return max(-40, min(60, 13 - (E >> 1)));
+}
+__device__ __forceinline__ float mf_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// eight scaled components as two planes of halves
+__device__ __forceinline__ void mf_split8(const float4 a, const float4 b, float s, v8h& hi, v8h& lo) {
+    const float x[8] = {a.x * s, a.y * s, a.z * s, a.w * s, b.x * s, b.y * s, b.z * s, b.w * s};
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        hi[j] = (_Float16)x[j];
+        lo[j] = (_Float16)(x[j] - (float)hi[j]);
+    }
 }
 
 // |x|^2 per row, and the largest of them (as the bit pattern of a non-negative float)
@@ -62,42 +86,69 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict_
     }
 }
 
+// The queries as the tile kernel reads them: per tile of 256 queries and stage of 16 dimensions, the hi plane and the
+// lo plane, each [256 rows][16 halves] -- a stage of a tile is 16 KB in the order in which it lies in LDS.  Rows beyond
+// the batch and dimensions beyond dim are zero.
+__global__ __launch_bounds__(256) void split_queries_kernel(const float* __restrict__ queries, int nq, int dim, int stages,
+                                                           const float* __restrict__ qn, _Float16* __restrict__ out) {
+    const int st = blockIdx.x, row = threadIdx.x;
+    const int64_t q = (int64_t)blockIdx.y * MT + row;
+    _Float16* dst = out + ((size_t)blockIdx.y * stages + st) * kStageA + row * BK;
+    const float s = q < nq ? mf_pow2(mf_scale_exp(qn[q])) : 0.0f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float4 v[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = st * BK + 8 * h + 4 * u;
+            v[u] = make_float4(0, 0, 0, 0);
+            if (q < nq && k < dim) v[u] = *reinterpret_cast<const float4*>(queries + (size_t)q * dim + k);
+        }
+        v8h hi, lo;
+        mf_split8(v[0], v[1], s, hi, lo);
+        *reinterpret_cast<v8h*>(dst + 8 * h) = hi;
+        *reinterpret_cast<v8h*>(dst + MT * BK + 8 * h) = lo;
+    }
+}
+
 // D[q][b] ~ signed distance (smaller is closer): |q|^2 + |b|^2 - 2 q.b for L2, -q.b for IP; +inf for tombstoned
-// ids.  One workgroup per 128 x 128 tile (the mapping of blockIdx to tiles is at the head of the kernel), 256
-// threads = 4 wavefronts in 2 x 2, each 64 x 64 of the tile as 2 x 2 MFMA blocks of 32 x 32.  Operands go through
-// LDS dimension-major, so that the 32 lanes of an MFMA operand read consecutive words.
-#ifndef CORAL_MFMA_WAVES
-#define CORAL_MFMA_WAVES 4
-#endif
-// FUSED = false writes the tile into D (column bt * 128 + ..., where bt counts the tiles this launch computes:
-// tile_stride > 1 takes every tile_stride-th tile of the base, a sample whose columns lie side by side in D).
+// ids.  One workgroup per 256 x 128 tile (the mapping of blockIdx to tiles is at the head of the kernel), 256
+// threads = 4 wavefronts in 2 x 2, each 128 x 64 of the tile as 4 x 2 MFMA blocks of 32 x 32.
+// FUSED = false writes the tile into D (column bt * 128 + ..., where bt counts the tiles this launch computes).
 // FUSED = true writes no matrix: an entry goes, as the key ord(value) << 32 | id, to the list of its query if it does
-// not exceed the query's bound tau[q] -- cnt[q] entries so far, at most cap kept (a count beyond cap tells the
-// caller that the list is incomplete).  A tile's entries are first gathered in LDS, so that the global counters see
-// one round of atomics per tile instead of one per accumulator register.
+// not exceed the query's bound tau[q] -- cnt[q * kCntStride] entries so far, at most cap kept (a count beyond cap
+// tells the caller that the list is incomplete).  A tile's entries are first gathered in LDS, so that the global
+// counters see one round of atomics per tile instead of one per accumulator register.
+// The tiles of a launch: tile_step > 0 takes tiles 0, tile_step, 2 tile_step ... of the base, tile_step < 0 the tiles
+// between those (all that are no multiple of -tile_step).
+//
+// Bound by the matrix cores in principle (three half-precision products per pair and dimension, 833 TFLOP/s of
+// pair-dimensions at the card's dense rate), in practice by LDS: a wavefront reads 12 KB per 24 multiplications
+// (768 cycles of its matrix core; the reads of a CU's four wavefronts take 384 cycles of its LDS, parking the next
+// stage 192), which is why a wavefront has a 128 x 64 tile and not the 64 x 64 that the fp32 form had.  The queries
+// come split (split_queries_kernel: every query tile is read by thousands of workgroups); the base is split here, on
+// its way to LDS, eight components per thread and stage under the other wavefronts' multiplications: a split copy of
+// the base would double the index or cost a pass over it per call, which small batches would feel.
 template <bool FUSED, bool L2>
-__global__ __launch_bounds__(256, CORAL_MFMA_WAVES) void approx_tile_mfma_kernel(const float* __restrict__ queries,
+__global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16* __restrict__ queries,
                                                               const float* __restrict__ base, int nq, int64_t nb,
                                                               int dim, const float* __restrict__ qn,
                                                               const float* __restrict__ bn,
                                                               const uint32_t* __restrict__ deleted, int64_t base_id0,
-                                                              int64_t ntiles, int64_t tile_stride, int hq,
+                                                              int64_t ntiles, int tile_step, int hq,
                                                               float* __restrict__ D, int64_t ldD,
                                                               const float* __restrict__ tau,
                                                               unsigned long long* __restrict__ lists, int64_t cap,
                                                               unsigned int* __restrict__ cnt) {
-    // Operands in LDS row-major, the BK = 8 dimensions of a row side by side (32 bytes): a thread parks the 16 bytes
-    // it fetched with one write, and the 16 bytes a lane reads hold its operands of four multiplications -- lane
-    // (kh, m) supplies row m's dimension kh * 4 + j to step j, so a step multiplies the dimension pair (j, 4 + j) of
-    // the stage.  The 64 lanes of either access cover consecutive addresses: no bank conflicts, no padding.
-    __shared__ __align__(16) float sa[2][MT][RS];
-    __shared__ __align__(16) float sb[2][NT][RS];
-    static_assert(BK % 8 == 0, "a stage is made of 16-byte pieces, one per thread, operand and eight dimensions");
+    // A row's 16 dimensions of a plane lie side by side (32 bytes); lane (kh, m) of a wavefront supplies row m's
+    // dimensions kh * 8 .. + 7, one 16-byte read, and the 64 lanes of a read cover 2 KB of consecutive addresses.
+    __shared__ __align__(16) _Float16 sa[2][kStageA];
+    __shared__ __align__(16) _Float16 sb[2][kStageB];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wr = wave >> 1, wc = wave & 1;
     // Workgroups go to the eight XCDs in turn, each with an L2 of its own (4 MB).  An XCD takes every eighth tile of
     // base points and walks, for one block of hq query tiles after the other, through all its base tiles: the
-    // workgroups in flight on it share those hq query tiles (hq x 100 KB at dim 200) and a handful of base tiles,
+    // workgroups in flight on it share those hq query tiles (hq x 213 KB at dim 200) and a handful of base tiles,
     // so both operands come from that L2 and each base tile from memory once per block of queries.
     // grid.x = 8 x ceil(base tiles / 8) x query blocks x hq.
     const int nqt = (nq + MT - 1) / MT;
@@ -106,161 +157,161 @@ __global__ __launch_bounds__(256, CORAL_MFMA_WAVES) void approx_tile_mfma_kernel
     const unsigned qb = place / (nbt8 * (unsigned)hq), rem = place - qb * nbt8 * (unsigned)hq;
     const int64_t bt = (int64_t)(rem / (unsigned)hq) * 8 + xcd;
     const int qt = (int)(qb * (unsigned)hq + rem % (unsigned)hq);
-    const int64_t b0 = bt * tile_stride * NT;
+    const int64_t b0 = (tile_step > 0 ? bt * tile_step : bt + bt / (-tile_step - 1) + 1) * NT;
     const int q0 = qt * MT;
     if (bt >= ntiles || b0 >= nb || qt >= nqt) return;  // padding: the last group of eight base tiles, the last query block
-    const int lrow = tid >> 1, lk = (tid & 1) * 4;  // staging: thread t loads row t/2, dimensions (t&1)*4 .. +4
-    // rows beyond the end read the last row instead: their results are never written
-    const float* pa = queries + (size_t)min(q0 + lrow, nq - 1) * dim + lk;
-    const float* pb = base + (size_t)min(b0 + lrow, nb - 1) * dim + lk;
-    float4 va[NS], vb[NS];
-    auto park = [&](int buf) {
+    const int full = dim / BK, tail = dim % BK;
+    const int stages = full + (tail ? 1 : 0);
+    // staging: thread t copies 4 x 16 bytes of the query stage and splits row t/2, dimensions (t&1)*8 .. +8 of the
+    // base; rows beyond the end read the last row instead: their results are never written
+    const int lrow = tid >> 1, lk = (tid & 1) * 8;
+    const _Float16* pa = queries + (size_t)qt * stages * kStageA + tid * 8;
+    const int64_t brow = min(b0 + lrow, nb - 1);
+    const float* pb = base + (size_t)brow * dim + lk;
+    const float bscale = mf_pow2(mf_scale_exp(bn[brow]));
+    v8h va[4];
+    float4 vb[2];
+    auto fetch = [&](int st) {
 #pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            *reinterpret_cast<float4*>(&sa[buf][lrow][8 * u + lk]) = va[u];
-            *reinterpret_cast<float4*>(&sb[buf][lrow][8 * u + lk]) = vb[u];
+        for (int u = 0; u < 4; ++u) va[u] = *reinterpret_cast<const v8h*>(pa + (size_t)st * kStageA + u * 2048);
+        if (st < full) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) vb[u] = *reinterpret_cast<const float4*>(pb + st * BK + 4 * u);
+        } else {  // part of a stage (dim is a multiple of 4): what is missing is zero
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                vb[u] = make_float4(0, 0, 0, 0);
+                if (lk + 4 * u < tail) vb[u] = *reinterpret_cast<const float4*>(pb + st * BK + 4 * u);
+            }
         }
     };
-    v16f acc[2][2];
+    auto park = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<v8h*>(&sa[buf][u * 2048 + tid * 8]) = va[u];
+        v8h hi, lo;
+        mf_split8(vb[0], vb[1], bscale, hi, lo);
+        *reinterpret_cast<v8h*>(&sb[buf][lrow * BK + lk]) = hi;
+        *reinterpret_cast<v8h*>(&sb[buf][NT * BK + lrow * BK + lk]) = lo;
+    };
+    v16f acc[4][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-    const int kh = lane >> 5, m = lane & 31;  // an MFMA operand: lane = row (or column) m of dimension kh
-    // the last stage may hold half a row (dim is a multiple of 4): its missing half is zero
-    const int full = dim / BK, tail = dim % BK;
-    auto fetch = [&](int st) {
-#pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            va[u] = *reinterpret_cast<const float4*>(pa + st * BK + 8 * u);
-            vb[u] = *reinterpret_cast<const float4*>(pb + st * BK + 8 * u);
-        }
-    };
-    auto fetch_tail = [&]() {
-#pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            va[u] = make_float4(0, 0, 0, 0), vb[u] = make_float4(0, 0, 0, 0);
-            if (8 * u + lk < tail) {
-                va[u] = *reinterpret_cast<const float4*>(pa + full * BK + 8 * u);
-                vb[u] = *reinterpret_cast<const float4*>(pb + full * BK + 8 * u);
-            }
-        }
-    };
+    const int kh = lane >> 5, m = lane & 31;  // an MFMA operand: lane = row (or column) m, dimensions kh * 8 .. + 7
     auto multiply = [&](int buf) {
+        const _Float16* A = &sa[buf][(wr * 128 + m) * BK + kh * 8];
+        const _Float16* B = &sb[buf][(wc * 64 + m) * BK + kh * 8];
+        v8h ah[4], al[4], bh[2], bl[2];
 #pragma unroll
-        for (int u = 0; u < NS; ++u) {
-            const float4 a0 = *reinterpret_cast<const float4*>(&sa[buf][wr * 64 + m][8 * u + kh * 4]);
-            const float4 a1 = *reinterpret_cast<const float4*>(&sa[buf][wr * 64 + 32 + m][8 * u + kh * 4]);
-            const float4 c0 = *reinterpret_cast<const float4*>(&sb[buf][wc * 64 + m][8 * u + kh * 4]);
-            const float4 c1 = *reinterpret_cast<const float4*>(&sb[buf][wc * 64 + 32 + m][8 * u + kh * 4]);
-#define CORAL_MFMA_STEP(X)                                                                  \
-        acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.X, c0.X, acc[0][0], 0, 0, 0); \
-        acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0.X, c1.X, acc[0][1], 0, 0, 0); \
-        acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.X, c0.X, acc[1][0], 0, 0, 0); \
-        acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1.X, c1.X, acc[1][1], 0, 0, 0);
-            CORAL_MFMA_STEP(x)
-            CORAL_MFMA_STEP(y)
-            CORAL_MFMA_STEP(z)
-            CORAL_MFMA_STEP(w)
-#undef CORAL_MFMA_STEP
-        }
+        for (int j = 0; j < 2; ++j) bh[j] = *reinterpret_cast<const v8h*>(B + j * 32 * BK);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ah[i] = *reinterpret_cast<const v8h*>(A + i * 32 * BK);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) bl[j] = *reinterpret_cast<const v8h*>(B + NT * BK + j * 32 * BK);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) al[i] = *reinterpret_cast<const v8h*>(A + MT * BK + i * 32 * BK);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
     };
-    const int stages = full + (tail ? 1 : 0);
-    if (full > 0)
-        fetch(0);
-    else
-        fetch_tail();
+    fetch(0);
     park(0);
     __syncthreads();
     int cur = 0;
     for (int st = 0; st < stages; ++st) {
         const bool more = st + 1 < stages;
-        if (st + 1 < full)
-            fetch(st + 1);
-        else if (more)
-            fetch_tail();
+        if (more) fetch(st + 1);
         multiply(cur);
         if (more) park(cur ^ 1);
         __syncthreads();
         cur ^= 1;
     }
     // a 32 x 32 block's 16 registers: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32.
-    // The norms of the tile's rows and columns (+inf for a tombstoned column) come through LDS, fetched once per
-    // workgroup instead of by 64 dependent global loads per lane.
-    float* srow = &sa[0][0][0];  // the operand buffers are free after the last barrier of the loop
-    float* scol = &sb[0][0][0];
-    float* stau = srow + MT;
-    // (FUSED) the tile's entries that pass: ord(value) << 32 | place, where place = accumulator register << 8 |
-    // thread names the entry's row and column; they lie behind the norms
-    unsigned long long* shit = reinterpret_cast<unsigned long long*>(scol + NT);
-    constexpr int kHitCap = (2 * NT * RS - NT) / 2;
-    unsigned int& s_nhit = *reinterpret_cast<unsigned int*>(stau + MT);
+    // What the tile's rows and columns contribute comes through LDS, fetched once per workgroup instead of by
+    // dependent global loads per lane: norm and inverse scale of every row and column (times -2 or -1), the bounds.
+    float* srow = reinterpret_cast<float*>(&sa[0][0]);  // the operand buffers are free after the last barrier of the loop
+    float* srsc = srow + MT;
+    float* stau = srsc + MT;
+    float* scol = stau + MT;
+    float* scsc = scol + NT;
+    unsigned int& s_nhit = *reinterpret_cast<unsigned int*>(scsc + NT);
+    // (FUSED) the tile's entries that pass: ord(value) << 32 | row << 8 | column
+    unsigned long long* shit = reinterpret_cast<unsigned long long*>(&sb[0][0]);
+    constexpr int kHitCap = 2 * kStageB * 2 / 8;
     const float inf = __int_as_float(0x7f800000), nan = __int_as_float(0x7fc00000);
-    if (tid < MT) {
+    {
         const int r = q0 + tid;
-        srow[tid] = (L2 && r < nq) ? qn[r] : 0.0f;
+        const float n2 = r < nq ? qn[r] : 0.0f;
+        srow[tid] = L2 ? n2 : 0.0f;
+        srsc[tid] = mf_pow2(-mf_scale_exp(n2));
         if constexpr (FUSED) stau[tid] = r < nq ? tau[r] : -inf;
-    } else if (tid < MT + NT) {
+    }
+    if (tid < NT) {
         // what a column adds to its entries: |b|^2 (L2) or 0, +inf for a tombstoned id; (FUSED) NaN beyond the end of
         // the base, which no comparison passes
-        const int64_t c = b0 + (tid - MT);
-        float v = FUSED ? nan : 0.0f;
+        const int64_t c = b0 + tid;
+        float v = FUSED ? nan : 0.0f, n2 = 0.0f;
         if (c < nb) {
-            v = L2 ? bn[c] : 0.0f;
+            n2 = bn[c];
+            v = L2 ? n2 : 0.0f;
             if (deleted) {
                 const int64_t id = base_id0 + c;
                 if ((deleted[id >> 5] >> (id & 31)) & 1u) v = inf;
             }
         }
-        scol[tid - MT] = v;
+        scol[tid] = v;
+        scsc[tid] = (L2 ? -2.0f : -1.0f) * mf_pow2(-mf_scale_exp(n2));
     }
     if (tid == 0) s_nhit = 0u;
     __syncthreads();
-    // register v of block (ti, tj) in thread t: row and column inside the tile
-    auto row_of = [&](int t, int ti, int v) { return ((t >> 6) >> 1) * 64 + ti * 32 + 8 * (v >> 2) + 4 * ((t & 63) >> 5) + (v & 3); };
-    auto col_of = [&](int t, int tj) { return ((t >> 6) & 1) * 64 + tj * 32 + (t & 31); };
-    auto emit = [&](int rl, int cl, float sv) {
+    auto emit = [&](int rl, int cl, uint32_t ov) {
         const int r = q0 + rl;
-        const unsigned pos = atomicAdd(&cnt[r], 1u);
-        if (pos < (unsigned)cap)
-            lists[(size_t)r * cap + pos] = ((unsigned long long)mf_ord32(sv) << 32) | (uint32_t)(base_id0 + b0 + cl);
+        const unsigned pos = atomicAdd(&cnt[(size_t)r * kCntStride], 1u);
+        if (pos < (unsigned)cap) lists[(size_t)r * cap + pos] = ((unsigned long long)ov << 32) | (uint32_t)(base_id0 + b0 + cl);
     };
 #pragma unroll
-    for (int ti = 0; ti < 2; ++ti) {
-        float4 rown[4];  // |q|^2 of the 16 rows this lane holds of a block: four runs of four
-        float4 taun[4];
+    for (int ti = 0; ti < 4; ++ti) {
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            rown[g] = *reinterpret_cast<const float4*>(srow + wr * 64 + ti * 32 + 8 * g + 4 * kh);
-            if constexpr (FUSED) taun[g] = *reinterpret_cast<const float4*>(stau + wr * 64 + ti * 32 + 8 * g + 4 * kh);
-        }
+        for (int g = 0; g < 4; ++g) {  // the 16 rows this lane holds of a block: four runs of four
+            const int rl0 = wr * 128 + ti * 32 + 8 * g + 4 * kh;
+            const float4 rn4 = *reinterpret_cast<const float4*>(srow + rl0);
+            const float4 rs4 = *reinterpret_cast<const float4*>(srsc + rl0);
+            float4 tq4 = make_float4(0, 0, 0, 0);
+            if constexpr (FUSED) tq4 = *reinterpret_cast<const float4*>(stau + rl0);
+            const float rn[4] = {rn4.x, rn4.y, rn4.z, rn4.w}, rs[4] = {rs4.x, rs4.y, rs4.z, rs4.w};
+            const float tq[4] = {tq4.x, tq4.y, tq4.z, tq4.w};
 #pragma unroll
-        for (int tj = 0; tj < 2; ++tj) {
-            const int cl = wc * 64 + tj * 32 + m;
-            const int64_t c = b0 + cl;
-            const float bnc = scol[cl];
+            for (int tj = 0; tj < 2; ++tj) {
+                const int cl = wc * 64 + tj * 32 + m;
+                const float bnc = scol[cl], csc = scsc[cl];
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float4 rn4 = rown[v >> 2];
-                const float rn = (v & 3) == 0 ? rn4.x : (v & 3) == 1 ? rn4.y : (v & 3) == 2 ? rn4.z : rn4.w;
-                const float dot = acc[ti][tj][v];
-                // (|q|^2 + |b|^2) - 2 q.b, or -q.b; a tombstoned column's +inf survives both forms
-                const float sv = L2 ? __fmaf_rn(-2.0f, dot, rn + bnc) : bnc - dot;
-                if constexpr (FUSED) {
-                    const float4 t4 = taun[v >> 2];
-                    const float tq = (v & 3) == 0 ? t4.x : (v & 3) == 1 ? t4.y : (v & 3) == 2 ? t4.z : t4.w;
-                    if (sv <= tq) {  // rows beyond nq have tau = -inf, columns beyond nb give NaN
-                        const unsigned pos = atomicAdd(&s_nhit, 1u);
-                        if (pos < (unsigned)kHitCap)
-                            shit[pos] = ((unsigned long long)mf_ord32(sv) << 32) | (unsigned)(((ti * 2 + tj) * 16 + v) << 8) | (unsigned)tid;
-                        else  // more hits than the tile's buffer holds: straight to the list
-                            emit(row_of(tid, ti, v), cl, sv);
+                for (int w = 0; w < 4; ++w) {
+                    // (|q|^2 + |b|^2) - 2 q.b, or -q.b; a tombstoned column's +inf survives both forms
+                    const float sv = __fmaf_rn(acc[ti][tj][4 * g + w], rs[w] * csc, L2 ? rn[w] + bnc : bnc);
+                    if constexpr (FUSED) {
+                        if (sv <= tq[w]) {  // rows beyond nq have tau = -inf, columns beyond nb give NaN
+                            const unsigned pos = atomicAdd(&s_nhit, 1u);
+                            if (pos < (unsigned)kHitCap)
+                                shit[pos] = ((unsigned long long)mf_ord32(sv) << 32) | (unsigned)((rl0 + w) << 8) | (unsigned)cl;
+                            else  // more hits than the tile's buffer holds: straight to the list
+                                emit(rl0 + w, cl, mf_ord32(sv));
+                        }
+                    } else {
+                        const int r = q0 + rl0 + w;
+                        if (r < nq && b0 + cl < nb) D[(size_t)r * ldD + bt * NT + cl] = sv;
                     }
-                } else {
-                    const int r = q0 + row_of(tid, ti, v);
-                    if (r < nq && c < nb) D[(size_t)r * ldD + bt * NT + cl] = sv;
                 }
             }
         }
@@ -270,8 +321,7 @@ __global__ __launch_bounds__(256, CORAL_MFMA_WAVES) void approx_tile_mfma_kernel
         const int nhit = (int)min(s_nhit, (unsigned)kHitCap);
         for (int i = tid; i < nhit; i += 256) {
             const unsigned long long h = shit[i];
-            const int t = (int)(h & 0xffu), reg = (int)((h >> 8) & 0x3fu);
-            emit(row_of(t, reg >> 5, reg & 15), col_of(t, (reg >> 4) & 1), mf_unord32((uint32_t)(h >> 32)));
+            emit((int)((h >> 8) & 0xffu), (int)(h & 0xffu), (uint32_t)(h >> 32));
         }
     }
 }
@@ -355,7 +405,7 @@ __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ q
         // k-th of them lies clear of the worst candidate's approximate distance
         if (cand_ids[(size_t)q * kc + kc - 1] >= 0) {
             const float worst = cand_d[(size_t)q * kc + kc - 1];
-            const float delta = 8.0f * (float)(dim + 2) * 5.9604645e-8f * (qn[q] + __uint_as_float(*bn_max_bits));
+            const float delta = 8.0f * (float)(dim + 4) * 5.9604645e-8f * (qn[q] + __uint_as_float(*bn_max_bits));
             const unsigned long long kth = rkeys[k - 1];
             const float sk = mf_unord32((uint32_t)(kth >> 32));
             if (kth == ~0ull || !(sk < worst - delta)) bad = 1;
@@ -385,37 +435,61 @@ hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint
     return hipGetLastError();
 }
 
-#ifndef CORAL_MFMA_HQ
-#define CORAL_MFMA_HQ 16
-#endif
-constexpr int64_t kQueryTilesPerBlock = CORAL_MFMA_HQ;  // query tiles an XCD keeps in its L2 while it walks the base
+size_t split_queries_bytes(int nq, int dim) {
+    return (size_t)((nq + MT - 1) / MT) * ((dim + BK - 1) / BK) * kStageA * sizeof(_Float16);
+}
 
-hipError_t launch_approx_tile(const float* queries, const float* base, int nq, int64_t nb, int dim, int metric,
-                              const float* qn, const float* bn, const uint32_t* deleted, int64_t base_id0, float* D,
-                              int64_t ldD, hipStream_t stream, int64_t sample_tiles, int64_t tile_stride) {
-    const int64_t nbt = sample_tiles > 0 ? sample_tiles : (nb + NT - 1) / NT, nqt = (nq + MT - 1) / MT;
-    const int64_t qblocks = (nqt + kQueryTilesPerBlock - 1) / kQueryTilesPerBlock, hq = (nqt + qblocks - 1) / qblocks;
-    const int64_t wgs = (nbt + 7) / 8 * 8 * qblocks * hq;
-    if (wgs <= 0 || wgs > 0x7fffffff || tile_stride < 1) return hipErrorInvalidValue;
-    dim3 grid((unsigned)wgs);
-    auto kernel = metric == 0 ? approx_tile_mfma_kernel<false, true> : approx_tile_mfma_kernel<false, false>;
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, queries, base, nq, nb, dim, qn, bn, deleted, base_id0, nbt,
-                       tile_stride, (int)hq, D, ldD, (const float*)nullptr, (unsigned long long*)nullptr, (int64_t)0,
-                       (unsigned int*)nullptr);
+hipError_t launch_split_queries(const float* queries, int nq, int dim, const float* qn, void* out, hipStream_t stream) {
+    const int stages = (dim + BK - 1) / BK, tiles = (nq + MT - 1) / MT;
+    if (nq <= 0 || tiles > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(split_queries_kernel, dim3((unsigned)stages, (unsigned)tiles), dim3(MT), 0, stream, queries, nq, dim,
+                       stages, qn, static_cast<_Float16*>(out));
     return hipGetLastError();
 }
 
-hipError_t launch_approx_filter(const float* queries, const float* base, int nq, int64_t nb, int dim, int metric,
+namespace {
+// the launch geometry: query tiles an XCD keeps in its L2 while it walks the base (about 2 MB of them), and the grid
+bool tile_grid(int nq, int dim, int64_t ntiles, int64_t* hq, unsigned* wgs) {
+    const int64_t nqt = (nq + MT - 1) / MT;
+    const int64_t per_tile = (int64_t)((dim + BK - 1) / BK) * kStageA * (int64_t)sizeof(_Float16);
+    const int64_t want = std::max<int64_t>(1, ((int64_t)2 << 20) / per_tile);
+    const int64_t qblocks = (nqt + want - 1) / want;
+    *hq = (nqt + qblocks - 1) / qblocks;
+    const int64_t total = (ntiles + 7) / 8 * 8 * qblocks * *hq;
+    *wgs = (unsigned)total;
+    return nq > 0 && ntiles > 0 && total <= 0x7fffffff;
+}
+}  // namespace
+
+hipError_t launch_approx_tile(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric,
+                              const float* qn, const float* bn, const uint32_t* deleted, int64_t base_id0, float* D,
+                              int64_t ldD, hipStream_t stream, int64_t sample_tiles, int tile_stride) {
+    const int64_t ntiles = sample_tiles > 0 ? sample_tiles : (nb + NT - 1) / NT;
+    int64_t hq = 0;
+    unsigned wgs = 0;
+    if (!tile_grid(nq, dim, ntiles, &hq, &wgs) || tile_stride < 1) return hipErrorInvalidValue;
+    auto kernel = metric == 0 ? approx_tile_mfma_kernel<false, true> : approx_tile_mfma_kernel<false, false>;
+    hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
+                       bn, deleted, base_id0, ntiles, tile_stride, (int)hq, D, ldD, (const float*)nullptr,
+                       (unsigned long long*)nullptr, (int64_t)0, (unsigned int*)nullptr);
+    return hipGetLastError();
+}
+
+hipError_t launch_approx_filter(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric,
                                 const float* qn, const float* bn, const uint32_t* deleted, const float* tau,
-                                unsigned long long* lists, int64_t cap, unsigned int* cnt, hipStream_t stream) {
-    const int64_t nbt = (nb + NT - 1) / NT, nqt = (nq + MT - 1) / MT;
-    const int64_t qblocks = (nqt + kQueryTilesPerBlock - 1) / kQueryTilesPerBlock, hq = (nqt + qblocks - 1) / qblocks;
-    const int64_t wgs = (nbt + 7) / 8 * 8 * qblocks * hq;
-    if (wgs <= 0 || wgs > 0x7fffffff || nb > 0x7fffffff) return hipErrorInvalidValue;
-    dim3 grid((unsigned)wgs);
+                                unsigned long long* lists, int64_t cap, unsigned int* cnt, int tile_step,
+                                hipStream_t stream) {
+    const int64_t all = (nb + NT - 1) / NT;
+    const int64_t step = tile_step < 0 ? -(int64_t)tile_step : tile_step;
+    if (tile_step == 0 || tile_step == -1 || nb > 0x7fffffff) return hipErrorInvalidValue;
+    const int64_t multiples = (all + step - 1) / step, ntiles = tile_step > 0 ? multiples : all - multiples;
+    if (ntiles == 0) return hipSuccess;  // no tile between the multiples
+    int64_t hq = 0;
+    unsigned wgs = 0;
+    if (!tile_grid(nq, dim, ntiles, &hq, &wgs)) return hipErrorInvalidValue;
     auto kernel = metric == 0 ? approx_tile_mfma_kernel<true, true> : approx_tile_mfma_kernel<true, false>;
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, queries, base, nq, nb, dim, qn, bn, deleted, (int64_t)0, nbt,
-                       (int64_t)1, (int)hq, (float*)nullptr, (int64_t)0, tau, lists, cap, cnt);
+    hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
+                       bn, deleted, (int64_t)0, ntiles, tile_step, (int)hq, (float*)nullptr, (int64_t)0, tau, lists, cap, cnt);
     return hipGetLastError();
 }
 

@@ -95,6 +95,41 @@ def test_bruteforce_exact_against_oracle(orc, n, dim, Q, k, metric, tomb):
     assert np.allclose(dists[live], td[live], rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("n,dim,Q,k,metric,law", [
+    (8192, 4, 1, 1, "l2", "plain"),            # one query in a tile of 256, a quarter of one stage of 16 dimensions
+    (8319, 12, 255, 10, "ip", "plain"),        # last base tile one short, last query tile one short
+    (8321, 16, 256, 10, "l2", "plain"),        # last base tile of one point; whole tile of queries, whole stage
+    (9000, 20, 257, 33, "ip", "plain"),        # a second query tile of one
+    (20483, 36, 1025, 10, "l2", "plain"),      # two passes over the base with a tightened bound
+    (20483, 24, 1024, 100, "ip", "plain"),
+    (20483, 24, 1024, 10, "l2", "row_scales"),  # rows from 1e-12 to 1e12 in one base
+    (20483, 24, 300, 10, "ip", "row_scales"),
+    (8500, 24, 130, 10, "l2", "tiny"),         # squared norms at the end of the range: scales are clamped
+    (8500, 24, 130, 10, "ip", "tiny"),
+    (8500, 24, 40, 10, "ip", "huge_row"),      # a squared norm that overflows: nothing can be vouched for
+])
+def test_screening_on_split_halves_at_the_edges_of_its_tiles(orc, n, dim, Q, k, metric, law):
+    """Sizes around the tiles (256 queries, 128 points, 16 dimensions) and magnitudes around the ends of the scaling;
+    the result is defined bit for bit, so there is nothing to tolerate."""
+    m = capi.IP if metric == "ip" else capi.L2
+    base = synth.gaussian_matrix(n + 3 * dim, n, dim)
+    q = synth.shifted_queries(Q, dim, 13, 14, 15)
+    rs = np.random.RandomState(n)
+    if law == "row_scales":
+        base *= (10.0 ** rs.uniform(-12, 12, (n, 1))).astype(np.float32)
+    elif law == "tiny":
+        base *= np.float32(1e-19)
+        q *= np.float32(1e-19)
+    elif law == "huge_row":
+        base[n // 2] *= np.float32(1e20)
+    idx = capi.Index(base, None, None, m)
+    ids, dists, _ = idx.bruteforce(q, k)
+    idx.close()
+    oi, od = orc.bruteforce(base, q, k, m, order=SEQ)
+    assert np.array_equal(ids, oi)
+    assert dists.tobytes() == od.tobytes()
+
+
 def test_randomised_knn_problems_equal_the_oracle(orc):
     """Seeded random sizes, k, metrics, tombstones and laws of the data (ties on a lattice, repeated vectors, large
     and small magnitudes, a common offset that makes the screening's error bound bite): the screened path and the
