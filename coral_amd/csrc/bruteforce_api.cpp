@@ -78,14 +78,17 @@ int knn_passes(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, i
     return CORAL_OK;
 }
 
+}  // namespace
+
+namespace coral {
 // |b|^2 of the base, once per index
 int ensure_base_norms(coral_index* idx, hipStream_t stream) {
     if (idx->d_bnorm) return CORAL_OK;
     if (!idx->d_bnorm_max) HIP_TRY(hipMalloc(&idx->d_bnorm_max, sizeof(uint32_t)));
     float* norms = nullptr;
     HIP_TRY(hipMalloc(&norms, (size_t)idx->n * sizeof(float)));
-    hipError_t e = coral::launch_fill_u32(idx->d_bnorm_max, 1, 0u, stream);
-    if (e == hipSuccess) e = coral::launch_row_norms(idx->d_vec, idx->n, idx->dim, norms, idx->d_bnorm_max, stream);
+    hipError_t e = launch_fill_u32(idx->d_bnorm_max, 1, 0u, stream);
+    if (e == hipSuccess) e = launch_row_norms(idx->d_vec, idx->n, idx->dim, norms, idx->d_bnorm_max, stream);
     if (e != hipSuccess) {
         (void)hipFree(norms);
         HIP_TRY(e);
@@ -94,6 +97,9 @@ int ensure_base_norms(coral_index* idx, hipStream_t stream) {
     return CORAL_OK;
 }
 
+}  // namespace coral
+
+namespace {
 constexpr int kScreenSlack = 32;  // candidates kept beyond k
 constexpr int64_t kListCap = 16384;  // keys a query's candidate list holds in the fused screening
 
@@ -236,7 +242,7 @@ int coral_bruteforce_knn_gpu(coral_index* idx, const float* d_queries, int32_t Q
                       hipGetErrorString(e));
             return false;
         };
-        if ((rc = ensure_base_norms(idx, stream)) == CORAL_OK &&
+        if ((rc = coral::ensure_base_norms(idx, stream)) == CORAL_OK &&
             ok(hipMalloc(&d_qn, (size_t)Q * sizeof(float)), "hipMalloc") &&
             ok(hipMalloc(&d_cid, (size_t)Q * kc * sizeof(int32_t)), "hipMalloc") &&
             ok(hipMalloc(&d_cd, (size_t)Q * kc * sizeof(float)), "hipMalloc") &&

@@ -9,31 +9,26 @@
 // than a bound on what the two ways of rounding can differ by; otherwise it is flagged and goes through the exact
 // search.
 //
-// The inner products.  A row x is scaled by a power of two that puts |x| into [2^13, 2^14) and every scaled component
-// is split into two halves, hi = half(x) and lo = half(x - hi); x - hi is exact, so hi + lo is x to 22 bits.  Then
-// q.b = hi.hi + hi.lo + lo.hi on v_mfma_f32_32x32x16_f16 (products exact, fp32 accumulation): three multiplications at
-// sixteen times the rate of the fp32 form.
+// The inner products: rows are split into two planes of halves (mfma_split.h, with the bound on what that and the
+// accumulation lose), and q.b = hi.hi + hi.lo + lo.hi on v_mfma_f32_32x32x16_f16: three multiplications at sixteen
+// times the rate of the fp32 form.
 //
-// Error bound, with u = 2^-24.  Splitting: each component is off by at most 2^-22 of itself, and lo.lo is left out:
-// 12 u |q| |b| over the sum (components below 2^-28 of their row's norm lose more, but of less: sqrt(dim) 2^-38 |q| |b|
-// in all).  Accumulation: 3 dim additions, within 2 u of the running sum each even if the hardware truncates:
-// 6 dim u |q| |b|.  The inner product enters twice: (6 dim + 12) u (|q|^2 + |b|^2).  The two norms are within dim u of
-// themselves, the final additions add 4 u (|q|^2 + |b|^2), the reference-order distance is within (dim + 2) u of the
-// true one.  Together the approximate and the reference-order value of a pair differ by less than
-// 8 (dim + 4) u (|q|^2 + |b|^2); the check takes the largest |b|^2 of the index.
+// Error bound, with u = 2^-24.  The inner product is within (6 dim + 12) u |q| |b| and enters twice:
+// (6 dim + 12) u (|q|^2 + |b|^2).  The two norms are within dim u of themselves, the final additions add
+// 4 u (|q|^2 + |b|^2), the reference-order distance is within (dim + 2) u of the true one.  Together the approximate
+// and the reference-order value of a pair differ by less than 8 (dim + 4) u (|q|^2 + |b|^2); the check takes the
+// largest |b|^2 of the index.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <algorithm>
 
 #include "bruteforce.h"
+#include "mfma_split.h"
 
 namespace coral {
 
 namespace {
-
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int MT = 256, NT = 128, BK = 16;  // tile of queries x base points per workgroup, dimensions per LDS stage
 constexpr int kStageA = 2 * MT * BK, kStageB = 2 * NT * BK;  // halves per stage: the hi plane, then the lo plane
@@ -45,25 +40,6 @@ __device__ __forceinline__ uint32_t mf_ord32(float s) {
 __device__ __forceinline__ float mf_unord32(uint32_t o) {
     const uint32_t u = (o & 0x80000000u) ? (o ^ 0x80000000u) : ~o;
     return __uint_as_float(u);
-}
-
-// e with |x| 2^e in [2^13, 2^14) for a row of squared norm n2; within [-40, 60], which rows of norm 0, of norms whose
-// square leaves the normal range, and of infinite norms meet (the last are never accepted: their error bound is
-// infinite), so that no product of two such powers overflows
-__device__ __forceinline__ int mf_scale_exp(float n2) {
-    const int E = (int)((__float_as_uint(n2) >> 23) & 0xffu) - 127;  // n2 in [2^E, 2^(E+1))
-    return max(-40, min(60, 13 - (E >> 1)));
-}
-__device__ __forceinline__ float mf_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
-
-// eight scaled components as two planes of halves
-__device__ __forceinline__ void mf_split8(const float4 a, const float4 b, float s, v8h& hi, v8h& lo) {
-    const float x[8] = {a.x * s, a.y * s, a.z * s, a.w * s, b.x * s, b.y * s, b.z * s, b.w * s};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        hi[j] = (_Float16)x[j];
-        lo[j] = (_Float16)(x[j] - (float)hi[j]);
-    }
 }
 
 // |x|^2 per row, and the largest of them (as the bit pattern of a non-negative float)

@@ -25,12 +25,13 @@
 
 #include "coral_search.h"
 #include "graph_build.h"
+#include "mfma_split.h"
 
 namespace coral {
 
 namespace {
 
-constexpr int kThreads = 256;
+constexpr int kThreads = 512;  // eight pivots of a cluster side by side: 1.10 ms -> 0.88 ms per 1024 clusters against four
 constexpr int kWaves = kThreads / 64;
 constexpr int kChunk = 32;                         // dimensions staged per step of the member-pair distances
 constexpr int kMaxCand = kBuildMaxKb + kBuildMaxR;  // candidates of one pivot
@@ -53,12 +54,13 @@ __device__ __forceinline__ void wave_sync() {
 // one lane walks both rows: the accumulation order of include/utils.cuh:254-275 (L2) and :307-323 (IP).  The rows
 // are fetched eight float4 at a time ahead of the additions, so a lane waits for memory once per 32 dimensions
 // instead of once per 4; the chain of additions itself stays strictly in dimension order.
+template <int kAhead = 8>
 __device__ __forceinline__ float seq_dist(const float* __restrict__ a, const float* __restrict__ b, int dim, int metric) {
-    constexpr int kAhead = 8;
     const float4* a4 = reinterpret_cast<const float4*>(a);
     const float4* b4 = reinterpret_cast<const float4*>(b);
     const int n4 = dim / 4;
     float acc = 0.0f;
+#pragma unroll 1
     for (int i0 = 0; i0 < n4; i0 += kAhead) {
         float4 x[kAhead], y[kAhead];
 #pragma unroll
@@ -104,6 +106,8 @@ struct WaveCands {
     int32_t id[kMaxCand];
     int16_t col[kMaxCand];
     uint8_t st[kMaxCand];
+    int32_t ret[kBuildMaxR];  // ids of the retained ones, in order
+    float4 rows[2][2][8];     // of the retained ones and of a block's: squared norms, inverse scales
 };
 
 // bytes of the region that holds the staging rows first and the candidate lists afterwards
@@ -118,7 +122,7 @@ __device__ __forceinline__ unsigned long long cand_key(float dist, int col, int 
 }
 
 // rank-by-counting sort of the C assembled entries; returns the number of candidates (invalid ones drop out)
-__device__ int sort_cands(WaveCands& S, int C, int lane) {
+__device__ __forceinline__ int sort_cands(WaveCands& S, int C, int lane) {
     wave_sync();
     int m = 0;
     for (int e0 = 0; e0 < C; e0 += 64) {
@@ -141,10 +145,10 @@ __device__ int sort_cands(WaveCands& S, int C, int lane) {
 
 // candidate_ignore_kernel (src/upd_gpu.cu:203-247, src/enhance.cu:334-380): in order of distance a candidate not yet
 // ruled out is retained and rules out every later one that is closer to it than to the pivot; duplicates of an id
-// are marked.  Stops once R are retained.  G (optional) holds the member-pair distances by pair of columns.
-template <bool HAVE_G>
-__device__ void prune_cands(WaveCands& S, int m, int lane, const float* __restrict__ vec, int dim, int metric, int R,
-                            const float* G, int kb) {
+// are marked.  Stops once R are retained.  Two forms of the rule, with the same outcome.
+//
+// Here every candidate is a member of the cluster: G holds the distances by pair of columns.
+__device__ __forceinline__ void prune_members(WaveCands& S, int m, int lane, int metric, int R, const float* G, int kb) {
     int nbr_num = 0;
     for (int i = 0; i < m && nbr_num < R; ++i) {
         const uint8_t st = S.st[i];
@@ -152,19 +156,11 @@ __device__ void prune_cands(WaveCands& S, int m, int lane, const float* __restri
         if (st == ST_INITIAL) {
             ++nbr_num;
             const int coli = S.col[i];
-            const float* vi = vec + (size_t)idi * dim;
             for (int j = i + 1 + lane; j < m; j += 64) {
-                const int32_t idj = S.id[j];
-                if (idj == idi) {
+                if (S.id[j] == idi) {
                     S.st[j] = ST_REPEATED;
                 } else if (S.st[j] == ST_INITIAL) {
-                    const int colj = S.col[j];
-                    float d;
-                    if (HAVE_G && coli < kb && colj < kb)
-                        d = G[pair_index(coli, colj, kb)];
-                    else
-                        d = seq_dist(vi, vec + (size_t)idj * dim, dim, metric);
-                    if (closer(S.dist[j], d, metric)) S.st[j] = ST_DISCARDED;
+                    if (closer(S.dist[j], G[pair_index(coli, S.col[j], kb)], metric)) S.st[j] = ST_DISCARDED;
                 }
             }
             if (lane == 0) S.st[i] = ST_RETAINED;
@@ -176,9 +172,162 @@ __device__ void prune_cands(WaveCands& S, int m, int lane, const float* __restri
     }
 }
 
+// By how much is the candidate at (exact) distance dj from the pivot closer to another candidate than to the pivot?
+// dot: the inner product of the two from split halves, n2: the sum of their squared norms.  The answer is certain where
+// it lies beyond +- slack * n2 + 1e-36: the reference-order distance is within 8 (dim + 8) u n2 of n2 - 2 dot (L2:
+// twice the bound of mfma_split.h, the norms', the reference order's and this difference's own rounding), the
+// reference-order product within half that of dot; 1e-36 covers what underflow adds.  Infinities and NaN are certain
+// of nothing.
+template <bool L2>
+__device__ __forceinline__ float margin(float dj, float dot, float n2) { return L2 ? fmaf(2.0f, dot, dj - n2) : dot - dj; }
+
+// Here the candidates are any nodes.  The rule only compares distances, and the comparison is nearly always clear of
+// rounding: the candidates are taken in blocks of 32, the distances of a block to everything retained before it and
+// inside the block come from two 32 x 32 products on the matrix cores (split halves, rows gathered straight into
+// operand registers: lane (kh, m) holds dimensions kh * 8 .. + 7 of row m of every stage of 16), and only a
+// comparison within the error bound is decided by the reference-order chain.  A candidate is ruled out by what was
+// retained before it, so the state of a block is a scan over 32 masks.
+//
+// Bound by the gather (two rows of dim * 4 bytes per candidate, from L2 and the memory-side cache).  One lane walking
+// each pair in the reference's order instead, a load of 16 bytes per line and a chain of waits per retained candidate,
+// took 453 us (200 floats, L2) and 3670 us (512 floats, inner product) per 4096 lists of 100 and 132; this takes 120
+// and 284 us.  At 128 registers (four wavefronts per SIMD; 13 spilled) against 168 or 256: 120 / 150 / 150 us.
+template <bool L2>
+__device__ __forceinline__ void prune_any(WaveCands& S, int m, int lane, const float* __restrict__ vec, const float* __restrict__ norms,
+                          int dim, int R) {
+    constexpr int metric = L2 ? CORAL_L2 : CORAL_IP;
+    const int l = lane & 31, kh = lane >> 5;
+    const float slack = (L2 ? 8.0f : 4.0f) * (float)(dim + 8) * 5.9604645e-8f;
+    int nbr_num = 0;
+    for (int j0 = 0; j0 < m && nbr_num < R; j0 += 32) {
+        const int cnt = min(32, m - j0), j = j0 + l;
+        const bool valid = l < cnt;
+        const int32_t idj = S.id[valid ? j : j0];
+        const int32_t idr = nbr_num > 0 ? S.ret[min(l, nbr_num - 1)] : idj;
+        const float nj = norms[idj], nr = norms[idr], dj = S.dist[valid ? j : j0];
+        const int ej = mf_scale_exp(nj), er = mf_scale_exp(nr);
+        const float sj = mf_pow2(ej), sr = mf_pow2(er), usj = mf_pow2(-ej), usr = mf_pow2(-er);
+        if (kh == 0) {
+            reinterpret_cast<float*>(S.rows[0][0])[l] = nr, reinterpret_cast<float*>(S.rows[0][1])[l] = usr;
+            reinterpret_cast<float*>(S.rows[1][0])[l] = nj, reinterpret_cast<float*>(S.rows[1][1])[l] = usj;
+        }
+        wave_sync();
+        v16f pr, pb;  // retained x block, block x block
+#pragma unroll
+        for (int v = 0; v < 16; ++v) pr[v] = 0.0f, pb[v] = 0.0f;
+        const float* pj = vec + (size_t)idj * dim + kh * 8;
+        const float* pq = vec + (size_t)idr * dim + kh * 8;
+        const int k0 = kh * 8;
+        constexpr int kAhead = 2;  // stages of 16 dimensions in flight: a cache line of every row
+#pragma unroll 1
+        for (int d0 = 0; d0 < dim; d0 += 16 * kAhead) {
+            float4 x[kAhead][2], y[kAhead][2];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    x[u][h] = make_float4(0, 0, 0, 0), y[u][h] = make_float4(0, 0, 0, 0);
+                    const int d = d0 + 16 * u + 4 * h;
+                    if (d + k0 < dim) {  // dim is a multiple of 4
+                        x[u][h] = *reinterpret_cast<const float4*>(pj + d);
+                        if (nbr_num > 0) y[u][h] = *reinterpret_cast<const float4*>(pq + d);
+                    }
+                }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                if (d0 + 16 * u < dim) {
+                    v8h bh, bl, rh, rl;
+                    mf_split8(x[u][0], x[u][1], sj, bh, bl);
+                    pb = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, bh, pb, 0, 0, 0);
+                    pb = __builtin_amdgcn_mfma_f32_32x32x16_f16(bh, bl, pb, 0, 0, 0);
+                    pb = __builtin_amdgcn_mfma_f32_32x32x16_f16(bl, bh, pb, 0, 0, 0);
+                    if (nbr_num > 0) {
+                        mf_split8(y[u][0], y[u][1], sr, rh, rl);
+                        pr = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, bh, pr, 0, 0, 0);
+                        pr = __builtin_amdgcn_mfma_f32_32x32x16_f16(rh, bl, pr, 0, 0, 0);
+                        pr = __builtin_amdgcn_mfma_f32_32x32x16_f16(rl, bh, pr, 0, 0, 0);
+                    }
+                }
+            }
+        }
+        // an id that stands anywhere before is a duplicate: its first place was retained or ruled out
+        bool rep = false;
+        for (int f = kh; f < j0 + cnt; f += 2) rep |= f < j && S.id[f] == idj;
+        rep |= __shfl_xor((int)rep, 32, 64) != 0;
+        // register v of lane (kh, l): row 8 (v / 4) + 4 kh + v % 4, column l.  First what the products decide, then --
+        // with the products out of the registers -- the chains for what they left open.
+        uint32_t yes_r = 0u;                // retained ones that rule this lane's column out
+        uint32_t open_r = 0u, open_b = 0u;  // retained ones, candidates of the block that this lane could not decide on
+        uint32_t mask = 0u;                 // candidates of the block that rule this lane's column out, if retained
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            auto at = [](const float4& q, int w) { return w == 0 ? q.x : w == 1 ? q.y : w == 2 ? q.z : q.w; };
+            if (nbr_num > 0) {
+                const float4 n4 = S.rows[0][0][2 * g + kh], s4 = S.rows[0][1][2 * g + kh];
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const int r = 8 * g + 4 * kh + w;
+                    const float n2 = nj + at(n4, w), e = fmaf(slack, n2, 1e-36f);
+                    const float t = margin<L2>(dj, pr[4 * g + w] * (usj * at(s4, w)), n2);
+                    yes_r |= t > e ? 1u << r : 0u;
+                    open_r |= t < -e ? 0u : 1u << r;
+                }
+            }
+            const float4 n4 = S.rows[1][0][2 * g + kh], s4 = S.rows[1][1][2 * g + kh];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int r = 8 * g + 4 * kh + w;
+                const float n2 = nj + at(n4, w), e = fmaf(slack, n2, 1e-36f);
+                const float t = margin<L2>(dj, pb[4 * g + w] * (usj * at(s4, w)), n2);
+                mask |= t > e ? 1u << r : 0u;
+                open_b |= t < -e ? 0u : 1u << r;
+            }
+        }
+        const uint32_t have = nbr_num >= 32 ? 0xffffffffu : (1u << nbr_num) - 1u, ahead = (1u << l) - 1u;
+        yes_r &= have, mask &= ahead;
+        open_r &= have & ~yes_r, open_b &= ahead & ~mask;
+        bool disc = yes_r != 0u;
+        disc |= __shfl_xor((int)disc, 32, 64) != 0;
+        if (!valid || rep || disc) open_r = 0u;
+#pragma unroll 1
+        while (open_r) {
+            const int r = __ffs((int)open_r) - 1;
+            open_r &= open_r - 1u;
+            if (closer(dj, seq_dist<4>(vec + (size_t)S.ret[r] * dim, vec + (size_t)idj * dim, dim, metric), metric)) {
+                disc = true;
+                open_r = 0u;
+            }
+        }
+        disc |= __shfl_xor((int)disc, 32, 64) != 0;
+        const uint32_t live = (uint32_t)__ballot(valid && !rep && !disc);  // the same in both halves
+        open_b = (live >> l) & 1u ? open_b & live : 0u;
+#pragma unroll 1
+        while (open_b) {
+            const int r = __ffs((int)open_b) - 1;
+            open_b &= open_b - 1u;
+            if (closer(dj, seq_dist<4>(vec + (size_t)S.id[j0 + r] * dim, vec + (size_t)idj * dim, dim, metric), metric))
+                mask |= 1u << r;
+        }
+        mask |= (uint32_t)__shfl_xor((int)mask, 32, 64);
+        uint32_t kept = 0u;
+        const int before = nbr_num;
+        for (int i = 0; i < cnt && nbr_num < R; ++i) {
+            const uint32_t mi = (uint32_t)__builtin_amdgcn_readlane((int)mask, i);
+            if (((live >> i) & 1u) && !(mi & kept)) kept |= 1u << i, ++nbr_num;
+        }
+        // behind the R-th retained one the states no longer matter: the row is full
+        if (kh == 0 && valid) {
+            const bool keep = (kept >> l) & 1u;
+            S.st[j] = keep ? ST_RETAINED : rep ? ST_REPEATED : (disc || (mask & kept)) ? ST_DISCARDED : ST_INITIAL;
+            if (keep) S.ret[before + __popc(kept & ((1u << l) - 1u))] = idj;
+        }
+        wave_sync();
+    }
+}
+
 // update_new_nbrs_kernel (src/upd_gpu.cu:102-156) / update_iso_nbrs_kernel (src/enhance.cu:528-568): the retained
 // candidates and, with fill, the nearest discarded ones up to R, in order of distance.  Returns the row length.
-__device__ int emit_row(const WaveCands& S, int m, int lane, int R, bool fill, int32_t* __restrict__ out_ids,
+__device__ __forceinline__ int emit_row(const WaveCands& S, int m, int lane, int R, bool fill, int32_t* __restrict__ out_ids,
                         float* __restrict__ out_dists) {
     const unsigned long long below = (1ull << lane) - 1ull;
     int retained = 0;
@@ -214,8 +363,9 @@ __global__ void claim_kernel(const int32_t* __restrict__ ids, int64_t count, int
 
 // one workgroup per cluster; dynamic LDS: G[kb(kb-1)/2] | stage[kb][kChunk+4] or WaveCands[kWaves] | ids[kb] | deg[kb]
 // (the staging rows of the distance phase and the candidate lists of the pivot phase are never live together)
-__global__ void __launch_bounds__(kThreads)
-nap_cluster_kernel(const float* __restrict__ vec, int dim, int metric, int R, const int32_t* __restrict__ nbrs,
+template <bool L2>
+__global__ void __launch_bounds__(kThreads, 4)
+nap_cluster_kernel(const float* __restrict__ vec, const float* __restrict__ norms, int dim, int metric, int R, const int32_t* __restrict__ nbrs,
                    const float* __restrict__ dists, const int32_t* __restrict__ deg, const int32_t* __restrict__ owner,
                    const int32_t* __restrict__ knn, int batch, int kb, int need_discard, int32_t* __restrict__ new_ids,
                    float* __restrict__ new_dists, int32_t* __restrict__ new_deg) {
@@ -325,7 +475,10 @@ nap_cluster_kernel(const float* __restrict__ vec, int dim, int metric, int R, co
                 S.udist[q] = d;
             }
             const int m = sort_cands(S, C, lane);
-            prune_cands<true>(S, m, lane, vec, dim, metric, R, G, kb);
+            if (rdeg == 0)  // all candidates are members: their distances are in LDS
+                prune_members(S, m, lane, metric, R, G, kb);
+            else
+                prune_any<L2>(S, m, lane, vec, norms, dim, R);
             const int nd = emit_row(S, m, lane, R, need_discard != 0, new_ids + (size_t)p * R, new_dists + (size_t)p * R);
             if (lane == 0) new_deg[p] = nd;
             wave_sync();
@@ -463,8 +616,9 @@ __global__ void enh_reverse_kernel(const float* __restrict__ vec, int dim, int m
 }
 
 // the isolated node's own row from its found list (src/enhance.cu:334-380, 519-575); one wavefront per node
-__global__ void __launch_bounds__(kThreads)
-enh_rows_kernel(const float* __restrict__ vec, int dim, int metric, int R, int32_t* __restrict__ nbrs,
+template <bool L2>
+__global__ void __launch_bounds__(kThreads, 4)
+enh_rows_kernel(const float* __restrict__ vec, const float* __restrict__ norms, int dim, int metric, int R, int32_t* __restrict__ nbrs,
                 float* __restrict__ dists, int32_t* __restrict__ deg, const int32_t* __restrict__ iso_ids,
                 const int32_t* __restrict__ knn_ids, const float* __restrict__ knn_dists,
                 const int32_t* __restrict__ len, int batch, int kn) {
@@ -482,7 +636,7 @@ enh_rows_kernel(const float* __restrict__ vec, int dim, int metric, int R, int32
             S.udist[q] = d;
         }
         const int m = sort_cands(S, kn, lane);
-        prune_cands<false>(S, m, lane, vec, dim, metric, R, nullptr, 0);
+        prune_any<L2>(S, m, lane, vec, norms, dim, R);
         int32_t* row = nbrs + (size_t)iso * R;
         float* rowd = dists + (size_t)iso * R;
         const int nd = emit_row(S, m, lane, R, true, row, rowd);
@@ -561,40 +715,42 @@ size_t nap_lds_bytes(int kb) {
     return g + nap_union_bytes(kb) + (size_t)kb * 8;
 }
 
-hipError_t launch_nap_batch(const float* vec, int dim, int metric, int R, int32_t* nbrs, float* dists, int32_t* deg,
+hipError_t launch_nap_batch(const float* vec, const float* norms, int dim, int metric, int R, int32_t* nbrs, float* dists, int32_t* deg,
                             int32_t* owner, const int32_t* knn, int batch, int kb, int need_discard, int32_t* new_ids,
                             float* new_dists, int32_t* new_deg, hipStream_t st) {
     const int64_t P = (int64_t)batch * kb;
     const size_t lds = nap_lds_bytes(kb);
     static bool attr_set = false;
     if (!attr_set) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(nap_cluster_kernel),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
-        if (e != hipSuccess) return e;
+        for (const void* k : {reinterpret_cast<const void*>(nap_cluster_kernel<true>),
+                              reinterpret_cast<const void*>(nap_cluster_kernel<false>)}) {
+            hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 256);
+            if (e != hipSuccess) return e;
+        }
         attr_set = true;
     }
+    auto cluster = metric == CORAL_L2 ? nap_cluster_kernel<true> : nap_cluster_kernel<false>;
     int blocks = (int)((P + 255) / 256);
     hipLaunchKernelGGL(claim_kernel, dim3(blocks > 2048 ? 2048 : blocks), dim3(256), 0, st, knn, P, owner);
-    hipLaunchKernelGGL(nap_cluster_kernel, dim3(batch), dim3(kThreads), lds, st, vec, dim, metric, R, nbrs, dists, deg,
+    hipLaunchKernelGGL(cluster, dim3(batch), dim3(kThreads), lds, st, vec, norms, dim, metric, R, nbrs, dists, deg,
                        owner, knn, batch, kb, need_discard, new_ids, new_dists, new_deg);
     hipLaunchKernelGGL(nap_commit_kernel, dim3((unsigned)((P * 32 + 255) / 256)), dim3(256), 0, st, knn, P, R, owner,
                        new_ids, new_dists, new_deg, nbrs, dists, deg);
     return hipGetLastError();
 }
 
-hipError_t launch_enhance_batch(const float* vec, int dim, int metric, int R, int32_t* nbrs, float* dists, int32_t* deg,
+hipError_t launch_enhance_batch(const float* vec, const float* norms, int dim, int metric, int R, int32_t* nbrs, float* dists, int32_t* deg,
                                 int32_t* owner, const int32_t* iso_ids, const int32_t* knn_ids, const float* knn_dists,
                                 int batch, int kn, int32_t* len, const int32_t* rev_len, unsigned long long* stats,
                                 hipStream_t st) {
-    const int waves_per_block = 4;
-    int blocks = (batch + waves_per_block - 1) / waves_per_block;
-    hipLaunchKernelGGL(enh_claim_kernel, dim3(blocks), dim3(256), 0, st, knn_ids, batch, kn, len, rev_len, owner);
+    hipLaunchKernelGGL(enh_claim_kernel, dim3((batch + 3) / 4), dim3(256), 0, st, knn_ids, batch, kn, len, rev_len, owner);
     const int64_t pairs = (int64_t)batch * kn;
     int64_t rb = (pairs * 32 + 255) / 256;
     rb = rb > 8192 ? 8192 : rb;
     hipLaunchKernelGGL(enh_reverse_kernel, dim3((unsigned)rb), dim3(256), 0, st, vec, dim, metric, R, nbrs, dists, deg,
                        owner, iso_ids, knn_ids, knn_dists, len, rev_len, batch, kn, stats);
-    hipLaunchKernelGGL(enh_rows_kernel, dim3(blocks), dim3(kThreads), 0, st, vec, dim, metric, R, nbrs, dists, deg,
+    auto rows = metric == CORAL_L2 ? enh_rows_kernel<true> : enh_rows_kernel<false>;
+    hipLaunchKernelGGL(rows, dim3((batch + kWaves - 1) / kWaves), dim3(kThreads), 0, st, vec, norms, dim, metric, R, nbrs, dists, deg,
                        iso_ids, knn_ids, knn_dists, len, batch, kn);
     return hipGetLastError();
 }

@@ -178,6 +178,7 @@ int coral_build_begin(coral_index* idx, int32_t R) {
     HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_deg, n, 0u, idx->stream));
     HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_owner, n, (uint32_t)INT_MAX, idx->stream));
     HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_build_stats, 8, 0u, idx->stream));
+    if (int rc = coral::ensure_base_norms(idx, idx->stream)) return rc;
     HIP_TRY(hipStreamSynchronize(idx->stream));
     idx->building = true;
     return CORAL_OK;
@@ -234,7 +235,7 @@ int coral_build_nap_batch(coral_index* idx, const int32_t* d_knn_ids, int32_t ba
     if (int rc = check_ids(idx, d_knn_ids, (int64_t)batch * k_b, false, "cluster ids")) return rc;
     idx->rows_unique = -1;
     HIP_TRY(coral::launch_count_hits(d_knn_ids, (int64_t)batch * k_b, idx->d_hits, idx->stream));
-    HIP_TRY(coral::launch_nap_batch(idx->d_vec, idx->dim, idx->metric, idx->R, idx->d_nbrs, idx->d_nbr_dists, idx->d_deg,
+    HIP_TRY(coral::launch_nap_batch(idx->d_vec, idx->d_bnorm, idx->dim, idx->metric, idx->R, idx->d_nbrs, idx->d_nbr_dists, idx->d_deg,
                                     idx->d_owner, d_knn_ids, batch, k_b, need_discard, idx->d_new_ids, idx->d_new_dists,
                                     idx->d_new_deg, idx->stream));
     HIP_TRY(hipStreamSynchronize(idx->stream));
@@ -254,7 +255,7 @@ static int enhance_lists(coral_index* idx, const int32_t* d_node_ids, const int3
     }
     idx->rows_unique = -1;
     HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_build_stats, 4, 0u, idx->stream));
-    HIP_TRY(coral::launch_enhance_batch(idx->d_vec, idx->dim, idx->metric, idx->R, idx->d_nbrs, idx->d_nbr_dists,
+    HIP_TRY(coral::launch_enhance_batch(idx->d_vec, idx->d_bnorm, idx->dim, idx->metric, idx->R, idx->d_nbrs, idx->d_nbr_dists,
                                         idx->d_deg, idx->d_owner, d_node_ids, d_ids, d_dists, batch, kn, idx->d_len,
                                         d_rev_len, idx->d_build_stats, idx->stream));
     unsigned long long st[2] = {0, 0};

@@ -123,5 +123,6 @@ struct coral_index {
 
 namespace coral {
 void free_build_state(coral_index* idx);
+int ensure_base_norms(coral_index* idx, hipStream_t stream);  // d_bnorm, d_bnorm_max (bruteforce_api.cpp)
 }
 

@@ -93,6 +93,52 @@ def test_enhance_batches_equal_the_oracle(orc, metric, R, kn, seed):
     idx.close()
 
 
+@pytest.mark.parametrize("dim,R,kn,metric,law", [
+    (4, 32, 31, capi.L2, "lattice"),     # ties everywhere: comparisons that only the reference order decides
+    (20, 32, 32, capi.IP, "lattice"),
+    (36, 31, 33, capi.L2, "offset"),     # norms a million times the distances: no comparison is clear of the bound
+    (132, 32, 64, capi.L2, "plain"),     # a block boundary of the candidate list; dimensions that end inside a stage
+    (516, 32, 65, capi.IP, "plain"),
+    (24, 8, 96, capi.L2, "scales"),      # rows from 1e-15 to 1e15 in one base
+    (24, 32, 97, capi.IP, "scales"),
+    (12, 16, 40, capi.L2, "tiny"),       # squared norms below the normal range
+])
+def test_pruning_on_matrix_core_products_equals_the_oracle(orc, dim, R, kn, metric, law):
+    """Rows of nodes with neighbours outside their cluster, and of found lists, are pruned on products of split
+    halves; the outcome is defined bit for bit, whatever the data leaves open."""
+    rng = np.random.RandomState(dim + kn)
+    n, linked_n, kb = 1500, 1200, 30
+    base = synth.gaussian_matrix(400 + dim, n, dim)
+    if law == "lattice":
+        base = np.round(base)
+    elif law == "offset":
+        base = (base + 1000.0).astype(np.float32)
+    elif law == "scales":
+        base *= (10.0 ** rng.uniform(-15, 15, (n, 1))).astype(np.float32)
+    elif law == "tiny":
+        base *= np.float32(3e-21)
+    idx = capi.Index(base, None, None, metric=metric)
+    idx.build_begin(R)
+    st = orc.GraphState(n, R)
+    for it in range(4):
+        pool = rng.choice(linked_n, linked_n if it < 2 else 90, replace=False)
+        knn = np.stack([rng.choice(pool, kb, replace=False) for _ in range(40)]).astype(np.int32)
+        t_knn = dev(knn)
+        idx.build_nap_batch(t_knn.data_ptr(), 40, kb, 1)
+        orc.nap_batch(base, st, knn, metric=metric, need_discard=1)
+        assert_same_state(idx, st)
+    linked = np.where(st.deg > 0)[0].astype(np.int32)
+    iso = np.arange(linked_n, linked_n + 70, dtype=np.int32)
+    ids, dd = orc.bruteforce(base[linked], base[iso], kn, metric, order=SEQ)
+    ids = linked[ids]
+    t_iso, t_ids, t_dd = dev(iso), dev(ids), dev(dd)
+    ins, rej = idx.build_enhance_batch(t_iso.data_ptr(), t_ids.data_ptr(), t_dd.data_ptr(), iso.size, kn)
+    stats = orc.enhance_batch(base, st, iso, ids, dd, metric=metric)
+    assert (ins, rej) == (stats[0], stats[1])
+    assert_same_state(idx, st)
+    idx.close()
+
+
 def test_randomised_shapes_of_both_steps_equal_the_oracle(orc):
     """Seeded random sizes, widths, cluster sizes, metrics and fill modes, small enough for the oracle; each case
     runs a few batch updates and one enhancement batch."""
