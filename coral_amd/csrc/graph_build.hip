@@ -567,11 +567,12 @@ __global__ void enh_reverse_kernel(const float* __restrict__ vec, int dim, int m
         if (have) {
             nb = nbrs[(size_t)v * R + l];
             rd = dists[(size_t)v * R + l];
-            dij = seq_dist(vec + (size_t)iso * dim, vec + (size_t)nb * dim, dim, metric);
         }
         // the newcomer goes in front of the first entry that is not strictly closer than it
         const uint32_t ahead = (uint32_t)(__ballot(have && closer(vd, rd, metric)) >> shift);
         const int pos = ahead == 0xffffffffu ? 32 : __ffs((int)~ahead) - 1;
+        // distances to the row's entries decide only where a full row has to give one up
+        if (have && d == R && pos < d) dij = seq_dist(vec + (size_t)iso * dim, vec + (size_t)nb * dim, dim, metric);
         // an entry in front that is closer to the newcomer than the row's owner is: the newcomer is occluded
         const uint32_t occl = (uint32_t)(__ballot(have && l < pos && closer(vd, dij, metric)) >> shift);
         // entries behind that the newcomer occludes
