@@ -1,5 +1,6 @@
 // start_nodes_api.cpp -- coral_start_ids_fps: Graph::FPS (src/start.cu:74-145) on the resident graph;
 // coral_index_mark_deleted: GPUFuncs::del_node_mark (src/update.cu:660-672).
+#include <algorithm>
 #include <climits>
 #include <vector>
 
@@ -17,12 +18,14 @@ extern "C" int coral_start_ids_fps(coral_index* idx, int32_t first_id, int32_t M
     hipStream_t st = idx->stream;
     const int64_t n = idx->n;
     const int nblocks = 512;
-    int *hops = nullptr, *min_hops = nullptr, *fa = nullptr, *fb = nullptr, *sizes = nullptr;
+    constexpr int kLevelsPerLook = 32;
+    int *hops = nullptr, *min_hops = nullptr, *fa = nullptr, *fb = nullptr;
     uint32_t* seen = nullptr;
+    // what the host reads after a search, in one piece: the maxima of the argmax launch, then the frontier sizes
     unsigned long long* partial = nullptr;
     auto release = [&]() {
         (void)hipFree(hops), (void)hipFree(min_hops), (void)hipFree(fa), (void)hipFree(fb);
-        (void)hipFree(sizes), (void)hipFree(partial), (void)hipFree(seen);
+        (void)hipFree(partial), (void)hipFree(seen);
     };
 #define TRY_R(expr)                                                                      \
     do {                                                                                 \
@@ -38,31 +41,38 @@ extern "C" int coral_start_ids_fps(coral_index* idx, int32_t first_id, int32_t M
     TRY_R(hipMalloc(&fa, n * sizeof(int)));
     TRY_R(hipMalloc(&fb, n * sizeof(int)));
     TRY_R(hipMalloc(&seen, (((size_t)n + 31) / 32 + 1) * sizeof(uint32_t)));
-    TRY_R(hipMalloc(&sizes, 2 * sizeof(int)));
-    TRY_R(hipMalloc(&partial, nblocks * sizeof(unsigned long long)));
+    const size_t back = nblocks * sizeof(unsigned long long) + coral::kBfsSlots * sizeof(int);
+    TRY_R(hipMalloc(&partial, back));
+    int* sizes = reinterpret_cast<int*>(partial + nblocks);
     TRY_R(coral::launch_fill_u32((uint32_t*)min_hops, (size_t)n, (uint32_t)INT_MAX, st));
-    std::vector<unsigned long long> h_partial(nblocks);
+    std::vector<unsigned long long> h_back((back + 7) / 8);
+    const int* h_sizes = reinterpret_cast<const int*>(h_back.data() + nblocks);
     int start = first_id, count = 0;
+    int levels = 8;  // launched before the host looks: what the search before needed and one more
     out_ids[count++] = start;
     while (count < M) {
         // one breadth-first search from the id selected last (src/start.cu:53-72)
-        TRY_R(coral::launch_bfs_init(hops, seen, fa, start, n, st));
-        int fsize = 1, level = 1;
+        TRY_R(coral::launch_bfs_init(hops, seen, fa, sizes, start, n, st));
         int *cur = fa, *next = fb;
-        while (fsize > 0) {
-            TRY_R(coral::launch_fill_u32((uint32_t*)sizes, 1, 0u, st));
-            TRY_R(coral::launch_bfs_expand(idx->d_nbrs, idx->R, cur, fsize, next, sizes, hops, seen, level++, st));
-            TRY_R(hipMemcpyAsync(&fsize, sizes, sizeof(int), hipMemcpyDeviceToHost, st));
+        int level = 0;
+        do {
+            for (int i = 0; i < levels; ++i) {
+                TRY_R(coral::launch_bfs_expand(idx->d_nbrs, idx->R, cur, next, sizes, hops, seen, ++level, n, st));
+                std::swap(cur, next);
+            }
+            // (launched before it is known whether the frontier is empty: a second time over more levels is no other)
+            TRY_R(coral::launch_update_min_hop(hops, min_hops, n, st));
+            TRY_R(coral::launch_argmax(min_hops, n, partial, nblocks, st));
+            TRY_R(hipMemcpyAsync(h_back.data(), partial, back, hipMemcpyDeviceToHost, st));
             TRY_R(hipStreamSynchronize(st));
-            std::swap(cur, next);
-        }
-        TRY_R(coral::launch_update_min_hop(hops, min_hops, n, st));
-        TRY_R(coral::launch_argmax(min_hops, n, partial, nblocks, st));
-        TRY_R(hipMemcpyAsync(h_partial.data(), partial, nblocks * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                             st));
-        TRY_R(hipStreamSynchronize(st));
+            levels = kLevelsPerLook;
+        } while (h_sizes[level % coral::kBfsSlots] > 0);
+        // the first empty frontier among the levels whose sizes are still there
+        int depth = level;
+        while (depth > 1 && level - depth < coral::kBfsSlots - 2 && h_sizes[(depth - 1) % coral::kBfsSlots] == 0) --depth;
+        levels = std::min(depth + 1, kLevelsPerLook);
         unsigned long long best = 0ull;
-        for (unsigned long long p : h_partial) best = p > best ? p : best;
+        for (int i = 0; i < nblocks; ++i) best = std::max(best, h_back[(size_t)i]);
         start = (int)(~(uint32_t)best);
         out_ids[count++] = start;
     }

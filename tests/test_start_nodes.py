@@ -74,6 +74,18 @@ def test_gpu_fps_equals_oracle(orc, n, R, M, seed):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 8, 9, 32, 33, 62, 63, 64, 65, 97, 1000])
+def test_gpu_fps_on_paths_as_deep_as_they_are_long(orc, n):
+    """Searches of every depth around the levels launched at a time and the frontier sizes kept (64)."""
+    from coral_amd import capi
+    g = path_graph(n)
+    idx = capi.Index(np.zeros((n, 4), np.float32), g, np.array([0], np.int32))
+    got = idx.start_ids_fps(n // 3, min(n, 5))
+    idx.close()
+    assert got.tolist() == orc.fps(g, n // 3, min(n, 5)).tolist()
+
+
+@pytest.mark.gpu
 def test_gpu_mark_deleted_accumulates_like_the_host_mask():
     # src/update.cu:406-412: bit (id & 31) of word (id >> 5), OR-ed in; two batches with repeats
     from coral_amd import capi, synth
