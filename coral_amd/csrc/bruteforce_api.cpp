@@ -1,7 +1,9 @@
 // bruteforce_api.cpp -- coral_bruteforce_knn*: exact k nearest neighbours of a batch of
 // queries among the index's resident vectors (kernels in bruteforce.hip, bruteforce_mfma.hip).
 #include <algorithm>
+#include <atomic>
 #include <cstring>
+#include <utility>
 #include <vector>
 
 #include "beam_search.h"
@@ -101,7 +103,53 @@ int ensure_base_norms(coral_index* idx, hipStream_t stream) {
 
 namespace {
 constexpr int kScreenSlack = 32;  // candidates kept beyond k
-constexpr int64_t kListCap = 16384;  // keys a query's candidate list holds in the fused screening
+constexpr int64_t kListCap = 16384;  // keys a query's candidate list holds at most in the fused screening
+constexpr size_t kKnnKeepBytes = (size_t)384 << 20;
+
+// Scratch of one call, carved from one block.  A block of up to kKnnKeepBytes stays with the index until it is
+// destroyed: a dozen allocations and releases were 150 of the 274 us of a call with 100 queries.  Every call waits for
+// its stream before it returns, so a call on another stream finds the block idle; a call that finds it taken by another
+// thread, or needs more, has a block of its own.
+class KnnScratch {
+public:
+    explicit KnnScratch(coral_index* idx) : idx_(idx) {}
+    KnnScratch(const KnnScratch&) = delete;
+    KnnScratch& operator=(const KnnScratch&) = delete;
+    ~KnnScratch() {
+        if (kept_)
+            idx_->knn_block_taken.store(false, std::memory_order_release);
+        else
+            (void)hipFree(base_);
+    }
+    template <typename T>
+    void reserve(T** p, size_t count) {
+        parts_.push_back({reinterpret_cast<void**>(p), total_});
+        total_ += (count * sizeof(T) + 255) & ~(size_t)255;
+    }
+    hipError_t allocate() {
+        if (total_ <= kKnnKeepBytes && !idx_->knn_block_taken.exchange(true, std::memory_order_acquire)) {
+            kept_ = true;
+            if (idx_->knn_block_bytes < total_) {
+                (void)hipFree(idx_->knn_block);
+                idx_->knn_block = nullptr, idx_->knn_block_bytes = 0;
+                if (hipError_t e = hipMalloc(&idx_->knn_block, total_)) return e;
+                idx_->knn_block_bytes = total_;
+            }
+            base_ = idx_->knn_block;
+        } else if (hipError_t e = hipMalloc(&base_, total_)) {
+            return e;
+        }
+        for (auto& p : parts_) *p.first = static_cast<char*>(base_) + p.second;
+        return hipSuccess;
+    }
+
+private:
+    coral_index* idx_;
+    std::vector<std::pair<void**, size_t>> parts_;
+    size_t total_ = 0;
+    void* base_ = nullptr;
+    bool kept_ = false;
+};
 
 // The screening with the selection inside the matrix-core kernel: no distance matrix goes to memory.  Per block of
 // queries: (1) the distances to a sample of the base (every stride-th tile of 128 points) as a small matrix, whose
@@ -110,84 +158,89 @@ constexpr int64_t kListCap = 16384;  // keys a query's candidate list holds in t
 // them) -- or two, where the base is many times the sample: first every step-th tile, whose kc smallest entries give
 // a tighter bound for the rest, then the tiles between; (3) the kc smallest keys of every list.  The kept candidates
 // are those of knn_passes(screen = true): the same approximate values, the kc smallest under (value, id).
-// *used = false when the shape does not suit (kc beyond what list_select_kernel takes, a base too small to sample) or
-// a list overflowed (sample unlike the base, rows of equal values, too few live points in the sample): the caller
-// then goes through the matrix.
-int knn_screen_fused(coral_index* idx, const float* d_queries, int32_t Q, int32_t kc, int32_t have_delete,
-                     const float* d_qn, int32_t* d_cid, float* d_cd, hipStream_t stream, bool* used) {
-    *used = false;
-    const int64_t n = idx->n, full_tiles = n / 128;
-    int64_t tiles = (2 * (int64_t)kc * full_tiles + kListCap - 1) / kListCap;
-    tiles = std::max<int64_t>(8, (tiles + 7) & ~(int64_t)7);
-    if (kc > 1024 || tiles * 8 > full_tiles || n > 0x7fffffff) return CORAL_OK;
-    // A larger sample than the lists need: an entry that passes costs an atomic and a scattered write.  A sixteenth of
-    // the base, up to 16 384 points.
-    tiles = std::max(tiles, std::min<int64_t>(128, (full_tiles / 16) & ~(int64_t)7));
-    const int64_t stride = full_tiles / tiles, ns = tiles * 128;
-    // Two passes with bounds from ns and then from n / step points let through kc (n / step / ns + step) entries per
-    // query instead of kc n / ns; step balances the two.  Worth a pass more only where the appending weighs more than
-    // the launches.
-    int step = 1;
-    if (Q >= 1024 && stride >= 16)
-        while ((step + 1) * (step + 1) <= stride) ++step;
-    int64_t qc = std::min<int64_t>(kListCap, (kBufferFloats / ns) & ~(int64_t)127);
-    qc = std::min<int64_t>(qc, ((int64_t)Q + 127) & ~(int64_t)127);
+struct FusedScreen {
+    bool suits = false;  // the shape does: kc within what list_select_kernel takes, a base large enough to sample
+    int64_t tiles = 0, stride = 0, ns = 0, qc = 0, qs = 0, cap = 0;
+    int step = 1, kc = 0;
     float *D = nullptr, *tau = nullptr;
     unsigned long long *keys = nullptr, *lists = nullptr;
     unsigned int* cnt = nullptr;
     int *redo = nullptr, *overflow = nullptr;
-    void* d_split = nullptr;
-    auto release = [&]() {
-        (void)hipFree(D), (void)hipFree(tau), (void)hipFree(keys), (void)hipFree(lists);
-        (void)hipFree(cnt), (void)hipFree(redo), (void)hipFree(overflow), (void)hipFree(d_split);
-    };
-#define HIP_TRY_R(expr)                                                                  \
-    do {                                                                                 \
-        hipError_t e_ = (expr);                                                          \
-        if (e_ != hipSuccess) {                                                          \
-            release();                                                                   \
-            return fail(e_ == hipErrorOutOfMemory ? CORAL_ERR_MEMORY : CORAL_ERR_DEVICE, \
-                        "%s failed: %s", #expr, hipGetErrorString(e_));                  \
-        }                                                                                \
-    } while (0)
-    HIP_TRY_R(hipMalloc(&D, (size_t)qc * ns * sizeof(float)));
-    HIP_TRY_R(hipMalloc(&tau, (size_t)qc * sizeof(float)));
-    HIP_TRY_R(hipMalloc(&keys, (size_t)qc * kc * sizeof(unsigned long long)));
-    HIP_TRY_R(hipMalloc(&lists, (size_t)qc * kListCap * sizeof(unsigned long long)));
-    HIP_TRY_R(hipMalloc(&cnt, (size_t)qc * coral::kCntStride * sizeof(unsigned int)));
-    HIP_TRY_R(hipMalloc(&d_split, coral::split_queries_bytes((int)qc, idx->dim)));
-    HIP_TRY_R(hipMalloc(&redo, (size_t)qc * sizeof(int)));
-    HIP_TRY_R(hipMalloc(&overflow, sizeof(int)));
-    HIP_TRY_R(coral::launch_fill_u32(reinterpret_cast<uint32_t*>(overflow), 1, 0u, stream));
-    const uint32_t* del = have_delete ? idx->d_deleted : nullptr;
-    for (int64_t q0 = 0; q0 < Q; q0 += qc) {
-        const int nq = (int)std::min<int64_t>(qc, Q - q0);
-        const float* qp = d_queries + (size_t)q0 * idx->dim;
-        HIP_TRY_R(coral::launch_split_queries(qp, nq, idx->dim, d_qn + q0, d_split, stream));
-        HIP_TRY_R(coral::launch_approx_tile(d_split, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm, del,
-                                            0, D, ns, stream, tiles, (int)stride));
-        HIP_TRY_R(coral::launch_row_select(D, ns, nq, ns, kc, 0, keys, kc, redo, stream));
-        HIP_TRY_R(coral::launch_bound_from_keys(keys, kc, kc - 1, nq, tau, stream));
-        HIP_TRY_R(coral::launch_fill_u32(cnt, (size_t)nq * coral::kCntStride, 0u, stream));
-        HIP_TRY_R(coral::launch_approx_filter(d_split, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm, del,
-                                              tau, lists, kListCap, cnt, step, stream));
-        if (step > 1) {
-            HIP_TRY_R(coral::launch_list_shrink(lists, kListCap, cnt, nq, kc, tau, overflow, stream));
-            HIP_TRY_R(coral::launch_approx_filter(d_split, idx->d_vec, nq, n, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm,
-                                                  del, tau, lists, kListCap, cnt, -step, stream));
-        }
-        HIP_TRY_R(coral::launch_list_select(lists, kListCap, cnt, nq, kc, keys, kc, overflow, stream));
-        HIP_TRY_R(coral::launch_merge_segments(keys, nq, 1, kc, /*signed distances*/ 0, d_cid + (size_t)q0 * kc,
-                                               d_cd + (size_t)q0 * kc, stream));
+    char* split = nullptr;
+
+    void plan(const coral_index* idx, int32_t Q, int32_t kc_) {
+        kc = kc_;
+        const int64_t n = idx->n, full_tiles = n / 128;
+        tiles = (2 * (int64_t)kc * full_tiles + kListCap - 1) / kListCap;
+        tiles = std::max<int64_t>(8, (tiles + 7) & ~(int64_t)7);
+        if (kc > 1024 || tiles * 8 > full_tiles || n > 0x7fffffff) return;
+        suits = true;
+        // A larger sample than the lists need: an entry that passes costs an atomic and a scattered write.  A
+        // sixteenth of the base, up to 16 384 points.
+        tiles = std::max(tiles, std::min<int64_t>(128, (full_tiles / 16) & ~(int64_t)7));
+        stride = full_tiles / tiles, ns = tiles * 128;
+        // Two passes with bounds from ns and then from n / step points let through kc (n / step / ns + step) entries
+        // per query instead of kc n / ns; step balances the two.  Worth a pass more only where the appending weighs
+        // more than the launches.
+        if (Q >= 1024 && stride >= 16)
+            while ((step + 1) * (step + 1) <= stride) ++step;
+        // three times the entries a list should see, of two passes the larger: kc to start with and kc * step more
+        const int64_t expect = kc * (step > 1 ? (stride + step - 1) / step + step : stride) + kc;
+        cap = 2048;
+        while (cap < 3 * expect && cap < kListCap) cap <<= 1;
+        // queries per block: what 4096 lists take is kept between calls, and a pass over the base for so many is
+        // hundreds of tiles per compute unit; the sample's matrix is made and read for 2048 at a time
+        const int64_t rows = ((int64_t)Q + 127) & ~(int64_t)127;
+        qc = std::min<int64_t>(4096, rows);
+        qs = std::min<int64_t>(2048, std::min(qc, std::max<int64_t>(128, (kBufferFloats / ns) & ~(int64_t)127)));
     }
-    int lost = 0;
-    HIP_TRY_R(hipMemcpyAsync(&lost, overflow, sizeof(int), hipMemcpyDeviceToHost, stream));
-    HIP_TRY_R(hipStreamSynchronize(stream));
-#undef HIP_TRY_R
-    release();
-    *used = lost == 0;
-    return CORAL_OK;
-}
+    void reserve(const coral_index* idx, KnnScratch& mem) {
+        if (!suits) return;
+        mem.reserve(&D, (size_t)qs * ns), mem.reserve(&tau, (size_t)qc), mem.reserve(&keys, (size_t)qc * kc);
+        mem.reserve(&lists, (size_t)qc * cap), mem.reserve(&cnt, (size_t)qc * coral::kCntStride);
+        mem.reserve(&redo, (size_t)qs), mem.reserve(&overflow, 1);
+        mem.reserve(&split, coral::split_queries_bytes((int)qc, idx->dim));
+    }
+    // *used = false when a list overflowed (sample unlike the base, rows of equal values, too few live points in the
+    // sample): the caller then goes through the matrix
+    int run(coral_index* idx, const float* d_queries, int32_t Q, int32_t have_delete, const float* d_qn, int32_t* d_cid,
+            float* d_cd, hipStream_t stream, bool* used) {
+        *used = false;
+        const int64_t n = idx->n;
+        HIP_TRY(coral::launch_fill_u32(reinterpret_cast<uint32_t*>(overflow), 1, 0u, stream));
+        const uint32_t* del = have_delete ? idx->d_deleted : nullptr;
+        for (int64_t q0 = 0; q0 < Q; q0 += qc) {
+            const int nq = (int)std::min<int64_t>(qc, Q - q0);
+            const float* qp = d_queries + (size_t)q0 * idx->dim;
+            const float* qn = d_qn + q0;
+            for (int64_t s0 = 0; s0 < nq; s0 += qs) {
+                const int ms = (int)std::min<int64_t>(qs, nq - s0);
+                HIP_TRY(coral::launch_split_queries(qp + (size_t)s0 * idx->dim, ms, idx->dim, qn + s0, split, stream));
+                HIP_TRY(coral::launch_approx_tile(split, idx->d_vec, ms, n, idx->dim, idx->metric, qn + s0, idx->d_bnorm, del,
+                                                  0, D, ns, stream, tiles, (int)stride));
+                HIP_TRY(coral::launch_row_select(D, ns, ms, ns, kc, 0, keys + (size_t)s0 * kc, kc, redo, stream));
+            }
+            if (nq > qs) HIP_TRY(coral::launch_split_queries(qp, nq, idx->dim, qn, split, stream));
+            HIP_TRY(coral::launch_bound_from_keys(keys, kc, kc - 1, nq, tau, stream));
+            HIP_TRY(coral::launch_fill_u32(cnt, (size_t)nq * coral::kCntStride, 0u, stream));
+            HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, qn, idx->d_bnorm, del, tau,
+                                                lists, cap, cnt, step, stream));
+            if (step > 1) {
+                HIP_TRY(coral::launch_list_shrink(lists, cap, cnt, nq, kc, tau, overflow, stream));
+                HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, qn, idx->d_bnorm, del,
+                                                    tau, lists, cap, cnt, -step, stream));
+            }
+            HIP_TRY(coral::launch_list_select(lists, cap, cnt, nq, kc, keys, kc, overflow, stream));
+            HIP_TRY(coral::launch_merge_segments(keys, nq, 1, kc, /*signed distances*/ 0, d_cid + (size_t)q0 * kc,
+                                                 d_cd + (size_t)q0 * kc, stream));
+        }
+        int lost = 0;
+        HIP_TRY(hipMemcpyAsync(&lost, overflow, sizeof(int), hipMemcpyDeviceToHost, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+        *used = lost == 0;
+        return CORAL_OK;
+    }
+};
 
 }  // namespace
 
@@ -204,53 +257,69 @@ int64_t coral_bruteforce_last_redone(coral_index* idx) { return idx ? idx->knn_l
 
 int32_t coral_bruteforce_last_fused(coral_index* idx) { return idx ? (int32_t)idx->knn_last_fused : -1; }
 
-int coral_bruteforce_knn_gpu(coral_index* idx, const float* d_queries, int32_t Q, int32_t k,
-                             int32_t have_delete, int32_t* d_ids, float* d_dists, void* stream_,
-                             double* time_s) {
-    if (!idx || !d_queries || !d_ids) return fail(CORAL_ERR_ARG, "null argument");
+static int check_knn(const coral_index* idx, int32_t Q, int32_t k, int32_t have_delete) {
     if (Q <= 0) return fail(CORAL_ERR_ARG, "Q must be positive");
     if (k <= 0 || k > 2048) return fail(CORAL_ERR_ARG, "k must be in 1..2048 (got %d)", k);
     if (have_delete && !idx->d_deleted)
         return fail(CORAL_ERR_STATE, "have_delete set but no tombstone mask was given");
-    HIP_TRY(hipSetDevice(idx->device));
-    hipStream_t stream = stream_ ? (hipStream_t)stream_ : idx->stream;
+    return CORAL_OK;
+}
+
+// The search of one call.  Host buffers (h_queries, h_ids, h_dists) are staged in the call's scratch; otherwise the
+// queries and results are d_queries, d_ids, d_dists.
+static int knn_call(coral_index* idx, const float* d_queries, const float* h_queries, int32_t Q, int32_t k,
+                    int32_t have_delete, int32_t* d_ids, int32_t* h_ids, float* d_dists, float* h_dists, hipStream_t stream,
+                    double* time_s) {
+    int rc = CORAL_OK;
+    const int kc = k + kScreenSlack;
+    const bool screen = !(idx->knn_mode == 1 || kc > 2048 || idx->n <= kc);
+    const size_t qb = (size_t)Q * idx->dim * sizeof(float), ib = (size_t)Q * k * sizeof(int32_t);
+    float *d_q = nullptr, *d_qn = nullptr, *d_cd = nullptr;
+    int32_t* d_cid = nullptr;
+    int* d_redo = nullptr;
+    FusedScreen fused_screen;
+    KnnScratch mem(idx);
+    if (h_queries) {
+        mem.reserve(&d_q, (size_t)Q * idx->dim), mem.reserve(&d_ids, (size_t)Q * k);
+        if (h_dists) mem.reserve(&d_dists, (size_t)Q * k);
+    }
+    if (screen) {
+        mem.reserve(&d_qn, (size_t)Q), mem.reserve(&d_cid, (size_t)Q * kc), mem.reserve(&d_cd, (size_t)Q * kc);
+        mem.reserve(&d_redo, (size_t)Q);
+        if (idx->knn_mode == 0) fused_screen.plan(idx, Q, kc);
+        fused_screen.reserve(idx, mem);
+    }
+    auto ok = [&](hipError_t e, const char* what) {
+        if (e == hipSuccess) return true;
+        rc = fail(e == hipErrorOutOfMemory ? CORAL_ERR_MEMORY : CORAL_ERR_DEVICE, "%s failed: %s", what, hipGetErrorString(e));
+        return false;
+    };
+    if ((h_queries || screen) && !ok(mem.allocate(), "hipMalloc")) return rc;
+    if (h_queries) {
+        if (!ok(hipMemcpy(d_q, h_queries, qb, hipMemcpyHostToDevice), "upload")) return rc;
+        d_queries = d_q;
+    }
     hipEvent_t ev0, ev1;
     HIP_TRY(hipEventCreate(&ev0));
     HIP_TRY(hipEventCreate(&ev1));
     HIP_TRY(hipEventRecord(ev0, stream));
-    int rc = CORAL_OK;
-    const int kc = k + kScreenSlack;
     idx->knn_last_redone = 0;
     idx->knn_last_fused = false;
-    if (idx->knn_mode == 1 || kc > 2048 || idx->n <= kc) {
+    if (!screen) {
         rc = knn_passes(idx, d_queries, Q, k, have_delete, false, nullptr, idx->metric, d_ids, d_dists, stream);
     } else {
         // screening on the matrix cores, exact distances for the kc candidates of each query, the exact passes for
         // the queries whose candidates cannot vouch for the result (bruteforce_mfma.hip)
-        float *d_qn = nullptr, *d_cd = nullptr, *d_rq = nullptr, *d_rd = nullptr;
-        int32_t *d_cid = nullptr, *d_rows = nullptr, *d_rid = nullptr;
-        int* d_redo = nullptr;
+        float *d_rq = nullptr, *d_rd = nullptr;
+        int32_t *d_rows = nullptr, *d_rid = nullptr;
         std::vector<int> redo((size_t)Q);
         std::vector<int32_t> rows;
-        auto release = [&]() {
-            (void)hipFree(d_qn), (void)hipFree(d_cd), (void)hipFree(d_cid), (void)hipFree(d_redo);
-            (void)hipFree(d_rows), (void)hipFree(d_rq), (void)hipFree(d_rid), (void)hipFree(d_rd);
-        };
-        auto ok = [&](hipError_t e, const char* what) {
-            if (e == hipSuccess) return true;
-            rc = fail(e == hipErrorOutOfMemory ? CORAL_ERR_MEMORY : CORAL_ERR_DEVICE, "%s failed: %s", what,
-                      hipGetErrorString(e));
-            return false;
-        };
+        auto release = [&]() { (void)hipFree(d_rows), (void)hipFree(d_rq), (void)hipFree(d_rid), (void)hipFree(d_rd); };
         if ((rc = coral::ensure_base_norms(idx, stream)) == CORAL_OK &&
-            ok(hipMalloc(&d_qn, (size_t)Q * sizeof(float)), "hipMalloc") &&
-            ok(hipMalloc(&d_cid, (size_t)Q * kc * sizeof(int32_t)), "hipMalloc") &&
-            ok(hipMalloc(&d_cd, (size_t)Q * kc * sizeof(float)), "hipMalloc") &&
-            ok(hipMalloc(&d_redo, (size_t)Q * sizeof(int)), "hipMalloc") &&
             ok(coral::launch_row_norms(d_queries, Q, idx->dim, d_qn, nullptr, stream), "query norms")) {
             bool fused = false;
-            if (idx->knn_mode == 0)
-                rc = knn_screen_fused(idx, d_queries, Q, kc, have_delete, d_qn, d_cid, d_cd, stream, &fused);
+            if (fused_screen.suits)
+                rc = fused_screen.run(idx, d_queries, Q, have_delete, d_qn, d_cid, d_cd, stream, &fused);
             idx->knn_last_fused = fused;
             if (rc == CORAL_OK && !fused)
                 rc = knn_passes(idx, d_queries, Q, kc, have_delete, true, d_qn, /*signed distances*/ 0, d_cid, d_cd, stream);
@@ -280,39 +349,37 @@ int coral_bruteforce_knn_gpu(coral_index* idx, const float* d_queries, int32_t Q
         release();
     }
     if (rc == CORAL_OK) {
-        HIP_TRY(hipEventRecord(ev1, stream));
-        HIP_TRY(hipEventSynchronize(ev1));
         float ms = 0.f;
-        HIP_TRY(hipEventElapsedTime(&ms, ev0, ev1));
-        if (time_s) *time_s = ms / 1000.0;
+        if (ok(hipEventRecord(ev1, stream), "event") && ok(hipEventSynchronize(ev1), "synchronize") &&
+            ok(hipEventElapsedTime(&ms, ev0, ev1), "event") && time_s)
+            *time_s = ms / 1000.0;
     }
     (void)hipEventDestroy(ev0);
     (void)hipEventDestroy(ev1);
+    if (rc == CORAL_OK && h_queries &&
+        (hipMemcpy(h_ids, d_ids, ib, hipMemcpyDeviceToHost) != hipSuccess ||
+         (h_dists && hipMemcpy(h_dists, d_dists, ib, hipMemcpyDeviceToHost) != hipSuccess)))
+        rc = fail(CORAL_ERR_DEVICE, "download failed");
+    if (rc != CORAL_OK) (void)hipStreamSynchronize(stream);  // nothing of this call is in flight when the scratch goes back
     return rc;
+}
+
+int coral_bruteforce_knn_gpu(coral_index* idx, const float* d_queries, int32_t Q, int32_t k,
+                             int32_t have_delete, int32_t* d_ids, float* d_dists, void* stream_,
+                             double* time_s) {
+    if (!idx || !d_queries || !d_ids) return fail(CORAL_ERR_ARG, "null argument");
+    if (int rc = check_knn(idx, Q, k, have_delete)) return rc;
+    HIP_TRY(hipSetDevice(idx->device));
+    return knn_call(idx, d_queries, nullptr, Q, k, have_delete, d_ids, nullptr, d_dists, nullptr,
+                    stream_ ? (hipStream_t)stream_ : idx->stream, time_s);
 }
 
 int coral_bruteforce_knn(coral_index* idx, const float* h_queries, int32_t Q, int32_t k, int32_t have_delete,
                          int32_t* h_ids, float* h_dists, double* time_s) {
     if (!idx || !h_queries || !h_ids) return fail(CORAL_ERR_ARG, "null argument");
-    if (Q <= 0 || k <= 0) return fail(CORAL_ERR_ARG, "Q and k must be positive");
+    if (int rc = check_knn(idx, Q, k, have_delete)) return rc;
     HIP_TRY(hipSetDevice(idx->device));
-    float* d_q = nullptr;
-    int32_t* d_ids = nullptr;
-    float* d_d = nullptr;
-    const size_t qb = (size_t)Q * idx->dim * sizeof(float), ib = (size_t)Q * k * sizeof(int32_t);
-    int rc = CORAL_OK;
-    if (hipMalloc(&d_q, qb) != hipSuccess || hipMalloc(&d_ids, ib) != hipSuccess ||
-        (h_dists && hipMalloc(&d_d, ib) != hipSuccess) ||
-        hipMemcpy(d_q, h_queries, qb, hipMemcpyHostToDevice) != hipSuccess)
-        rc = fail(CORAL_ERR_MEMORY, "device allocation or upload failed");
-    if (rc == CORAL_OK) rc = coral_bruteforce_knn_gpu(idx, d_q, Q, k, have_delete, d_ids, d_d, nullptr, time_s);
-    if (rc == CORAL_OK && (hipMemcpy(h_ids, d_ids, ib, hipMemcpyDeviceToHost) != hipSuccess ||
-                           (h_dists && hipMemcpy(h_dists, d_d, ib, hipMemcpyDeviceToHost) != hipSuccess)))
-        rc = fail(CORAL_ERR_DEVICE, "download failed");
-    (void)hipFree(d_q);
-    (void)hipFree(d_ids);
-    (void)hipFree(d_d);
-    return rc;
+    return knn_call(idx, nullptr, h_queries, Q, k, have_delete, nullptr, h_ids, nullptr, h_dists, idx->stream, time_s);
 }
 
 }  // extern "C"

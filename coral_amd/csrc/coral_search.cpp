@@ -207,6 +207,7 @@ void coral_index_destroy(coral_index* idx) {
     (void)hipFree(idx->d_bf_beams);
     (void)hipFree(idx->d_bnorm);
     (void)hipFree(idx->d_bnorm_max);
+    (void)hipFree(idx->knn_block);
     (void)hipFree(idx->d_io_q);
     (void)hipFree(idx->d_io_ids);
     (void)hipFree(idx->d_io_dists);

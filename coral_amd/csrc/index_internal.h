@@ -1,6 +1,7 @@
 // index_internal.h -- the library-private state behind a coral_index handle and the
 // error-propagation macro shared by the translation units that implement the C ABI.
 #pragma once
+#include <atomic>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -79,6 +80,10 @@ struct coral_index {
     uint32_t* d_bnorm_max = nullptr;
     int knn_mode = 0;             // 0: fused screening, 1: no screening, 2: screening through the distance matrix
     bool knn_last_fused = false;  // the last call's candidates came from the fused screening
+    // scratch of the exact kNN, kept between calls up to kKnnKeepBytes (bruteforce_api.cpp); one call has it at a time
+    void* knn_block = nullptr;
+    size_t knn_block_bytes = 0;
+    std::atomic<bool> knn_block_taken{false};
     int64_t knn_last_redone = 0;  // queries of the last call that went through the exact passes after screening
 
     // best-first on one wavefront per query: per-slot visited epochs in global memory
