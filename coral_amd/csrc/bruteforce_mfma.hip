@@ -136,8 +136,7 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     const int64_t b0 = (tile_step > 0 ? bt * tile_step : bt + bt / (-tile_step - 1) + 1) * NT;
     const int q0 = qt * MT;
     if (bt >= ntiles || b0 >= nb || qt >= nqt) return;  // padding: the last group of eight base tiles, the last query block
-    const int full = dim / BK, tail = dim % BK;
-    const int stages = full + (tail ? 1 : 0);
+    const int stages = (dim + BK - 1) / BK;
     // staging: thread t copies 4 x 16 bytes of the query stage and splits row t/2, dimensions (t&1)*8 .. +8 of the
     // base; rows beyond the end read the last row instead: their results are never written
     const int lrow = tid >> 1, lk = (tid & 1) * 8;
@@ -145,27 +144,33 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     const int64_t brow = min(b0 + lrow, nb - 1);
     const float* pb = base + (size_t)brow * dim + lk;
     const float bscale = mf_pow2(mf_scale_exp(bn[brow]));
-    v8h va[4];
-    float4 vb[2];
-    auto fetch = [&](int st) {
+    // A stage's loads are requested two stages ahead, with no condition, so that the wait for one stage's leaves the
+    // next one's in flight (against one stage ahead: 10 000 x 1 000 000 x 200 in 18.4 instead of 19.1 ms).
+    struct Staged {
+        v8h a[4];
+        float4 b[2];
+    } r0, r1;
+    auto fetch = [&](int st, Staged& r) {
+        st = min(st, stages - 1);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) va[u] = *reinterpret_cast<const v8h*>(pa + (size_t)st * kStageA + u * 2048);
-        if (st < full) {
+        for (int u = 0; u < 4; ++u) r.a[u] = *reinterpret_cast<const v8h*>(pa + (size_t)st * kStageA + u * 2048);
 #pragma unroll
-            for (int u = 0; u < 2; ++u) vb[u] = *reinterpret_cast<const float4*>(pb + st * BK + 4 * u);
-        } else {  // part of a stage (dim is a multiple of 4): what is missing is zero
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                vb[u] = make_float4(0, 0, 0, 0);
-                if (lk + 4 * u < tail) vb[u] = *reinterpret_cast<const float4*>(pb + st * BK + 4 * u);
-            }
+        for (int u = 0; u < 2; ++u) {
+            const int d = st * BK + 4 * u;  // beyond dim (a multiple of 4) the row's start is read and then dropped
+            r.b[u] = *reinterpret_cast<const float4*>(pb + (d + lk < dim ? d : -lk));
         }
     };
-    auto park = [&](int buf) {
+    auto park = [&](int st, int buf, const Staged& r) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) *reinterpret_cast<v8h*>(&sa[buf][u * 2048 + tid * 8]) = va[u];
+        for (int u = 0; u < 4; ++u) *reinterpret_cast<v8h*>(&sa[buf][u * 2048 + tid * 8]) = r.a[u];
+        float4 b[2] = {r.b[0], r.b[1]};
+        if ((st + 1) * BK > dim) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (st * BK + 4 * u + lk >= dim) b[u] = make_float4(0, 0, 0, 0);
+        }
         v8h hi, lo;
-        mf_split8(vb[0], vb[1], bscale, hi, lo);
+        mf_split8(b[0], b[1], bscale, hi, lo);
         *reinterpret_cast<v8h*>(&sb[buf][lrow * BK + lk]) = hi;
         *reinterpret_cast<v8h*>(&sb[buf][NT * BK + lrow * BK + lk]) = lo;
     };
@@ -202,18 +207,23 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
     };
-    fetch(0);
-    park(0);
+    fetch(0, r0);
+    fetch(1, r1);
+    park(0, 0, r0);
     __syncthreads();
-    int cur = 0;
-    for (int st = 0; st < stages; ++st) {
-        const bool more = st + 1 < stages;
-        if (more) fetch(st + 1);
-        multiply(cur);
-        if (more) park(cur ^ 1);
+#pragma unroll 1
+    for (int st = 0; st + 1 < stages; st += 2) {
+        fetch(st + 2, r0);
+        multiply(0);
+        park(st + 1, 1, r1);
         __syncthreads();
-        cur ^= 1;
+        fetch(st + 3, r1);
+        multiply(1);
+        park(min(st + 2, stages - 1), 0, r0);
+        __syncthreads();
     }
+    if (stages & 1) multiply(0);
+    __syncthreads();
     // a 32 x 32 block's 16 registers: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32.
     // What the tile's rows and columns contribute comes through LDS, fetched once per workgroup instead of by
     // dependent global loads per lane: norm and inverse scale of every row and column (times -2 or -1), the bounds.
