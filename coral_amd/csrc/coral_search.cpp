@@ -333,6 +333,14 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     // eight chunks of codes per lane is no faster than half precision: 103 k against 106 k QPS at 2048 floats, after
     // 382 k against 291 k at 1024)
     p.screen = !screen ? 0 : t.screening > 0 ? t.screening : (codes_possible && (idx->dim <= 1024 || idx->metric != CORAL_L2) ? 2 : 1);
+    // A batch of no more queries than the chip has CUs: every workgroup has a CU to itself whatever it takes of it, and
+    // the time of the launch is the longest query's chain of waits.  Such launches take 1024 threads, the bitmap
+    // wherever it fits and the look-ahead.  One query / 64 queries / 256 queries, before and after: 100 000 x 128,
+    // L = 64: 89 / 108 / 113 -> 64 / 75 / 79 us; 200 000 x 200, L = 128: 176 / 201 / 217 -> 117 / 141 / 158;
+    // 200 000 x 512, inner product, L = 256: 768 / 807 / 849 -> 360 / 403 / 640.  With 400 queries 1024 threads would
+    // cost 25 to 30 %, and going without the screening costs 12 % and more at every size.
+    const bool alone = !best_first && t.workgroups == 0 && t.cand_cap == 0 && Q <= idx->num_cu;
+    const bool any_form = t.visited_choices == 0;  // (a caller who names a form of the table gets a table)
     // ---- the visited structure.  Three forms: a table of 2^s 16-bit cells with an overflow bitmap in global memory
     // (visited_slots_log2 = s, or the library's choice), or a plain bitmap of all n ids in LDS (visited_slots_log2 =
     // -1, or the library's choice): one LDS atomic per test and nothing ever overflows, at n / 8 bytes -- 125 KB for
@@ -349,6 +357,7 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
         return fail(CORAL_ERR_ARG, "visited_choices must be 0, 1, 3 or 4 (got %d)", t.visited_choices);
     const int choices = t.visited_choices == 4 ? 3 : t.visited_choices;  // (4: the bucket form as tests want it)
     bool three = false;  // the table of cells in its bucket form
+    int plan_words = 0;  // words of visited state that the lists are sized beside, if more than there are
     int slots_log2 = t.visited_slots_log2;
     if (slots_log2 == -1) {
         if (!bitmap_possible || lds_bitmap(p.big, min_cap) > lds_max)
@@ -369,8 +378,13 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
         want += bump_log2;
         const bool table_holds = !p.big && want <= 16 && lds_table(false, want, min_cap) <= lds_max;
         const bool table_alone_on_cu = table_holds && lds_table(false, want, min_cap) > lds_max / 2;
-        if (bitmap_possible && !p.big && lds_bitmap(false, min_cap) <= lds_max && (!table_holds || table_alone_on_cu)) {
-            p.direct = 1;  // one workgroup per CU either way: the bitmap is the cheaper test and cannot overflow
+        const bool smaller = any_form && table_holds && bitmap_words <= (1 << want) >> 1;  // 200 000 ids: 25 KB against 32 KB at L = 128
+        if (bitmap_possible && !p.big && lds_bitmap(false, min_cap) <= lds_max &&
+            (!table_holds || table_alone_on_cu || (alone && any_form) || smaller)) {
+            p.direct = 1;  // no workgroup per CU less for it: the bitmap is the cheaper test and cannot overflow
+            // (the LDS a smaller bitmap leaves over goes unused: a list of 1024 instead of 512 costs the 512-float
+            // search at L = 256 1 %, see below)
+            if (smaller && !alone) plan_words = (1 << want) >> 1;
         } else if (bitmap_possible && !table_holds && !lds_beam_only && lds_bitmap(true, 1024) <= lds_max) {
             p.direct = 1, p.big = true;  // the beam gives its LDS to the bitmap (measured: +30 % at L = 1024 and 2048)
         } else {
@@ -434,7 +448,8 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
         // with the list, the beam's worst entry be refreshed half as often, and a 512-float inner-product search at
         // L = 256 lost 5 %)
         if (cap == 2048 && !(screen && wg_fit == 1 && p.big)) continue;
-        if (lds_for(cap, cap) <= lds_max && (int)(lds_max / lds_for(cap, cap)) >= std::min(wg_fit, 2)) {
+        const size_t need = lds_for(cap, cap) + (size_t)std::max(0, plan_words - p.table_words) * 4;
+        if (need <= lds_max && (int)(lds_max / need) >= (alone ? 1 : std::min(wg_fit, 2))) {
             tcap = cap;
             break;
         }
@@ -449,7 +464,7 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     }
     int threads = t.threads;
     if (threads == 0)
-        threads = p.big ? 1024 : best_first ? 256 : (lds_for(tcap, ccap) > lds_max / 2 ? 1024 : 512);
+        threads = p.big || alone ? 1024 : best_first ? 256 : (lds_for(tcap, ccap) > lds_max / 2 ? 1024 : 512);
     if (threads != 128 && threads != 256 && threads != 512 && threads != 1024)
         return fail(CORAL_ERR_ARG, "threads must be 128, 256, 512 or 1024");
     p.lds_bytes = coral::search_lds_bytes(L, idx->dim, p.table_words, tcap, ccap, ocap, p.big, screen);
@@ -469,7 +484,7 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     p.workgroups = std::min(workgroups, (int)Q);
     p.tcap = tcap, p.ccap = ccap, p.threads = threads, p.id_bits = id_bits, p.ocap = ocap;
     // graph rows a chunk ahead: pays where a workgroup is alone on its CU (nothing else covers the wait)
-    p.prefetch = t.prefetch_rows > 0 || (t.prefetch_rows == 0 && wg_per_cu == 1 && !best_first);
+    p.prefetch = t.prefetch_rows > 0 || (t.prefetch_rows == 0 && (wg_per_cu == 1 || alone) && !best_first);
     p.beam_stride = p.big ? coral::search_beam_stride(L) : 0;
     *out = p;
     return CORAL_OK;

@@ -41,6 +41,36 @@ def problem(n, dim, R, seed, metric="l2", n_start=16, ragged_seed=None, isolate=
     return base, nbrs, starts
 
 
+@pytest.mark.parametrize("n,dim,R,metric,L,k,M", [
+    (40, 20, 8, "l2", 16, 10, 3),        # the bitmap is two words, the beam holds nearly all there is
+    (9000, 68, 32, "ip", 64, 10, 16),
+    (9000, 200, 24, "l2", 300, 100, 16),  # rows that do not divide a pass of 1024 threads
+    (33000, 132, 32, "l2", 1100, 50, 7),  # the beam takes more than half of a CU's LDS
+])
+def test_batches_of_few_queries_take_another_launch_and_give_the_same(n, dim, R, metric, L, k, M):
+    """No more queries than CUs: 1024 threads and the bitmap of all ids; one more: what there was before.  Both against
+    a launch whose table, threads and look-ahead the caller names: ids, distance bits and counters are the same."""
+    import torch
+    base, nbrs, starts = problem(n, dim, R, 21, metric, M)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    q = synth.shifted_queries(cus + 1, dim, 5, 6, 7)
+    idx = capi.Index(base, nbrs, starts, capi.IP if metric == "ip" else capi.L2)
+    want = None
+    for Q, kw in ((cus + 1, dict(threads=512, visited_slots_log2=13, prefetch_rows=-1)), (cus + 1, {}), (cus, {}), (1, {})):
+        idx.prepare(Q, L, **kw)
+        plan = idx.plan_info()
+        if not kw:
+            assert plan.visited_form == 1
+            assert plan.beam_in_hbm or Q > cus or plan.threads == 1024
+        ids, dists, _ = idx.search(q[:Q], k, L)
+        cnt = idx.query_counters(Q)
+        if want is None:
+            want = ids, dists, cnt
+        assert np.array_equal(ids, want[0][:Q]) and np.array_equal(cnt, want[2][:Q])
+        assert dists.tobytes() == want[1][:Q].tobytes()
+    idx.close()
+
+
 CASES = [
     # n, dim, R, metric, policy, L, k, M, ragged, slots_log2, threads
     (20000, 200, 32, "l2", 0, 64, 10, 16, None, 0, 0),
