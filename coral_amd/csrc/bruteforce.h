@@ -7,9 +7,11 @@ namespace coral {
 hipError_t launch_distance_tile(const float* queries, const float* base, int nq, int64_t nb, int dim,
                                 int metric, const uint32_t* deleted, int64_t base_id0, float* D,
                                 int64_t ldD, hipStream_t stream);
+// tau: only the value of the k-th smallest of every row (+inf if there are fewer); out is not written then
 // redo: int[nq] scratch for the rows the fast path hands over (null: radix path for every row)
 hipError_t launch_row_select(const float* D, int64_t ldD, int nq, int64_t n, int k, int64_t id0,
-                             unsigned long long* out, int64_t out_stride, int* redo, hipStream_t stream);
+                             unsigned long long* out, int64_t out_stride, int* redo, hipStream_t stream,
+                             float* tau = nullptr);
 hipError_t launch_merge_segments(const unsigned long long* part, int nq, int nseg, int k, int metric,
                                  int32_t* ids, float* dists, hipStream_t stream);
 // --- the screening pass on the matrix cores (bruteforce_mfma.hip) ---
@@ -32,12 +34,10 @@ hipError_t launch_approx_filter(const void* queries, const float* base, int nq, 
                                 const float* qn, const float* bn, const uint32_t* deleted, const float* tau,
                                 unsigned long long* lists, int64_t cap, unsigned int* cnt, int tile_step,
                                 hipStream_t stream);
-// tau[q] = value of keys[q * stride + j], +inf where that key is the "none" key
-hipError_t launch_bound_from_keys(const unsigned long long* keys, int64_t stride, int j, int nq, float* tau,
-                                  hipStream_t stream);
-// the k (<= 1024) smallest keys of every list, sorted; *overflow (zero before) counts the lists that could not be done
-hipError_t launch_list_select(const unsigned long long* lists, int64_t cap, const unsigned int* cnt, int nq, int k,
-                              unsigned long long* out, int64_t out_stride, int* overflow, hipStream_t stream);
+// the k (<= 1024) smallest keys of every list, sorted, as ids [nq][k] (-1: none) and values; *overflow (zero before)
+// counts the lists that could not be done
+hipError_t launch_list_select(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, int32_t* ids,
+                              float* dists, int* overflow, hipStream_t stream);
 // the same selection in place, between two launches that append: the list shrinks to its k smallest keys, tau[q]
 // becomes the value of the k-th (+inf if there are fewer)
 hipError_t launch_list_shrink(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, float* tau,

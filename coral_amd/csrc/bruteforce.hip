@@ -165,15 +165,19 @@ __global__ __launch_bounds__(256) void distance_tile_kernel(const float* __restr
 // collects the entries up to that value into LDS, a sort by (value, index) finishes.  Two coalesced reads of the
 // row, no atomics on the way.  A row with so many ties at the threshold that the candidates outgrow LDS is
 // flagged and left to row_select_radix_kernel, which makes no such assumption.
-constexpr int kSelThreads = 1024;
+// T threads: 1024, or 256 where k is small (kFewK): the minima of 256 threads bound the k-th smallest a little more
+// loosely, and their sort and its barriers are a third of the time of either kernel otherwise.
+constexpr int kSelThreads = 1024, kFewThreads = 256, kFewK = 160;
 constexpr int kSelCap = 4096;  // candidate keys in LDS
+// (out or tau: the keys, or only the value of the k-th, +inf if there are fewer)
 
-__global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __restrict__ D, int64_t ldD, int64_t n,
-                                                                 int k, int64_t id0,
-                                                                 unsigned long long* __restrict__ out,
-                                                                 int64_t out_stride, int* __restrict__ redo) {
+template <int T>
+__global__ __launch_bounds__(T) void row_select_kernel(const float* __restrict__ D, int64_t ldD, int64_t n, int k,
+                                                       int64_t id0, unsigned long long* __restrict__ out,
+                                                       int64_t out_stride, int* __restrict__ redo,
+                                                       float* __restrict__ tau) {
     __shared__ unsigned long long skeys[kSelCap];
-    __shared__ uint32_t smin[kSelThreads];
+    __shared__ uint32_t smin[T];
     __shared__ unsigned int s_count;
     const int tid = threadIdx.x;
     const float* row = D + (size_t)blockIdx.x * ldD;
@@ -182,20 +186,20 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __
     const float4* row4 = reinterpret_cast<const float4*>(row);  // rows start 16-byte aligned (ldD % 4 == 0)
     // pass 1: per-thread minimum
     uint32_t m = 0xffffffffu;
-    for (int64_t i = tid; i < n4; i += 2 * kSelThreads) {
+    for (int64_t i = tid; i < n4; i += 2 * T) {
         const float4 v0 = row4[i];
-        const float4 v1 = i + kSelThreads < n4 ? row4[i + kSelThreads] : v0;
+        const float4 v1 = i + T < n4 ? row4[i + T] : v0;
         m = min(m, min(min(bf_ord32(v0.x), bf_ord32(v0.y)), min(bf_ord32(v0.z), bf_ord32(v0.w))));
         m = min(m, min(min(bf_ord32(v1.x), bf_ord32(v1.y)), min(bf_ord32(v1.z), bf_ord32(v1.w))));
     }
-    for (int64_t i = (n4 << 2) + tid; i < n; i += kSelThreads) m = min(m, bf_ord32(row[i]));
+    for (int64_t i = (n4 << 2) + tid; i < n; i += T) m = min(m, bf_ord32(row[i]));
     smin[tid] = m;
     if (tid == 0) s_count = 0u;
     __syncthreads();
     // the kk-th smallest of the minima: bitonic sort of 1024 values
-    for (int k2 = 2; k2 <= kSelThreads; k2 <<= 1)
+    for (int k2 = 2; k2 <= T; k2 <<= 1)
         for (int j = k2 >> 1; j > 0; j >>= 1) {
-            if (tid < kSelThreads / 2) {
+            if (tid < T / 2) {
                 const int i = 2 * tid - (tid & (j - 1)), x = i + j;
                 const bool asc = (i & k2) == 0;
                 const uint32_t a = smin[i], b = smin[x];
@@ -203,9 +207,9 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __
             }
             __syncthreads();
         }
-    const uint32_t thr = kk <= kSelThreads ? smin[kk - 1] : 0xffffffffu;
+    const uint32_t thr = kk <= T ? smin[kk - 1] : 0xffffffffu;
     // pass 2: everything up to the threshold
-    for (int64_t i0 = 0; i0 < n4; i0 += kSelThreads) {
+    for (int64_t i0 = 0; i0 < n4; i0 += T) {
         const int64_t i = i0 + tid;
         float4 v = make_float4(0, 0, 0, 0);
         bool hit = false;
@@ -226,7 +230,7 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __
                 }
         }
     }
-    for (int64_t i = (n4 << 2) + tid; i < n; i += kSelThreads) {
+    for (int64_t i = (n4 << 2) + tid; i < n; i += T) {
         const uint32_t o = bf_ord32(row[i]);
         if (o <= thr) {
             const unsigned pos = atomicAdd(&s_count, 1u);
@@ -242,11 +246,11 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __
     if (tid == 0) redo[blockIdx.x] = 0;
     int P = 2;
     while (P < (int)count) P <<= 1;
-    for (int i = (int)count + tid; i < P; i += kSelThreads) skeys[i] = ~0ull;
+    for (int i = (int)count + tid; i < P; i += T) skeys[i] = ~0ull;
     __syncthreads();
     for (int k2 = 2; k2 <= P; k2 <<= 1)
         for (int j = k2 >> 1; j > 0; j >>= 1) {
-            for (int t = tid; t < (P >> 1); t += kSelThreads) {
+            for (int t = tid; t < (P >> 1); t += T) {
                 const int i = 2 * t - (t & (j - 1)), x = i + j;
                 const bool asc = (i & k2) == 0;
                 const unsigned long long ka = skeys[i], kb = skeys[x];
@@ -254,8 +258,12 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __
             }
             __syncthreads();
         }
+    if (tau) {  // (a tombstoned k-th is +inf as it is)
+        if (tid == 0) tau[blockIdx.x] = kk == k ? bf_unord32((uint32_t)(skeys[k - 1] >> 32)) : __int_as_float(0x7f800000);
+        return;
+    }
     unsigned long long* dst = out + (size_t)blockIdx.x * out_stride;
-    for (int i = tid; i < k; i += kSelThreads) {
+    for (int i = tid; i < k; i += T) {
         unsigned long long key = i < kk ? skeys[i] : ~0ull;
         if ((uint32_t)(key >> 32) == bf_ord32(__int_as_float(0x7f800000))) key = ~0ull;  // tombstoned
         dst[i] = key;
@@ -266,15 +274,15 @@ __global__ __launch_bounds__(kSelThreads) void row_select_kernel(const float* __
 // id), sorted, into out.  The scheme of row_select_kernel on keys: the k-th smallest of the per-thread minima bounds
 // the k-th smallest key from above, a second pass collects what lies up to it, a sort finishes.  *overflow is raised
 // when a list lost entries (cnt[q] > cap) or the collection outgrows LDS; the caller then takes another path.
-// SHRINK: the result replaces the list (out = lists, out_stride = cap) and its count, and tau[q] becomes the value
-// of the k-th key.
-template <bool SHRINK>
-__global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned long long* lists, int64_t cap,
-                                                                  unsigned int* cnt, int k, unsigned long long* out,
-                                                                  int64_t out_stride, float* __restrict__ tau,
-                                                                  int* __restrict__ overflow) {
+// The result goes out as ids (-1: none) and values; SHRINK: it replaces the list and its count, and tau[q] becomes the
+// value of the k-th key.
+template <int T, bool SHRINK>
+__global__ __launch_bounds__(T) void list_select_kernel(unsigned long long* __restrict__ lists, int64_t cap,
+                                                        unsigned int* __restrict__ cnt, int k, int32_t* __restrict__ ids,
+                                                        float* __restrict__ dists, float* __restrict__ tau,
+                                                        int* __restrict__ overflow) {
     __shared__ unsigned long long skeys[kSelCap];
-    __shared__ unsigned long long smin[kSelThreads];
+    __shared__ unsigned long long smin[T];
     __shared__ unsigned int s_count;
     const int tid = threadIdx.x;
     const unsigned int have = cnt[(size_t)blockIdx.x * kCntStride];
@@ -283,16 +291,16 @@ __global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned
         return;
     }
     const int n = (int)have;
-    const unsigned long long* list = lists + (size_t)blockIdx.x * cap;
+    unsigned long long* list = lists + (size_t)blockIdx.x * cap;
     const int kk = min(k, n);
     unsigned long long m = ~0ull;
-    for (int i = tid; i < n; i += kSelThreads) m = min(m, list[i]);
+    for (int i = tid; i < n; i += T) m = min(m, list[i]);
     smin[tid] = m;
     if (tid == 0) s_count = 0u;
     __syncthreads();
-    for (int k2 = 2; k2 <= kSelThreads; k2 <<= 1)
+    for (int k2 = 2; k2 <= T; k2 <<= 1)
         for (int j = k2 >> 1; j > 0; j >>= 1) {
-            if (tid < kSelThreads / 2) {
+            if (tid < T / 2) {
                 const int i = 2 * tid - (tid & (j - 1)), x = i + j;
                 const bool asc = (i & k2) == 0;
                 const unsigned long long a = smin[i], b = smin[x];
@@ -300,8 +308,8 @@ __global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned
             }
             __syncthreads();
         }
-    const unsigned long long thr = kk > 0 ? smin[kk - 1] : 0ull;  // k <= kSelThreads (launcher)
-    for (int i = tid; i < n; i += kSelThreads) {
+    const unsigned long long thr = kk > 0 ? smin[kk - 1] : 0ull;  // k <= T (launcher)
+    for (int i = tid; i < n; i += T) {
         const unsigned long long key = list[i];
         if (kk > 0 && key <= thr) {
             const unsigned pos = atomicAdd(&s_count, 1u);
@@ -316,11 +324,11 @@ __global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned
     }
     int P = 2;
     while (P < (int)count) P <<= 1;
-    for (int i = (int)count + tid; i < P; i += kSelThreads) skeys[i] = ~0ull;
+    for (int i = (int)count + tid; i < P; i += T) skeys[i] = ~0ull;
     __syncthreads();
     for (int k2 = 2; k2 <= P; k2 <<= 1)
         for (int j = k2 >> 1; j > 0; j >>= 1) {
-            for (int t = tid; t < (P >> 1); t += kSelThreads) {
+            for (int t = tid; t < (P >> 1); t += T) {
                 const int i = 2 * t - (t & (j - 1)), x = i + j;
                 const bool asc = (i & k2) == 0;
                 const unsigned long long ka = skeys[i], kb = skeys[x];
@@ -328,19 +336,19 @@ __global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned
             }
             __syncthreads();
         }
-    unsigned long long* dst = out + (size_t)blockIdx.x * out_stride;
     if constexpr (SHRINK) {  // every thread has read the list: the barriers of the sort lie in between
-        for (int i = tid; i < kk; i += kSelThreads) dst[i] = skeys[i];
+        for (int i = tid; i < kk; i += T) list[i] = skeys[i];
         if (tid == 0) {
             cnt[(size_t)blockIdx.x * kCntStride] = (unsigned)kk;
             tau[blockIdx.x] = kk == k ? bf_unord32((uint32_t)(skeys[k - 1] >> 32)) : __int_as_float(0x7f800000);
         }
-        return;
-    }
-    for (int i = tid; i < k; i += kSelThreads) {
-        unsigned long long key = i < kk ? skeys[i] : ~0ull;
-        if ((uint32_t)(key >> 32) == bf_ord32(__int_as_float(0x7f800000))) key = ~0ull;  // tombstoned
-        dst[i] = key;
+    } else {
+        for (int i = tid; i < k; i += T) {
+            const unsigned long long key = i < kk ? skeys[i] : ~0ull;
+            const bool none = (uint32_t)(key >> 32) == bf_ord32(__int_as_float(0x7f800000)) || key == ~0ull;  // tombstoned, or fewer
+            ids[(size_t)blockIdx.x * k + i] = none ? -1 : (int32_t)(uint32_t)key;
+            dists[(size_t)blockIdx.x * k + i] = none ? 3.402823466e+38f : bf_unord32((uint32_t)(key >> 32));
+        }
     }
 }
 
@@ -349,7 +357,8 @@ __global__ __launch_bounds__(kSelThreads) void list_select_kernel(const unsigned
 __global__ __launch_bounds__(256) void row_select_radix_kernel(const float* __restrict__ D, int64_t ldD,
                                                                int64_t n, int k, int64_t id0,
                                                                unsigned long long* __restrict__ out,
-                                                               int64_t out_stride, const int* __restrict__ redo) {
+                                                               int64_t out_stride, const int* __restrict__ redo,
+                                                               float* __restrict__ tau) {
     extern __shared__ unsigned long long skeys[];  // pow2 >= k keys
     __shared__ unsigned int hist[256];
     __shared__ unsigned int s_prefix, s_need, s_count, s_base;
@@ -468,6 +477,10 @@ __global__ __launch_bounds__(256) void row_select_radix_kernel(const float* __re
             }
             __syncthreads();
         }
+    if (tau) {
+        if (tid == 0) tau[blockIdx.x] = kk == k ? bf_unord32((uint32_t)(skeys[k - 1] >> 32)) : __int_as_float(0x7f800000);
+        return;
+    }
     unsigned long long* dst = out + (size_t)blockIdx.x * out_stride;
     for (int i = tid; i < k; i += 256) {
         unsigned long long key = i < kk ? skeys[i] : ~0ull;
@@ -520,31 +533,36 @@ hipError_t launch_distance_tile(const float* queries, const float* base, int nq,
 }
 
 hipError_t launch_row_select(const float* D, int64_t ldD, int nq, int64_t n, int k, int64_t id0,
-                             unsigned long long* out, int64_t out_stride, int* redo, hipStream_t stream) {
+                             unsigned long long* out, int64_t out_stride, int* redo, hipStream_t stream, float* tau) {
     int P = 2;
     while (P < k) P <<= 1;
     const bool fast = redo != nullptr && k <= kSelThreads;
-    if (fast)
-        hipLaunchKernelGGL(row_select_kernel, dim3(nq), dim3(kSelThreads), 0, stream, D, ldD, n, k, id0, out, out_stride,
-                           redo);
+    if (fast && k <= kFewK && n <= 32768)  // (longer rows want the loads of 1024 threads)
+        hipLaunchKernelGGL(row_select_kernel<kFewThreads>, dim3(nq), dim3(kFewThreads), 0, stream, D, ldD, n, k, id0, out,
+                           out_stride, redo, tau);
+    else if (fast)
+        hipLaunchKernelGGL(row_select_kernel<kSelThreads>, dim3(nq), dim3(kSelThreads), 0, stream, D, ldD, n, k, id0, out,
+                           out_stride, redo, tau);
     hipLaunchKernelGGL(row_select_radix_kernel, dim3(nq), dim3(256), (size_t)P * 8, stream, D, ldD, n, k, id0, out,
-                       out_stride, fast ? redo : nullptr);
+                       out_stride, fast ? redo : nullptr, tau);
     return hipGetLastError();
 }
 
-hipError_t launch_list_select(const unsigned long long* lists, int64_t cap, const unsigned int* cnt, int nq, int k,
-                              unsigned long long* out, int64_t out_stride, int* overflow, hipStream_t stream) {
+hipError_t launch_list_select(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, int32_t* ids,
+                              float* dists, int* overflow, hipStream_t stream) {
     if (k > kSelThreads) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(list_select_kernel<false>, dim3(nq), dim3(kSelThreads), 0, stream, lists, cap,
-                       const_cast<unsigned int*>(cnt), k, out, out_stride, (float*)nullptr, overflow);
+    auto kernel = k <= kFewK ? list_select_kernel<kFewThreads, false> : list_select_kernel<kSelThreads, false>;
+    hipLaunchKernelGGL(kernel, dim3(nq), dim3(k <= kFewK ? kFewThreads : kSelThreads), 0, stream, lists, cap, cnt, k, ids,
+                       dists, (float*)nullptr, overflow);
     return hipGetLastError();
 }
 
 hipError_t launch_list_shrink(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, float* tau,
                               int* overflow, hipStream_t stream) {
     if (k > kSelThreads || k > cap) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(list_select_kernel<true>, dim3(nq), dim3(kSelThreads), 0, stream, lists, cap, cnt, k, lists, cap, tau,
-                       overflow);
+    auto kernel = k <= kFewK ? list_select_kernel<kFewThreads, true> : list_select_kernel<kSelThreads, true>;
+    hipLaunchKernelGGL(kernel, dim3(nq), dim3(k <= kFewK ? kFewThreads : kSelThreads), 0, stream, lists, cap, cnt, k,
+                       (int32_t*)nullptr, (float*)nullptr, tau, overflow);
     return hipGetLastError();
 }
 

@@ -163,7 +163,7 @@ struct FusedScreen {
     int64_t tiles = 0, stride = 0, ns = 0, qc = 0, qs = 0, cap = 0;
     int step = 1, kc = 0;
     float *D = nullptr, *tau = nullptr;
-    unsigned long long *keys = nullptr, *lists = nullptr;
+    unsigned long long* lists = nullptr;
     unsigned int* cnt = nullptr;
     int *redo = nullptr, *overflow = nullptr;
     char* split = nullptr;
@@ -196,7 +196,7 @@ struct FusedScreen {
     }
     void reserve(const coral_index* idx, KnnScratch& mem) {
         if (!suits) return;
-        mem.reserve(&D, (size_t)qs * ns), mem.reserve(&tau, (size_t)qc), mem.reserve(&keys, (size_t)qc * kc);
+        mem.reserve(&D, (size_t)qs * ns), mem.reserve(&tau, (size_t)qc);
         mem.reserve(&lists, (size_t)qc * cap), mem.reserve(&cnt, (size_t)qc * coral::kCntStride);
         mem.reserve(&redo, (size_t)qs), mem.reserve(&overflow, 1);
         mem.reserve(&split, coral::split_queries_bytes((int)qc, idx->dim));
@@ -218,10 +218,9 @@ struct FusedScreen {
                 HIP_TRY(coral::launch_split_queries(qp + (size_t)s0 * idx->dim, ms, idx->dim, qn + s0, split, stream));
                 HIP_TRY(coral::launch_approx_tile(split, idx->d_vec, ms, n, idx->dim, idx->metric, qn + s0, idx->d_bnorm, del,
                                                   0, D, ns, stream, tiles, (int)stride));
-                HIP_TRY(coral::launch_row_select(D, ns, ms, ns, kc, 0, keys + (size_t)s0 * kc, kc, redo, stream));
+                HIP_TRY(coral::launch_row_select(D, ns, ms, ns, kc, 0, nullptr, 0, redo, stream, tau + s0));
             }
             if (nq > qs) HIP_TRY(coral::launch_split_queries(qp, nq, idx->dim, qn, split, stream));
-            HIP_TRY(coral::launch_bound_from_keys(keys, kc, kc - 1, nq, tau, stream));
             HIP_TRY(coral::launch_fill_u32(cnt, (size_t)nq * coral::kCntStride, 0u, stream));
             HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, qn, idx->d_bnorm, del, tau,
                                                 lists, cap, cnt, step, stream));
@@ -230,9 +229,8 @@ struct FusedScreen {
                 HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, qn, idx->d_bnorm, del,
                                                     tau, lists, cap, cnt, -step, stream));
             }
-            HIP_TRY(coral::launch_list_select(lists, cap, cnt, nq, kc, keys, kc, overflow, stream));
-            HIP_TRY(coral::launch_merge_segments(keys, nq, 1, kc, /*signed distances*/ 0, d_cid + (size_t)q0 * kc,
-                                                 d_cd + (size_t)q0 * kc, stream));
+            HIP_TRY(coral::launch_list_select(lists, cap, cnt, nq, kc, d_cid + (size_t)q0 * kc, d_cd + (size_t)q0 * kc,
+                                              overflow, stream));
         }
         int lost = 0;
         HIP_TRY(hipMemcpyAsync(&lost, overflow, sizeof(int), hipMemcpyDeviceToHost, stream));

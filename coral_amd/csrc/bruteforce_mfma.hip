@@ -312,16 +312,6 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     }
 }
 
-// tau[q] = value of the key keys[q * stride + j] (the j-th smallest of a sample of the row), +inf where the sample
-// has no j-th entry
-__global__ void bound_from_keys_kernel(const unsigned long long* __restrict__ keys, int64_t stride, int j, int nq,
-                                       float* __restrict__ tau) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nq) return;
-    const unsigned long long key = keys[(size_t)q * stride + j];
-    tau[q] = key == ~0ull ? __int_as_float(0x7f800000) : mf_unord32((uint32_t)(key >> 32));
-}
-
 // One workgroup per query: the kc candidates (ids, -1 = none; approximate signed distances, ascending) are measured
 // in the reference's order (one thread walks the dimensions of one candidate with one fused multiply-add each,
 // include/utils.cuh:254-275, 307-323: the arithmetic of distance_tile_kernel), sorted by (distance, id), and the k
@@ -476,12 +466,6 @@ hipError_t launch_approx_filter(const void* queries, const float* base, int nq, 
     auto kernel = metric == 0 ? approx_tile_mfma_kernel<true, true> : approx_tile_mfma_kernel<true, false>;
     hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
                        bn, deleted, (int64_t)0, ntiles, tile_step, (int)hq, (float*)nullptr, (int64_t)0, tau, lists, cap, cnt);
-    return hipGetLastError();
-}
-
-hipError_t launch_bound_from_keys(const unsigned long long* keys, int64_t stride, int j, int nq, float* tau,
-                                  hipStream_t stream) {
-    hipLaunchKernelGGL(bound_from_keys_kernel, dim3((nq + 255) / 256), dim3(256), 0, stream, keys, stride, j, nq, tau);
     return hipGetLastError();
 }
 
