@@ -392,8 +392,12 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
             while (slots_log2 > 12 && lds_table(p.big, slots_log2, min_cap) > lds_max) --slots_log2;
         }
     } else if (slots_log2 == 0) {
-        // best-first on this kernel: about 31 first visits per beam entry, 48 cells
-        if (p.big && bitmap_possible && lds_bitmap(true, min_cap) <= lds_max) {
+        // best-first on this kernel: about 31 first visits per beam entry, 48 cells; the bitmap where the batch leaves
+        // every CU one or two workgroups and it fits as often (L = 128, 97 queries on 200 000 x 200: 847 -> 698 us)
+        const size_t per_cu = ((size_t)Q + idx->num_cu - 1) / idx->num_cu;
+        const bool few = any_form && !p.big && t.workgroups == 0 && per_cu <= 2 && bitmap_possible &&
+                         per_cu * lds_bitmap(false, min_cap) <= lds_max;
+        if (few || (p.big && bitmap_possible && lds_bitmap(true, min_cap) <= lds_max)) {
             p.direct = 1;
         } else {
             slots_log2 = 12;
@@ -552,7 +556,16 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     // (measured at a million nodes: the two forms cross between L = 1024 and 1536)
     const bool long_form = best_first && !t.best_first_in_lds &&
                            (t.best_first_long > 0 || (t.best_first_long == 0 && L > kLongBeamFrom));
-    const bool wave_form = best_first && !t.best_first_in_lds && !long_form && !plan.big &&
+    // A step of a lone wavefront is bound by its own instructions.  Where the batch leaves every CU one or two queries,
+    // rows are wide and the visited ids fit a bitmap, the four wavefronts of the workgroup-per-query kernel share them
+    // (97 / 512 queries, wavefront against workgroup: 200 000 x 200, L = 128: 888 / 1034 -> 698 / 802 us, L = 512:
+    // 2591 / 2648 -> 2411 / 2484; 100 000 x 512, L = 256: 1501 / 1514 -> 1185 / 1262; at 96 floats the wavefront stays
+    // ahead: 536 / 555 against 561 / 590).  A caller who names any part of the launch keeps the wavefronts.
+    const bool named = t.visited_slots_log2 || t.workgroups || t.threads || t.best_first_packed || t.best_first_table_log2 ||
+                       t.beam_in_hbm || t.cand_cap || t.best_first_long || t.best_first_buffer || t.screening ||
+                       t.visited_choices || t.prefetch_rows;
+    const bool shared_steps = best_first && !named && idx->dim / 4 > 32 && Q <= 2 * idx->num_cu && plan.direct && !plan.big;
+    const bool wave_form = best_first && !t.best_first_in_lds && !long_form && !plan.big && !shared_steps &&
                            coral::best_first_wave_lds_bytes(L, 0, 0) * 4 <= (size_t)kMaxLdsBytes;
     // rows of 68 .. 128 floats are screened (on codes) only when the caller asks for it by name; the coded query then
     // takes the LDS a table of visited ids would fill

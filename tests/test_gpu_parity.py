@@ -71,6 +71,28 @@ def test_batches_of_few_queries_take_another_launch_and_give_the_same(n, dim, R,
     idx.close()
 
 
+@pytest.mark.parametrize("n,dim,metric,L", [(9000, 128, "l2", 64), (9000, 132, "l2", 16), (33000, 200, "ip", 700)])
+def test_few_best_first_queries_share_a_step_between_wavefronts(n, dim, metric, L):
+    """Up to two queries per CU on rows of more than 128 floats run in workgroups; narrower rows, larger batches and
+    launches the caller names run a wavefront per query.  Ids, distance bits and counters are the same."""
+    import torch
+    base, nbrs, starts = problem(n, dim, 32, 22, metric)
+    few = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    q = synth.shifted_queries(few + 1, dim, 5, 6, 7)
+    idx = capi.Index(base, nbrs, starts, capi.IP if metric == "ip" else capi.L2)
+    want = None
+    for Q, kw in ((few + 1, {}), (few, dict(best_first_packed=True)), (few, {}), (1, {})):
+        idx.prepare(Q, L, policy=capi.POLICY_BEST_FIRST, **kw)
+        assert idx.plan_info().kernel == (0 if Q <= few and not kw and dim > 128 else 1)
+        ids, dists, _ = idx.search(q[:Q], 10, L, policy=capi.POLICY_BEST_FIRST)
+        cnt = idx.query_counters(Q)
+        if want is None:
+            want = ids, dists, cnt
+        assert np.array_equal(ids, want[0][:Q]) and np.array_equal(cnt, want[2][:Q])
+        assert dists.tobytes() == want[1][:Q].tobytes()
+    idx.close()
+
+
 CASES = [
     # n, dim, R, metric, policy, L, k, M, ragged, slots_log2, threads
     (20000, 200, 32, "l2", 0, 64, 10, 16, None, 0, 0),
