@@ -102,6 +102,10 @@ def test_bruteforce_exact_against_oracle(orc, n, dim, Q, k, metric, tomb):
     (9000, 20, 257, 33, "ip", "plain"),        # a second query tile of one
     (20483, 36, 1025, 10, "l2", "plain"),      # two passes over the base with a tightened bound
     (20483, 24, 1024, 100, "ip", "plain"),
+    (9000, 24, 40, 128, "l2", "plain"),        # 160 kept candidates: the last that 256 threads select
+    (9000, 24, 40, 129, "l2", "plain"),
+    (9000, 24, 4097, 5, "ip", "plain"),        # a second block of queries, of one
+    (9000, 24, 2049, 5, "l2", "plain"),        # a second piece of the sample, of one
     (20483, 24, 1024, 10, "l2", "row_scales"),  # rows from 1e-12 to 1e12 in one base
     (20483, 24, 300, 10, "ip", "row_scales"),
     (8500, 24, 130, 10, "l2", "tiny"),         # squared norms at the end of the range: scales are clamped
