@@ -384,7 +384,7 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
             p.direct = 1;  // no workgroup per CU less for it: the bitmap is the cheaper test and cannot overflow
             // (the LDS a smaller bitmap leaves over goes unused: a list of 1024 instead of 512 costs the 512-float
             // search at L = 256 1 %, see below)
-            if (smaller && !alone) plan_words = (1 << want) >> 1;
+            if (smaller && !alone && !table_alone_on_cu) plan_words = (1 << want) >> 1;
         } else if (bitmap_possible && !table_holds && !lds_beam_only && lds_bitmap(true, 1024) <= lds_max) {
             p.direct = 1, p.big = true;  // the beam gives its LDS to the bitmap (measured: +30 % at L = 1024 and 2048)
         } else {
@@ -487,8 +487,11 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     int workgroups = t.workgroups > 0 ? t.workgroups : wg_per_cu * idx->num_cu;
     p.workgroups = std::min(workgroups, (int)Q);
     p.tcap = tcap, p.ccap = ccap, p.threads = threads, p.id_bits = id_bits, p.ocap = ocap;
-    // graph rows a chunk ahead: pays where a workgroup is alone on its CU (nothing else covers the wait)
-    p.prefetch = t.prefetch_rows > 0 || (t.prefetch_rows == 0 && (wg_per_cu == 1 || alone) && !best_first);
+    // graph rows a chunk ahead: pays where a workgroup is alone on its CU (nothing else covers the wait), and where no
+    // workgroup has a second query (257 .. 512 on 200 000 x 200: 2 % at L = 32, 4 % at L = 128, 5 % at L = 1024; 0 .. 3 %
+    // at 512 floats); 1024 queries of 512 floats lose up to 4 %, a full batch 5 % and more
+    p.prefetch = t.prefetch_rows > 0 ||
+                 (t.prefetch_rows == 0 && !best_first && (wg_per_cu == 1 || (int64_t)Q <= 2 * (int64_t)idx->num_cu));
     p.beam_stride = p.big ? coral::search_beam_stride(L) : 0;
     *out = p;
     return CORAL_OK;
