@@ -10,10 +10,10 @@
 //
 // Here one workgroup owns one cluster: the member-pair distances are computed once into LDS (every pivot of the
 // cluster reuses them), and one wavefront per pivot keeps its candidate list in LDS from assembly to the final
-// row: rank-by-counting sort, occlusion loop with the later candidates spread over the lanes, ballot-prefix
-// emission.  Only distances to a pivot's current neighbours are evaluated on the fly.  Every distance is the
-// sequential fp32 chain of include/utils.cuh:254-275 / :307-323, so rows are bit-identical to a CPU statement
-// of the same rules.
+// row: rank-by-counting sort, occlusion rule, ballot-prefix emission.  Distances to a pivot's current neighbours are
+// only compared, never stored: they come from the matrix cores with an error bound, and comparisons inside the bound
+// are decided by the sequential fp32 chain of include/utils.cuh:254-275 / :307-323.  Every stored distance is that
+// chain, so rows are bit-identical to a CPU statement of the same rules.
 //
 // Two outcomes that the reference leaves to thread timing are fixed: ties of the sort keep column order (its
 // cub::DeviceSegmentedSort::SortPairs is not stable), and a base id that several clusters of one batch contain
