@@ -376,12 +376,15 @@ __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ q
         }
     }
     if (tid == 0) {
-        int bad = 0;
-        // every live point is a candidate unless the list is full; a full list vouches for the k best only if the
-        // k-th of them lies clear of the worst candidate's approximate distance
-        if (cand_ids[(size_t)q * kc + kc - 1] >= 0) {
+        // Where |q|^2 + |b|^2 is infinite or NaN, or twice it is, approximate distances may be so too: such points were
+        // dropped like tombstoned ones, and a list that is not full says nothing.
+        const float n2 = qn[q] + __uint_as_float(*bn_max_bits);
+        int bad = !(n2 <= 1.5e38f);
+        // otherwise every live point is a candidate unless the list is full; a full list vouches for the k best only if
+        // the k-th of them lies clear of the worst candidate's approximate distance
+        if (!bad && cand_ids[(size_t)q * kc + kc - 1] >= 0) {
             const float worst = cand_d[(size_t)q * kc + kc - 1];
-            const float delta = 8.0f * (float)(dim + 4) * 5.9604645e-8f * (qn[q] + __uint_as_float(*bn_max_bits));
+            const float delta = 8.0f * (float)(dim + 4) * 5.9604645e-8f * n2;
             const unsigned long long kth = rkeys[k - 1];
             const float sk = mf_unord32((uint32_t)(kth >> 32));
             if (kth == ~0ull || !(sk < worst - delta)) bad = 1;

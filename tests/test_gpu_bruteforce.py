@@ -134,6 +134,34 @@ def test_screening_on_split_halves_at_the_edges_of_its_tiles(orc, n, dim, Q, k, 
     assert dists.tobytes() == od.tobytes()
 
 
+@pytest.mark.parametrize("n,dim,Q,k,metric,scale_q,scale_b,redone", [
+    (9000, 24, 40, 10, "l2", 1e18, 1.0, "all"),     # finite norms beyond a power of two of 2^-40 for the halves
+    (20483, 24, 1030, 10, "ip", 1e18, 1.0, "all"),  # (two passes over the base)
+    (9000, 24, 40, 10, "ip", 1e20, 1.0, "all"),     # |q|^2 overflows, every product is finite
+    (9000, 24, 40, 10, "ip", 1.0, 1e20, "all"),     # |b|^2 overflows for every point
+    (9000, 24, 40, 10, "l2", 1e17, 1e17, "few"),    # the screening vouches: its products are right at this scale
+    (9000, 24, 40, 10, "ip", 1e18, 1e18, "few"),
+    (9000, 24, 40, 10, "l2", 7e17, 7e17, "few"),
+])
+def test_screening_answers_for_large_magnitudes(orc, n, dim, Q, k, metric, scale_q, scale_b, redone):
+    """Every component is finite and so is every distance: k neighbours, the oracle's, whatever the screening can
+    vouch for.  Fused screening, screening through the matrix and the exact passes alike."""
+    m = capi.IP if metric == "ip" else capi.L2
+    base = synth.gaussian_matrix(n, n, dim) * np.float32(scale_b)
+    q = synth.shifted_queries(Q, dim, 13, 14, 15) * np.float32(scale_q)
+    oi, od = orc.bruteforce(base, q, k, m, order=SEQ)
+    assert np.isfinite(od).all() and (oi >= 0).all()
+    idx = capi.Index(base, None, None, m)
+    for mode in (0, 2, 1):
+        idx.bruteforce_exact_only(mode)
+        ids, dists, _ = idx.bruteforce(q, k)
+        assert np.array_equal(ids, oi) and dists.tobytes() == od.tobytes(), "mode %d" % mode
+        if mode != 1:
+            count = idx.bruteforce_last_redone()
+            assert count == Q if redone == "all" else count <= Q // 4
+    idx.close()
+
+
 def test_randomised_knn_problems_equal_the_oracle(orc):
     """Seeded random sizes, k, metrics, tombstones and laws of the data (ties on a lattice, repeated vectors, large
     and small magnitudes, a common offset that makes the screening's error bound bite): the screened path and the
