@@ -176,8 +176,12 @@ __device__ __forceinline__ void prune_members(WaveCands& S, int m, int lane, int
 // dot: the inner product of the two from split halves, n2: the sum of their squared norms.  The answer is certain where
 // it lies beyond +- slack * n2 + 1e-36: the reference-order distance is within 8 (dim + 8) u n2 of n2 - 2 dot (L2:
 // twice the bound of mfma_split.h, the norms', the reference order's and this difference's own rounding), the
-// reference-order product within half that of dot; 1e-36 covers what underflow adds.  Infinities and NaN are certain
-// of nothing.
+// reference-order product within half that of dot; 1e-36 covers what underflow adds.  A NaN is certain of nothing.
+//
+// dj may be infinite, and so may the distance measured here, of which finite norms say nothing: two rows a and b need
+// |a|^2 + |b|^2 of 2^127 or more for that, so one of them has a squared norm of 2^126 and, with at most 2048 floats, a
+// component of 2^57.5.  kLeastScale leaves that component beyond 65 504: dot is NaN, and the chain decides.
+constexpr int kLeastScale = -40;
 template <bool L2>
 __device__ __forceinline__ float margin(float dj, float dot, float n2) { return L2 ? fmaf(2.0f, dot, dj - n2) : dot - dj; }
 
@@ -205,7 +209,7 @@ __device__ __forceinline__ void prune_any(WaveCands& S, int m, int lane, const f
         const int32_t idj = S.id[valid ? j : j0];
         const int32_t idr = nbr_num > 0 ? S.ret[min(l, nbr_num - 1)] : idj;
         const float nj = norms[idj], nr = norms[idr], dj = S.dist[valid ? j : j0];
-        const int ej = mf_scale_exp(nj), er = mf_scale_exp(nr);
+        const int ej = mf_scale_exp<kLeastScale>(nj), er = mf_scale_exp<kLeastScale>(nr);
         const float sj = mf_pow2(ej), sr = mf_pow2(er), usj = mf_pow2(-ej), usr = mf_pow2(-er);
         if (kh == 0) {
             reinterpret_cast<float*>(S.rows[0][0])[l] = nr, reinterpret_cast<float*>(S.rows[0][1])[l] = usr;

@@ -17,13 +17,15 @@ namespace coral {
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-// e with |x| 2^e in [2^13, 2^14) for a row of squared norm n2; at least -51, which every finite norm stays above, so that
-// no component of such a row leaves the range of a half and no product of two inverse scales overflows; at most 60, which
-// rows of norm 0 and of norms whose square leaves the normal range meet.  A row whose squared norm is infinite or NaN has
-// products that may be NaN, which pass no comparison: callers must not take the absence of such a row for an answer.
+// e with |x| 2^e in [2^13, 2^14) for a row of squared norm n2; at most 60, which rows of norm 0 and of norms whose square
+// leaves the normal range meet; at least kLeast.  -51 is what no finite norm falls below, so that no component of such a
+// row leaves the range of a half and no product of two inverse scales overflows.  A row whose squared norm is infinite or
+// NaN, or that a larger kLeast leaves with a component beyond 65 504, has hi = inf and lo = -inf there, and every product
+// with it is NaN, which passes no comparison: callers must not take the absence of such a row for an answer.
+template <int kLeast = -51>
 __device__ __forceinline__ int mf_scale_exp(float n2) {
     const int E = (int)((__float_as_uint(n2) >> 23) & 0xffu) - 127;  // n2 in [2^E, 2^(E+1))
-    return max(-51, min(60, 13 - (E >> 1)));
+    return max(kLeast, min(60, 13 - (E >> 1)));
 }
 __device__ __forceinline__ float mf_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 

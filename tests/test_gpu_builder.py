@@ -139,6 +139,41 @@ def test_pruning_on_matrix_core_products_equals_the_oracle(orc, dim, R, kn, metr
     idx.close()
 
 
+def test_pruning_of_a_found_list_whose_distances_overflow(orc):
+    """Two groups of linked nodes, opposite each other, and isolated nodes to the side of both: every norm and every sum
+    of two linked nodes' squared norms is finite, the distances between the groups and to the isolated nodes are not.
+    Within a group a neighbour rules the others out; a node of the other group, as infinitely far, is kept."""
+    dim, R, kb, kn, each, n_iso = 24, 16, 30, 64, 240, 70
+    n = 2 * each + n_iso
+    base = synth.gaussian_matrix(31, n, dim) * np.float32(1e17)
+    base[:each, 0] += np.float32(1.1e19)
+    base[each:2 * each, 0] -= np.float32(1.1e19)
+    base[2 * each:, 1] += np.float32(1.6e19)
+    idx = capi.Index(base, None, None)
+    idx.build_begin(R)
+    st = orc.GraphState(n, R)
+    rng = np.random.RandomState(4)
+    for it in range(2):
+        knn = np.concatenate([rng.permutation(each).reshape(-1, kb) + g * each for g in (0, 1)]).astype(np.int32)
+        t_knn = dev(knn)
+        idx.build_nap_batch(t_knn.data_ptr(), knn.shape[0], kb, 1)
+        orc.nap_batch(base, st, knn, need_discard=1)
+    assert np.isfinite(st.dists).all() and (st.deg[:2 * each] > 0).all()
+    assert_same_state(idx, st)
+    # 40 nodes of the first group, then 24 of the second, all at an infinite distance
+    ids = np.stack([np.concatenate([rng.permutation(each)[:40], each + rng.permutation(each)[:24]]) for _ in range(n_iso)])
+    ids = ids.astype(np.int32)
+    iso = np.arange(2 * each, n, dtype=np.int32)
+    dd = np.full((n_iso, kn), np.inf, np.float32)
+    t_iso, t_ids, t_dd = dev(iso), dev(ids), dev(dd)
+    ins, rej = idx.build_enhance_batch(t_iso.data_ptr(), t_ids.data_ptr(), t_dd.data_ptr(), n_iso, kn)
+    stats = orc.enhance_batch(base, st, iso, ids, dd)
+    assert (ins, rej) == (stats[0], stats[1])
+    assert_same_state(idx, st)
+    assert (st.nbrs[iso] >= each).any(1).all()
+    idx.close()
+
+
 def test_randomised_shapes_of_both_steps_equal_the_oracle(orc):
     """Seeded random sizes, widths, cluster sizes, metrics and fill modes, small enough for the oracle; each case
     runs a few batch updates and one enhancement batch."""
