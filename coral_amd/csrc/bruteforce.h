@@ -39,7 +39,7 @@ hipError_t launch_approx_filter(const void* queries, const float* base, int nq, 
 hipError_t launch_list_select(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, int32_t* ids,
                               float* dists, int* overflow, hipStream_t stream);
 // the same selection in place, between two launches that append: the list shrinks to its k smallest keys, tau[q]
-// becomes the value of the k-th (+inf if there are fewer)
+// becomes the value of the k-th (and stays what it was if there are fewer)
 hipError_t launch_list_shrink(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, float* tau,
                               int* overflow, hipStream_t stream);
 // cand_ids / cand_d [nq][kc] (ascending approximate signed distance, -1 = none) -> the exact k best per query in the

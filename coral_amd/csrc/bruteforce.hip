@@ -275,7 +275,9 @@ __global__ __launch_bounds__(T) void row_select_kernel(const float* __restrict__
 // the k-th smallest key from above, a second pass collects what lies up to it, a sort finishes.  *overflow is raised
 // when a list lost entries (cnt[q] > cap) or the collection outgrows LDS; the caller then takes another path.
 // The result goes out as ids (-1: none) and values; SHRINK: it replaces the list and its count, and tau[q] becomes the
-// value of the k-th key.
+// value of the k-th key -- or stays, where the list has fewer: the bound that let them through holds for the whole row
+// whether its k smallest lie in the tiles seen so far or not.  (Without it every entry of the tiles to come would pass;
+// of a base stored cluster by cluster a few queries in a hundred meet this.)
 template <int T, bool SHRINK>
 __global__ __launch_bounds__(T) void list_select_kernel(unsigned long long* __restrict__ lists, int64_t cap,
                                                         unsigned int* __restrict__ cnt, int k, int32_t* __restrict__ ids,
@@ -340,7 +342,7 @@ __global__ __launch_bounds__(T) void list_select_kernel(unsigned long long* __re
         for (int i = tid; i < kk; i += T) list[i] = skeys[i];
         if (tid == 0) {
             cnt[(size_t)blockIdx.x * kCntStride] = (unsigned)kk;
-            tau[blockIdx.x] = kk == k ? bf_unord32((uint32_t)(skeys[k - 1] >> 32)) : __int_as_float(0x7f800000);
+            if (kk == k) tau[blockIdx.x] = bf_unord32((uint32_t)(skeys[k - 1] >> 32));
         }
     } else {
         for (int i = tid; i < k; i += T) {

@@ -291,6 +291,33 @@ def test_bruteforce_candidate_lists_that_overflow_go_through_the_matrix(orc):
     idx.close()
 
 
+def clustered(n, dim, size, Q, seed):
+    """Clusters of `size` consecutive rows, well apart, and queries that belong to one each."""
+    centres = 3.0 * synth.gaussian_matrix(seed, (n + size - 1) // size, dim)
+    base = np.repeat(centres, size, axis=0)[:n] + synth.gaussian_matrix(seed + 1, n, dim)
+    own = np.random.RandomState(seed).randint(0, centres.shape[0], Q)
+    q = centres[own] + synth.gaussian_matrix(seed + 2, Q, dim)
+    return base.astype(np.float32), q.astype(np.float32)
+
+
+@pytest.mark.parametrize("n,size,Q", [
+    (300000, 200, 1024),  # two passes whose first takes every 4th tile, after a sample of every 18th
+    (20000, 64, 1024),    # every 4th and every 19th; clusters of half a tile
+])
+def test_two_screening_passes_over_a_base_stored_cluster_by_cluster(orc, n, size, Q):
+    """The tiles of the first pass are not those of the sample: it may meet nothing of the cluster that a query's bound
+    came from.  The bound still holds, and no list overflows."""
+    dim, k = 16, 10
+    base, q = clustered(n, dim, size, Q, 900)
+    idx = capi.Index(base, None, None)
+    ids, dists, _ = idx.bruteforce(q, k)
+    fused = idx.bruteforce_last_fused()
+    idx.close()
+    oi, od = orc.bruteforce(base, q, k, order=SEQ)
+    assert np.array_equal(ids, oi) and dists.tobytes() == od.tobytes()
+    assert fused == 1
+
+
 def test_bruteforce_segments(orc):
     # more base points than one pass holds (4M): per-segment winners are merged
     n, dim, Q, k = 5 * 1000 * 1000, 8, 40, 50
