@@ -174,9 +174,10 @@ __device__ __forceinline__ void prune_members(WaveCands& S, int m, int lane, int
 
 // By how much is the candidate at (exact) distance dj from the pivot closer to another candidate than to the pivot?
 // dot: the inner product of the two from split halves, n2: the sum of their squared norms.  The answer is certain where
-// it lies beyond +- slack * n2 + 1e-36: the reference-order distance is within 8 (dim + 8) u n2 of n2 - 2 dot (L2:
-// twice the bound of mfma_split.h, the norms', the reference order's and this difference's own rounding), the
-// reference-order product within half that of dot; 1e-36 covers what underflow adds.  A NaN is certain of nothing.
+// it lies beyond +- slack * n2 + 1e-36.  L2: n2 - 2 dot is within (6 dim + 12) u n2 (mfma_split.h) and dim u n2 (the norms)
+// of the true distance; the reference-order one within (dim + 2) u of that, which is up to 2 n2; this difference's own
+// rounding adds 4 u: (9 dim + 20) u n2 in all, and slack is 10 (dim + 8) u.  Inner product: (3 dim + 6) u n2 and half a
+// dim u n2 for the reference order, and slack is 4 (dim + 8) u.  1e-36 covers what underflow adds.  A NaN is certain of nothing.
 //
 // dj may be infinite, and so may the distance measured here, of which finite norms say nothing: two rows a and b need
 // |a|^2 + |b|^2 of 2^127 or more for that, so one of them has a squared norm of 2^126 and, with at most 2048 floats, a
@@ -201,7 +202,7 @@ __device__ __forceinline__ void prune_any(WaveCands& S, int m, int lane, const f
                           int dim, int R) {
     constexpr int metric = L2 ? CORAL_L2 : CORAL_IP;
     const int l = lane & 31, kh = lane >> 5;
-    const float slack = (L2 ? 8.0f : 4.0f) * (float)(dim + 8) * 5.9604645e-8f;
+    const float slack = (L2 ? 10.0f : 4.0f) * (float)(dim + 8) * 5.9604645e-8f;
     int nbr_num = 0;
     for (int j0 = 0; j0 < m && nbr_num < R; j0 += 32) {
         const int cnt = min(32, m - j0), j = j0 + l;

@@ -162,6 +162,24 @@ def test_screening_answers_for_large_magnitudes(orc, n, dim, Q, k, metric, scale
     idx.close()
 
 
+@pytest.mark.parametrize("metric", ["l2", "ip"])
+def test_screening_of_distances_below_the_normal_range(orc, metric):
+    """Products and squares of a few units of 2^-149: the reference order rounds each of them, the screening rounds
+    their sum, and the two differ by more than neighbouring ranks do."""
+    n, dim, Q, k = 9000, 24, 40, 200
+    base = synth.gaussian_matrix(n, n, dim) * np.float32(5e-23)
+    q = synth.shifted_queries(Q, dim, 13, 14, 15) * np.float32(5e-23)
+    m = capi.IP if metric == "ip" else capi.L2
+    oi, od = orc.bruteforce(base, q, k, m, order=SEQ)
+    assert 0.0 < np.abs(od).max() < 1.2e-38
+    idx = capi.Index(base, None, None, m)
+    for mode in (0, 2, 1):
+        idx.bruteforce_exact_only(mode)
+        ids, dists, _ = idx.bruteforce(q, k)
+        assert np.array_equal(ids, oi) and dists.tobytes() == od.tobytes(), "mode %d" % mode
+    idx.close()
+
+
 def test_randomised_knn_problems_equal_the_oracle(orc):
     """Seeded random sizes, k, metrics, tombstones and laws of the data (ties on a lattice, repeated vectors, large
     and small magnitudes, a common offset that makes the screening's error bound bite): the screened path and the
