@@ -106,7 +106,11 @@ def test_bruteforce_exact_against_oracle(orc, n, dim, Q, k, metric, tomb):
     (9000, 24, 40, 129, "l2", "plain"),
     (9000, 24, 4097, 5, "ip", "plain"),        # a second block of queries, of one
     (9000, 24, 2049, 5, "l2", "plain"),        # a second piece of the sample, of one
-    (20483, 24, 1024, 10, "l2", "row_scales"),  # rows from 1e-12 to 1e12 in one base
+    (20483, 24, 4097, 5, "l2", "plain"),       # both, in two passes over the base
+    (20483, 24, 2049, 5, "ip", "plain"),
+    (20483, 24, 1024, 10, "l2", "spread"),     # rows from 0.1 to 10 in one base, each on a scale of its own
+    (20483, 24, 300, 10, "ip", "spread"),
+    (20483, 24, 1024, 10, "l2", "row_scales"),  # rows from 1e-12 to 1e12: nothing can be vouched for
     (20483, 24, 300, 10, "ip", "row_scales"),
     (8500, 24, 130, 10, "l2", "tiny"),         # squared norms at the end of the range: scales are clamped
     (8500, 24, 130, 10, "ip", "tiny"),
@@ -121,6 +125,8 @@ def test_screening_on_split_halves_at_the_edges_of_its_tiles(orc, n, dim, Q, k, 
     rs = np.random.RandomState(n)
     if law == "row_scales":
         base *= (10.0 ** rs.uniform(-12, 12, (n, 1))).astype(np.float32)
+    elif law == "spread":
+        base *= (10.0 ** rs.uniform(-1, 1, (n, 1))).astype(np.float32)
     elif law == "tiny":
         base *= np.float32(1e-19)
         q *= np.float32(1e-19)
@@ -128,10 +134,13 @@ def test_screening_on_split_halves_at_the_edges_of_its_tiles(orc, n, dim, Q, k, 
         base[n // 2] *= np.float32(1e20)
     idx = capi.Index(base, None, None, m)
     ids, dists, _ = idx.bruteforce(q, k)
+    redone, fused = idx.bruteforce_last_redone(), idx.bruteforce_last_fused()
     idx.close()
     oi, od = orc.bruteforce(base, q, k, m, order=SEQ)
     assert np.array_equal(ids, oi)
     assert dists.tobytes() == od.tobytes()
+    # (in 64 bits, no query of the other laws comes within the error bound of its last candidate)
+    assert fused == 1 and redone == (Q if law in ("row_scales", "huge_row") else 0)
 
 
 @pytest.mark.parametrize("n,dim,Q,k,metric,scale_q,scale_b,redone", [
