@@ -159,9 +159,9 @@ __global__ __launch_bounds__(256) void distance_tile_kernel(const float* __restr
 // keys ord32(value) << 32 | (id0 + index).  Fewer than k finite entries: padded with ~0.
 // Entries equal to +inf (tombstones) never win over finite ones and are dropped at the end.
 //
-// row_select_kernel is the fast path.  Every thread keeps the smallest value of the entries it reads; the k-th
-// smallest of those 1024 minima is a value that at least k entries of the row do not exceed (the minima are
-// distinct entries), and in a row of independent values hardly more than k do (about k + k^2/2048).  A second pass
+// row_select_kernel is the fast path.  Each of T threads keeps the smallest value of the entries it reads; the k-th
+// smallest of those T minima is a value that at least k entries of the row do not exceed (the minima are
+// distinct entries), and in a row of independent values hardly more than k do (about k + k^2/2T).  A second pass
 // collects the entries up to that value into LDS, a sort by (value, index) finishes.  Two coalesced reads of the
 // row, no atomics on the way.  A row with so many ties at the threshold that the candidates outgrow LDS is
 // flagged and left to row_select_radix_kernel, which makes no such assumption.
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(T) void row_select_kernel(const float* __restrict__
     smin[tid] = m;
     if (tid == 0) s_count = 0u;
     __syncthreads();
-    // the kk-th smallest of the minima: bitonic sort of 1024 values
+    // the kk-th smallest of the minima: bitonic sort of T values
     for (int k2 = 2; k2 <= T; k2 <<= 1)
         for (int j = k2 >> 1; j > 0; j >>= 1) {
             if (tid < T / 2) {

@@ -337,8 +337,11 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     // the time of the launch is the longest query's chain of waits.  Such launches take 1024 threads, the bitmap
     // wherever it fits and the look-ahead.  One query / 64 queries / 256 queries, before and after: 100 000 x 128,
     // L = 64: 89 / 108 / 113 -> 64 / 75 / 79 us; 200 000 x 200, L = 128: 176 / 201 / 217 -> 117 / 141 / 158;
-    // 200 000 x 512, inner product, L = 256: 768 / 807 / 849 -> 360 / 403 / 640.  With 400 queries 1024 threads would
-    // cost 25 to 30 %, and going without the screening costs 12 % and more at every size.
+    // 200 000 x 512, inner product, L = 256: 768 / 807 / 849 -> 360 / 403 / 640.  A bitmap of a million ids, 125 KB, is
+    // still the better form: 1M x 200, L = 64: 120 / 150 / 161 -> 89 / 116 / 125, L = 256: 403 / 432 / 453 -> 230 / 258 /
+    // 288 (from L = 512 on it stood before); 1M x 512, inner product, L = 128: 334 / 380 / 445 -> 221 / 282 / 385;
+    // 1.2M x 96, L = 128: 250 / 271 / 289 -> 181 / 204 / 222.  With 400 queries 1024 threads would cost 25 to 30 %, and
+    // going without the screening costs 12 % and more at every size.
     const bool alone = !best_first && t.workgroups == 0 && t.cand_cap == 0 && Q <= idx->num_cu;
     const bool any_form = t.visited_choices == 0;  // (a caller who names a form of the table gets a table)
     // ---- the visited structure.  Three forms: a table of 2^s 16-bit cells with an overflow bitmap in global memory
@@ -489,7 +492,7 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     p.tcap = tcap, p.ccap = ccap, p.threads = threads, p.id_bits = id_bits, p.ocap = ocap;
     // graph rows a chunk ahead: pays where a workgroup is alone on its CU (nothing else covers the wait), and where no
     // workgroup has a second query (257 .. 512 on 200 000 x 200: 2 % at L = 32, 4 % at L = 128, 5 % at L = 1024; 0 .. 3 %
-    // at 512 floats); 1024 queries of 512 floats lose up to 4 %, a full batch 5 % and more
+    // at 512 floats and on a million nodes); 1024 queries of 512 floats lose up to 4 %, a full batch 5 % and more
     p.prefetch = t.prefetch_rows > 0 ||
                  (t.prefetch_rows == 0 && !best_first && (wg_per_cu == 1 || (int64_t)Q <= 2 * (int64_t)idx->num_cu));
     p.beam_stride = p.big ? coral::search_beam_stride(L) : 0;
@@ -562,8 +565,11 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     // A step of a lone wavefront is bound by its own instructions.  Where the batch leaves every CU one or two queries,
     // rows are wide and the visited ids fit a bitmap, the four wavefronts of the workgroup-per-query kernel share them
     // (97 / 512 queries, wavefront against workgroup: 200 000 x 200, L = 128: 888 / 1034 -> 698 / 802 us, L = 512:
-    // 2591 / 2648 -> 2411 / 2484; 100 000 x 512, L = 256: 1501 / 1514 -> 1185 / 1262; at 96 floats the wavefront stays
-    // ahead: 536 / 555 against 561 / 590).  A caller who names any part of the launch keeps the wavefronts.
+    // 2591 / 2648 -> 2411 / 2484; 100 000 x 512, L = 256: 1501 / 1514 -> 1185 / 1262; just beyond the line, 100 000 x 132,
+    // L = 128: 764 / 777 -> 666 / 720; at 96 floats the wavefront stays ahead: 536 / 555 against 561 / 590).  At a million
+    // nodes LDS holds one bitmap, so the rule ends at one query per CU there (97 / 256 queries: 1M x 200, L = 128:
+    // 992 / 1026 -> 712 / 734, L = 512: 3007 / 3092 -> 2696 / 2699).  A caller who names any part of the launch keeps the
+    // wavefronts.
     const bool named = t.visited_slots_log2 || t.workgroups || t.threads || t.best_first_packed || t.best_first_table_log2 ||
                        t.beam_in_hbm || t.cand_cap || t.best_first_long || t.best_first_buffer || t.screening ||
                        t.visited_choices || t.prefetch_rows;

@@ -177,7 +177,8 @@ __device__ __forceinline__ void prune_members(WaveCands& S, int m, int lane, int
 // it lies beyond +- slack * n2 + 1e-36.  L2: n2 - 2 dot is within (6 dim + 12) u n2 (mfma_split.h) and dim u n2 (the norms)
 // of the true distance; the reference-order one within (dim + 2) u of that, which is up to 2 n2; this difference's own
 // rounding adds 4 u: (9 dim + 20) u n2 in all, and slack is 10 (dim + 8) u.  Inner product: (3 dim + 6) u n2 and half a
-// dim u n2 for the reference order, and slack is 4 (dim + 8) u.  1e-36 covers what underflow adds.  A NaN is certain of nothing.
+// dim u n2 for the reference order, and slack is 4 (dim + 8) u.  1e-36 covers what underflow adds.  A NaN is certain of
+// nothing.
 //
 // dj may be infinite, and so may the distance measured here, of which finite norms say nothing: two rows a and b need
 // |a|^2 + |b|^2 of 2^127 or more for that, so one of them has a squared norm of 2^126 and, with at most 2048 floats, a
@@ -196,7 +197,8 @@ __device__ __forceinline__ float margin(float dj, float dot, float n2) { return 
 // Bound by the gather (two rows of dim * 4 bytes per candidate, from L2 and the memory-side cache).  One lane walking
 // each pair in the reference's order instead, a load of 16 bytes per line and a chain of waits per retained candidate,
 // took 453 us (200 floats, L2) and 3670 us (512 floats, inner product) per 4096 lists of 100 and 132; this takes 120
-// and 284 us.  At 128 registers (four wavefronts per SIMD; 13 spilled) against 168 or 256: 120 / 150 / 150 us.
+// and 291 us.  At 128 registers (four wavefronts per SIMD; 11 to 13 spilled in enh_rows_kernel, 38 in nap_cluster_kernel)
+// against 168 or 256, enh_rows_kernel at 200 floats: 120 / 150 / 150 us.
 template <bool L2>
 __device__ __forceinline__ void prune_any(WaveCands& S, int m, int lane, const float* __restrict__ vec, const float* __restrict__ norms,
                           int dim, int R) {

@@ -262,7 +262,9 @@ CORAL_API int coral_search_verify(coral_index* idx, const int32_t* d_ids_res, co
  * the builder's k_b-NN (src/knn.cu:174-193).  Ordered by (distance, id); every distance is
  * accumulated in dimension order by fused multiply-adds, the arithmetic of
  * include/utils.cuh:254-275 / :307-323.  have_delete leaves tombstoned ids out.  Unfilled
- * slots: id -1, +-FLT_MAX.  The *_gpu form takes device pointers (d_dists may be NULL). */
+ * slots: id -1, +-FLT_MAX.  The *_gpu form takes device pointers (d_dists may be NULL).
+ * Scratch of up to 384 MB is kept with the index for the next call and given back by coral_index_destroy; a call that
+ * needs more allocates its own and frees it before it returns. */
 CORAL_API int coral_bruteforce_knn_gpu(coral_index* idx, const float* d_queries, int32_t Q, int32_t k,
                                        int32_t have_delete, int32_t* d_ids, float* d_dists, void* stream,
                                        double* time_s);
