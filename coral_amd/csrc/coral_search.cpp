@@ -565,15 +565,27 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     // A step of a lone wavefront is bound by its own instructions.  Where the batch leaves every CU one or two queries,
     // rows are wide and the visited ids fit a bitmap, the four wavefronts of the workgroup-per-query kernel share them
     // (97 / 512 queries, wavefront against workgroup: 200 000 x 200, L = 128: 888 / 1034 -> 698 / 802 us, L = 512:
-    // 2591 / 2648 -> 2411 / 2484; 100 000 x 512, L = 256: 1501 / 1514 -> 1185 / 1262; just beyond the line, 100 000 x 132,
-    // L = 128: 764 / 777 -> 666 / 720; at 96 floats the wavefront stays ahead: 536 / 555 against 561 / 590).  At a million
-    // nodes LDS holds one bitmap, so the rule ends at one query per CU there (97 / 256 queries: 1M x 200, L = 128:
-    // 992 / 1026 -> 712 / 734, L = 512: 3007 / 3092 -> 2696 / 2699).  A caller who names any part of the launch keeps the
-    // wavefronts.
+    // 2591 / 2648 -> 2411 / 2484; 100 000 x 512, L = 256: 1501 / 1514 -> 1185 / 1262; at 96 floats the wavefront stays
+    // ahead: 536 / 555 against 561 / 590).  At a million nodes LDS holds one bitmap, so the rule ends at one query per CU
+    // there (97 / 256 queries: 1M x 200, L = 128: 992 / 1026 -> 712 / 734, L = 512: 3007 / 3092 -> 2696 / 2699).
+    // What the wavefronts share are the new rows of a step, and a small graph has few: most neighbours have been seen.
+    // There the barriers of the workgroup cost more than it gains (512 queries, L = 1024: 5000 x 512, inner product,
+    // 1057 -> 1774 us; 8000 x 1024, L2, 1.74 times the wavefront's time; 3000 x 200, 2489 -> 3118).  The inner product
+    // leads a query past more new rows than L2 does.  Workgroup against wavefront, worst of L = 32 .. 1024 and 1 .. 512
+    // queries on either side of the lines below: inner product, 24 000 nodes of 132 / 1536 floats 1.00 / 1.03, 60 000 of
+    // them 0.95 / 0.87; L2, n dim of 14 / 16 million floats 1.05 / 1.01 (single queries at L = 512; the mean of either is
+    // 0.92); 24 000 / 60 000 nodes of 1024 floats 1.10 / 0.96; of 1536 floats 1.05 / 0.85 with up to a query per CU and,
+    // with two, 60 000 / 150 000 nodes 1.12 / 0.95.
+    const int64_t nodes_shared = idx->metric == CORAL_IP ? (int64_t)1 << 15
+                                 : idx->dim <= 512                    ? ((int64_t)1 << 24) / idx->dim
+                                 : idx->dim > 1024 && Q > idx->num_cu ? (int64_t)1 << 17
+                                                                      : (int64_t)1 << 16;
+    // A caller who names any part of the launch keeps the wavefronts.
     const bool named = t.visited_slots_log2 || t.workgroups || t.threads || t.best_first_packed || t.best_first_table_log2 ||
                        t.beam_in_hbm || t.cand_cap || t.best_first_long || t.best_first_buffer || t.screening ||
                        t.visited_choices || t.prefetch_rows;
-    const bool shared_steps = best_first && !named && idx->dim / 4 > 32 && Q <= 2 * idx->num_cu && plan.direct && !plan.big;
+    const bool shared_steps = best_first && !named && idx->dim / 4 > 32 && Q <= 2 * idx->num_cu && idx->n >= nodes_shared &&
+                              plan.direct && !plan.big;
     const bool wave_form = best_first && !t.best_first_in_lds && !long_form && !plan.big && !shared_steps &&
                            coral::best_first_wave_lds_bytes(L, 0, 0) * 4 <= (size_t)kMaxLdsBytes;
     // rows of 68 .. 128 floats are screened (on codes) only when the caller asks for it by name; the coded query then

@@ -71,10 +71,21 @@ def test_batches_of_few_queries_take_another_launch_and_give_the_same(n, dim, R,
     idx.close()
 
 
-@pytest.mark.parametrize("n,dim,metric,L", [(9000, 128, "l2", 64), (9000, 132, "l2", 16), (33000, 200, "ip", 700)])
-def test_few_best_first_queries_share_a_step_between_wavefronts(n, dim, metric, L):
-    """Up to two queries per CU on rows of more than 128 floats run in workgroups; narrower rows, larger batches and
-    launches the caller names run a wavefront per query.  Ids, distance bits and counters are the same."""
+@pytest.mark.parametrize("n,dim,metric,L,shared", [
+    (9000, 128, "l2", 64, False),
+    (9000, 132, "l2", 16, False),        # few nodes: a step finds few new rows
+    (33000, 200, "ip", 700, True),
+    (32767, 132, "ip", 32, False),       # the first number of nodes that shares a step, and one less
+    (32768, 132, "ip", 32, True),
+    (32767, 512, "l2", 64, False),       # L2: 2^24 floats
+    (32768, 512, "l2", 64, True),
+    (65535, 516, "l2", 32, False),       # rows of more than 512 floats, and of more than 1024
+    (65536, 516, "l2", 32, True),
+    (70000, 1028, "l2", 32, None),       # two queries per CU need more nodes than one
+])
+def test_few_best_first_queries_share_a_step_between_wavefronts(n, dim, metric, L, shared):
+    """Up to two queries per CU on rows of more than 128 floats run in workgroups where the graph has nodes enough;
+    narrower rows, smaller graphs, larger batches and launches the caller names run a wavefront per query.  Ids, distance bits and counters are the same."""
     import torch
     base, nbrs, starts = problem(n, dim, 32, 22, metric)
     few = 2 * torch.cuda.get_device_properties(0).multi_processor_count
@@ -83,7 +94,7 @@ def test_few_best_first_queries_share_a_step_between_wavefronts(n, dim, metric, 
     want = None
     for Q, kw in ((few + 1, {}), (few, dict(best_first_packed=True)), (few, {}), (1, {})):
         idx.prepare(Q, L, policy=capi.POLICY_BEST_FIRST, **kw)
-        assert idx.plan_info().kernel == (0 if Q <= few and not kw and dim > 128 else 1)
+        assert idx.plan_info().kernel == (0 if Q <= few and not kw and (Q == 1 if shared is None else shared) else 1)
         ids, dists, _ = idx.search(q[:Q], 10, L, policy=capi.POLICY_BEST_FIRST)
         cnt = idx.query_counters(Q)
         if want is None:
