@@ -492,9 +492,12 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     p.tcap = tcap, p.ccap = ccap, p.threads = threads, p.id_bits = id_bits, p.ocap = ocap;
     // graph rows a chunk ahead: pays where a workgroup is alone on its CU (nothing else covers the wait), and where no
     // workgroup has a second query (257 .. 512 on 200 000 x 200: 2 % at L = 32, 4 % at L = 128, 5 % at L = 1024; 0 .. 3 %
-    // at 512 floats and on a million nodes); 1024 queries of 512 floats lose up to 4 %, a full batch 5 % and more
+    // at 512 floats and on a million nodes); 1024 queries of 512 floats lose up to 4 %, a full batch 5 % and more.  Wider
+    // rows lose at every batch of up to two queries per CU (100 000 nodes of 516, 576, 640 or 768 floats, L = 32 .. 512,
+    // 1 .. 512 queries: 1 to 4 %; 200 000 x 1024, one / 64 / 256 queries at L = 32: 103 / 137 / 145 -> 105 / 141 / 150 us).
     p.prefetch = t.prefetch_rows > 0 ||
-                 (t.prefetch_rows == 0 && !best_first && (wg_per_cu == 1 || (int64_t)Q <= 2 * (int64_t)idx->num_cu));
+                 (t.prefetch_rows == 0 && !best_first &&
+                  ((wg_per_cu == 1 && !alone) || (idx->dim <= 512 && (int64_t)Q <= 2 * (int64_t)idx->num_cu)));
     p.beam_stride = p.big ? coral::search_beam_stride(L) : 0;
     *out = p;
     return CORAL_OK;

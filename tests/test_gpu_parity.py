@@ -46,6 +46,8 @@ def problem(n, dim, R, seed, metric="l2", n_start=16, ragged_seed=None, isolate=
     (9000, 68, 32, "ip", 64, 10, 16),
     (9000, 200, 24, "l2", 300, 100, 16),  # rows that do not divide a pass of 1024 threads
     (33000, 132, 32, "l2", 1100, 50, 7),  # the beam takes more than half of a CU's LDS
+    (9000, 512, 32, "l2", 64, 10, 16),    # the widest rows whose graph rows are requested ahead, and the next
+    (9000, 516, 32, "l2", 64, 10, 16),
 ])
 def test_batches_of_few_queries_take_another_launch_and_give_the_same(n, dim, R, metric, L, k, M):
     """No more queries than CUs: 1024 threads and the bitmap of all ids; one more: what there was before.  Both against
