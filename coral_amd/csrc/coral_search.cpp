@@ -335,14 +335,19 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     p.screen = !screen ? 0 : t.screening > 0 ? t.screening : (codes_possible && (idx->dim <= 1024 || idx->metric != CORAL_L2) ? 2 : 1);
     // A batch of no more queries than the chip has CUs: every workgroup has a CU to itself whatever it takes of it, and
     // the time of the launch is the longest query's chain of waits.  Such launches take 1024 threads, the bitmap
-    // wherever it fits and the look-ahead.  One query / 64 queries / 256 queries, before and after: 100 000 x 128,
+    // wherever it fits and, for rows of up to 512 floats, the look-ahead.  One query / 64 queries / 256 queries, before and after: 100 000 x 128,
     // L = 64: 89 / 108 / 113 -> 64 / 75 / 79 us; 200 000 x 200, L = 128: 176 / 201 / 217 -> 117 / 141 / 158;
     // 200 000 x 512, inner product, L = 256: 768 / 807 / 849 -> 360 / 403 / 640.  A bitmap of a million ids, 125 KB, is
     // still the better form: 1M x 200, L = 64: 120 / 150 / 161 -> 89 / 116 / 125, L = 256: 403 / 432 / 453 -> 230 / 258 /
     // 288 (from L = 512 on it stood before); 1M x 512, inner product, L = 128: 334 / 380 / 445 -> 221 / 282 / 385;
     // 1.2M x 96, L = 128: 250 / 271 / 289 -> 181 / 204 / 222.  With 400 queries 1024 threads would cost 25 to 30 %, and
     // going without the screening costs 12 % and more at every size.
-    const bool alone = !best_first && t.workgroups == 0 && t.cand_cap == 0 && Q <= idx->num_cu;
+    // Under the inner product, which leads a query past two to three times the rows, a full chip of such workgroups on
+    // wide rows is memory's again: the rule ends at seven eighths of the CUs there (224 / 256 queries, L = 256, before and
+    // after: 60 000 x 2048: 3769 / 3935 -> 3635 / 4192 us; 100 000 x 1024: 1081 / 1213 -> 1078 / 1243; L2, 200 000 x 2048:
+    // 3431 / 3506 -> 2477 / 2641).
+    const int most_alone = idx->metric == CORAL_IP && idx->dim > 512 ? idx->num_cu - idx->num_cu / 8 : idx->num_cu;
+    const bool alone = !best_first && t.workgroups == 0 && t.cand_cap == 0 && Q <= most_alone;
     const bool any_form = t.visited_choices == 0;  // (a caller who names a form of the table gets a table)
     // ---- the visited structure.  Three forms: a table of 2^s 16-bit cells with an overflow bitmap in global memory
     // (visited_slots_log2 = s, or the library's choice), or a plain bitmap of all n ids in LDS (visited_slots_log2 =

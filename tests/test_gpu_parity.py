@@ -48,22 +48,24 @@ def problem(n, dim, R, seed, metric="l2", n_start=16, ragged_seed=None, isolate=
     (33000, 132, 32, "l2", 1100, 50, 7),  # the beam takes more than half of a CU's LDS
     (9000, 512, 32, "l2", 64, 10, 16),    # the widest rows whose graph rows are requested ahead, and the next
     (9000, 516, 32, "l2", 64, 10, 16),
+    (9000, 516, 32, "ip", 64, 10, 16),    # inner product on wide rows: up to seven eighths of the CUs
 ])
 def test_batches_of_few_queries_take_another_launch_and_give_the_same(n, dim, R, metric, L, k, M):
-    """No more queries than CUs: 1024 threads and the bitmap of all ids; one more: what there was before.  Both against
+    """No more queries than CUs: 1024 threads and the bitmap of all ids; one more: another launch.  Both against
     a launch whose table, threads and look-ahead the caller names: ids, distance bits and counters are the same."""
     import torch
     base, nbrs, starts = problem(n, dim, R, 21, metric, M)
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     q = synth.shifted_queries(cus + 1, dim, 5, 6, 7)
     idx = capi.Index(base, nbrs, starts, capi.IP if metric == "ip" else capi.L2)
+    most = cus - cus // 8 if metric == "ip" and dim > 512 else cus
     want = None
-    for Q, kw in ((cus + 1, dict(threads=512, visited_slots_log2=13, prefetch_rows=-1)), (cus + 1, {}), (cus, {}), (1, {})):
+    for Q, kw in ((cus + 1, dict(threads=512, visited_slots_log2=13, prefetch_rows=-1)), (most + 1, {}), (most, {}), (1, {})):
         idx.prepare(Q, L, **kw)
         plan = idx.plan_info()
         if not kw:
             assert plan.visited_form == 1
-            assert plan.beam_in_hbm or Q > cus or plan.threads == 1024
+            assert plan.beam_in_hbm or (plan.threads == 1024) == (Q <= most)
         ids, dists, _ = idx.search(q[:Q], k, L)
         cnt = idx.query_counters(Q)
         if want is None:
