@@ -13,13 +13,17 @@
 // accumulation lose), and q.b = hi.hi + hi.lo + lo.hi on v_mfma_f32_32x32x16_f16: three multiplications at sixteen
 // times the rate of the fp32 form.
 //
-// Error bound, with u = 2^-24 and n2 = |q|^2 + |b|^2.  The inner product is within (6 dim + 12) u |q| |b| and enters
-// twice: (6 dim + 12) u n2.  The two norms are within dim u of themselves, the final additions add 4 u n2.  The
-// reference-order distance is within (dim + 2) u of the true one, which is 2 n2 where q and b point apart:
-// (2 dim + 4) u n2.  Together the approximate and the reference-order value of a pair differ by at most (9 dim + 20) u n2,
-// and by 2^-149 for each of these operations whose result leaves the normal range (what the clamped scale of rows shorter
-// than 2^-47 loses is less than either).  For the inner product half of the first and a quarter of the last term are left.
-// The check takes 10 (dim + 4) (u n2 + 2^-149), with the largest |b|^2 of the index.
+// Error bound, with u = 2^-24 and n2 = |q|^2 + |b|^2.
+// L2.  The inner product is within (6 dim + 12) u |q| |b| and enters twice: (6 dim + 12) u n2.  The two norms are within
+// dim u of themselves, the final additions add 3 u n2, and terms of second order come to less than 14 u n2 at 2048
+// dimensions: the approximate distance is within E = (7 dim + 32) u n2 of the true one.  The reference-order distance is
+// within (dim + 2) u of the true one, relative to that.  So a point whose approximate distance is no less than `worst` has
+// a reference-order distance of at least worst - E - (dim + 2) u worst; the check takes (dim + 8) u worst for the last
+// term, which leaves room for its own rounding.
+// Inner product.  (3 dim + 6) u n2 for the product, u n2 / 2 for the last rounding, dim u n2 / 2 for the reference order:
+// the check takes 4 (dim + 8) u n2.
+// Either way 2^-149 is added for each operation whose result may leave the normal range, 10 (dim + 4) of them (what the
+// clamped scale of rows shorter than 2^-47 loses is less), and the largest |b|^2 of the index stands for |b|^2.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -386,7 +390,10 @@ __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ q
         // the k-th of them lies clear of the worst candidate's approximate distance
         if (!bad && cand_ids[(size_t)q * kc + kc - 1] >= 0) {
             const float worst = cand_d[(size_t)q * kc + kc - 1];
-            const float delta = 10.0f * (float)(dim + 4) * (5.9604645e-8f * n2 + 1.4e-45f);
+            const float u = 5.9604645e-8f, un2 = u * n2;
+            const float delta = (metric == 0 ? (float)(7 * dim + 32) * un2 + (float)(dim + 8) * (u * fmaxf(worst, 0.0f))
+                                             : (float)(4 * dim + 32) * un2) +
+                                (float)(10 * dim + 40) * 1.4e-45f;
             const unsigned long long kth = rkeys[k - 1];
             const float sk = mf_unord32((uint32_t)(kth >> 32));
             if (kth == ~0ull || !(sk < worst - delta)) bad = 1;
