@@ -70,6 +70,8 @@ struct BestFirstArgs {
     int32_t rows_in_flight;  // 8, 16 or 32: float4 registers of vector data a lane requests before it adds them up
     int32_t rows_unique;     // no graph row lists an id twice (checked by launch_find_repeated_ids)
     int32_t packed;          // visited is [slots][stride] of 32-bit words, 8 bits of epoch over 24 node flags each
+    int32_t bitmap_words;    // the visited set is a bitmap of all ids in LDS (32-bit words per wavefront, a multiple of 4);
+                             // 0: it is not, and what follows and the state above hold it
     int32_t bloom_log2;      // log2 of the bits of the per-wavefront Bloom filter in LDS, 0 = none
     // first level of the visited set: an exact table of 2^table_log2 16-bit cells per wavefront in LDS (0 = none) in
     // buckets of four; rem_bits = the bits of the mixed id (id_bits wide) that a cell stores, at most 14; what
@@ -84,14 +86,20 @@ struct BestFirstArgs {
     int32_t coded_bytes;
 };
 
-// LDS bytes of one wavefront: a beam of L keys, 32 candidate keys, two lists of 32 ids, L byte counters, a Bloom filter of
-// 2^bloom_log2 bits over the visited ids in HBM (bloom_log2 = 0: none) and a table of 2^table_log2 16-bit cells
-// (table_log2 = 0: none)
-__host__ __device__ inline size_t best_first_wave_lds_bytes(int L, int bloom_log2, int table_log2 = 0, int coded_bytes = 0) {
+constexpr int kMaxWaveBeam = 2048;  // 32 keys per lane
+
+// LDS bytes of one wavefront: two lists of 32 ids, a Bloom filter of 2^bloom_log2 bits over the visited ids in HBM
+// (bloom_log2 = 0: none), a table of 2^table_log2 16-bit cells (table_log2 = 0: none), a bitmap of all ids
+__host__ __device__ inline size_t best_first_wave_lds_bytes(int bloom_log2, int table_log2, int coded_bytes, int bitmap_words) {
     const size_t bloom = bloom_log2 ? ((size_t)1 << bloom_log2) / 8 : 0;
     const size_t table = table_log2 ? (size_t)2 << table_log2 : 0;
-    return ((size_t)((L + 3) & ~3) * 9 + 32 * 8 + 2 * 32 * 4 + bloom + table + (size_t)coded_bytes + 15) & ~(size_t)15;
+    return (2 * 32 * 4 + bloom + table + (size_t)bitmap_words * 4 + (size_t)coded_bytes + 15) & ~(size_t)15;
 }
+// what four wavefronts that share a step exchange beside that: 32 candidate keys, counts, three more lists of 32 ids
+constexpr int kSharedStepBytes = 32 * 8 + 32 + 3 * 32 * 4;
+size_t best_first_shared_lds_bytes(int coded_bytes, int bitmap_words);
+hipError_t best_first_shared_prepare(int dim, int L, int screen, size_t lds, int* max_wg_per_cu);
+hipError_t launch_best_first_shared(const SearchArgs& a, const BestFirstArgs& b, hipStream_t stream);  // slots: workgroups
 // LDS of a wavefront's query in integer codes for the screening on eight-bit rows: two bytes per dimension
 __host__ __device__ inline int coded_query_bytes(int dim) { return 2 * ((dim + 15) & ~15); }
 // the filter size for a beam of L: 128 bits per beam entry rounded up to a power of two, halved while that would leave
@@ -99,12 +107,11 @@ __host__ __device__ inline int coded_query_bytes(int dim) { return 2 * ((dim + 1
 __host__ inline int best_first_bloom_log2(int L, int coded_bytes = 0) {
     int lg = 12;
     while (((size_t)1 << lg) < (size_t)128 * L && lg < 17) ++lg;
-    while (lg >= 12 && best_first_wave_lds_bytes(L, lg, 0, coded_bytes) > (size_t)10 * 1024) --lg;
+    while (lg >= 12 && best_first_wave_lds_bytes(lg, 0, coded_bytes, 0) > (size_t)10 * 1024) --lg;
     return lg >= 12 ? lg : 0;
 }
 // screen: 0 none, 1 rows are first measured in half precision, 2 in eight-bit codes (rows of up to 512 floats)
-hipError_t best_first_prepare(int dim, int L, int rows_in_flight, bool packed, int screen, int bloom_log2,
-                              int table_log2, int* max_wg_per_cu);
+hipError_t best_first_prepare(int dim, int L, int rows_in_flight, int screen, size_t wave_lds, int* max_wg_per_cu);
 hipError_t launch_best_first(const SearchArgs& a, const BestFirstArgs& b, hipStream_t stream);
 // *flag (a device word, zero before) becomes nonzero if a row of nbrs [n][R] holds the same id twice
 hipError_t launch_find_repeated_ids(const int32_t* nbrs, int64_t n, int R, uint32_t* flag, hipStream_t stream);

@@ -450,7 +450,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
 #pragma unroll
                     for (int u = 0; u < U8; ++u)
                         if (r0 + u >= T) vid[u] = -1;
-                    const int mi = r0 + gl8;
+                    const int mi = r0 + (gl8 < U8 ? filed_row<16, U8>(lane) : 0);
                     int myid = (int)list[mi];  // the row this lane files (inside the lists' LDS)
                     if (gl8 >= U8 || mi >= T) myid = -1;
                     const bool valid = myid >= 0;

@@ -228,7 +228,7 @@ __global__ __launch_bounds__(kWavesPerWg * 64, WGS) void best_first_long_kernel(
                         const int r0 = base + grp8 * U8;
 #pragma unroll
                         for (int u = 0; u < U8; ++u) vid[u] = r0 + u < T ? (int)todo[r0 + u] : -1;
-                        const int mi = r0 + gl8;
+                        const int mi = r0 + filed_row<16, U8>(lane);
                         const int myid = (gl8 < U8 && mi < T) ? (int)todo[mi] : -1;  // the row this lane files
                         const bool valid = myid >= 0;
                         float lo, hi;

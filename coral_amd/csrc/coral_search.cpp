@@ -48,14 +48,14 @@ int bf_table_rem_bits(int id_bits, int table_log2) { return std::max(0, id_bits 
 
 // First level of the visited set of the wavefront-per-query best-first kernel: an exact table of 16-bit cells per
 // wavefront in LDS, where one that holds most of a query's first visits (20 to 30 per beam entry) still leaves a CU
-// eight wavefronts -- what the HBM-resident state costs in requests is worth more than the wavefronts given up.
+// fewest_waves wavefronts, eight or more -- what the HBM-resident state costs in requests is worth more than the wavefronts given up.
 // Sixteen wavefronts if 24 cells per entry fit with them, else twelve, else eight with 20 cells per entry; no table
 // (0) for longer beams, or when the ids are wider than a cell can tell apart.  wanted: the caller's
 // coral_tuning.best_first_table_log2.
-int choose_bf_table(int L, int id_bits, int wanted, int* table_log2) {
+int choose_bf_table(int L, int id_bits, int wanted, int coded, int fewest_waves, int* table_log2) {
     *table_log2 = 0;
     if (wanted > 0) {
-        if (wanted < 8 || wanted > 14 || coral::best_first_wave_lds_bytes(L, 0, wanted) * 4 > (size_t)kMaxLdsBytes)
+        if (wanted < 8 || wanted > 14 || coral::best_first_wave_lds_bytes(0, wanted, coded, 0) * 4 > (size_t)kMaxLdsBytes)
             return fail(CORAL_ERR_ARG, "best_first_table_log2 must be in 8..14 and fit LDS with the beam");
         if (bf_table_rem_bits(id_bits, wanted) > 14)
             return fail(CORAL_ERR_ARG, "ids of %d bits do not fit the cells of a 2^%d table", id_bits, wanted);
@@ -64,7 +64,7 @@ int choose_bf_table(int L, int id_bits, int wanted, int* table_log2) {
         const struct { int waves, cells_per_entry; } plans[] = {{16, 24}, {12, 24}, {8, 20}};
         for (const auto& pl : plans)
             for (int lg = 14; lg >= 10 && !*table_log2; --lg)
-                if (coral::best_first_wave_lds_bytes(L, 0, lg) * pl.waves <= (size_t)kMaxLdsBytes &&
+                if (pl.waves >= fewest_waves && coral::best_first_wave_lds_bytes(0, lg, coded, 0) * pl.waves <= (size_t)kMaxLdsBytes &&
                     (1 << lg) >= pl.cells_per_entry * L && bf_table_rem_bits(id_bits, lg) <= 14)
                     *table_log2 = lg;
     }
@@ -570,20 +570,13 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     // (measured at a million nodes: the two forms cross between L = 1024 and 1536)
     const bool long_form = best_first && !t.best_first_in_lds &&
                            (t.best_first_long > 0 || (t.best_first_long == 0 && L > kLongBeamFrom));
-    // A step of a lone wavefront is bound by its own instructions.  Where the batch leaves every CU one or two queries,
-    // rows are wide and the visited ids fit a bitmap, the four wavefronts of the workgroup-per-query kernel share them
-    // (97 / 512 queries, wavefront against workgroup: 200 000 x 200, L = 128: 888 / 1034 -> 698 / 802 us, L = 512:
-    // 2591 / 2648 -> 2411 / 2484; 100 000 x 512, L = 256: 1501 / 1514 -> 1185 / 1262; at 96 floats the wavefront stays
-    // ahead: 536 / 555 against 561 / 590).  At a million nodes LDS holds one bitmap, so the rule ends at one query per CU
-    // there (97 / 256 queries: 1M x 200, L = 128: 992 / 1026 -> 712 / 734, L = 512: 3007 / 3092 -> 2696 / 2699).
-    // What the wavefronts share are the new rows of a step, and a small graph has few: most neighbours have been seen.
-    // There the barriers of the workgroup cost more than it gains (512 queries, L = 1024: 5000 x 512, inner product,
-    // 1057 -> 1774 us; 8000 x 1024, L2, 1.74 times the wavefront's time; 3000 x 200, 2489 -> 3118).  The inner product
-    // leads a query past more new rows than L2 does.  Workgroup against wavefront, worst of L = 32 .. 1024 and 1 .. 512
-    // queries on either side of the lines below: inner product, 24 000 nodes of 132 / 1536 floats 1.00 / 1.03, 60 000 of
-    // them 0.95 / 0.87; L2, n dim of 14 / 16 million floats 1.05 / 1.01 (single queries at L = 512; the mean of either is
-    // 0.92); 24 000 / 60 000 nodes of 1024 floats 1.10 / 0.96; of 1536 floats 1.05 / 0.85 with up to a query per CU and,
-    // with two, 60 000 / 150 000 nodes 1.12 / 0.95.
+    // Four wavefronts per query (best_first_shared.hip), where the batch leaves every CU one or two queries, rows are wide
+    // and a step finds new rows enough to share.  Against a wavefront per query, at L = 32 .. 1000: 70 000 x 1028, inner
+    // product, 1 / 97 / 512 queries 0.47 .. 0.57 / 0.45 .. 0.54 / 0.59 .. 0.69 of the time (such rows are not screened); 1M x 200,
+    // where LDS holds one bitmap per CU but not four, 0.77 .. 0.85 with up to a query per CU; up to 512 floats on fewer
+    // nodes the same time within 5 % for up to a query per CU, but with two each copy of a long beam costs more than the
+    // rows spare (200 000 x 200, 512 queries, L = 32 / 512 / 1000: 0.98 / 1.08 / 1.18), so that case ends at L = 768.  A
+    // graph has nodes enough where a step finds more than a handful of new rows.
     const int64_t nodes_shared = idx->metric == CORAL_IP ? (int64_t)1 << 15
                                  : idx->dim <= 512                    ? ((int64_t)1 << 24) / idx->dim
                                  : idx->dim > 1024 && Q > idx->num_cu ? (int64_t)1 << 17
@@ -591,17 +584,48 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     // A caller who names any part of the launch keeps the wavefronts.
     const bool named = t.visited_slots_log2 || t.workgroups || t.threads || t.best_first_packed || t.best_first_table_log2 ||
                        t.beam_in_hbm || t.cand_cap || t.best_first_long || t.best_first_buffer || t.screening ||
-                       t.visited_choices || t.prefetch_rows;
-    const bool shared_steps = best_first && !named && idx->dim / 4 > 32 && Q <= 2 * idx->num_cu && idx->n >= nodes_shared &&
-                              plan.direct && !plan.big;
-    const bool wave_form = best_first && !t.best_first_in_lds && !long_form && !plan.big && !shared_steps &&
-                           coral::best_first_wave_lds_bytes(L, 0, 0) * 4 <= (size_t)kMaxLdsBytes;
+                       t.visited_choices || t.prefetch_rows || t.best_first_in_lds;
+    const bool shared_steps = best_first && !named && !long_form && !plan.big && L <= coral::kMaxWaveBeam && idx->dim / 4 > 32 &&
+                              Q <= 2 * idx->num_cu && idx->n >= nodes_shared &&
+                              (L <= 768 || Q <= idx->num_cu || idx->dim > coral::kMaxByteRowDim);
+    const bool wave_form = best_first && !t.best_first_in_lds && !long_form && !plan.big && L <= coral::kMaxWaveBeam;
     // rows of 68 .. 128 floats are screened (on codes) only when the caller asks for it by name; the coded query then
     // takes the LDS a table of visited ids would fill
     const bool narrow_codes = best_first && t.screening == 2 && idx->dim / 4 > 16 && idx->dim / 4 <= 32;
-    int table_log2 = 0;
-    if (wave_form)
-        if (int rc = choose_bf_table(L, id_bits, narrow_codes ? -1 : t.best_first_table_log2, &table_log2)) return rc;
+    int table_log2 = 0, bitmap_words = 0, bf_form = 0;
+    bool shared = false;
+    if (wave_form) {
+        // Rows are screened on the copy in eight-bit codes where it applies (half precision, which only L2 has, has to be
+        // asked for by name: on rows of more than 512 floats it costs).  The rows it spares are worth its wait at every
+        // beam length (sixteen wavefronts per CU or one; 200 000 x 200, L = 64 / 512, one query: 226 / 1600 without, 147 /
+        // 1321 us with; 5000 queries: 774 / 6469, 551 / 4549) -- except on graphs so small for the beam that most
+        // neighbours have been visited and a step has few rows to read (one query, 40 000 x 300: L = 400 941 / 963, L =
+        // 512 1147 / 1230; 30 000 x 512, L = 1000 2241 / 2697; 100 000 x 512 under the inner product, L = 1000, still
+        // 4407 / 4349, and 5000 queries 35 100 / 19 600).
+        const int form = t.screening == 1 || idx->dim > coral::kMaxByteRowDim ? 1 : 2;
+        const bool can = (idx->dim / 4 > 32 || narrow_codes) && (form == 2 || idx->metric == CORAL_L2);
+        if (can && (t.screening > 0 || (t.screening == 0 && form == 2 && idx->n >= (int64_t)80 * L))) bf_form = form;
+        const int coded = bf_form == 2 ? coral::coded_query_bytes(idx->dim) : 0;
+        // The visited set: a bitmap of all ids in LDS where every wavefront that the batch gives a CU finds room for one
+        // (one atomic per id, nothing to hash or probe; 200 000 x 200, L = 128, one query: 244 us, the table 314, the
+        // state in HBM 311).
+        const int bits = (int)(((idx->n + 127) / 128) * 4);
+        const int wgs_wanted = (int)std::min<int64_t>(((int64_t)Q + 4 * idx->num_cu - 1) / (4 * idx->num_cu), L <= 512 ? 4 : L <= 1280 ? 3 : 2);
+        const size_t shared_lds = coral::best_first_shared_lds_bytes(coded, bits);
+        if (shared_steps && bf_form != 1 && idx->n <= ((int64_t)1 << 21) && shared_lds * (Q > idx->num_cu ? 2 : 1) <= (size_t)kMaxLdsBytes) {
+            bitmap_words = bits, shared = true;
+        } else if (t.best_first_table_log2 == 0 && !t.best_first_packed && t.workgroups == 0 && idx->n <= ((int64_t)1 << 21) &&
+            coral::best_first_wave_lds_bytes(0, 0, coded, bits) * 4 * wgs_wanted <= (size_t)kMaxLdsBytes) {
+            bitmap_words = bits;
+        } else {
+            // (a full chip of narrow rows wants its sixteen wavefronts per CU more than a table that leaves eight:
+            // 200 000 x 200, 5000 queries, L = 256 / 330 / 400: 2456 / 3361 / 4164 us with it, 2400 / 3030 / 3632 without;
+            // rows of 256 floats: 3601 / 4880 / 5824, 4024 / 5160 / 6076; 2048 queries gain by it everywhere)
+            const int fewest_waves = idx->dim <= 208 && L > 256 && Q > 8 * idx->num_cu ? 12 : 8;
+            if (int rc = choose_bf_table(L, id_bits, narrow_codes ? -1 : t.best_first_table_log2, coded, fewest_waves, &table_log2))
+                return rc;
+        }
+    }
     // from here on buffers are replaced: a failure part-way leaves the index unprepared, not half-prepared
     idx->prepared = false;
     const size_t need_words = plan.spill_words * (size_t)workgroups;
@@ -632,7 +656,7 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     // Best-first, one wavefront per query: the visited state lives in HBM, n bytes per wavefront (n / 6 in the packed
     // form), up to a third of what is free and 64 GiB.  wg_per_cu: what the chosen kernel's occupancy allows;
     // reprepare(packed): sets that kernel up in the packed form and returns its occupancy.
-    idx->bf_ready = false, idx->bf_long = false, idx->bf_screen = 0;
+    idx->bf_ready = false, idx->bf_long = false, idx->bf_shared = false, idx->bf_screen = 0;
     // Best-first with the beam in LDS screens rows in half precision too, where a CU holds sixteen wavefronts (beams
     // without the LDS table: L > 409): +12 % at L = 512 and 1024.  With the table (eight wavefronts per CU) the extra
     // wait per step costs more than the bytes it spares (L = 256 / 320: -27 %), so those launches go without unless
@@ -651,16 +675,10 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
             HIP_TRY(e);
         }
     }
-    // eight-bit codes where they apply; launches with the LDS table (whose size was chosen to fill LDS) and rows of
-    // more than 512 floats screen in half precision, which only the L2 metric has
-    const int form = t.screening == 1 || idx->dim > coral::kMaxByteRowDim || table_log2 != 0 ? 1 : 2;
-    // (rows of more than 512 floats, which this kernel can only screen in half precision, go without unless asked by
-    // name: 156 k against 211 k QPS at 1024 floats and L = 512, 51 k against 111 k at 2048)
-    if (wave_form && (idx->dim / 4 > 32 || narrow_codes) && (form == 2 || idx->metric == CORAL_L2) &&
-        (t.screening > 0 || (t.screening == 0 && table_log2 == 0 && idx->dim <= coral::kMaxByteRowDim))) {
-        const hipError_t e = form == 2 ? ensure_vec8() : ensure_vec16();
+    if (bf_form != 0) {
+        const hipError_t e = bf_form == 2 ? ensure_vec8() : ensure_vec16();
         if (e == hipSuccess) {
-            idx->bf_screen = form;
+            idx->bf_screen = bf_form;
         } else if (e == hipErrorOutOfMemory && t.screening == 0) {
             (void)hipGetLastError();
         } else {
@@ -708,27 +726,33 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         }
         return CORAL_OK;
     };
-    if (wave_form) {
+    if (shared) {
+        // (neither the state in HBM nor the epochs exist for this form: its bitmap holds every id)
+        const int coded = idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0;
+        idx->bf_bitmap_words = bitmap_words;
+        const size_t lds = coral::best_first_shared_lds_bytes(coded, bitmap_words);
+        int per_cu = 0;
+        HIP_TRY(coral::best_first_shared_prepare(idx->dim, L, idx->bf_screen, lds, &per_cu));
+        if (per_cu <= 0) return fail(CORAL_ERR_DEVICE, "kernel does not fit the device");
+        idx->bf_shared = true, idx->bf_shared_lds = (int)lds, idx->bf_slots = std::min(per_cu * idx->num_cu, (int)Q);
+    } else if (wave_form) {
         int bf_wg_per_cu = 0;
-        const int chunks = idx->dim / 4;
         idx->bf_table_log2 = table_log2;
         idx->bf_table_rem_bits = table_log2 ? bf_table_rem_bits(id_bits, table_log2) : 0;
-        // 16 rows requested per wavefront before any is added up where that fits 128 registers without spilling; a
-        // launch whose LDS leaves a CU eight wavefronts may as well use 256 registers per lane: all 32 rows of a step
-        int rif = (chunks > 16 && chunks <= 256) ? 16 : 8;
-        if (idx->bf_screen != 0 && table_log2 == 0) rif = 8;  // (the screening leaves few rows to read in fp32)
-        if (table_log2 && coral::best_first_wave_lds_bytes(L, 0, table_log2) * 12 > (size_t)kMaxLdsBytes && chunks > 16 &&
-            chunks <= 64)
-            rif = 32;
-        idx->bf_rows_in_flight = rif;
-        // with a table the filter would only cover what outgrew it, and its LDS is worth more as cells
+        idx->bf_bitmap_words = bitmap_words;
         const int coded = idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0;
-        const int bloom_log2 = table_log2 ? 0 : coral::best_first_bloom_log2(L, coded);
+        // with a table the filter would only cover what outgrew it, and its LDS is worth more as cells
+        const int bloom_log2 = table_log2 || bitmap_words ? 0 : coral::best_first_bloom_log2(L, coded);
         idx->bf_bloom_log2 = bloom_log2;
-        HIP_TRY(coral::best_first_prepare(idx->dim, L, rif, false, idx->bf_screen, bloom_log2, table_log2, &bf_wg_per_cu));
-        auto reprepare = [&](int* occ) {
-            return coral::best_first_prepare(idx->dim, L, rif, true, idx->bf_screen, bloom_log2, table_log2, occ);
-        };
+        const size_t wave_lds = coral::best_first_wave_lds_bytes(bloom_log2, table_log2, coded, idx->bf_bitmap_words);
+        // 16 rows requested per wavefront before any is added up; a launch whose LDS, or whose batch, leaves a CU eight
+        // wavefronts may as well use 256 registers per lane: all 32 rows of a step.  Where a screening leaves few rows
+        // to read in fp32, 8.
+        const bool eight = wave_lds * 12 > (size_t)kMaxLdsBytes || Q <= 8 * idx->num_cu;
+        const int rif = eight && L <= 1024 && idx->bf_screen != 1 ? 32 : idx->bf_screen != 0 ? 8 : 16;
+        idx->bf_rows_in_flight = rif;
+        HIP_TRY(coral::best_first_prepare(idx->dim, L, rif, idx->bf_screen, wave_lds, &bf_wg_per_cu));
+        auto reprepare = [&](int*) -> hipError_t { return hipSuccess; };  // (one kernel for both forms)
         if (int rc = visited_slots(bf_wg_per_cu, reprepare, 0)) return rc;
     } else if (long_form) {
         // the insert buffer: 512 keys unless the caller names a size; a sample of at most 128 keys of the long run
@@ -853,6 +877,7 @@ int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, f
         coral::BestFirstArgs b;
         b.rows_unique = idx->rows_unique == 1;
         b.packed = idx->bf_packed;
+        b.bitmap_words = idx->bf_bitmap_words;
         b.bloom_log2 = idx->bf_bloom_log2;
         b.table_log2 = idx->bf_table_log2;
         b.id_bits = plan.id_bits, b.rem_bits = idx->bf_table_rem_bits;
@@ -863,6 +888,13 @@ int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, f
         b.vec8 = idx->bf_screen == 2 ? idx->d_vec8 : nullptr, b.stride8 = coral::byte_row_stride(idx->dim);
         b.coded_bytes = idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0;
         HIP_TRY(coral::launch_best_first(a, b, stream));
+    } else if (policy == CORAL_POLICY_BEST_FIRST && idx->bf_shared) {
+        coral::BestFirstArgs b;
+        std::memset(&b, 0, sizeof b);
+        b.bitmap_words = idx->bf_bitmap_words, b.slots = std::min(idx->bf_slots, (int)Q);
+        b.vec8 = idx->bf_screen == 2 ? idx->d_vec8 : nullptr, b.stride8 = coral::byte_row_stride(idx->dim);
+        b.coded_bytes = idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0;
+        HIP_TRY(coral::launch_best_first_shared(a, b, stream));
     } else {
         const int wgs = std::min(plan.workgroups, (int)Q);
         HIP_TRY(coral::launch_search(a, plan.big, wgs, plan.threads, plan.lds_bytes, stream));
@@ -906,7 +938,7 @@ int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, f
     // there, the next launches get a table twice the size.  (The bucket form turns away only the ids that find their
     // three buckets full, a handful per query at a load where linear probing freezes the table: it takes the larger
     // table only when more than a fiftieth of all first visits went to the bitmap.)
-    const bool lds_table = !(policy == CORAL_POLICY_BEST_FIRST && idx->bf_ready) && !plan.big;
+    const bool lds_table = !(policy == CORAL_POLICY_BEST_FIRST && (idx->bf_ready || idx->bf_shared)) && !plan.big;
     bool grow = lds_table && idx->tuning.visited_slots_log2 == 0 && (int64_t)scal[1] * 20 > Q && plan.slots_log2 < 16;
     if (grow && plan.choices != 0 && sum.visited_requests / 2 * 50 <= sum.dist_evals) {
         // few ids left LDS: the larger table is worth taking only if it costs the CU no workgroup
@@ -1015,13 +1047,18 @@ int coral_search_plan_info(const coral_index* idx, coral_plan_info* out) {
             idx->bf_long
                 ? coral::best_first_long_lds_bytes(idx->bf_bcap, idx->bf_scap,
                                                    idx->bf_screen == 2 ? coral::best_first_long_coded_bytes(idx->dim) : 0)
-                : coral::best_first_wave_lds_bytes(idx->L, idx->bf_bloom_log2, idx->bf_table_log2,
-                                                   idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0);
+                : coral::best_first_wave_lds_bytes(idx->bf_bloom_log2, idx->bf_table_log2,
+                                                   idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0,
+                                                   idx->bf_bitmap_words);
         out->lds_bytes = (int32_t)(per_wave * 4);
         out->screening = idx->bf_screen;
-        out->visited_form = !idx->bf_long && idx->bf_table_log2 ? 4 : idx->bf_packed ? 3 : 2;
+        out->visited_form = !idx->bf_long && idx->bf_bitmap_words ? 1 : !idx->bf_long && idx->bf_table_log2 ? 4 : idx->bf_packed ? 3 : 2;
         out->visited_slots_log2 = idx->bf_long ? 0 : idx->bf_table_log2;
         out->beam_in_hbm = idx->bf_long;
+    } else if (idx->prepared_policy == CORAL_POLICY_BEST_FIRST && idx->bf_shared) {
+        out->kernel = 0;  // (a workgroup per query)
+        out->threads = 256, out->workgroups = out->query_slots = idx->bf_slots, out->lds_bytes = idx->bf_shared_lds;
+        out->screening = idx->bf_screen, out->visited_form = 1;
     } else {
         out->kernel = 0;
         out->threads = p.threads, out->workgroups = p.workgroups, out->lds_bytes = (int32_t)p.lds_bytes;

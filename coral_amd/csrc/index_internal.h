@@ -91,7 +91,8 @@ struct coral_index {
     uint8_t* d_bf_visited = nullptr;
     uint32_t* d_bf_epochs = nullptr;
     size_t bf_stride = 0, bf_alloc_bytes = 0;
-    int bf_slots = 0, bf_alloc_slots = 0, bf_rows_in_flight = 8, bf_packed = 0, bf_bloom_log2 = 0;
+    int bf_slots = 0, bf_alloc_slots = 0, bf_rows_in_flight = 8, bf_packed = 0, bf_bitmap_words = 0, bf_shared_lds = 0, bf_bloom_log2 = 0;
+    bool bf_shared = false;  // best-first: four wavefronts share a query's steps
     int bf_table_log2 = 0, bf_table_rem_bits = 0;
     // ... or, for long beams, with an insert buffer in LDS and the long sorted run of every slot in global memory
     int bf_screen = 0;  // the kernel with the beam in LDS screens rows: 1 in half precision (d_vec16), 2 in eight-bit codes (d_vec8)

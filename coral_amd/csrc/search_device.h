@@ -35,6 +35,65 @@ __device__ __forceinline__ int dpp_mov_i(int x) {
     return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xF, 0xF, true);
 }
 
+// ---- Sums over the lanes of a row, several rows at once.
+//
+// The sum of a row's lane values is the butterfly p[l] += p[l ^ off], off = 1, 2, 4, ..., G / 2 (addition commutes, so
+// every lane ends with the same bits).  Only one lane needs a row's sum, so with N rows to add up each level halves
+// their number: a lane keeps one of two rows and hands the other to its partner, which does the opposite.  N rows cost
+// about 3 N instructions (and a choice is made on the way) instead of N per level and 2 N to choose.
+// Inside a row of 16 lanes the partner is reached by DPP: l ^ 1, l ^ 2 (quad_perm), l ^ 7 (row_half_mirror) and l ^ 15
+// (row_mirror); b0 .. b3 below are bits of the lane such that each of the four flips the bit of its own level only.
+template <int CTRL>
+__device__ __forceinline__ float dpp_lane(float x) {
+    return dpp_mov<CTRL>(x);
+}
+template <int CTRL>
+__device__ __forceinline__ int dpp_lane(int x) {
+    return dpp_mov_i<CTRL>(x);
+}
+template <int CTRL, int N, typename T>
+__device__ __forceinline__ void rows_fold(T* x, bool odd) {
+    if constexpr (N == 1) {
+        x[0] = x[0] + dpp_lane<CTRL>(x[0]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N / 2; ++i) {
+            const T mine = odd ? x[2 * i + 1] : x[2 * i], other = odd ? x[2 * i] : x[2 * i + 1];
+            x[i] = mine + dpp_lane<CTRL>(other);
+        }
+    }
+}
+// which of its group's N rows (N a power of two) the lane ends with; lanes 0 .. N - 1 of a group hold all of them
+template <int G, int N>
+__device__ __forceinline__ int filed_row(int lane) {
+    const int b0 = (lane ^ (lane >> 2)) & 1, b1 = (lane >> 1 ^ lane >> 2) & 1, b2 = (lane >> 2 ^ lane >> 3) & 1;
+    const int row = b0 | b1 << 1 | b2 << 2 | (lane & 8) | (lane & 16);
+    return row & (N - 1);
+}
+__device__ __forceinline__ float lane_bits(float, uint32_t u) { return __uint_as_float(u); }
+__device__ __forceinline__ int lane_bits(int, uint32_t u) { return (int)u; }
+__device__ __forceinline__ uint32_t lane_word(float x) { return __float_as_uint(x); }
+__device__ __forceinline__ uint32_t lane_word(int x) { return (uint32_t)x; }
+template <int G, int N, typename T>
+__device__ __forceinline__ T rows_sum(T (&x)[N]) {
+    static_assert(N <= G && (N & (N - 1)) == 0 && N <= 32, "a lane for every row");
+    const int lane = threadIdx.x & 63;
+    rows_fold<0xB1, N>(x, ((lane ^ (lane >> 2)) & 1) != 0);                          // quad_perm [1,0,3,2]
+    rows_fold<0x4E, (N > 2 ? N / 2 : 1)>(x, ((lane >> 1 ^ lane >> 2) & 1) != 0);      // quad_perm [2,3,0,1]
+    rows_fold<0x141, (N > 4 ? N / 4 : 1)>(x, ((lane >> 2 ^ lane >> 3) & 1) != 0);     // row_half_mirror
+    rows_fold<0x140, (N > 8 ? N / 8 : 1)>(x, (lane & 8) != 0);                        // row_mirror
+    if constexpr (G >= 32) {
+        // lanes 16 apart: the two halves of the exchange are added; two rows are dealt out to even and odd sixteens
+        const auto r = __builtin_amdgcn_permlane16_swap(lane_word(x[0]), lane_word(x[N > 16 ? 1 : 0]), false, false);
+        x[0] = lane_bits(x[0], r[0]) + lane_bits(x[0], r[1]);
+    }
+    if constexpr (G >= 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(lane_word(x[0]), lane_word(x[0]), false, false);
+        x[0] = lane_bits(x[0], r[0]) + lane_bits(x[0], r[1]);
+    }
+    return x[0];
+}
+
 // ---- Screening on rows in eight-bit codes (the copy byte_rows_kernel makes).  Row x is stored as codes k_i in
 // [-127, 127] with x~_i = s k_i, s = max |x_i| / 127, followed by s, |x~|^2 and e >= |x - x~| (rounded up; infinite for
 // rows that take no part).  The query is coded as q~_i = sq (128 h_i + l_i), bytes h_i in [-127, 127] and l_i in
@@ -99,8 +158,8 @@ __device__ __forceinline__ void load_coded_query(const signed char* qh8, const s
 // Rows vid[0..U8) (-1: none) of one group of sixteen lanes, in three steps so that a caller with more rows to come can
 // request the next ones before it finishes these: request (all loads back to back), dots (the integer sums, which
 // wait for the loads and leave their registers free), finish (the lane that files a row gets the bounds
-// lo <= d <= hi of its exact distance).  Lane gl8 < U8 of the group files row vid[gl8]; the caller hands it that id as
-// myid (-1: the lane files none; lo and hi are then worthless).  A row that takes no part has lo = 0 and hi = inf; a
+// lo <= d <= hi of its exact distance).  Lane gl8 < U8 of the group files row filed_row<16, U8>; the caller hands it
+// that id as myid (-1: the lane files none; lo and hi are then worthless).  A row that takes no part has lo = 0 and hi = inf; a
 // NaN anywhere fails every comparison a caller makes with the bounds.
 //
 // Inner product (metric 1; the signed distance is -q.x): q.x = q~.x~ + q~.(x - x~) + (q - q~).x, so
@@ -178,23 +237,6 @@ __device__ __forceinline__ void coded_rows_dots_wide(const CodedRows<CPL8, U8>& 
     }
 }
 
-// the sum over the sixteen lanes of a row, for the lane that files it
-template <int U8>
-__device__ __forceinline__ int coded_rows_reduce(int (&acc)[U8], int gl8) {
-#pragma unroll
-    for (int u = 0; u < U8; ++u) {
-        acc[u] = acc[u] + dpp_mov_i<0xB1>(acc[u]);   // quad_perm [1,0,3,2]
-        acc[u] = acc[u] + dpp_mov_i<0x4E>(acc[u]);   // quad_perm [2,3,0,1]
-        acc[u] = acc[u] + dpp_mov_i<0x141>(acc[u]);  // row_half_mirror
-        acc[u] = acc[u] + dpp_mov_i<0x140>(acc[u]);  // row_mirror
-    }
-    int mine = acc[0];
-#pragma unroll
-    for (int u = 1; u < U8; ++u)
-        if (gl8 == u) mine = acc[u];
-    return mine;
-}
-
 // bounds from the integer sum as a float; WIDE: rows of more than 512 codes (two more roundings on the way to the
 // sum, and a longer exact inner product to allow for)
 template <bool WIDE>
@@ -219,9 +261,9 @@ __device__ __forceinline__ void coded_bounds(float isum, const float4& fig, floa
 }
 
 template <int U8>
-__device__ __forceinline__ void coded_rows_finish(int (&acc)[U8], int gl8, const float4& fig, float qq, float sq, float eq,
+__device__ __forceinline__ void coded_rows_finish(int (&acc)[U8], const float4& fig, float qq, float sq, float eq,
                                                   int metric, float& lo, float& hi) {
-    const int mine = coded_rows_reduce<U8>(acc, gl8);
+    const int mine = rows_sum<16, U8>(acc);
     coded_bounds<false>((float)mine, fig, qq, sq, eq, metric, lo, hi);
 }
 
@@ -234,7 +276,7 @@ __device__ __forceinline__ void coded_rows_bounds(const unsigned char* vec8, uin
     coded_rows_request<CPL8, U8>(vec8, st8, nck, gl8, vid, myid, r);
     int acc[U8];
     coded_rows_dots<CPL8, U8>(r, q, acc);
-    coded_rows_finish<U8>(acc, gl8, r.fig, qq, sq, eq, metric, lo, hi);
+    coded_rows_finish<U8>(acc, r.fig, qq, sq, eq, metric, lo, hi);
 }
 
 // rows of more than 512 codes: the query's codes come from LDS (qh8, ql8)
@@ -247,7 +289,7 @@ __device__ __forceinline__ void coded_rows_bounds_wide(const unsigned char* vec8
     coded_rows_request<CPL8, U8>(vec8, st8, nck, gl8, vid, myid, r);
     int acch[U8], accl[U8];
     coded_rows_dots_wide<CPL8, U8>(r, qh8, ql8, nck, gl8, acch, accl);
-    const int mh = coded_rows_reduce<U8>(acch, gl8), ml = coded_rows_reduce<U8>(accl, gl8);
+    const int mh = rows_sum<16, U8>(acch), ml = rows_sum<16, U8>(accl);
     coded_bounds<true>(128.0f * (float)mh + (float)ml, r.fig, qq, sq, eq, metric, lo, hi);
 }
 

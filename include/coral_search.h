@@ -116,9 +116,10 @@ typedef struct {
                                    24 flags: n / 6 bytes per slot, about 5 % slower); 1 = the packed form always */
     int32_t best_first_table_log2; /* the wavefront-per-query kernel keeps the first visits of a query in an exact
                                    table of 16-bit cells in LDS (the cells of the ROUNDS kernel's table) and only
-                                   what outgrows it in HBM: log2 of the cells per query, 8..14; 0 = chosen from L
-                                   where 8192 cells hold most of a query's visits (L <= 409 at up to 2^25 nodes),
-                                   none otherwise; -1 = none */
+                                   what outgrows it in HBM: log2 of the cells per query, 8..14; 0 = a bitmap of all ids
+                                   where the batch leaves LDS for one per wavefront, else chosen from L where 8192
+                                   cells hold most of a query's visits (L <= 409 at up to 2^25 nodes), none otherwise;
+                                   -1 = neither */
     int32_t beam_in_hbm;        /* 1 = keep the beam in global memory whatever L is (the form beams longer than
                                    CORAL_MAX_LDS_BEAM always take, and shorter ones when that frees the LDS a bitmap of
                                    all ids needs) */
@@ -126,7 +127,7 @@ typedef struct {
                                    0 = where a workgroup has its CU to itself */
     int32_t cand_cap;           /* capacity of the candidate buffer in LDS (a power of two, at least the todo list's);
                                    0 = chosen */
-    int32_t best_first_long;    /* best-first with a wavefront per query keeps beams up to 1280 entries in LDS and longer
+    int32_t best_first_long;    /* best-first with a wavefront per query keeps beams up to 1280 entries in registers and longer
                                    ones as a sorted insert buffer in LDS in front of a long run in global memory (two
                                    runs of L keys per query slot): 1 = that form whatever L is, -1 = never (beams
                                    beyond CORAL_MAX_LDS_BEAM then run on the workgroup-per-query kernel), 0 = by L */
@@ -226,7 +227,9 @@ CORAL_API int coral_search_row_counters(coral_index* idx, int32_t* host_out, int
 
 /* The launch geometry the last coral_search_prepare chose (what a search call on this index runs with). */
 typedef struct {
-    int32_t kernel;          /* 0 beam_search_kernel (workgroup per query), 1 best_first_wave_kernel, 2 best_first_long_kernel */
+    int32_t kernel;          /* 0 a workgroup per query (beam_search_kernel; best-first with 256 threads: the wavefronts of
+                                best_first_wave_kernel, four to a query), 1 best_first_wave_kernel, a wavefront per
+                                query, 2 best_first_long_kernel */
     int32_t threads;         /* per workgroup */
     int32_t workgroups;      /* persistent workgroups (the wavefront kernels: query slots / 4) */
     int32_t lds_bytes;       /* per workgroup */

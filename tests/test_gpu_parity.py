@@ -893,3 +893,51 @@ def test_randomised_shapes(orc):
         assert np.array_equal(ids, oi), case
         assert dists.tobytes() == od.tobytes(), case
         assert np.array_equal(cnt, os_), case
+
+
+@pytest.mark.parametrize("n,dim,metric,L,M,Q,kw", [
+    # the largest beam of every number of keys per lane and the smallest of the next
+    (9000, 96, "l2", 1, 1, 40, {}), (9000, 96, "l2", 127, 7, 40, {}), (9000, 96, "l2", 128, 33, 40, {}),
+    (9000, 96, "ip", 129, 64, 40, {}), (9000, 200, "l2", 256, 65, 40, {}), (9000, 200, "ip", 257, 1, 40, {}),
+    (9000, 200, "l2", 512, 16, 20, {}), (9000, 520, "l2", 513, 16, 20, {}), (9000, 200, "l2", 1024, 300, 12, {}),
+    (9000, 64, "ip", 1025, 16, 12, {}), (9000, 64, "l2", 1280, 16, 12, {}),
+    (9000, 132, "l2", 1281, 16, 12, dict(best_first_long=-1)), (9000, 1036, "l2", 2048, 16, 8, dict(best_first_long=-1)),
+    # rows of one, of two and of four to a wavefront, with a last chunk that is part padding
+    (9000, 4, "l2", 40, 3, 40, {}), (9000, 68, "l2", 40, 3, 40, {}), (6000, 2044, "ip", 40, 3, 20, {}),
+    # more queries than one workgroup per CU takes; the forms of the visited set behind the bitmap
+    (9000, 96, "l2", 100, 16, 1100, {}), (9000, 200, "l2", 100, 16, 300, dict(best_first_table_log2=8)),
+    (9000, 200, "l2", 300, 16, 100, dict(best_first_table_log2=-1)), (9000, 200, "l2", 300, 16, 100, dict(best_first_packed=True)),
+    # four wavefronts per query: beams of every number of keys per lane, one query and several per workgroup
+    (33000, 132, "ip", 48, 40, 3, {}), (33000, 132, "ip", 200, 5, 300, {}), (33000, 516, "ip", 300, 5, 40, {}),
+    (33000, 260, "ip", 600, 70, 20, {}), (33000, 132, "ip", 1280, 5, 12, {}), (33000, 1028, "ip", 100, 5, 40, {}),
+    (33000, 260, "ip", 412, 3, 40, {}), (33000, 260, "ip", 413, 3, 40, {}),  # 80 nodes per entry: screened, and not
+])
+def test_best_first_with_the_beam_in_registers_at_the_edges_of_its_sizes(orc, n, dim, metric, L, M, Q, kw):
+    """Beams that fill the places of their lanes and beams one longer, start ids beyond a list of 32, ragged rows with
+    repeated ids, tombstones: ids, distance bits and counters equal the oracle's."""
+    print("registers", n, dim, metric, L, M, Q, kw, flush=True)
+    m = capi.IP if metric == "ip" else capi.L2
+    rng = np.random.RandomState(L + dim)
+    base = synth.gaussian_matrix(71, n, dim)
+    if metric == "ip":
+        base = synth.normalize_rows(base)
+    nbrs = rng.randint(0, n, (n, 32)).astype(np.int32)  # repeated ids now and then
+    nbrs[::7, 5] = nbrs[::7, 3]
+    nbrs[::5, 20:] = -1
+    starts = rng.choice(n, M, replace=False).astype(np.int32)
+    mask = synth.tombstone_mask(n, 9, modulo=4)
+    q = make_queries(Q, dim, 55, metric)
+    k = min(L, 100)
+    oi, od, os_, _ = orc.search_A(orc.Problem(base, nbrs, starts, mask), q, k, L, metric=m, order=WAVE64)
+    idx = capi.Index(base, nbrs, starts, m)
+    idx.set_deleted(mask)
+    idx.prepare(Q, L, policy=1, **kw)
+    shared = n > 32768
+    assert idx.plan_info().kernel == (0 if shared else 1)
+    for _ in range(2):
+        ids, dists, st = idx.search(q, k, L, policy=1, have_delete=True)
+        assert np.array_equal(ids, oi) and dists.tobytes() == od.tobytes()
+        assert np.array_equal(idx.query_counters(Q), os_)
+        rows = idx.row_counters(Q)
+        assert ((rows[:, 0] + rows[:, 1] >= os_[:, 2]) & (rows[:, 1] <= os_[:, 2])).all()
+    idx.close()
