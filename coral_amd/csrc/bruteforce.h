@@ -15,22 +15,26 @@ hipError_t launch_row_select(const float* D, int64_t ldD, int nq, int64_t n, int
 hipError_t launch_merge_segments(const unsigned long long* part, int nq, int nseg, int k, int metric,
                                  int32_t* ids, float* dists, hipStream_t stream);
 // --- the screening pass on the matrix cores (bruteforce_mfma.hip) ---
-// out[r] = |x_r|^2; *max_bits (optional, zero before) = bit pattern of the largest of them
-hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, hipStream_t stream);
-// the queries in the form the two launches below take them (split into halves, tile by tile); out: that many bytes
-size_t split_queries_bytes(int nq, int dim);
-hipError_t launch_split_queries(const float* queries, int nq, int dim, const float* qn, void* out, hipStream_t stream);
+// out[r] (optional) = |x_r|^2; *max_bits (optional, zero before) = bit pattern of the largest of them; res[r], *res_max (optional):
+// the same for a bound on |x_r - hi(x_r)|, what one half per component leaves out
+hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, float* res, uint32_t* res_max,
+                            hipStream_t stream);
+// the queries in the form the two launches below take them (split into halves, tile by tile); out: that many bytes.
+// products: 3 (hi.hi + hi.lo + lo.hi, about fp32 accuracy) or 1 (hi.hi alone), the same in all launches of a call
+size_t split_queries_bytes(int nq, int dim, int products);
+hipError_t launch_split_queries(const float* queries, int nq, int dim, int products, const float* qn, void* out,
+                                hipStream_t stream);
 // as launch_distance_tile, with D[q][b] = |q|^2 + |b|^2 - 2 q.b (L2) or -q.b (IP) from inner products on the matrix
 // cores; queries: what launch_split_queries wrote.
 // sample_tiles > 0: only that many tiles of 128 base points, every tile_stride-th of the base, side by side in D
-hipError_t launch_approx_tile(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric,
+hipError_t launch_approx_tile(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, int products,
                               const float* qn, const float* bn, const uint32_t* deleted, int64_t base_id0, float* D,
                               int64_t ldD, hipStream_t stream, int64_t sample_tiles = 0, int tile_stride = 1);
 // the same distances, no matrix: every entry <= tau[q] is appended to lists[q * cap ...] as ord(value) << 32 | id
 // (cnt[q * kCntStride] counts them, also those beyond cap that were dropped).  tile_step > 0: tiles 0, tile_step,
 // 2 tile_step ... of 128 base points; tile_step < 0: the tiles between those
 constexpr int kCntStride = 16;  // a 64-byte line per counter: workgroups append to many queries at a time
-hipError_t launch_approx_filter(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric,
+hipError_t launch_approx_filter(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, int products,
                                 const float* qn, const float* bn, const uint32_t* deleted, const float* tau,
                                 unsigned long long* lists, int64_t cap, unsigned int* cnt, int tile_step,
                                 hipStream_t stream);
@@ -45,8 +49,13 @@ hipError_t launch_list_shrink(unsigned long long* lists, int64_t cap, unsigned i
 // cand_ids / cand_d [nq][kc] (ascending approximate signed distance, -1 = none) -> the exact k best per query in the
 // reference's summation order; redo[q] = 1 where the candidates cannot vouch for the result
 hipError_t launch_rerank(const float* queries, const float* base, int nq, int dim, int metric, const int32_t* cand_ids,
-                         const float* cand_d, int kc, int k, const float* qn, const uint32_t* bn_max_bits, int32_t* ids,
-                         float* dists, int* redo, hipStream_t stream);
+                         const float* cand_d, int kc, int k, const float* qn, const uint32_t* bn_max_bits, const float* qres,
+                         const uint32_t* bres_max_bits, int32_t* ids, float* dists, int* redo, hipStream_t stream);
+// (qres, *bres_max_bits: what launch_row_norms gave, for candidates chosen on one product; else null)
+// *extra += the entries of D's rows, beyond kc, that one product cannot tell from those up to tau
+hipError_t launch_count_close(const float* D, int64_t ldD, int nq, int64_t n, int kc, int metric, const float* qn,
+                              const uint32_t* bn_max_bits, const float* qres, const uint32_t* bres_max_bits, const float* tau,
+                              int* extra, hipStream_t stream);
 hipError_t launch_scatter_results(const int32_t* rows, int count, int k, const int32_t* src_ids, const float* src_d,
                                   int32_t* dst_ids, float* dst_d, hipStream_t stream);
 }  // namespace coral

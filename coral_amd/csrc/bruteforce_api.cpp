@@ -2,6 +2,7 @@
 // queries among the index's resident vectors (kernels in bruteforce.hip, bruteforce_mfma.hip).
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstring>
 #include <utility>
 #include <vector>
@@ -54,18 +55,18 @@ int knn_passes(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, i
     HIP_TRY_R(hipMalloc(&D, (size_t)qc * ld * sizeof(float)));
     HIP_TRY_R(hipMalloc(&part, (size_t)Q * nseg * k * sizeof(unsigned long long)));
     HIP_TRY_R(hipMalloc(&redo, (size_t)qc * sizeof(int)));
-    if (screen) HIP_TRY_R(hipMalloc(&d_split, coral::split_queries_bytes((int)qc, idx->dim)));
+    if (screen) HIP_TRY_R(hipMalloc(&d_split, coral::split_queries_bytes((int)qc, idx->dim, 3)));
     for (int64_t q0 = 0; q0 < Q; q0 += qc) {
         const int nq = (int)std::min<int64_t>(qc, Q - q0);
         if (screen)
-            HIP_TRY_R(coral::launch_split_queries(d_queries + (size_t)q0 * idx->dim, nq, idx->dim, d_qn + q0, d_split, stream));
+            HIP_TRY_R(coral::launch_split_queries(d_queries + (size_t)q0 * idx->dim, nq, idx->dim, 3, d_qn + q0, d_split, stream));
         for (int64_t s = 0; s < nseg; ++s) {
             const int64_t b0 = s * seg, nb = std::min(seg, n - b0);
             const float* qp = d_queries + (size_t)q0 * idx->dim;
             const float* bp = idx->d_vec + (size_t)b0 * idx->dim;
             const uint32_t* del = have_delete ? idx->d_deleted : nullptr;
             if (screen)
-                HIP_TRY_R(coral::launch_approx_tile(d_split, bp, nq, nb, idx->dim, idx->metric, d_qn + q0, idx->d_bnorm + b0, del,
+                HIP_TRY_R(coral::launch_approx_tile(d_split, bp, nq, nb, idx->dim, idx->metric, 3, d_qn + q0, idx->d_bnorm + b0, del,
                                                     b0, D, ld, stream));
             else
                 HIP_TRY_R(coral::launch_distance_tile(qp, bp, nq, nb, idx->dim, idx->metric, del, b0, D, ld, stream));
@@ -86,16 +87,26 @@ namespace coral {
 // |b|^2 of the base, once per index
 int ensure_base_norms(coral_index* idx, hipStream_t stream) {
     if (idx->d_bnorm) return CORAL_OK;
-    if (!idx->d_bnorm_max) HIP_TRY(hipMalloc(&idx->d_bnorm_max, sizeof(uint32_t)));
+    if (!idx->d_bnorm_max) HIP_TRY(hipMalloc(&idx->d_bnorm_max, 2 * sizeof(uint32_t)));  // the largest norm; the largest loss
     float* norms = nullptr;
     HIP_TRY(hipMalloc(&norms, (size_t)idx->n * sizeof(float)));
-    hipError_t e = launch_fill_u32(idx->d_bnorm_max, 1, 0u, stream);
-    if (e == hipSuccess) e = launch_row_norms(idx->d_vec, idx->n, idx->dim, norms, idx->d_bnorm_max, stream);
+    hipError_t e = launch_fill_u32(idx->d_bnorm_max, 2, 0u, stream);
+    if (e == hipSuccess) e = launch_row_norms(idx->d_vec, idx->n, idx->dim, norms, idx->d_bnorm_max, nullptr, nullptr, stream);
     if (e != hipSuccess) {
         (void)hipFree(norms);
         HIP_TRY(e);
     }
     idx->d_bnorm = norms;  // kept only once its kernel is on the stream
+    return CORAL_OK;
+}
+
+// what the base's rows lose at most when they are rounded to halves (d_bnorm_max[1]), once per index; after
+// ensure_base_norms
+static int ensure_base_loss(coral_index* idx, hipStream_t stream) {
+    if (idx->bloss_ready) return CORAL_OK;
+    HIP_TRY(launch_row_norms(idx->d_vec, idx->n, idx->dim, nullptr, nullptr, nullptr, idx->d_bnorm_max + 1, stream));
+    HIP_TRY(hipStreamSynchronize(stream));
+    idx->bloss_ready = true;
     return CORAL_OK;
 }
 
@@ -161,15 +172,15 @@ private:
 struct FusedScreen {
     bool suits = false;  // the shape does: kc within what list_select_kernel takes, a base large enough to sample
     int64_t tiles = 0, stride = 0, ns = 0, qc = 0, qs = 0, cap = 0;
-    int step = 1, kc = 0;
+    int step = 1, kc = 0, products = 3;
     float *D = nullptr, *tau = nullptr;
     unsigned long long* lists = nullptr;
     unsigned int* cnt = nullptr;
     int *redo = nullptr, *overflow = nullptr;
     char* split = nullptr;
 
-    void plan(const coral_index* idx, int32_t Q, int32_t kc_) {
-        kc = kc_;
+    void plan(const coral_index* idx, int32_t Q, int32_t kc_, int products_) {
+        kc = kc_, products = products_;
         const int64_t n = idx->n, full_tiles = n / 128;
         tiles = (2 * (int64_t)kc * full_tiles + kListCap - 1) / kListCap;
         tiles = std::max<int64_t>(8, (tiles + 7) & ~(int64_t)7);
@@ -198,35 +209,54 @@ struct FusedScreen {
         if (!suits) return;
         mem.reserve(&D, (size_t)qs * ns), mem.reserve(&tau, (size_t)qc);
         mem.reserve(&lists, (size_t)qc * cap), mem.reserve(&cnt, (size_t)qc * coral::kCntStride);
-        mem.reserve(&redo, (size_t)qs), mem.reserve(&overflow, 1);
-        mem.reserve(&split, coral::split_queries_bytes((int)qc, idx->dim));
+        mem.reserve(&redo, (size_t)qs), mem.reserve(&overflow, 2);
+        mem.reserve(&split, coral::split_queries_bytes((int)qc, idx->dim, 3));  // (the larger form: one product may give way to three)
     }
     // *used = false when a list overflowed (sample unlike the base, rows of equal values, too few live points in the
-    // sample): the caller then goes through the matrix
-    int run(coral_index* idx, const float* d_queries, int32_t Q, int32_t have_delete, const float* d_qn, int32_t* d_cid,
-            float* d_cd, hipStream_t stream, bool* used) {
+    // sample): the caller then goes through the matrix; and with one product when the sample says that too many entries
+    // lie where it cannot tell them apart (d_qres: what it loses per query)
+    int run(coral_index* idx, const float* d_queries, int32_t Q, int32_t have_delete, const float* d_qn, const float* d_qres,
+            int32_t* d_cid, float* d_cd, hipStream_t stream, bool* used) {
         *used = false;
         const int64_t n = idx->n;
-        HIP_TRY(coral::launch_fill_u32(reinterpret_cast<uint32_t*>(overflow), 1, 0u, stream));
+        HIP_TRY(coral::launch_fill_u32(reinterpret_cast<uint32_t*>(overflow), 2, 0u, stream));
         const uint32_t* del = have_delete ? idx->d_deleted : nullptr;
+        if (products == 1) {
+            // The kc kept are meant to hold the k best whatever one product lost: kScreenSlack entries may lie too close.
+            // How many do is asked of the sample and 64 queries first: at its kc-th entry; the k-th of the whole base
+            // lies further out, where entries thin out up to twice as fast (as the 1.6th power: 1e-2 against 1e-4 of a
+            // Gaussian).  (Costs 60 us whatever the answer.)
+            const int probe = std::min(Q, 64);
+            int extra = 0;
+            HIP_TRY(coral::launch_split_queries(d_queries, probe, idx->dim, 1, d_qn, split, stream));
+            HIP_TRY(coral::launch_approx_tile(split, idx->d_vec, probe, n, idx->dim, idx->metric, 1, d_qn, idx->d_bnorm, del, 0, D,
+                                              ns, stream, tiles, (int)stride));
+            HIP_TRY(coral::launch_row_select(D, ns, probe, ns, kc, 0, nullptr, 0, redo, stream, tau));
+            HIP_TRY(coral::launch_count_close(D, ns, probe, ns, kc, idx->metric, d_qn, idx->d_bnorm_max, d_qres,
+                                              idx->d_bnorm_max + 1, tau, overflow + 1, stream));
+            HIP_TRY(hipMemcpyAsync(&extra, overflow + 1, sizeof extra, hipMemcpyDeviceToHost, stream));
+            HIP_TRY(hipStreamSynchronize(stream));
+            const double grown = 1.0 + (double)extra / ((double)probe * kc);
+            if ((kc - kScreenSlack) * (std::pow(grown, 1.6) - 1.0) > 0.6 * kScreenSlack) return CORAL_OK;
+        }
         for (int64_t q0 = 0; q0 < Q; q0 += qc) {
             const int nq = (int)std::min<int64_t>(qc, Q - q0);
             const float* qp = d_queries + (size_t)q0 * idx->dim;
             const float* qn = d_qn + q0;
             for (int64_t s0 = 0; s0 < nq; s0 += qs) {
                 const int ms = (int)std::min<int64_t>(qs, nq - s0);
-                HIP_TRY(coral::launch_split_queries(qp + (size_t)s0 * idx->dim, ms, idx->dim, qn + s0, split, stream));
-                HIP_TRY(coral::launch_approx_tile(split, idx->d_vec, ms, n, idx->dim, idx->metric, qn + s0, idx->d_bnorm, del,
+                HIP_TRY(coral::launch_split_queries(qp + (size_t)s0 * idx->dim, ms, idx->dim, products, qn + s0, split, stream));
+                HIP_TRY(coral::launch_approx_tile(split, idx->d_vec, ms, n, idx->dim, idx->metric, products, qn + s0, idx->d_bnorm, del,
                                                   0, D, ns, stream, tiles, (int)stride));
                 HIP_TRY(coral::launch_row_select(D, ns, ms, ns, kc, 0, nullptr, 0, redo, stream, tau + s0));
             }
-            if (nq > qs) HIP_TRY(coral::launch_split_queries(qp, nq, idx->dim, qn, split, stream));
+            if (nq > qs) HIP_TRY(coral::launch_split_queries(qp, nq, idx->dim, products, qn, split, stream));
             HIP_TRY(coral::launch_fill_u32(cnt, (size_t)nq * coral::kCntStride, 0u, stream));
-            HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, qn, idx->d_bnorm, del, tau,
+            HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, products, qn, idx->d_bnorm, del, tau,
                                                 lists, cap, cnt, step, stream));
             if (step > 1) {
                 HIP_TRY(coral::launch_list_shrink(lists, cap, cnt, nq, kc, tau, overflow, stream));
-                HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, qn, idx->d_bnorm, del,
+                HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, products, qn, idx->d_bnorm, del,
                                                     tau, lists, cap, cnt, -step, stream));
             }
             HIP_TRY(coral::launch_list_select(lists, cap, cnt, nq, kc, d_cid + (size_t)q0 * kc, d_cd + (size_t)q0 * kc,
@@ -263,6 +293,95 @@ static int check_knn(const coral_index* idx, int32_t Q, int32_t k, int32_t have_
     return CORAL_OK;
 }
 
+namespace {
+
+// One product per pair pays where the products are what a call takes its time for, from about 0.7 ms of them on (one
+// product against three, k = 10 / 200: 300 000 x 200, 1000 queries (6e10) 598 / 916 us against 642 / 866, 3000 queries 1247 /
+// 2019 against 1625 / 2210; 1M x 200, 10 000 queries 8.9 / 13.4 ms against 15.0 / 19.0; 100 000 x 64, 3000 queries (1.9e10) the
+// same).
+bool one_product_pays(const coral_index* idx, int32_t Q) { return Q >= 256 && (double)Q * (double)idx->n * idx->dim >= 1e11; }
+
+// Screening on the matrix cores, exact distances for the kc candidates of each query, and for the queries whose
+// candidates cannot vouch for the result (bruteforce_mfma.hip): after the screening on one product the one on three,
+// after that the exact passes.
+struct Screening {
+    int products = 3, kc = 0;
+    float *d_qn = nullptr, *d_qres = nullptr, *d_cd = nullptr;
+    int32_t* d_cid = nullptr;
+    int* d_redo = nullptr;
+    FusedScreen fused_screen;
+
+    void reserve(const coral_index* idx, int32_t Q, int32_t k, int products_, KnnScratch& mem) {
+        products = products_, kc = k + kScreenSlack;
+        mem.reserve(&d_qn, (size_t)Q), mem.reserve(&d_qres, (size_t)Q), mem.reserve(&d_cid, (size_t)Q * kc);
+        mem.reserve(&d_cd, (size_t)Q * kc), mem.reserve(&d_redo, (size_t)Q);
+        if (idx->knn_mode == 0) fused_screen.plan(idx, Q, kc, products);
+        fused_screen.reserve(idx, mem);
+    }
+
+    int run(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, int32_t have_delete, int32_t* d_ids, float* d_dists,
+            hipStream_t stream) {
+        if (int rc = coral::ensure_base_norms(idx, stream)) return rc;
+        if (products == 1)
+            if (int rc = coral::ensure_base_loss(idx, stream)) return rc;
+        const float* qres = products == 1 ? d_qres : nullptr;
+        HIP_TRY(coral::launch_row_norms(d_queries, Q, idx->dim, d_qn, nullptr, products == 1 ? d_qres : nullptr, nullptr, stream));
+        bool fused = false;
+        while (fused_screen.suits && !fused) {
+            if (int rc = fused_screen.run(idx, d_queries, Q, have_delete, d_qn, qres, d_cid, d_cd, stream, &fused)) return rc;
+            if (fused || products == 3) break;
+            products = fused_screen.products = 3, qres = nullptr;  // in the same scratch, from the start
+        }
+        if (!fused) products = 3, qres = nullptr;
+        idx->knn_last_fused = fused;
+        if (!fused)
+            if (int rc = knn_passes(idx, d_queries, Q, kc, have_delete, true, d_qn, /*signed distances*/ 0, d_cid, d_cd, stream))
+                return rc;
+        std::vector<int> redo((size_t)Q);
+        HIP_TRY(coral::launch_rerank(d_queries, idx->d_vec, Q, idx->dim, idx->metric, d_cid, d_cd, kc, k, d_qn, idx->d_bnorm_max,
+                                     qres, idx->d_bnorm_max + 1, d_ids, d_dists, d_redo, stream));
+        HIP_TRY(hipMemcpyAsync(redo.data(), d_redo, (size_t)Q * sizeof(int), hipMemcpyDeviceToHost, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+        std::vector<int32_t> rows;
+        for (int32_t q = 0; q < Q; ++q)
+            if (redo[(size_t)q]) rows.push_back(q);
+        if (products == 3) idx->knn_last_redone = (int64_t)rows.size();
+        if (rows.empty()) return CORAL_OK;
+        const int m = (int)rows.size();
+        float *d_rq = nullptr, *d_rd = nullptr;
+        int32_t *d_rows = nullptr, *d_rid = nullptr;
+        KnnScratch mem(idx);
+        mem.reserve(&d_rows, (size_t)m), mem.reserve(&d_rq, (size_t)m * idx->dim);
+        mem.reserve(&d_rid, (size_t)m * k), mem.reserve(&d_rd, (size_t)m * k);
+        HIP_TRY(mem.allocate());
+        int rc = CORAL_OK;
+        hipError_t e = hipMemcpyAsync(d_rows, rows.data(), (size_t)m * sizeof(int32_t), hipMemcpyHostToDevice, stream);
+        if (e == hipSuccess) e = coral::launch_gather_rows(d_queries, idx->dim, d_rows, m, d_rq, stream);
+        if (e == hipSuccess) {
+            rc = products == 1 ? run_on_three(idx, d_rq, m, k, have_delete, d_rid, d_rd, stream)
+                               : knn_passes(idx, d_rq, m, k, have_delete, false, nullptr, idx->metric, d_rid, d_rd, stream);
+            if (rc == CORAL_OK) e = coral::launch_scatter_results(d_rows, m, k, d_rid, d_rd, d_ids, d_dists, stream);
+        }
+        const hipError_t done = hipStreamSynchronize(stream);  // before the scratch and `rows` go
+        if (rc == CORAL_OK) HIP_TRY(e);
+        if (rc == CORAL_OK) HIP_TRY(done);
+        return rc;
+    }
+
+    static int run_on_three(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, int32_t have_delete, int32_t* d_ids,
+                            float* d_dists, hipStream_t stream) {
+        Screening next;
+        KnnScratch mem(idx);
+        next.reserve(idx, Q, k, 3, mem);
+        HIP_TRY(mem.allocate());
+        const int rc = next.run(idx, d_queries, Q, k, have_delete, d_ids, d_dists, stream);
+        if (rc != CORAL_OK) (void)hipStreamSynchronize(stream);  // nothing is in flight when the scratch goes back
+        return rc;
+    }
+};
+
+}  // namespace
+
 // The search of one call.  Host buffers (h_queries, h_ids, h_dists) are staged in the call's scratch; otherwise the
 // queries and results are d_queries, d_ids, d_dists.
 static int knn_call(coral_index* idx, const float* d_queries, const float* h_queries, int32_t Q, int32_t k,
@@ -272,21 +391,14 @@ static int knn_call(coral_index* idx, const float* d_queries, const float* h_que
     const int kc = k + kScreenSlack;
     const bool screen = !(idx->knn_mode == 1 || kc > 2048 || idx->n <= kc);
     const size_t qb = (size_t)Q * idx->dim * sizeof(float), ib = (size_t)Q * k * sizeof(int32_t);
-    float *d_q = nullptr, *d_qn = nullptr, *d_cd = nullptr;
-    int32_t* d_cid = nullptr;
-    int* d_redo = nullptr;
-    FusedScreen fused_screen;
+    float* d_q = nullptr;
+    Screening screening;
     KnnScratch mem(idx);
     if (h_queries) {
         mem.reserve(&d_q, (size_t)Q * idx->dim), mem.reserve(&d_ids, (size_t)Q * k);
         if (h_dists) mem.reserve(&d_dists, (size_t)Q * k);
     }
-    if (screen) {
-        mem.reserve(&d_qn, (size_t)Q), mem.reserve(&d_cid, (size_t)Q * kc), mem.reserve(&d_cd, (size_t)Q * kc);
-        mem.reserve(&d_redo, (size_t)Q);
-        if (idx->knn_mode == 0) fused_screen.plan(idx, Q, kc);
-        fused_screen.reserve(idx, mem);
-    }
+    if (screen) screening.reserve(idx, Q, k, idx->knn_mode == 0 && one_product_pays(idx, Q) ? 1 : 3, mem);
     auto ok = [&](hipError_t e, const char* what) {
         if (e == hipSuccess) return true;
         rc = fail(e == hipErrorOutOfMemory ? CORAL_ERR_MEMORY : CORAL_ERR_DEVICE, "%s failed: %s", what, hipGetErrorString(e));
@@ -303,49 +415,10 @@ static int knn_call(coral_index* idx, const float* d_queries, const float* h_que
     HIP_TRY(hipEventRecord(ev0, stream));
     idx->knn_last_redone = 0;
     idx->knn_last_fused = false;
-    if (!screen) {
+    if (!screen)
         rc = knn_passes(idx, d_queries, Q, k, have_delete, false, nullptr, idx->metric, d_ids, d_dists, stream);
-    } else {
-        // screening on the matrix cores, exact distances for the kc candidates of each query, the exact passes for
-        // the queries whose candidates cannot vouch for the result (bruteforce_mfma.hip)
-        float *d_rq = nullptr, *d_rd = nullptr;
-        int32_t *d_rows = nullptr, *d_rid = nullptr;
-        std::vector<int> redo((size_t)Q);
-        std::vector<int32_t> rows;
-        auto release = [&]() { (void)hipFree(d_rows), (void)hipFree(d_rq), (void)hipFree(d_rid), (void)hipFree(d_rd); };
-        if ((rc = coral::ensure_base_norms(idx, stream)) == CORAL_OK &&
-            ok(coral::launch_row_norms(d_queries, Q, idx->dim, d_qn, nullptr, stream), "query norms")) {
-            bool fused = false;
-            if (fused_screen.suits)
-                rc = fused_screen.run(idx, d_queries, Q, have_delete, d_qn, d_cid, d_cd, stream, &fused);
-            idx->knn_last_fused = fused;
-            if (rc == CORAL_OK && !fused)
-                rc = knn_passes(idx, d_queries, Q, kc, have_delete, true, d_qn, /*signed distances*/ 0, d_cid, d_cd, stream);
-        }
-        if (rc == CORAL_OK &&
-            ok(coral::launch_rerank(d_queries, idx->d_vec, Q, idx->dim, idx->metric, d_cid, d_cd, kc, k, d_qn,
-                                    idx->d_bnorm_max, d_ids, d_dists, d_redo, stream), "rerank") &&
-            ok(hipMemcpyAsync(redo.data(), d_redo, (size_t)Q * sizeof(int), hipMemcpyDeviceToHost, stream), "hipMemcpy") &&
-            ok(hipStreamSynchronize(stream), "synchronize")) {
-            for (int32_t q = 0; q < Q; ++q)
-                if (redo[(size_t)q]) rows.push_back(q);
-        }
-        if (rc == CORAL_OK && !rows.empty()) {
-            const int m = (int)rows.size();
-            if (ok(hipMalloc(&d_rows, (size_t)m * sizeof(int32_t)), "hipMalloc") &&
-                ok(hipMalloc(&d_rq, (size_t)m * idx->dim * sizeof(float)), "hipMalloc") &&
-                ok(hipMalloc(&d_rid, (size_t)m * k * sizeof(int32_t)), "hipMalloc") &&
-                ok(hipMalloc(&d_rd, (size_t)m * k * sizeof(float)), "hipMalloc") &&
-                ok(hipMemcpyAsync(d_rows, rows.data(), (size_t)m * sizeof(int32_t), hipMemcpyHostToDevice, stream), "hipMemcpy") &&
-                ok(coral::launch_gather_rows(d_queries, idx->dim, d_rows, m, d_rq, stream), "gather"))
-                rc = knn_passes(idx, d_rq, m, k, have_delete, false, nullptr, idx->metric, d_rid, d_rd, stream);
-            if (rc == CORAL_OK &&
-                ok(coral::launch_scatter_results(d_rows, m, k, d_rid, d_rd, d_ids, d_dists, stream), "scatter"))
-                ok(hipStreamSynchronize(stream), "synchronize");
-        }
-        idx->knn_last_redone = (int64_t)rows.size();
-        release();
-    }
+    else
+        rc = screening.run(idx, d_queries, Q, k, have_delete, d_ids, d_dists, stream);
     if (rc == CORAL_OK) {
         float ms = 0.f;
         if (ok(hipEventRecord(ev1, stream), "event") && ok(hipEventSynchronize(ev1), "synchronize") &&

@@ -13,6 +13,14 @@
 // accumulation lose), and q.b = hi.hi + hi.lo + lo.hi on v_mfma_f32_32x32x16_f16: three multiplications at sixteen
 // times the rate of the fp32 form.
 //
+// Large batches are first screened on hi.hi alone, a third of the products.  No value of that screening goes anywhere
+// but into the choice of candidates, and the choice stays rigorous: what the missing products amount to is bounded by
+// |q - hi(q)| |b| + |hi(q)| |b - hi(b)| (row_norms_kernel measures both factors; about 3e-4 |q| |b|), the check
+// below takes that much more, and queries that fail it go through the screening on three products.  k + 32 candidates
+// leave room for the entries that one product cannot tell apart wherever distances spread by more than a few
+// thousandths of |q| |b|; whether they do is read off the sample before the base is walked (count_close_kernel).
+// 10 000 x 1 000 000 x 200, k = 100: 18.2 -> 12.0 ms.
+//
 // Error bound, with u = 2^-24 and n2 = |q|^2 + |b|^2.
 // L2.  The inner product is within (6 dim + 12) u |q| |b| and enters twice: (6 dim + 12) u n2.  The two norms are within
 // dim u of themselves, the final additions add 3 u n2, and terms of second order come to less than 14 u n2 at 2048
@@ -37,7 +45,11 @@ namespace coral {
 namespace {
 
 constexpr int MT = 256, NT = 128, BK = 16;  // tile of queries x base points per workgroup, dimensions per LDS stage
-constexpr int kStageA = 2 * MT * BK, kStageB = 2 * NT * BK;  // halves per stage: the hi plane, then the lo plane
+constexpr int kStageA = 2 * MT * BK, kStageB = 2 * NT * BK;  // halves per stage: two planes
+// NP: products per pair and dimension.  3: the planes are the hi and the lo halves of 16 dimensions; 1: the hi halves of
+// 32 dimensions
+template <int NP>
+constexpr int kStageDims = NP == 1 ? 2 * BK : BK;
 
 __device__ __forceinline__ uint32_t mf_ord32(float s) {
     const uint32_t u = __float_as_uint(s);
@@ -48,9 +60,13 @@ __device__ __forceinline__ float mf_unord32(uint32_t o) {
     return __uint_as_float(u);
 }
 
-// |x|^2 per row, and the largest of them (as the bit pattern of a non-negative float)
+// |x|^2 per row, and the largest of them (as the bit pattern of a non-negative float); with res or res_max also a bound on
+// what the row loses when each component of it, scaled as the tile kernel scales it, becomes one half: |x - half(x)|.
+// (Halves below the format's normal range count as lost whole, so the bound holds whether or not the matrix cores
+// take them for zero.  A row of infinite or NaN norm gives an infinite or NaN bound, which no comparison passes.)
 __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict__ x, int64_t n, int dim,
-                                                       float* __restrict__ out, uint32_t* __restrict__ max_bits) {
+                                                       float* __restrict__ out, uint32_t* __restrict__ max_bits,
+                                                       float* __restrict__ res, uint32_t* __restrict__ res_max) {
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     float s = 0.0f;
     if (r < n) {
@@ -59,7 +75,36 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict_
             const float4 v = p[c];
             s = __fmaf_rn(v.x, v.x, s), s = __fmaf_rn(v.y, v.y, s), s = __fmaf_rn(v.z, v.z, s), s = __fmaf_rn(v.w, v.w, s);
         }
-        out[r] = s;
+        if (out) out[r] = s;
+    }
+    if (res || res_max) {
+        float lost = 0.0f;
+        if (r < n) {
+            const int e = mf_scale_exp(s);
+            const float up = mf_pow2(e);
+            float l2 = 0.0f;
+            const float4* p = reinterpret_cast<const float4*>(x + (size_t)r * dim);
+            for (int c = 0; c < dim / 4; ++c) {
+                const float4 v = p[c];
+                const float w[4] = {v.x * up, v.y * up, v.z * up, v.w * up};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float h = (float)(_Float16)w[j];
+                    const float d = fabsf(h) < 6.2e-5f ? w[j] : w[j] - h;
+                    l2 = __fmaf_rn(d, d, l2);
+                }
+            }
+            // (2^-51 <= 2^e <= 2^60; the sum of squares is within dim 2^-24 of itself; the last term for squares that
+            // leave the normal range)
+            lost = (sqrtf(l2) * (1.0f + 2.0e-4f) + 1.0e-17f) * mf_pow2(-e);
+            if (!(s <= 3.0e38f)) lost = __int_as_float(0x7f800000);
+            if (res) res[r] = lost;
+        }
+        if (res_max) {
+            float m = lost;
+            for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+            if ((threadIdx.x & 63) == 0) atomicMax(res_max, __float_as_uint(m));
+        }
     }
     if (max_bits) {
         float m = s;
@@ -68,9 +113,10 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict_
     }
 }
 
-// The queries as the tile kernel reads them: per tile of 256 queries and stage of 16 dimensions, the hi plane and the
-// lo plane, each [256 rows][16 halves] -- a stage of a tile is 16 KB in the order in which it lies in LDS.  Rows beyond
-// the batch and dimensions beyond dim are zero.
+// The queries as the tile kernel reads them: per tile of 256 queries and stage, two planes of [256 rows][16 halves] --
+// a stage of a tile is 16 KB in the order in which it lies in LDS.  NP = 3: the hi and the lo plane of 16 dimensions;
+// NP = 1: the hi planes of 32.  Rows beyond the batch and dimensions beyond dim are zero.
+template <int NP>
 __global__ __launch_bounds__(256) void split_queries_kernel(const float* __restrict__ queries, int nq, int dim, int stages,
                                                            const float* __restrict__ qn, _Float16* __restrict__ out) {
     const int st = blockIdx.x, row = threadIdx.x;
@@ -81,15 +127,18 @@ __global__ __launch_bounds__(256) void split_queries_kernel(const float* __restr
     for (int h = 0; h < 2; ++h) {
         float4 v[2];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int k = st * BK + 8 * h + 4 * u;
-            v[u] = make_float4(0, 0, 0, 0);
-            if (q < nq && k < dim) v[u] = *reinterpret_cast<const float4*>(queries + (size_t)q * dim + k);
+        for (int plane = 0; plane < (NP == 1 ? 2 : 1); ++plane) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int k = st * kStageDims<NP> + plane * BK + 8 * h + 4 * u;
+                v[u] = make_float4(0, 0, 0, 0);
+                if (q < nq && k < dim) v[u] = *reinterpret_cast<const float4*>(queries + (size_t)q * dim + k);
+            }
+            v8h hi, lo;
+            mf_split8(v[0], v[1], s, hi, lo);
+            *reinterpret_cast<v8h*>(dst + plane * MT * BK + 8 * h) = hi;
+            if (NP == 3) *reinterpret_cast<v8h*>(dst + MT * BK + 8 * h) = lo;
         }
-        v8h hi, lo;
-        mf_split8(v[0], v[1], s, hi, lo);
-        *reinterpret_cast<v8h*>(dst + 8 * h) = hi;
-        *reinterpret_cast<v8h*>(dst + MT * BK + 8 * h) = lo;
     }
 }
 
@@ -111,7 +160,7 @@ __global__ __launch_bounds__(256) void split_queries_kernel(const float* __restr
 // come split (split_queries_kernel: every query tile is read by thousands of workgroups); the base is split here, on
 // its way to LDS, eight components per thread and stage under the other wavefronts' multiplications: a split copy of
 // the base would double the index or cost a pass over it per call, which small batches would feel.
-template <bool FUSED, bool L2>
+template <bool FUSED, bool L2, int NP>
 __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16* __restrict__ queries,
                                                               const float* __restrict__ base, int nq, int64_t nb,
                                                               int dim, const float* __restrict__ qn,
@@ -142,9 +191,10 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     const int64_t b0 = (tile_step > 0 ? bt * tile_step : bt + bt / (-tile_step - 1) + 1) * NT;
     const int q0 = qt * MT;
     if (bt >= ntiles || b0 >= nb || qt >= nqt) return;  // padding: the last group of eight base tiles, the last query block
-    const int stages = (dim + BK - 1) / BK;
-    // staging: thread t copies 4 x 16 bytes of the query stage and splits row t/2, dimensions (t&1)*8 .. +8 of the
-    // base; rows beyond the end read the last row instead: their results are never written
+    constexpr int KS = kStageDims<NP>, NB = NP == 1 ? 4 : 2;
+    const int stages = (dim + KS - 1) / KS;
+    // staging: thread t copies 4 x 16 bytes of the query stage and splits row t/2, dimensions (t&1)*8 .. +8 (of either
+    // half of the stage) of the base; rows beyond the end read the last row instead: their results are never written
     const int lrow = tid >> 1, lk = (tid & 1) * 8;
     const _Float16* pa = queries + (size_t)qt * stages * kStageA + tid * 8;
     const int64_t brow = min(b0 + lrow, nb - 1);
@@ -154,30 +204,33 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     // next one's in flight (against one stage ahead: 10 000 x 1 000 000 x 200 in 18.4 instead of 19.1 ms).
     struct Staged {
         v8h a[4];
-        float4 b[2];
+        float4 b[NB];
     } r0, r1;
     auto fetch = [&](int st, Staged& r) {
         st = min(st, stages - 1);
 #pragma unroll
         for (int u = 0; u < 4; ++u) r.a[u] = *reinterpret_cast<const v8h*>(pa + (size_t)st * kStageA + u * 2048);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int d = st * BK + 4 * u;  // beyond dim (a multiple of 4) the row's start is read and then dropped
+        for (int u = 0; u < NB; ++u) {
+            const int d = st * KS + (u >> 1) * BK + 4 * (u & 1);  // beyond dim (a multiple of 4) the row's start is read and then dropped
             r.b[u] = *reinterpret_cast<const float4*>(pb + (d + lk < dim ? d : -lk));
         }
     };
     auto park = [&](int st, int buf, const Staged& r) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) *reinterpret_cast<v8h*>(&sa[buf][u * 2048 + tid * 8]) = r.a[u];
-        float4 b[2] = {r.b[0], r.b[1]};
-        if ((st + 1) * BK > dim) {
+        float4 b[NB];
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
-                if (st * BK + 4 * u + lk >= dim) b[u] = make_float4(0, 0, 0, 0);
+        for (int u = 0; u < NB; ++u) b[u] = r.b[u];
+        if ((st + 1) * KS > dim) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+                if (st * KS + (u >> 1) * BK + 4 * (u & 1) + lk >= dim) b[u] = make_float4(0, 0, 0, 0);
         }
         v8h hi, lo;
         mf_split8(b[0], b[1], bscale, hi, lo);
         *reinterpret_cast<v8h*>(&sb[buf][lrow * BK + lk]) = hi;
+        if constexpr (NP == 1) mf_split8(b[2], b[3], bscale, lo, hi);  // (the plane behind it: the hi halves of 16 dimensions more)
         *reinterpret_cast<v8h*>(&sb[buf][NT * BK + lrow * BK + lk]) = lo;
     };
     v16f acc[4][2];
@@ -188,7 +241,7 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
     const int kh = lane >> 5, m = lane & 31;  // an MFMA operand: lane = row (or column) m, dimensions kh * 8 .. + 7
-    auto multiply = [&](int buf) {
+    auto multiply = [&](int buf, int st) {
         const _Float16* A = &sa[buf][(wr * 128 + m) * BK + kh * 8];
         const _Float16* B = &sb[buf][(wc * 64 + m) * BK + kh * 8];
         v8h ah[4], al[4], bh[2], bl[2];
@@ -204,14 +257,22 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+        if constexpr (NP == 1) {
+            if (st * KS + BK >= dim) return;  // the last stage of 16 dimensions or fewer
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bl[j], acc[i][j], 0, 0, 0);
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
+        }
     };
     fetch(0, r0);
     fetch(1, r1);
@@ -220,15 +281,15 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
 #pragma unroll 1
     for (int st = 0; st + 1 < stages; st += 2) {
         fetch(st + 2, r0);
-        multiply(0);
+        multiply(0, st);
         park(st + 1, 1, r1);
         __syncthreads();
         fetch(st + 3, r1);
-        multiply(1);
+        multiply(1, st + 1);
         park(min(st + 2, stages - 1), 0, r0);
         __syncthreads();
     }
-    if (stages & 1) multiply(0);
+    if (stages & 1) multiply(0, stages - 1);
     __syncthreads();
     // a 32 x 32 block's 16 registers: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32.
     // What the tile's rows and columns contribute comes through LDS, fetched once per workgroup instead of by
@@ -238,6 +299,7 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     float* stau = srsc + MT;
     float* scol = stau + MT;
     float* scsc = scol + NT;
+    float* spre = scsc + NT + 4;
     unsigned int& s_nhit = *reinterpret_cast<unsigned int*>(scsc + NT);
     // (FUSED) the tile's entries that pass: ord(value) << 32 | row << 8 | column
     unsigned long long* shit = reinterpret_cast<unsigned long long*>(&sb[0][0]);
@@ -248,7 +310,14 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
         const float n2 = r < nq ? qn[r] : 0.0f;
         srow[tid] = L2 ? n2 : 0.0f;
         srsc[tid] = mf_pow2(-mf_scale_exp(n2));
-        if constexpr (FUSED) stau[tid] = r < nq ? tau[r] : -inf;
+        if constexpr (FUSED) {
+            const float t = r < nq ? tau[r] : -inf;
+            stau[tid] = t;
+            // What acc rs csc + |b|^2 cannot exceed where the value below does not exceed t.  Either sum is within
+            // 2^-24 (2 |q|^2 + 3 |b|^2 + 2 t) of itself, and |b|^2 <= 2 (|q|^2 + t) wherever the value is at most t (the
+            // inner product's two are the same sum).
+            spre[tid] = L2 ? (t - n2) + 1.0e-6f * (n2 + fabsf(t)) : t;
+        }
     }
     if (tid < NT) {
         // what a column adds to its entries: |b|^2 (L2) or 0, +inf for a tombstoned id; (FUSED) NaN beyond the end of
@@ -280,14 +349,22 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
             const int rl0 = wr * 128 + ti * 32 + 8 * g + 4 * kh;
             const float4 rn4 = *reinterpret_cast<const float4*>(srow + rl0);
             const float4 rs4 = *reinterpret_cast<const float4*>(srsc + rl0);
-            float4 tq4 = make_float4(0, 0, 0, 0);
-            if constexpr (FUSED) tq4 = *reinterpret_cast<const float4*>(stau + rl0);
+            float4 tq4 = make_float4(0, 0, 0, 0), pre4 = tq4;
+            if constexpr (FUSED) tq4 = *reinterpret_cast<const float4*>(stau + rl0), pre4 = *reinterpret_cast<const float4*>(spre + rl0);
             const float rn[4] = {rn4.x, rn4.y, rn4.z, rn4.w}, rs[4] = {rs4.x, rs4.y, rs4.z, rs4.w};
-            const float tq[4] = {tq4.x, tq4.y, tq4.z, tq4.w};
+            const float tq[4] = {tq4.x, tq4.y, tq4.z, tq4.w}, pre[4] = {pre4.x, pre4.y, pre4.z, pre4.w};
 #pragma unroll
             for (int tj = 0; tj < 2; ++tj) {
                 const int cl = wc * 64 + tj * 32 + m;
                 const float bnc = scol[cl], csc = scsc[cl];
+                if constexpr (FUSED && NP == 1) {
+                    // (most fours hold nothing that passes: three instructions an entry and one branch for the four; 3 % of
+                    // the call on one product, nothing on three, which smaller batches with looser bounds take)
+                    bool any = false;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) any |= __fmaf_rn(acc[ti][tj][4 * g + w], rs[w] * csc, bnc) <= pre[w];
+                    if (__ballot(any) == 0ull) continue;
+                }
 #pragma unroll
                 for (int w = 0; w < 4; ++w) {
                     // (|q|^2 + |b|^2) - 2 q.b, or -q.b; a tombstoned column's +inf survives both forms
@@ -318,6 +395,33 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     }
 }
 
+// What one product of hi halves (NP = 1) is off by beside the accumulation: |q.b - hi(q).hi(b)| <= |q - hi(q)| |b| +
+// |hi(q)| |b - hi(b)|, for any row of the index.
+__device__ __forceinline__ float mf_hi_loss(float qn, float qres, const uint32_t* bn_max_bits, const uint32_t* bres_max_bits) {
+    const float bmax = sqrtf(__uint_as_float(*bn_max_bits)), bres = __uint_as_float(*bres_max_bits);
+    return (qres * bmax + (sqrtf(qn) + qres) * bres) * (1.0f + 1.0e-4f);
+}
+
+// How many entries of a sample of the base lie so close behind the bound that NP = 1 could not tell them from the
+// entries before it: one workgroup per query counts those up to tau + 2 loss; *extra += count - kc.
+__global__ __launch_bounds__(256) void count_close_kernel(const float* __restrict__ D, int64_t ldD, int64_t n, int kc, int metric,
+                                                        const float* __restrict__ qn, const uint32_t* __restrict__ bn_max_bits,
+                                                        const float* __restrict__ qres, const uint32_t* __restrict__ bres_max_bits,
+                                                        const float* __restrict__ tau, int* __restrict__ extra) {
+    const int q = blockIdx.x;
+    const float loss = (metric == 0 ? 2.0f : 1.0f) * mf_hi_loss(qn[q], qres[q], bn_max_bits, bres_max_bits);
+    const float upto = tau[q] + 2.0f * loss;
+    int c = 0;
+    __shared__ int s_count;
+    if (threadIdx.x == 0) s_count = 0;
+    __syncthreads();
+    for (int64_t i = threadIdx.x; i < n; i += 256) c += D[(size_t)q * ldD + i] <= upto;
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&s_count, c);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(extra, max(0, s_count - kc));
+}
+
 // One workgroup per query: the kc candidates (ids, -1 = none; approximate signed distances, ascending) are measured
 // in the reference's order (one thread walks the dimensions of one candidate with one fused multiply-add each,
 // include/utils.cuh:254-275, 307-323: the arithmetic of distance_tile_kernel), sorted by (distance, id), and the k
@@ -326,6 +430,7 @@ __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ q
                                                     int dim, int metric, const int32_t* __restrict__ cand_ids,
                                                     const float* __restrict__ cand_d, int kc, int k,
                                                     const float* __restrict__ qn, const uint32_t* __restrict__ bn_max_bits,
+                                                    const float* __restrict__ qres, const uint32_t* __restrict__ bres_max_bits,
                                                     int32_t* __restrict__ ids, float* __restrict__ dists,
                                                     int* __restrict__ redo) {
     extern __shared__ unsigned long long rkeys[];
@@ -393,7 +498,8 @@ __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ q
             const float u = 5.9604645e-8f, un2 = u * n2;
             const float delta = (metric == 0 ? (float)(7 * dim + 32) * un2 + (float)(dim + 8) * (u * fmaxf(worst, 0.0f))
                                              : (float)(4 * dim + 32) * un2) +
-                                (float)(10 * dim + 40) * 1.4e-45f;
+                                (float)(10 * dim + 40) * 1.4e-45f +
+                                (qres ? (metric == 0 ? 2.0f : 1.0f) * mf_hi_loss(qn[q], qres[q], bn_max_bits, bres_max_bits) : 0.0f);
             const unsigned long long kth = rkeys[k - 1];
             const float sk = mf_unord32((uint32_t)(kth >> 32));
             if (kth == ~0ull || !(sk < worst - delta)) bad = 1;
@@ -416,30 +522,37 @@ __global__ void scatter_results_kernel(const int32_t* __restrict__ rows, int cou
 
 }  // namespace
 
-hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, hipStream_t stream) {
+hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, float* res, uint32_t* res_max,
+                            hipStream_t stream) {
     const int64_t blocks = (n + 255) / 256;
     if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, dim, out, max_bits);
+    hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, dim, out, max_bits, res, res_max);
     return hipGetLastError();
 }
 
-size_t split_queries_bytes(int nq, int dim) {
-    return (size_t)((nq + MT - 1) / MT) * ((dim + BK - 1) / BK) * kStageA * sizeof(_Float16);
+namespace {
+int stages_of(int dim, int products) { return products == 1 ? (dim + kStageDims<1> - 1) / kStageDims<1> : (dim + BK - 1) / BK; }
+}  // namespace
+
+size_t split_queries_bytes(int nq, int dim, int products) {
+    return (size_t)((nq + MT - 1) / MT) * stages_of(dim, products) * kStageA * sizeof(_Float16);
 }
 
-hipError_t launch_split_queries(const float* queries, int nq, int dim, const float* qn, void* out, hipStream_t stream) {
-    const int stages = (dim + BK - 1) / BK, tiles = (nq + MT - 1) / MT;
+hipError_t launch_split_queries(const float* queries, int nq, int dim, int products, const float* qn, void* out,
+                                hipStream_t stream) {
+    const int stages = stages_of(dim, products), tiles = (nq + MT - 1) / MT;
     if (nq <= 0 || tiles > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(split_queries_kernel, dim3((unsigned)stages, (unsigned)tiles), dim3(MT), 0, stream, queries, nq, dim,
+    auto kernel = products == 1 ? split_queries_kernel<1> : split_queries_kernel<3>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)stages, (unsigned)tiles), dim3(MT), 0, stream, queries, nq, dim,
                        stages, qn, static_cast<_Float16*>(out));
     return hipGetLastError();
 }
 
 namespace {
 // the launch geometry: query tiles an XCD keeps in its L2 while it walks the base (about 2 MB of them), and the grid
-bool tile_grid(int nq, int dim, int64_t ntiles, int64_t* hq, unsigned* wgs) {
+bool tile_grid(int nq, int dim, int products, int64_t ntiles, int64_t* hq, unsigned* wgs) {
     const int64_t nqt = (nq + MT - 1) / MT;
-    const int64_t per_tile = (int64_t)((dim + BK - 1) / BK) * kStageA * (int64_t)sizeof(_Float16);
+    const int64_t per_tile = (int64_t)stages_of(dim, products) * kStageA * (int64_t)sizeof(_Float16);
     const int64_t want = std::max<int64_t>(1, ((int64_t)2 << 20) / per_tile);
     const int64_t qblocks = (nqt + want - 1) / want;
     *hq = (nqt + qblocks - 1) / qblocks;
@@ -449,21 +562,22 @@ bool tile_grid(int nq, int dim, int64_t ntiles, int64_t* hq, unsigned* wgs) {
 }
 }  // namespace
 
-hipError_t launch_approx_tile(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric,
+hipError_t launch_approx_tile(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, int products,
                               const float* qn, const float* bn, const uint32_t* deleted, int64_t base_id0, float* D,
                               int64_t ldD, hipStream_t stream, int64_t sample_tiles, int tile_stride) {
     const int64_t ntiles = sample_tiles > 0 ? sample_tiles : (nb + NT - 1) / NT;
     int64_t hq = 0;
     unsigned wgs = 0;
-    if (!tile_grid(nq, dim, ntiles, &hq, &wgs) || tile_stride < 1) return hipErrorInvalidValue;
-    auto kernel = metric == 0 ? approx_tile_mfma_kernel<false, true> : approx_tile_mfma_kernel<false, false>;
+    if (!tile_grid(nq, dim, products, ntiles, &hq, &wgs) || tile_stride < 1) return hipErrorInvalidValue;
+    auto kernel = products == 1 ? (metric == 0 ? approx_tile_mfma_kernel<false, true, 1> : approx_tile_mfma_kernel<false, false, 1>)
+                                : (metric == 0 ? approx_tile_mfma_kernel<false, true, 3> : approx_tile_mfma_kernel<false, false, 3>);
     hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
                        bn, deleted, base_id0, ntiles, tile_stride, (int)hq, D, ldD, (const float*)nullptr,
                        (unsigned long long*)nullptr, (int64_t)0, (unsigned int*)nullptr);
     return hipGetLastError();
 }
 
-hipError_t launch_approx_filter(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric,
+hipError_t launch_approx_filter(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, int products,
                                 const float* qn, const float* bn, const uint32_t* deleted, const float* tau,
                                 unsigned long long* lists, int64_t cap, unsigned int* cnt, int tile_step,
                                 hipStream_t stream) {
@@ -474,20 +588,29 @@ hipError_t launch_approx_filter(const void* queries, const float* base, int nq, 
     if (ntiles == 0) return hipSuccess;  // no tile between the multiples
     int64_t hq = 0;
     unsigned wgs = 0;
-    if (!tile_grid(nq, dim, ntiles, &hq, &wgs)) return hipErrorInvalidValue;
-    auto kernel = metric == 0 ? approx_tile_mfma_kernel<true, true> : approx_tile_mfma_kernel<true, false>;
+    if (!tile_grid(nq, dim, products, ntiles, &hq, &wgs)) return hipErrorInvalidValue;
+    auto kernel = products == 1 ? (metric == 0 ? approx_tile_mfma_kernel<true, true, 1> : approx_tile_mfma_kernel<true, false, 1>)
+                                : (metric == 0 ? approx_tile_mfma_kernel<true, true, 3> : approx_tile_mfma_kernel<true, false, 3>);
     hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
                        bn, deleted, (int64_t)0, ntiles, tile_step, (int)hq, (float*)nullptr, (int64_t)0, tau, lists, cap, cnt);
     return hipGetLastError();
 }
 
 hipError_t launch_rerank(const float* queries, const float* base, int nq, int dim, int metric, const int32_t* cand_ids,
-                         const float* cand_d, int kc, int k, const float* qn, const uint32_t* bn_max_bits, int32_t* ids,
-                         float* dists, int* redo, hipStream_t stream) {
+                         const float* cand_d, int kc, int k, const float* qn, const uint32_t* bn_max_bits, const float* qres,
+                         const uint32_t* bres_max_bits, int32_t* ids, float* dists, int* redo, hipStream_t stream) {
     int P = 2;
     while (P < kc) P <<= 1;
     hipLaunchKernelGGL(rerank_kernel, dim3(nq), dim3(256), (size_t)P * 8, stream, queries, base, dim, metric, cand_ids,
-                       cand_d, kc, k, qn, bn_max_bits, ids, dists, redo);
+                       cand_d, kc, k, qn, bn_max_bits, qres, bres_max_bits, ids, dists, redo);
+    return hipGetLastError();
+}
+
+hipError_t launch_count_close(const float* D, int64_t ldD, int nq, int64_t n, int kc, int metric, const float* qn,
+                              const uint32_t* bn_max_bits, const float* qres, const uint32_t* bres_max_bits, const float* tau,
+                              int* extra, hipStream_t stream) {
+    hipLaunchKernelGGL(count_close_kernel, dim3(nq), dim3(256), 0, stream, D, ldD, n, kc, metric, qn, bn_max_bits, qres,
+                       bres_max_bits, tau, extra);
     return hipGetLastError();
 }
 

@@ -77,6 +77,7 @@ struct coral_index {
     // exact kNN: |b|^2 of every base vector and the bit pattern of the largest (made on first use), and whether the
     // matrix-core screening pass is skipped
     float* d_bnorm = nullptr;
+    bool bloss_ready = false;  // d_bnorm_max[1] is there
     uint32_t* d_bnorm_max = nullptr;
     int knn_mode = 0;             // 0: fused screening, 1: no screening, 2: screening through the distance matrix
     bool knn_last_fused = false;  // the last call's candidates came from the fused screening

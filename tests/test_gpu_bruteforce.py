@@ -393,3 +393,53 @@ def test_bruteforce_ground_truth_at_full_size(orc):
     idx.bruteforce_device(tq.data_ptr(), d_ids.data_ptr(), None, 256, k)
     assert np.array_equal(d_ids.cpu().numpy(), ids[:256])
     idx.close()
+
+
+@pytest.mark.parametrize("law,metric,dim,k,dele", [
+    ("gauss", "l2", 100, 100, False), ("gauss", "l2", 120, 1, True), ("cone", "ip", 132, 10, False),
+    ("cone", "ip", 144, 200, True),
+    ("offset", "l2", 100, 100, False),   # norms far beyond the spread: one product cannot tell the rows apart
+    ("pairs", "l2", 100, 40, False),     # every row twice, and queries among them: ties at every place
+    ("lattice", "l2", 100, 10, False),   # exact in halves, thousands of equal distances
+    ("scales", "l2", 100, 20, False),    # rows of norms 1e-3 .. 1e3: a few decide the bound for all
+    ("tiny", "ip", 100, 20, False),      # components below what scaled halves hold
+])
+def test_screening_on_one_product_answers_what_the_plain_passes_answer(law, metric, dim, k, dele):
+    """Batches large enough to be screened on one product of halves per pair (1e11 pair dimensions; their last stage of
+    32 dimensions is whole, half or less): ids and distance bits are those of the search that measures every pair in
+    the reference's order, whether the candidates vouch for them or the queries go on to three products and beyond."""
+    n, Q = 300000, 3400
+    assert Q * n * dim >= 1e11
+    rng = np.random.RandomState(dim + k)
+    base = synth.gaussian_matrix(5, n, dim)
+    q = synth.shifted_queries(Q, dim, 6, 7, 8)
+    if law == "cone":
+        base = synth.normalize_rows(base)
+        q = synth.normalize_rows(q + 3.0)
+    if law == "offset":
+        base += np.float32(30.0)
+        q += np.float32(30.0)
+    if law == "pairs":
+        base[1::2] = base[::2]
+        q[::2] = base[rng.choice(n, Q // 2, replace=False)]
+    if law == "lattice":
+        base = rng.randint(-2, 3, (n, dim)).astype(np.float32)
+        q = rng.randint(-2, 3, (Q, dim)).astype(np.float32)
+    if law == "scales":
+        base *= (10.0 ** rng.randint(-3, 4, (n, 1))).astype(np.float32)
+    if law == "tiny":
+        base[:, 1:] *= np.float32(1e-7)
+    idx = capi.Index(base, None, None, metric=capi.IP if metric == "ip" else capi.L2)
+    if dele:
+        idx.mark_deleted(rng.choice(n, n // 5, replace=False).astype(np.int32))
+    print("one product", law, metric, dim, k, dele, flush=True)
+    ids, dists, _ = idx.bruteforce(q, k, have_delete=dele)
+    redone = idx.bruteforce_last_redone()
+    idx.bruteforce_exact_only(2)
+    ids3, dists3, _ = idx.bruteforce(q, k, have_delete=dele)
+    assert idx.bruteforce_last_redone() == redone  # what one product leaves open three decide as they did
+    idx.bruteforce_exact_only(True)
+    want_ids, want_d, _ = idx.bruteforce(q, k, have_delete=dele)
+    idx.close()
+    assert np.array_equal(ids, want_ids) and dists.tobytes() == want_d.tobytes()
+    assert np.array_equal(ids3, want_ids) and dists3.tobytes() == want_d.tobytes()
