@@ -183,5 +183,7 @@ void* static_scratch(int device);
 hipError_t launch_verify(const int32_t* res, const int32_t* gt, unsigned long long* hit, int Q, int k,
                          hipStream_t stream);
 hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t stream);
+// clears the four scalars of a launch and copies count floats from src (pinned host memory) to dst
+hipError_t launch_begin_search(uint32_t* scalars, const float* src, float* dst, size_t count, hipStream_t stream);
 
 }  // namespace coral

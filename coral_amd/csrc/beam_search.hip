@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -1095,6 +1096,14 @@ __global__ void fill_u32_kernel(uint32_t* p, size_t n, uint32_t v) {
         p[i] = v;
 }
 
+// count is a multiple of 4
+__global__ __launch_bounds__(256) void begin_search_kernel(uint32_t* scalars, const float4* __restrict__ src,
+                                                          float4* __restrict__ dst, size_t count4) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < 4) scalars[i] = 0u;
+    if (i < count4) dst[i] = src[i];
+}
+
 // ------------------------------------------------------------------ launchers
 
 typedef void (*kernel_fn)(const SearchArgs);
@@ -1282,6 +1291,14 @@ hipError_t launch_verify(const int32_t* res, const int32_t* gt, unsigned long lo
                          hipStream_t stream) {
     hipLaunchKernelGGL(ids_verify_kernel, dim3(Q < 1024 ? Q : 1024), dim3(64), 0, stream, res, gt, hit,
                        Q, k);
+    return hipGetLastError();
+}
+
+hipError_t launch_begin_search(uint32_t* scalars, const float* src, float* dst, size_t count, hipStream_t stream) {
+    const size_t blocks = std::max<size_t>(1, (count / 4 + 255) / 256);
+    if (count % 4 != 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(begin_search_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, scalars,
+                       reinterpret_cast<const float4*>(src), reinterpret_cast<float4*>(dst), count / 4);
     return hipGetLastError();
 }
 

@@ -40,6 +40,8 @@ using coral::fail;
 constexpr int kMaxL = CORAL_MAX_BEAM;  // beams beyond CORAL_MAX_LDS_BEAM live in global memory
 constexpr int kMaxLdsBytes = 160 * 1024;
 constexpr int kStaticLds = 128;  // what the workgroup kernel declares outside its dynamic block (counts, per-wave sums)
+constexpr int kDirectCounters = 1024;  // queries of a batch whose counters the kernels write to pinned memory themselves
+constexpr size_t kPinnedIo = (size_t)256 << 10;  // pinned memory of a call with host buffers: half queries, half results
 constexpr int kLongBeamFrom = 1280;  // best-first: beams longer than this take the long-beam kernel
 
 // bits of a mixed id that a cell of the wavefront kernel's table stores: what the bucket index (a quarter of the
@@ -215,6 +217,8 @@ void coral_index_destroy(coral_index* idx) {
         if (e) (void)hipEventDestroy(e);
     coral::free_build_state(idx);
     if (idx->h_counters) (void)hipHostFree(idx->h_counters);
+    if (idx->h_scalars) (void)hipHostFree(idx->h_scalars);
+    if (idx->h_io) (void)hipHostFree(idx->h_io);
     if (idx->stream) (void)hipStreamDestroy(idx->stream);
     delete idx;
 }
@@ -643,6 +647,7 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         HIP_TRY(hipMalloc(&idx->d_beam, need_beam * sizeof(uint64_t)));
         idx->beam_alloc_words = need_beam;
     }
+    if (!idx->h_scalars) HIP_TRY(hipHostMalloc(&idx->h_scalars, 4 * sizeof(int)));
     // per query: the four traversal counters, then (behind those of the whole batch) the four counts of what it read
     const size_t need_counters = (size_t)Q * 8;
     if (need_counters > idx->counters_alloc) {
@@ -820,10 +825,10 @@ static coral::SearchArgs search_args(const coral_index* idx, const coral_search_
     return a;
 }
 
-int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, float* d_dists,
-                     int32_t Q, int32_t k, int32_t policy, int32_t have_delete, void* stream_,
-                     coral_stats* stats) {
-    if (!idx || !d_queries || !d_ids) return fail(CORAL_ERR_ARG, "null argument");
+// h_queries: null, or queries in pinned memory that are to be brought to d_queries first; d_ids and d_dists may be pinned
+// memory too (all of it small: the kernels then read and write it where it lies)
+static int search_launch(coral_index* idx, const float* d_queries, const float* h_queries, int32_t* d_ids, float* d_dists,
+                         int32_t Q, int32_t k, int32_t policy, int32_t have_delete, void* stream_, coral_stats* stats) {
     if (!idx->prepared) return fail(CORAL_ERR_STATE, "coral_search_prepare has not been called");
     if (Q <= 0 || Q > idx->Q)
         return fail(CORAL_ERR_ARG, "Q=%d exceeds the prepared batch of %d", Q, idx->Q);
@@ -837,7 +842,10 @@ int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, f
 
     const coral_search_plan& plan = idx->plan;
     coral::SearchArgs a = search_args(idx, plan, d_queries, d_ids, d_dists, Q, k, policy, have_delete);
-    a.counters = idx->d_counters, a.spill = idx->d_spill, a.beam_scratch = idx->d_beam;
+    // The counters of a small batch go straight to pinned memory (32 bytes a query): the copy and its wait would take as
+    // long as many such searches.
+    const bool direct_counters = Q <= kDirectCounters;
+    a.counters = direct_counters ? idx->h_counters : idx->d_counters, a.spill = idx->d_spill, a.beam_scratch = idx->d_beam;
     a.next_qid = idx->d_scalars, a.spill_count = idx->d_scalars + 1;
 
     const bool wave_kernel = policy == CORAL_POLICY_BEST_FIRST && idx->bf_ready;
@@ -854,7 +862,8 @@ int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, f
     for (hipEvent_t& e : idx->ev)
         if (!e) HIP_TRY(hipEventCreate(&e));
     hipEvent_t ev0 = idx->ev[0], evk = idx->ev[1], ev1 = idx->ev[2];
-    HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_scalars, 4, 0u, stream));
+    HIP_TRY(coral::launch_begin_search((uint32_t*)idx->d_scalars, h_queries, const_cast<float*>(d_queries),
+                                       h_queries ? (size_t)Q * idx->dim : 0, stream));
 #ifdef CORAL_PHASE_TIMERS
     if (!idx->d_phase) HIP_TRY(hipMalloc(&idx->d_phase, 8 * sizeof(unsigned long long)));
     HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_phase, 16, 0u, stream));
@@ -900,16 +909,23 @@ int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, f
         HIP_TRY(coral::launch_search(a, plan.big, wgs, plan.threads, plan.lds_bytes, stream));
     }
     HIP_TRY(hipEventRecord(evk, stream));
-    HIP_TRY(hipMemcpyAsync(idx->h_counters, idx->d_counters, (size_t)Q * 8 * sizeof(int32_t),
-                           hipMemcpyDeviceToHost, stream));
-    HIP_TRY(hipEventRecord(ev1, stream));
-    HIP_TRY(hipEventSynchronize(ev1));
+    // what outgrew a table in LDS is counted in device memory; a bitmap of all ids, and the wavefront kernels, never do
+    const bool wants_scalars = !wave_kernel && !(policy == CORAL_POLICY_BEST_FIRST && idx->bf_shared) && !plan.direct;
+    if (!direct_counters)
+        HIP_TRY(hipMemcpyAsync(idx->h_counters, idx->d_counters, (size_t)Q * 8 * sizeof(int32_t), hipMemcpyDeviceToHost, stream));
+    int* scal = idx->h_scalars;
+    scal[1] = scal[2] = 0;
+    if (wants_scalars) HIP_TRY(hipMemcpyAsync(scal, idx->d_scalars, 3 * sizeof(int), hipMemcpyDeviceToHost, stream));
+    hipEvent_t last = evk;
+    if (!direct_counters || wants_scalars) {
+        HIP_TRY(hipEventRecord(ev1, stream));
+        last = ev1;
+    }
+    HIP_TRY(hipEventSynchronize(last));
     float ms = 0.f, ms_kernel = 0.f;
-    HIP_TRY(hipEventElapsedTime(&ms, ev0, ev1));
     HIP_TRY(hipEventElapsedTime(&ms_kernel, ev0, evk));
-    int scal[3] = {0, 0, 0};
-    HIP_TRY(hipMemcpyAsync(scal, idx->d_scalars, sizeof scal, hipMemcpyDeviceToHost, stream));
-    HIP_TRY(hipStreamSynchronize(stream));
+    ms = ms_kernel;
+    if (last != evk) HIP_TRY(hipEventElapsedTime(&ms, ev0, ev1));
 #ifdef CORAL_PHASE_TIMERS
     {
         unsigned long long t[8];
@@ -959,6 +975,13 @@ int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, f
     }
     if (stats) *stats = sum;
     return CORAL_OK;
+}
+
+int coral_search_gpu(coral_index* idx, const float* d_queries, int32_t* d_ids, float* d_dists,
+                     int32_t Q, int32_t k, int32_t policy, int32_t have_delete, void* stream_,
+                     coral_stats* stats) {
+    if (!idx || !d_queries || !d_ids) return fail(CORAL_ERR_ARG, "null argument");
+    return search_launch(idx, d_queries, nullptr, d_ids, d_dists, Q, k, policy, have_delete, stream_, stats);
 }
 
 int coral_search_gpu_noalloc(coral_index* idx, const float* d_queries, int32_t* d_ids, float* d_dists, int32_t Q,
@@ -1100,6 +1123,25 @@ int coral_search(coral_index* idx, const float* h_queries, int32_t Q, int32_t k,
     const size_t qbytes = (size_t)Q * idx->dim * sizeof(float);
     const size_t ibytes = (size_t)Q * k * sizeof(int32_t), dbytes = (size_t)Q * k * sizeof(float);
     HIP_TRY(grow((void**)&idx->d_io_q, &idx->io_q_bytes, qbytes));
+    // A small call goes through one block of pinned memory: the queries are copied into it here and fetched by the kernel
+    // that clears the launch's counters, the results are written to it by the search itself.  Five copies and as many
+    // waits through the runtime took longer than the search of one query (100 000 x 128, L = 64: kernel 64 us, call 162 us;
+    // now 91).
+    if (qbytes <= kPinnedIo / 2 && ibytes + dbytes <= kPinnedIo / 2) {
+        if (!idx->h_io) HIP_TRY(hipHostMalloc(&idx->h_io, kPinnedIo));
+        unsigned char* io = static_cast<unsigned char*>(idx->h_io);
+        float* hq = reinterpret_cast<float*>(io);
+        int32_t* hi = reinterpret_cast<int32_t*>(io + kPinnedIo / 2);
+        float* hd = reinterpret_cast<float*>(io + kPinnedIo / 2 + ibytes);
+        std::memcpy(hq, h_queries, qbytes);
+        const int rc = search_launch(idx, idx->d_io_q, hq, hi, h_dists ? hd : nullptr, Q, k, policy, have_delete, nullptr, stats);
+        if (rc != CORAL_OK) return rc;
+        std::memcpy(h_ids, hi, ibytes);
+        if (h_dists) std::memcpy(h_dists, hd, dbytes);
+        return CORAL_OK;
+    }
+    HIP_TRY(grow((void**)&idx->d_io_ids, &idx->io_ids_bytes, ibytes));
+    if (h_dists) HIP_TRY(grow((void**)&idx->d_io_dists, &idx->io_dists_bytes, dbytes));
     HIP_TRY(grow((void**)&idx->d_io_ids, &idx->io_ids_bytes, ibytes));
     if (h_dists) HIP_TRY(grow((void**)&idx->d_io_dists, &idx->io_dists_bytes, dbytes));
     HIP_TRY(hipMemcpy(idx->d_io_q, h_queries, qbytes, hipMemcpyHostToDevice));

@@ -61,6 +61,8 @@ struct coral_index {
     unsigned long long* d_hit = nullptr;
     unsigned long long* d_phase = nullptr;  // debug builds only
     int32_t* h_counters = nullptr;  // pinned, counters_alloc entries
+    int* h_scalars = nullptr;       // pinned, what d_scalars held after a launch
+    void* h_io = nullptr;           // pinned: queries and results of small calls with host buffers
     int last_Q = 0;
     // the entry point that allocates nothing: its last plan (kernel attributes and occupancy are looked up once per
     // (Q, L, policy, screening form)), and whether a launch of it may still be in flight on a stream of the caller's

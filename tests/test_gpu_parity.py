@@ -941,3 +941,25 @@ def test_best_first_with_the_beam_in_registers_at_the_edges_of_its_sizes(orc, n,
         rows = idx.row_counters(Q)
         assert ((rows[:, 0] + rows[:, 1] >= os_[:, 2]) & (rows[:, 1] <= os_[:, 2])).all()
     idx.close()
+
+
+@pytest.mark.parametrize("Q,k,dim", [(1, 1, 4), (31, 100, 1028), (63, 257, 512), (64, 256, 512), (64, 257, 512), (65, 40, 512),
+                                     (1024, 16, 32), (1025, 8, 28)])
+def test_small_calls_with_host_buffers_take_one_block_of_pinned_memory(Q, k, dim):
+    """Queries and results up to and beyond the halves of that block, counters up to and beyond what the kernels write
+    to pinned memory themselves; larger and smaller calls in turn; with and without distances."""
+    n, L = 6000, 300
+    base, nbrs, starts = problem(n, dim, 32, seed=3)
+    q = make_queries(Q, dim, 4)
+    idx = capi.Index(base, nbrs, starts)
+    for policy in (0, 1):
+        big, big_d, _ = idx.search(np.repeat(q, 1200 // Q + 1, axis=0), k, L, policy=policy)  # through the larger buffers
+        cnt = idx.query_counters(Q)
+        step = 1200 // Q + 1
+        ids, dists, st = idx.search(q, k, L, policy=policy)
+        assert np.array_equal(ids, big[::step]) and dists.tobytes() == np.ascontiguousarray(big_d[::step]).tobytes()
+        assert st.hops == int(idx.query_counters(Q)[:, 0].sum()) and st.kernel_s > 0 and st.time_s >= st.kernel_s
+        assert np.array_equal(idx.query_counters(1), cnt[:1])
+        only, none, _ = idx.search(q, k, L, policy=policy, want_dists=False)
+        assert np.array_equal(only, ids) and none is None
+    idx.close()
