@@ -59,6 +59,13 @@ struct SearchArgs {
     // rem_bits is then id_bits - (slots_log2 - 2), at most 14, and dmax is unused.  4: the same with the bucket picked
     // by the inserting wavefront's number instead of by load (for tests of what follows concurrent inserts of one id)
     int32_t bucket_choices;
+    // levels: the visited set is four bits per id in LDS (table_words words): 15 visited, else the level that the row of
+    // levels of the query (level_pitch bytes apart, in memory) gives the id; ranges: what the levels mean (bruteforce.h).
+    // The launch answers queries q_begin .. q_end - 1; the rows of levels and ranges start at q_begin.
+    const unsigned char* levels;
+    const float4* ranges;
+    size_t level_pitch;
+    int32_t q_begin, q_end;
 };
 
 // What the wavefront-per-query best-first kernel (best_first.hip) needs beyond SearchArgs.
@@ -165,7 +172,7 @@ constexpr int kMaxByteRowDimRounds = 2048;  // ... in the workgroup-per-query ke
 hipError_t launch_half_rows(const float* vec, int64_t n, int dim, unsigned char* out, hipStream_t stream);
 // 64-bit words of global scratch one workgroup of a BIG launch needs for a beam of capacity L
 size_t search_beam_stride(int L);
-hipError_t search_kernel_prepare(int dim, bool big, size_t lds_bytes, int threads, int* max_wg_per_cu);
+hipError_t search_kernel_prepare(int dim, bool big, bool levels, size_t lds_bytes, int threads, int* max_wg_per_cu);
 hipError_t launch_search(const SearchArgs& a, bool big, int workgroups, int threads, size_t lds_bytes,
                          hipStream_t stream);
 

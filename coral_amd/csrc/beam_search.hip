@@ -218,8 +218,11 @@ struct WgState {
     uint64_t live;    // key of the worst entry of a full beam, else kKeyMax
 };
 
-template <int G, int CPL, bool BIG>
+// LEVELS: the launch comes with four bits per (query, node) that bound the distance (bruteforce.h), made on the matrix
+// cores for the whole batch.  They are the visited set as well, and nothing is read of most rows a search visits.
+template <int G, int CPL, bool BIG, bool LEVELS>
 __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
+    static_assert(!(BIG && LEVELS), "the levels of all nodes leave LDS no room for what a long beam keeps there");
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, NT = blockDim.x;
     const int lane = tid & 63, wave = tid >> 6, NW = NT >> 6;
@@ -251,6 +254,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
     }
     float* qs = (float*)(olist + a.ocap);
 
+    __shared__ int s_new;  // (levels) new ids of the query
     __shared__ int s_qid, s_ntodo, s_ntodo2, s_ncand, s_nexp, s_cntf, s_cursor, s_nover, s_dup;
     __shared__ int s_wcnt[16];
     // what the query read, by class (thread 0 alone adds to these and writes them out): rows measured on the smaller
@@ -276,13 +280,18 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
 
     for (;;) {
         __syncthreads();
-        if (tid == 0) s_qid = atomicAdd(a.next_qid, 1);
+        if (tid == 0) s_qid = a.q_begin + atomicAdd(a.next_qid, 1), s_new = 0;
         __syncthreads();
         const int qid = s_qid;
-        if (qid >= a.Q) break;
+        if (qid >= a.q_end) break;
         PHASE_DECL;
 
-        for (int i = tid; i < a.table_words; i += NT) table[i] = 0u;
+        if constexpr (LEVELS) {
+            const uint4* row = reinterpret_cast<const uint4*>(a.levels + (size_t)(qid - a.q_begin) * a.level_pitch);
+            for (int i = tid; i < (a.table_words >> 2); i += NT) reinterpret_cast<uint4*>(table)[i] = row[i];
+        } else {
+            for (int i = tid; i < a.table_words; i += NT) table[i] = 0u;
+        }
         for (int i = tid; i < dim; i += NT) qs[i] = a.queries[(size_t)qid * dim + i];
         if (tid == 0) s_ncand = 0, s_cntf = 0, s_nover = 0, s_cursor = 0, s_ntodo2 = 0, s_dup = 0;
         if (tid == 0) s_rows_screened = 0, s_rows_exact = 0, s_beam_words = 0;
@@ -294,11 +303,22 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
             const int c = gl + G * t;
             qreg[t] = c < chunks ? reinterpret_cast<const float4*>(qs)[c] : make_float4(0, 0, 0, 0);
         }
+        // (levels) lane l < 15 of every wavefront: the interval of level l.  A rounding of its ends is covered by the last
+        // factor; level 0 has no ends, level 14 no upper one.
+        float lev_lo = -3.402823466e+38f, lev_hi = __int_as_float(0x7f800000);
+        int my_new = 0;  // new ids that this wavefront met
+        if constexpr (LEVELS) {
+            const float4 range = a.ranges[qid - a.q_begin];
+            const float lo = range.x + (float)lane * range.z, hi = range.x + (float)(lane + 1) * range.z;
+            const float slack = range.w + 1.0e-6f * (fabsf(range.x) + 16.0f * range.z);
+            if (range.y != 0.0f && lane >= 1 && lane < 15) lev_lo = lo - slack;
+            if (range.y != 0.0f && lane >= 1 && lane < 14) lev_hi = hi + slack;
+        }
         // The query in integer codes for the screening on eight-bit rows (search_device.h).  Written by wave 0 alone;
         // first read after the barriers of the seeds' merge.
         signed char* qh8 = reinterpret_cast<signed char*>(qs + ((dim + 3) & ~3));
         signed char* ql8 = qh8 + ((dim + 15) & ~15);
-        if (a.vec8 != nullptr && wave == 0) {
+        if (!LEVELS && a.vec8 != nullptr && wave == 0) {
             float qq, sq, eq;
             code_query(qs, dim, lane, qh8, ql8, qq, sq, eq);
             if (lane == 0) s_qq = qq, s_qscale = sq, s_qerr = eq;
@@ -757,7 +777,8 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
 
         // ---- the rows the screening left open, todo2[0..s_ntodo2): exact distances (entered by every thread after a
         // barrier; the candidates they add must fit the buffer)
-        const bool screening = (a.vec16 != nullptr || a.vec8 != nullptr) && a.policy == 0;
+        const bool screening = !LEVELS && (a.vec16 != nullptr || a.vec8 != nullptr) && a.policy == 0;
+        const int policy = LEVELS ? 0 : a.policy;
         auto flush_exact = [&]() {
             const int n2 = ntodo2_u;
             if (n2 == 0) return;
@@ -800,7 +821,10 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
         const int M = a.M;
         for (int i = tid; i < M; i += NT) {
             const uint32_t id = (uint32_t)a.start_ids[i];
-            vs.test_and_set(id, false);
+            if constexpr (LEVELS)
+                atomicOr(&table[id >> 3], 15u << (4 * (id & 7)));
+            else
+                vs.test_and_set(id, false);
             todo[i] = id;
         }
         __syncthreads();
@@ -809,7 +833,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
         PHASE_MARK(1);
         if (tid == 0) s_cntf = 0, s_rows_exact += M;
         nd = M, nvis = M;
-        if (a.policy == 1) hops = M;
+        if (policy == 1) hops = M;
 
         // ---- rounds
         for (;;) {
@@ -817,7 +841,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
             const int nb0 = st.nb;
             if (tid == 0) s_nexp = 0;
             __syncthreads();
-            if (a.policy == 0) {
+            if (policy == 0) {
                 for (int i0 = 0; i0 < nb0; i0 += NT) {
                     const int i = i0 + tid;
                     uint64_t key = 0;
@@ -863,12 +887,12 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
             __syncthreads();
             const int nexp = s_nexp;
             // (rounds: the scan read the beam's nb0 keys and flagged nexp of them; the expand list is written, then read)
-            if (BIG && tid == 0) s_beam_words += (a.policy == 0 ? 2 * nb0 : 128) + 4 * nexp;
+            if (BIG && tid == 0) s_beam_words += (policy == 0 ? 2 * nb0 : 128) + 4 * nexp;
             PHASE_MARK(2);
             if (nexp == 0) {
                 // a round that finds every entry expanded still counts: the candidates of the round that first
                 // overfilled the beam can all have fallen behind its L entries
-                if (a.policy == 0) ++rounds;
+                if (policy == 0) ++rounds;
                 break;
             }
 
@@ -877,7 +901,8 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
             // ids are requested one chunk ahead -- and the entry whose row they come from two chunks ahead -- so
             // that both waits pass while the chunk before is being measured.  With two workgroups per CU the other
             // workgroup covers those waits and the look-ahead only costs (measured); with one it pays.
-            const int ech = (screening ? min(TCAP, NT) : TCAP) / R;
+            // (levels leave few ids of a chunk: half the list is left free for the next chunk's, so that they collect)
+            const int ech = (LEVELS ? min(TCAP / 2, NT) : screening ? min(TCAP, NT) : TCAP) / R;
             ne += nexp;
             const bool ahead = a.prefetch_rows != 0 && ech * R <= NT;
             const int pe = tid / R, pj = tid - pe * R;  // this thread's entry of a chunk and neighbour slot
@@ -897,6 +922,14 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                 if (tid == 0 && tprev == 0) s_ntodo = 0;
                 __syncthreads();
                 const int total = min(ech, nexp - e0) * R;
+                // (levels) what the round's threshold and the beam's worst entry make of each level: beyond the
+                // threshold, or below it and beyond the worst entry -- counted, and no entry whatever its distance
+                uint32_t lev_gone = 0, lev_counted = 0;
+                if constexpr (LEVELS) {
+                    const float s_live = st.live == kKeyMax ? 3.402823466e+38f : key_s(st.live);
+                    lev_gone = (uint32_t)__ballot(lane < 15 && lev_lo > thr);
+                    lev_counted = (uint32_t)__ballot(lane < 15 && !(lev_lo > thr) && lev_hi < thr && lev_lo > s_live);
+                }
                 for (int f0 = 0; f0 < total; f0 += NT) {
                     const int f = f0 + tid;
                     int v = -1;
@@ -907,7 +940,18 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                         v = a.nbrs[(size_t)elist[e0 + e] * R + (f - e * R)];
                     }
                     bool isnew = false;
-                    if (v >= 0) isnew = vs.test_and_set((uint32_t)v, spill) != 0;
+                    if constexpr (LEVELS) {
+                        // one atomic tells whether the id is new and, if it is, its level
+                        uint32_t level = 15u;
+                        if (v >= 0) level = (atomicOr(&table[v >> 3], 15u << (4 * (v & 7))) >> (4 * (v & 7))) & 15u;
+                        my_new += __popcll(__ballot(level != 15u));
+                        const bool counted = ((lev_counted >> level) & 1u) != 0u;
+                        const uint64_t mc = __ballot(counted);
+                        if (mc && lane == 0) atomicAdd(&s_cntf, __popcll(mc));
+                        isnew = level != 15u && !counted && ((lev_gone >> level) & 1u) == 0u;
+                    } else if (v >= 0) {
+                        isnew = vs.test_and_set((uint32_t)v, spill) != 0;
+                    }
                     const uint64_t m = __ballot(isnew);
                     if (m) {
                         int pos = 0;
@@ -918,7 +962,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                 }
                 __syncthreads();
                 int tall = s_ntodo;
-                if (vs.buckets) {
+                if (!LEVELS && vs.buckets) {
                     // (read by every thread behind the barrier above; the next chunk's inserts lie behind the barrier
                     // at its start)
                     if (s_dup != 0) {
@@ -950,7 +994,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                 const int T = tall - tprev;
                 nd += T;
                 PHASE_MARK(3);
-                if (!screening && ncand_u + T > CCAP) merge();  // merge() starts and ends with a barrier
+                if (!screening && !LEVELS && ncand_u + T > CCAP) merge();  // merge() starts and ends with a barrier
                 PHASE_MARK(5);
                 nvis += T;
                 if (ahead) {
@@ -969,6 +1013,18 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                     } else {
                         tprev = tall;
                     }
+                } else if constexpr (LEVELS) {
+                    // what the levels leave open collects over the chunks of a round, like the screening's
+                    if (e0 + ech >= nexp || tall + ech * R > TCAP) {
+                        if (ncand_u + tall > CCAP) merge();
+                        distance_phase(todo, tall);
+                        __syncthreads();
+                        if (tid == 0) s_rows_exact += tall;
+                        ncand_u = s_ncand;
+                        tprev = 0;
+                    } else {
+                        tprev = tall;
+                    }
                 } else {
                     distance_phase(todo, T);
                     __syncthreads();
@@ -980,7 +1036,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
             if (screening) flush_exact();
             ++rounds;
             const int cntf = s_cntf;
-            if (a.policy == 0) {
+            if (policy == 0) {
                 if (cntf == 0) break;
                 hops += cntf;
             } else {
@@ -989,12 +1045,14 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
             merge();
             PHASE_MARK(5);
             if (tid == 0) s_cntf = 0;
-            if (a.policy == 0 && nb0 + cntf > L) thr = key_s((st.cur ? beam1 : beam0)[L - 1]);
+            if (policy == 0 && nb0 + cntf > L) thr = key_s((st.cur ? beam1 : beam0)[L - 1]);
         }
 
         // ---- output: the k closest live entries, closest first
         {
+            if (LEVELS && lane == 0) atomicAdd(&s_new, my_new);
             __syncthreads();
+            if (LEVELS) nd = M + s_new;
             const uint64_t* beam = st.cur ? beam1 : beam0;
             int32_t* ids_out = a.ids_out + (size_t)qid * a.k;
             float* dists_out = a.dists_out ? a.dists_out + (size_t)qid * a.k : nullptr;
@@ -1038,7 +1096,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                 // unfilled slots: the farthest sentinel (rounds: +-FLT_MAX as the CUDA kernel pads its
                 // beam, src/search_gpu.cu:408; best-first: +-infinity, src/search_in_cpu.cpp:33-35)
                 if (dists_out) {
-                    const float far = a.policy == 1 ? __int_as_float(0x7f800000) : 3.402823466e+38f;
+                    const float far = policy == 1 ? __int_as_float(0x7f800000) : 3.402823466e+38f;
                     dists_out[i] = a.metric == 0 ? far : -far;
                 }
             }
@@ -1048,12 +1106,12 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                 {
                     int32_t* rc = a.counters + ((size_t)a.Q + qid) * 4;
                     // (ids sent to the bitmap in global memory: one atomic each; the clean-up writes them once more)
-                    rc[0] = s_rows_screened, rc[1] = s_rows_exact, rc[2] = s_beam_words, rc[3] = 2 * s_nover;
+                    rc[0] = s_rows_screened, rc[1] = s_rows_exact, rc[2] = s_beam_words, rc[3] = LEVELS ? 0 : 2 * s_nover;
                 }
-                if (s_nover > 0) atomicAdd(a.spill_count, 1);
+                if (!LEVELS && s_nover > 0) atomicAdd(a.spill_count, 1);
             }
             // leave the global bitmap clean: word by word from the list, or all of it
-            const int nover = s_nover;
+            const int nover = LEVELS ? 0 : s_nover;
             if (nover > a.ocap) {
                 for (size_t i = tid; i < a.spill_words; i += NT) vs.bitmap[i] = 0u;
             } else {
@@ -1108,19 +1166,21 @@ __global__ __launch_bounds__(256) void begin_search_kernel(uint32_t* scalars, co
 
 typedef void (*kernel_fn)(const SearchArgs);
 
-template <bool BIG>
+template <bool BIG, bool LEVELS>
 static kernel_fn pick_kernel_form(int chunks) {
-    if (chunks <= 16) return beam_search_kernel<16, 1, BIG>;
-    if (chunks <= 32) return beam_search_kernel<32, 1, BIG>;
-    if (chunks <= 64) return beam_search_kernel<64, 1, BIG>;
-    if (chunks <= 128) return beam_search_kernel<64, 2, BIG>;
-    if (chunks <= 256) return beam_search_kernel<64, 4, BIG>;
-    if (chunks <= 512) return beam_search_kernel<64, 8, BIG>;
+    if (chunks <= 16) return beam_search_kernel<16, 1, BIG, LEVELS>;
+    if (chunks <= 32) return beam_search_kernel<32, 1, BIG, LEVELS>;
+    if (chunks <= 64) return beam_search_kernel<64, 1, BIG, LEVELS>;
+    if (chunks <= 128) return beam_search_kernel<64, 2, BIG, LEVELS>;
+    if (chunks <= 256) return beam_search_kernel<64, 4, BIG, LEVELS>;
+    if (chunks <= 512) return beam_search_kernel<64, 8, BIG, LEVELS>;
     return nullptr;
 }
 
-static kernel_fn pick_kernel(int dim, bool big) {
-    return big ? pick_kernel_form<true>(dim / 4) : pick_kernel_form<false>(dim / 4);
+static kernel_fn pick_kernel(int dim, bool big, bool levels) {
+    return levels ? (big ? nullptr : pick_kernel_form<false, true>(dim / 4))
+           : big  ? pick_kernel_form<true, false>(dim / 4)
+                  : pick_kernel_form<false, false>(dim / 4);
 }
 
 size_t search_lds_bytes(int L, int dim, int table_words, int tcap, int ccap, int ocap, bool big, bool screening) {
@@ -1137,8 +1197,8 @@ size_t search_beam_stride(int L) {
     return (2 * Lp + Lp / 2 + 15) & ~(size_t)15;  // [2][Lp] keys + Lp 32-bit ids, a multiple of 128 bytes
 }
 
-hipError_t search_kernel_prepare(int dim, bool big, size_t lds_bytes, int threads, int* max_wg_per_cu) {
-    kernel_fn fn = pick_kernel(dim, big);
+hipError_t search_kernel_prepare(int dim, bool big, bool levels, size_t lds_bytes, int threads, int* max_wg_per_cu) {
+    kernel_fn fn = pick_kernel(dim, big, levels);
     if (!fn) return hipErrorInvalidValue;
     // The limit on a kernel's dynamic LDS is only ever raised: a launch planned earlier (the entry point that
     // allocates nothing keeps its plan) must stay valid after a later plan for a shorter beam.
@@ -1167,8 +1227,11 @@ hipError_t search_kernel_prepare(int dim, bool big, size_t lds_bytes, int thread
 
 hipError_t launch_search(const SearchArgs& a, bool big, int workgroups, int threads, size_t lds_bytes,
                          hipStream_t stream) {
-    kernel_fn fn = pick_kernel(a.dim, big);
+    kernel_fn fn = pick_kernel(a.dim, big, a.levels != nullptr);
     if (!fn) return hipErrorInvalidValue;
+    if (a.levels && (a.policy != 0 || !a.ranges || a.level_pitch % 16 != 0 || (int64_t)a.level_pitch * 2 < a.n ||
+                     (size_t)a.table_words * 4 != a.level_pitch || a.tcap < 2 * a.R))
+        return hipErrorInvalidValue;
     hipLaunchKernelGGL(fn, dim3(workgroups), dim3(threads), lds_bytes, stream, a);
     return hipGetLastError();
 }

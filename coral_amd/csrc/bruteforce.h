@@ -56,6 +56,18 @@ hipError_t launch_rerank(const float* queries, const float* base, int nq, int di
 hipError_t launch_count_close(const float* D, int64_t ldD, int nq, int64_t n, int kc, int metric, const float* qn,
                               const uint32_t* bn_max_bits, const float* qres, const uint32_t* bres_max_bits, const float* tau,
                               int* extra, hipStream_t stream);
+// --- levels: four bits per (query, base point) that bound the distance from below and above (bruteforce_mfma.hip) ---
+// Level l in 0 .. 14 of an entry means: its exact signed distance lies in [origin + l step - E, origin + (l + 1) step + E],
+// the lower end void for l = 0 and the upper one for l = 0 and l = 14; ranges[q] = origin, 1 / step, step, E (1 / step = 0: all
+// levels are 0).  Point i of query q: bits 4 (i & 1) of byte levels[q * level_pitch(n) + i / 2].
+size_t level_pitch(int64_t n);
+// D: [nq][n] approximate distances to a sample of the base, made on one product
+hipError_t launch_level_ranges(const float* D, int64_t ldD, int nq, int n, int dim, int metric, const float* qn,
+                               const uint32_t* bn_max_bits, const float* qres, const uint32_t* bres_max_bits, float4* ranges,
+                               hipStream_t stream);
+// queries: split for one product
+hipError_t launch_levels(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, const float* qn,
+                         const float* bn, const float4* ranges, unsigned char* levels, hipStream_t stream);
 hipError_t launch_scatter_results(const int32_t* rows, int count, int k, const int32_t* src_ids, const float* src_d,
                                   int32_t* dst_ids, float* dst_d, hipStream_t stream);
 }  // namespace coral

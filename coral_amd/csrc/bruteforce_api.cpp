@@ -102,7 +102,7 @@ int ensure_base_norms(coral_index* idx, hipStream_t stream) {
 
 // what the base's rows lose at most when they are rounded to halves (d_bnorm_max[1]), once per index; after
 // ensure_base_norms
-static int ensure_base_loss(coral_index* idx, hipStream_t stream) {
+int ensure_base_loss(coral_index* idx, hipStream_t stream) {
     if (idx->bloss_ready) return CORAL_OK;
     HIP_TRY(launch_row_norms(idx->d_vec, idx->n, idx->dim, nullptr, nullptr, nullptr, idx->d_bnorm_max + 1, stream));
     HIP_TRY(hipStreamSynchronize(stream));

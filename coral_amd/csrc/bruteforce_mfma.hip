@@ -44,6 +44,7 @@ namespace coral {
 
 namespace {
 
+constexpr int kMatrix = 0, kFused = 1, kLevels = 2;  // what a launch of the tile kernel writes
 constexpr int MT = 256, NT = 128, BK = 16;  // tile of queries x base points per workgroup, dimensions per LDS stage
 constexpr int kStageA = 2 * MT * BK, kStageB = 2 * NT * BK;  // halves per stage: two planes
 // NP: products per pair and dimension.  3: the planes are the hi and the lo halves of 16 dimensions; 1: the hi halves of
@@ -64,27 +65,29 @@ __device__ __forceinline__ float mf_unord32(uint32_t o) {
 // what the row loses when each component of it, scaled as the tile kernel scales it, becomes one half: |x - half(x)|.
 // (Halves below the format's normal range count as lost whole, so the bound holds whether or not the matrix cores
 // take them for zero.  A row of infinite or NaN norm gives an infinite or NaN bound, which no comparison passes.)
+// One wavefront per row, lane by lane side by side.  (A thread per row read 16 bytes of a line at a time: the norms of 1M x
+// 200 took 724 us, of a batch of 2000 x 512 as long as 45.)
 __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict__ x, int64_t n, int dim,
                                                        float* __restrict__ out, uint32_t* __restrict__ max_bits,
                                                        float* __restrict__ res, uint32_t* __restrict__ res_max) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    float s = 0.0f;
-    if (r < n) {
+    const int lane = threadIdx.x & 63, chunks = dim >> 2;
+    const int64_t waves = (int64_t)gridDim.x * 4;
+    float most = 0.0f, most_lost = 0.0f;
+    for (int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += waves) {
         const float4* p = reinterpret_cast<const float4*>(x + (size_t)r * dim);
-        for (int c = 0; c < dim / 4; ++c) {
+        float s = 0.0f;
+        for (int c = lane; c < chunks; c += 64) {
             const float4 v = p[c];
             s = __fmaf_rn(v.x, v.x, s), s = __fmaf_rn(v.y, v.y, s), s = __fmaf_rn(v.z, v.z, s), s = __fmaf_rn(v.w, v.w, s);
         }
-        if (out) out[r] = s;
-    }
-    if (res || res_max) {
-        float lost = 0.0f;
-        if (r < n) {
+        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        if (out && lane == 0) out[r] = s;
+        most = s > most ? s : (s != s ? s : most);  // (a NaN stays)
+        if (res || res_max) {
             const int e = mf_scale_exp(s);
             const float up = mf_pow2(e);
             float l2 = 0.0f;
-            const float4* p = reinterpret_cast<const float4*>(x + (size_t)r * dim);
-            for (int c = 0; c < dim / 4; ++c) {
+            for (int c = lane; c < chunks; c += 64) {
                 const float4 v = p[c];
                 const float w[4] = {v.x * up, v.y * up, v.z * up, v.w * up};
 #pragma unroll
@@ -94,22 +97,18 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict_
                     l2 = __fmaf_rn(d, d, l2);
                 }
             }
+            for (int off = 32; off > 0; off >>= 1) l2 += __shfl_xor(l2, off, 64);
             // (2^-51 <= 2^e <= 2^60; the sum of squares is within dim 2^-24 of itself; the last term for squares that
             // leave the normal range)
-            lost = (sqrtf(l2) * (1.0f + 2.0e-4f) + 1.0e-17f) * mf_pow2(-e);
+            float lost = (sqrtf(l2) * (1.0f + 2.0e-4f) + 1.0e-17f) * mf_pow2(-e);
             if (!(s <= 3.0e38f)) lost = __int_as_float(0x7f800000);
-            if (res) res[r] = lost;
-        }
-        if (res_max) {
-            float m = lost;
-            for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-            if ((threadIdx.x & 63) == 0) atomicMax(res_max, __float_as_uint(m));
+            if (res && lane == 0) res[r] = lost;
+            most_lost = fmaxf(most_lost, lost);
         }
     }
-    if (max_bits) {
-        float m = s;
-        for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-        if ((threadIdx.x & 63) == 0) atomicMax(max_bits, __float_as_uint(m));
+    if (lane == 0) {
+        if (max_bits) atomicMax(max_bits, __float_as_uint(most));
+        if (res_max) atomicMax(res_max, __float_as_uint(most_lost));
     }
 }
 
@@ -145,8 +144,12 @@ __global__ __launch_bounds__(256) void split_queries_kernel(const float* __restr
 // D[q][b] ~ signed distance (smaller is closer): |q|^2 + |b|^2 - 2 q.b for L2, -q.b for IP; +inf for tombstoned
 // ids.  One workgroup per 256 x 128 tile (the mapping of blockIdx to tiles is at the head of the kernel), 256
 // threads = 4 wavefronts in 2 x 2, each 128 x 64 of the tile as 4 x 2 MFMA blocks of 32 x 32.
-// FUSED = false writes the tile into D (column bt * 128 + ..., where bt counts the tiles this launch computes).
-// FUSED = true writes no matrix: an entry goes, as the key ord(value) << 32 | id, to the list of its query if it does
+// MODE = kMatrix writes the tile into D (column bt * 128 + ..., where bt counts the tiles this launch computes).
+// MODE = kLevels (NP = 1) writes four bits per entry: which of fifteen steps of the query's range (origin, step) the
+// value falls into, 0 and 14 open to below and above, entries of rows whose norm is not finite or beyond 1e37 always 0;
+// the matrix is computed with the operands exchanged, so that a lane holds four consecutive base points of one query and
+// packs them by itself.  The tile's levels leave through LDS, 64 bytes per query.
+// MODE = kFused writes no matrix: an entry goes, as the key ord(value) << 32 | id, to the list of its query if it does
 // not exceed the query's bound tau[q] -- cnt[q * kCntStride] entries so far, at most cap kept (a count beyond cap
 // tells the caller that the list is incomplete).  A tile's entries are first gathered in LDS, so that the global
 // counters see one round of atomics per tile instead of one per accumulator register.
@@ -160,7 +163,7 @@ __global__ __launch_bounds__(256) void split_queries_kernel(const float* __restr
 // come split (split_queries_kernel: every query tile is read by thousands of workgroups); the base is split here, on
 // its way to LDS, eight components per thread and stage under the other wavefronts' multiplications: a split copy of
 // the base would double the index or cost a pass over it per call, which small batches would feel.
-template <bool FUSED, bool L2, int NP>
+template <int MODE, bool L2, int NP>
 __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16* __restrict__ queries,
                                                               const float* __restrict__ base, int nq, int64_t nb,
                                                               int dim, const float* __restrict__ qn,
@@ -170,7 +173,10 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
                                                               float* __restrict__ D, int64_t ldD,
                                                               const float* __restrict__ tau,
                                                               unsigned long long* __restrict__ lists, int64_t cap,
-                                                              unsigned int* __restrict__ cnt) {
+                                                              unsigned int* __restrict__ cnt, const float4* __restrict__ ranges,
+                                                              unsigned char* __restrict__ levels, size_t pitch) {
+    constexpr bool FUSED = MODE == kFused;
+    static_assert(MODE != kLevels || NP == 1, "levels are made on one product");
     // A row's 16 dimensions of a plane lie side by side (32 bytes); lane (kh, m) of a wavefront supplies row m's
     // dimensions kh * 8 .. + 7, one 16-byte read, and the 64 lanes of a read cover 2 KB of consecutive addresses.
     __shared__ __align__(16) _Float16 sa[2][kStageA];
@@ -253,25 +259,23 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
         for (int j = 0; j < 2; ++j) bl[j] = *reinterpret_cast<const v8h*>(B + NT * BK + j * 32 * BK);
 #pragma unroll
         for (int i = 0; i < 4; ++i) al[i] = *reinterpret_cast<const v8h*>(A + MT * BK + i * 32 * BK);
+        auto product = [&](const v8h (&x)[4], const v8h (&y)[2]) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bh[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 2; ++j) {
+                    if constexpr (MODE == kLevels)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(y[j], x[i], acc[i][j], 0, 0, 0);
+                    else
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[i], y[j], acc[i][j], 0, 0, 0);
+                }
+        };
+        product(ah, bh);
         if constexpr (NP == 1) {
-            if (st * KS + BK >= dim) return;  // the last stage of 16 dimensions or fewer
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bl[j], acc[i][j], 0, 0, 0);
+            if (st * KS + BK < dim) product(al, bl);  // (the last stage may hold 16 dimensions or fewer)
         } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i], bl[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i], bh[j], acc[i][j], 0, 0, 0);
+            product(ah, bl);
+            product(al, bh);
         }
     };
     fetch(0, r0);
@@ -291,6 +295,54 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
     }
     if (stages & 1) multiply(0, stages - 1);
     __syncthreads();
+    if constexpr (MODE == kLevels) {
+        constexpr int kPitch = NT / 2 + 4;  // bytes of a query's levels in LDS, one bank on from query to query
+        float* scol = reinterpret_cast<float*>(&sb[0][0]);  // what a base point contributes: its inverse scale, |b|^2
+        float* sn2 = scol + NT;
+        unsigned char* slev = reinterpret_cast<unsigned char*>(&sa[0][0]);
+        static_assert(MT * kPitch <= (int)sizeof(sa) && 2 * NT * 4 <= (int)sizeof(sb), "the levels of a tile fit the operand buffers");
+        if (tid < NT) {
+            const int64_t c = b0 + tid;
+            const float n2 = c < nb ? bn[c] : 0.0f;
+            const bool takes_part = n2 <= 1.0e37f;
+            scol[tid] = takes_part ? mf_pow2(-mf_scale_exp(n2)) : 0.0f;
+            sn2[tid] = takes_part ? (L2 ? n2 : 0.0f) : -3.0e38f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int rl = wr * 128 + i * 32 + m, r = q0 + rl;
+            const float n2 = r < nq ? qn[r] : 0.0f;
+            const float4 range = r < nq ? ranges[r] : make_float4(0, 0, 0, 0);  // origin, 1 / step (0: everything is level 0)
+            const float inv = range.y;
+            const float scale = (L2 ? -2.0f : -1.0f) * mf_pow2(-mf_scale_exp(n2)) * inv, off = ((L2 ? n2 : 0.0f) - range.x) * inv;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const int cl = wc * 64 + j * 32 + 8 * g + 4 * kh;
+                    const float4 c4 = *reinterpret_cast<const float4*>(scol + cl), n4 = *reinterpret_cast<const float4*>(sn2 + cl);
+                    const float cs[4] = {c4.x, c4.y, c4.z, c4.w}, cn[4] = {n4.x, n4.y, n4.z, n4.w};
+                    uint32_t four = 0;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        // (a value below the origin, or NaN, converts to 0)
+                        const float u = __fmaf_rn(acc[i][j][4 * g + w] * cs[w], scale, __fmaf_rn(cn[w], inv, off));
+                        four |= (uint32_t)fminf(fmaxf(u, 0.0f), 14.0f) << (4 * w);
+                    }
+                    *reinterpret_cast<uint16_t*>(slev + rl * kPitch + (cl >> 1)) = (uint16_t)four;
+                }
+        }
+        __syncthreads();
+        for (int i = tid; i < MT * 4; i += 256) {
+            const int rl = i >> 2, piece = i & 3;
+            if (q0 + rl >= nq) continue;
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(slev + rl * kPitch + piece * 16);
+            *reinterpret_cast<uint4*>(levels + (size_t)(q0 + rl) * pitch + (size_t)(b0 >> 1) + piece * 16) =
+                make_uint4(src[0], src[1], src[2], src[3]);
+        }
+        return;
+    }
     // a 32 x 32 block's 16 registers: register v of lane l holds row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32.
     // What the tile's rows and columns contribute comes through LDS, fetched once per workgroup instead of by
     // dependent global loads per lane: norm and inverse scale of every row and column (times -2 or -1), the bounds.
@@ -400,6 +452,36 @@ __global__ __launch_bounds__(256, 2) void approx_tile_mfma_kernel(const _Float16
 __device__ __forceinline__ float mf_hi_loss(float qn, float qres, const uint32_t* bn_max_bits, const uint32_t* bres_max_bits) {
     const float bmax = sqrtf(__uint_as_float(*bn_max_bits)), bres = __uint_as_float(*bres_max_bits);
     return (qres * bmax + (sqrtf(qn) + qres) * bres) * (1.0f + 1.0e-4f);
+}
+
+// The range of a query's levels from the distances to a sample of the base (one wavefront per query): fourteen steps from
+// 3.5 standard deviations below the mean to 0.1 above, where a search's thresholds fall from its first round to its last.
+// ranges[q]: origin, 1 / step, step, and the bound E on |the tile kernel's value of an entry - its exact distance|:
+// what one product loses (mf_hi_loss); (7 dim + 32) u n2 for the accumulation, the norms and the final additions (head of
+// this file) and (dim + 8) u d for the reference order, d <= 2 n2; and what the value that is cut into steps is off by,
+// the roundings of its sums of |q|^2, |b|^2, 2 |q| |b| and the origin and of 1 / step, 32 u (n2 + |origin|).  A query or a sample that is
+// not finite gets 1 / step = 0: level 0 everywhere, which says nothing.
+__global__ __launch_bounds__(64) void level_ranges_kernel(const float* __restrict__ D, int64_t ldD, int n, int dim, int metric,
+                                                         const float* __restrict__ qn, const uint32_t* __restrict__ bn_max_bits,
+                                                         const float* __restrict__ qres, const uint32_t* __restrict__ bres_max_bits,
+                                                         float4* __restrict__ ranges) {
+    const int q = blockIdx.x, lane = threadIdx.x;
+    const float* row = D + (size_t)q * ldD;
+    float sum = 0.0f;
+    for (int i = lane; i < n; i += 64) sum += row[i];
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    const float mean = sum / (float)n;
+    float var = 0.0f;
+    for (int i = lane; i < n; i += 64) var = __fmaf_rn(row[i] - mean, row[i] - mean, var);
+    for (int off = 32; off > 0; off >>= 1) var += __shfl_xor(var, off, 64);
+    if (lane != 0) return;
+    const float sd = sqrtf(var / (float)n), origin = mean - 3.5f * sd, step = sd * (3.6f / 14.0f), inv = 1.0f / step;
+    const float n2 = qn[q] + fminf(__uint_as_float(*bn_max_bits), 1.0e37f);  // (larger rows take no part)
+    const float u = 5.9604645e-8f;
+    const float E = (metric == 0 ? 2.0f : 1.0f) * mf_hi_loss(qn[q], qres[q], bn_max_bits, bres_max_bits) +
+                    (float)(9 * dim + 64) * u * n2 + 32.0f * u * (n2 + fabsf(origin)) + 1.0e-30f;
+    const bool good = n2 <= 1.0e38f && E <= 1.0e38f && inv <= 1.0e20f && inv >= 1.0e-15f && fabsf(origin) <= 1.0e38f;
+    ranges[q] = good ? make_float4(origin, inv, step, E) : make_float4(0, 0, 0, 0);
 }
 
 // How many entries of a sample of the base lie so close behind the bound that NP = 1 could not tell them from the
@@ -524,8 +606,8 @@ __global__ void scatter_results_kernel(const int32_t* __restrict__ rows, int cou
 
 hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, float* res, uint32_t* res_max,
                             hipStream_t stream) {
-    const int64_t blocks = (n + 255) / 256;
-    if (blocks <= 0 || blocks > 0x7fffffff) return hipErrorInvalidValue;
+    if (n <= 0) return hipErrorInvalidValue;
+    const int64_t blocks = std::min<int64_t>((n + 3) / 4, 8192);
     hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, dim, out, max_bits, res, res_max);
     return hipGetLastError();
 }
@@ -569,11 +651,12 @@ hipError_t launch_approx_tile(const void* queries, const float* base, int nq, in
     int64_t hq = 0;
     unsigned wgs = 0;
     if (!tile_grid(nq, dim, products, ntiles, &hq, &wgs) || tile_stride < 1) return hipErrorInvalidValue;
-    auto kernel = products == 1 ? (metric == 0 ? approx_tile_mfma_kernel<false, true, 1> : approx_tile_mfma_kernel<false, false, 1>)
-                                : (metric == 0 ? approx_tile_mfma_kernel<false, true, 3> : approx_tile_mfma_kernel<false, false, 3>);
+    auto kernel = products == 1 ? (metric == 0 ? approx_tile_mfma_kernel<kMatrix, true, 1> : approx_tile_mfma_kernel<kMatrix, false, 1>)
+                                : (metric == 0 ? approx_tile_mfma_kernel<kMatrix, true, 3> : approx_tile_mfma_kernel<kMatrix, false, 3>);
     hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
                        bn, deleted, base_id0, ntiles, tile_stride, (int)hq, D, ldD, (const float*)nullptr,
-                       (unsigned long long*)nullptr, (int64_t)0, (unsigned int*)nullptr);
+                       (unsigned long long*)nullptr, (int64_t)0, (unsigned int*)nullptr, (const float4*)nullptr,
+                       (unsigned char*)nullptr, (size_t)0);
     return hipGetLastError();
 }
 
@@ -589,10 +672,35 @@ hipError_t launch_approx_filter(const void* queries, const float* base, int nq, 
     int64_t hq = 0;
     unsigned wgs = 0;
     if (!tile_grid(nq, dim, products, ntiles, &hq, &wgs)) return hipErrorInvalidValue;
-    auto kernel = products == 1 ? (metric == 0 ? approx_tile_mfma_kernel<true, true, 1> : approx_tile_mfma_kernel<true, false, 1>)
-                                : (metric == 0 ? approx_tile_mfma_kernel<true, true, 3> : approx_tile_mfma_kernel<true, false, 3>);
+    auto kernel = products == 1 ? (metric == 0 ? approx_tile_mfma_kernel<kFused, true, 1> : approx_tile_mfma_kernel<kFused, false, 1>)
+                                : (metric == 0 ? approx_tile_mfma_kernel<kFused, true, 3> : approx_tile_mfma_kernel<kFused, false, 3>);
     hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
-                       bn, deleted, (int64_t)0, ntiles, tile_step, (int)hq, (float*)nullptr, (int64_t)0, tau, lists, cap, cnt);
+                       bn, deleted, (int64_t)0, ntiles, tile_step, (int)hq, (float*)nullptr, (int64_t)0, tau, lists, cap, cnt,
+                       (const float4*)nullptr, (unsigned char*)nullptr, (size_t)0);
+    return hipGetLastError();
+}
+
+hipError_t launch_level_ranges(const float* D, int64_t ldD, int nq, int n, int dim, int metric, const float* qn,
+                               const uint32_t* bn_max_bits, const float* qres, const uint32_t* bres_max_bits, float4* ranges,
+                               hipStream_t stream) {
+    hipLaunchKernelGGL(level_ranges_kernel, dim3(nq), dim3(64), 0, stream, D, ldD, n, dim, metric, qn, bn_max_bits, qres,
+                       bres_max_bits, ranges);
+    return hipGetLastError();
+}
+
+size_t level_pitch(int64_t n) { return (size_t)((n + NT - 1) / NT) * (NT / 2); }
+
+hipError_t launch_levels(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, const float* qn,
+                         const float* bn, const float4* ranges, unsigned char* levels, hipStream_t stream) {
+    const int64_t ntiles = (nb + NT - 1) / NT;
+    int64_t hq = 0;
+    unsigned wgs = 0;
+    if (!tile_grid(nq, dim, 1, ntiles, &hq, &wgs)) return hipErrorInvalidValue;
+    auto kernel = metric == 0 ? approx_tile_mfma_kernel<kLevels, true, 1> : approx_tile_mfma_kernel<kLevels, false, 1>;
+    hipLaunchKernelGGL(kernel, dim3(wgs), dim3(256), 0, stream, static_cast<const _Float16*>(queries), base, nq, nb, dim, qn,
+                       bn, (const uint32_t*)nullptr, (int64_t)0, ntiles, 1, (int)hq, (float*)nullptr, (int64_t)0,
+                       (const float*)nullptr, (unsigned long long*)nullptr, (int64_t)0, (unsigned int*)nullptr, ranges, levels,
+                       level_pitch(nb));
     return hipGetLastError();
 }
 

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "beam_search.h"
+#include "bruteforce.h"
 #include "error.h"
 #include "index_internal.h"
 
@@ -42,6 +43,7 @@ constexpr int kMaxLdsBytes = 160 * 1024;
 constexpr int kStaticLds = 128;  // what the workgroup kernel declares outside its dynamic block (counts, per-wave sums)
 constexpr int kDirectCounters = 1024;  // queries of a batch whose counters the kernels write to pinned memory themselves
 constexpr size_t kPinnedIo = (size_t)256 << 10;  // pinned memory of a call with host buffers: half queries, half results
+constexpr size_t kLevelBytes = (size_t)1 << 30;  // levels made at a time
 constexpr int kLongBeamFrom = 1280;  // best-first: beams longer than this take the long-beam kernel
 
 // bits of a mixed id that a cell of the wavefront kernel's table stores: what the bucket index (a quarter of the
@@ -210,6 +212,7 @@ void coral_index_destroy(coral_index* idx) {
     (void)hipFree(idx->d_bnorm);
     (void)hipFree(idx->d_bnorm_max);
     (void)hipFree(idx->knn_block);
+    (void)hipFree(idx->d_level_block);
     (void)hipFree(idx->d_io_q);
     (void)hipFree(idx->d_io_ids);
     (void)hipFree(idx->d_io_dists);
@@ -485,14 +488,14 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
         return fail(CORAL_ERR_ARG, "threads must be 128, 256, 512 or 1024");
     p.lds_bytes = coral::search_lds_bytes(L, idx->dim, p.table_words, tcap, ccap, ocap, p.big, screen);
     int wg_per_cu = 0;
-    HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, p.lds_bytes, threads, &wg_per_cu));
+    HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, false, p.lds_bytes, threads, &wg_per_cu));
     if (wg_per_cu <= 0) return fail(CORAL_ERR_DEVICE, "kernel does not fit the device");
     // A small batch that the chip cannot take at once in workgroups of 512 threads, but can in workgroups of 256 (twice
     // as many per CU where LDS allows), runs in one go instead of two: 1000 queries on a 100 000-node graph at L = 64
     // take 276 us instead of 312.
     if (t.threads == 0 && threads == 512 && !best_first && Q > (int64_t)wg_per_cu * idx->num_cu) {
         int wg256 = 0;
-        if (coral::search_kernel_prepare(idx->dim, p.big, p.lds_bytes, 256, &wg256) == hipSuccess && wg256 > wg_per_cu &&
+        if (coral::search_kernel_prepare(idx->dim, p.big, false, p.lds_bytes, 256, &wg256) == hipSuccess && wg256 > wg_per_cu &&
             Q <= (int64_t)wg256 * idx->num_cu)
             threads = 256, wg_per_cu = wg256;
     }
@@ -508,6 +511,89 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
                  (t.prefetch_rows == 0 && !best_first &&
                   ((wg_per_cu == 1 && !alone) || (idx->dim <= 512 && (int64_t)Q <= 2 * (int64_t)idx->num_cu)));
     p.beam_stride = p.big ? coral::search_beam_stride(L) : 0;
+    *out = p;
+    return CORAL_OK;
+}
+
+// The scratch of the levels of `rows` queries: its bytes and, with a block, where its parts lie.
+struct LevelScratch {
+    unsigned char* levels;
+    float4* ranges;
+    float *qn, *qres, *D;
+    void* split;
+};
+constexpr int kLevelSampleTiles = 4;  // tiles of 128 base points whose distances set a query's range
+static size_t level_block(const coral_index* idx, int rows, void* block, LevelScratch* out) {
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        const size_t here = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return block ? static_cast<unsigned char*>(block) + here : nullptr;
+    };
+    LevelScratch s;
+    s.levels = take((size_t)rows * coral::level_pitch(idx->n));
+    s.ranges = reinterpret_cast<float4*>(take((size_t)rows * sizeof(float4)));
+    s.qn = reinterpret_cast<float*>(take((size_t)rows * sizeof(float)));
+    s.qres = reinterpret_cast<float*>(take((size_t)rows * sizeof(float)));
+    s.D = reinterpret_cast<float*>(take((size_t)rows * kLevelSampleTiles * 128 * sizeof(float)));
+    s.split = take(coral::split_queries_bytes(rows, idx->dim, 1));
+    if (out) *out = s;
+    return at;
+}
+
+// Do levels pay?  Per query they cost what the matrix cores and their way into LDS take of every node, about 0.65 + 0.002
+// dim picoseconds, and spare the rows (bytes each, on codes or in fp32) that a search reads without need, four in five, at
+// 7 TB/s: of x = 45 first visits per beam entry under L2, 1.7 times as many under the inner product, x / (1 + x / c n) as
+// the graph runs out of new nodes (c = 1 / 4 and 3 / 5).  The kernels for rows of more than 512 and 1024 floats spill
+// registers where this form does not: two and three times the bytes stand for that.
+// Measured over 144 launches (30 000 .. 280 000 nodes of 64 .. 1028 floats, L = 32 .. 800, 512 .. 5000 queries), the time with over the
+// time without: spared / cost 1.5 1.13 (100 000 x 128, L = 32); 2.5 0.97 (L = 100); 5.1 0.69 (L = 256); inner product, 1.7 0.84 (200 000 x 512, L = 100);
+// 3.1 0.58 (60 000 x 512, L = 64); 11 0.46 (L = 256); 80 000 x 1028, L = 256, 0.22.  From 3 on, 2 under the inner product.
+// A batch costs another 60 us for its norms, its sample and the launches: 512 queries and more, which spare three times
+// that.  With one workgroup per CU (more than about 140 000 nodes) the waits of a round stand where the rows of up to 256
+// floats were (200 000 x 200, L = 256 / 800: 1.15 / 1.05; under the inner product 512 floats 0.57 / 0.55, 120 000 x 256, L =
+// 800, 0.61).
+static bool levels_pay(const coral_index* idx, const coral_search_plan& base, int32_t Q, int32_t L) {
+    const bool ip = idx->metric == CORAL_IP;
+    const double row = base.screen == 2   ? (double)coral::byte_row_stride(idx->dim)
+                       : base.screen == 1 ? (double)coral::half_row_stride(idx->dim)
+                                          : 4.0 * idx->dim;
+    const double n = (double)idx->n, x = 45.0 * L * (ip ? 1.7 : 1.0), visits = x / (1.0 + x / ((ip ? 0.6 : 0.25) * n));
+    const double spared = 0.8 * visits * row / 7.0e12 * (idx->dim > 1024 ? 3.0 : idx->dim > 512 ? 2.0 : 1.0);
+    const double cost = n * (0.65 + 0.002 * idx->dim) * 1.0e-12;
+    return Q >= 512 && spared >= (ip ? 2.0 : 3.0) * cost && Q * (spared - cost) >= 1.8e-4;
+}
+
+// Levels (bruteforce.h) instead of the visited structure of `base`, for a batch of Q queries with a beam of L: p->levels
+// stays 0 where LDS has no room for them or they would not pay.
+static int plan_levels(coral_index* idx, int32_t Q, int32_t L, const coral_search_plan& base, coral_search_plan* out) {
+    coral_search_plan p = base;
+    const size_t pitch = coral::level_pitch(idx->n);
+    p.levels = 0, out->levels = 0;
+    if (base.big || pitch > (size_t)kMaxLdsBytes || !levels_pay(idx, base, Q, L)) return CORAL_OK;
+    p.direct = 0, p.choices = 0, p.screen = 0, p.slots_log2 = 0, p.spill_words = 0, p.dmax = -1, p.vis_limit = 0x7fffffff;
+    p.ocap = 4, p.table_words = (int)(pitch / 4), p.beam_stride = 0;
+    auto lds_for = [&](int cap) {
+        return coral::search_lds_bytes(L, idx->dim, p.table_words, cap, cap, p.ocap, false, false) + kStaticLds;
+    };
+    int least = 512;
+    while (least < idx->M || least < 2 * idx->R) least <<= 1;
+    if (lds_for(least) > (size_t)kMaxLdsBytes) return CORAL_OK;
+    const bool two = 2 * lds_for(std::max(least, idx->dim > 256 ? 512 : 1024)) <= (size_t)kMaxLdsBytes;
+    // Ids collect up to half the list's size before they are measured: the fewer, the sooner the beam's worst entry
+    // turns away what it can.  Two workgroups per CU want 512 on rows of more than 256 floats, 1024 on narrower ones (60 000
+    // x 512, inner product, L = 256, 10 000 queries, 512 / 1024 / 2048: 8.15 / 8.96 / 10.89 ms; 100 000 x 128: 3.67 / 3.06 /
+    // 3.24); one workgroup of 1024 threads 1024 (200 000 x 512: 13.1 / 12.5 / 13.3).
+    const int cap = std::max(least, two && idx->dim > 256 ? 512 : 1024);
+    if (lds_for(cap) > (size_t)kMaxLdsBytes || (!two && idx->dim <= (idx->metric == CORAL_IP ? 252 : 256))) return CORAL_OK;
+    p.tcap = p.ccap = cap, p.threads = two ? 512 : 1024;
+    p.lds_bytes = lds_for(cap) - kStaticLds;
+    int wg_per_cu = 0;
+    HIP_TRY(coral::search_kernel_prepare(idx->dim, false, true, p.lds_bytes, p.threads, &wg_per_cu));
+    if (wg_per_cu <= 0) return CORAL_OK;
+    p.workgroups = wg_per_cu * idx->num_cu;
+    p.prefetch = wg_per_cu == 1;
+    p.levels = 1;
     *out = p;
     return CORAL_OK;
 }
@@ -792,6 +878,36 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         idx->bf_long = idx->bf_ready;
         idx->bf_bcap = bcap, idx->bf_scap = scap, idx->bf_sshift = sshift, idx->bf_beam_stride = beam_stride;
     }
+    // levels for the whole batch, where the caller leaves the launch to the library
+    idx->level_plan = coral_search_plan{};
+    if (!best_first && !t.visited_slots_log2 && !t.workgroups && !t.threads && !t.beam_in_hbm && !t.prefetch_rows && !t.cand_cap &&
+        !t.screening && !t.visited_choices) {
+        coral_search_plan lp;
+        if (int rc = plan_levels(idx, Q, L, plan, &lp)) return rc;
+        if (lp.levels) {
+            const size_t pitch = coral::level_pitch(idx->n);
+            const int64_t fit = std::max<int64_t>(1, (int64_t)(kLevelBytes / pitch) / 256);
+            const int rows = (int)(std::min<int64_t>(fit, ((int64_t)Q + 255) / 256) * 256);
+            const size_t need = level_block(idx, rows, nullptr, nullptr);
+            if (need > idx->level_block_bytes) {
+                (void)hipFree(idx->d_level_block);
+                idx->d_level_block = nullptr, idx->level_block_bytes = 0;
+                const hipError_t e = hipMalloc(&idx->d_level_block, need);
+                if (e == hipSuccess) {
+                    idx->level_block_bytes = need;
+                } else {
+                    HIP_TRY(e == hipErrorOutOfMemory ? hipSuccess : e);
+                    (void)hipGetLastError();
+                    lp.levels = 0;  // the search runs without
+                }
+            }
+            if (lp.levels) {
+                if (int rc = coral::ensure_base_norms(idx, idx->stream)) return rc;
+                if (int rc = coral::ensure_base_loss(idx, idx->stream)) return rc;
+                idx->level_plan = lp, idx->level_rows = rows;
+            }
+        }
+    }
     HIP_TRY(hipStreamSynchronize(idx->stream));
     idx->Q = Q, idx->L = L, idx->plan = plan;
     idx->prepared_policy = t.policy;
@@ -822,6 +938,7 @@ static coral::SearchArgs search_args(const coral_index* idx, const coral_search_
     a.vec8 = p.screen == 2 ? idx->d_vec8 : nullptr, a.stride8 = coral::byte_row_stride(idx->dim);
     a.tcap2 = p.screen ? coral::search_exact_list_cap(p.tcap) : 0;
     a.scap = p.big ? coral::kBeamSampleKeys : 0;
+    a.q_begin = 0, a.q_end = Q;
     return a;
 }
 
@@ -841,7 +958,8 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
     hipStream_t stream = stream_ ? (hipStream_t)stream_ : idx->stream;
 
     const coral_search_plan& plan = idx->plan;
-    coral::SearchArgs a = search_args(idx, plan, d_queries, d_ids, d_dists, Q, k, policy, have_delete);
+    const bool use_levels = policy == CORAL_POLICY_ROUNDS && idx->level_plan.levels && levels_pay(idx, plan, Q, idx->L);
+    coral::SearchArgs a = search_args(idx, use_levels ? idx->level_plan : plan, d_queries, d_ids, d_dists, Q, k, policy, have_delete);
     // The counters of a small batch go straight to pinned memory (32 bytes a query): the copy and its wait would take as
     // long as many such searches.
     const bool direct_counters = Q <= kDirectCounters;
@@ -904,13 +1022,36 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
         b.vec8 = idx->bf_screen == 2 ? idx->d_vec8 : nullptr, b.stride8 = coral::byte_row_stride(idx->dim);
         b.coded_bytes = idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0;
         HIP_TRY(coral::launch_best_first_shared(a, b, stream));
+    } else if (use_levels) {
+        // the batch in pieces that the scratch holds the levels of
+        const coral_search_plan& lp = idx->level_plan;
+        LevelScratch w;
+        (void)level_block(idx, idx->level_rows, idx->d_level_block, &w);
+        const int64_t tiles = std::min<int64_t>(kLevelSampleTiles, std::max<int64_t>(1, idx->n / 128));
+        const int64_t sampled = std::min<int64_t>(tiles * 128, idx->n);
+        a.levels = w.levels, a.ranges = w.ranges, a.level_pitch = coral::level_pitch(idx->n);
+        for (int q0 = 0; q0 < Q; q0 += idx->level_rows) {
+            const int m = std::min(idx->level_rows, Q - q0);
+            const float* q = d_queries + (size_t)q0 * idx->dim;
+            if (q0) HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_scalars, 1, 0u, stream));
+            HIP_TRY(coral::launch_row_norms(q, m, idx->dim, w.qn, nullptr, w.qres, nullptr, stream));
+            HIP_TRY(coral::launch_split_queries(q, m, idx->dim, 1, w.qn, w.split, stream));
+            HIP_TRY(coral::launch_approx_tile(w.split, idx->d_vec, m, idx->n, idx->dim, idx->metric, 1, w.qn, idx->d_bnorm, nullptr, 0,
+                                              w.D, kLevelSampleTiles * 128, stream, tiles, (int)std::max<int64_t>(1, idx->n / 128 / tiles)));
+            HIP_TRY(coral::launch_level_ranges(w.D, kLevelSampleTiles * 128, m, (int)sampled, idx->dim, idx->metric, w.qn, idx->d_bnorm_max,
+                                               w.qres, idx->d_bnorm_max + 1, w.ranges, stream));
+            HIP_TRY(coral::launch_levels(w.split, idx->d_vec, m, idx->n, idx->dim, idx->metric, w.qn, idx->d_bnorm, w.ranges, w.levels,
+                                         stream));
+            a.q_begin = q0, a.q_end = q0 + m;
+            HIP_TRY(coral::launch_search(a, false, std::min(lp.workgroups, m), lp.threads, lp.lds_bytes, stream));
+        }
     } else {
         const int wgs = std::min(plan.workgroups, (int)Q);
         HIP_TRY(coral::launch_search(a, plan.big, wgs, plan.threads, plan.lds_bytes, stream));
     }
     HIP_TRY(hipEventRecord(evk, stream));
     // what outgrew a table in LDS is counted in device memory; a bitmap of all ids, and the wavefront kernels, never do
-    const bool wants_scalars = !wave_kernel && !(policy == CORAL_POLICY_BEST_FIRST && idx->bf_shared) && !plan.direct;
+    const bool wants_scalars = !wave_kernel && !(policy == CORAL_POLICY_BEST_FIRST && idx->bf_shared) && !plan.direct && !use_levels;
     if (!direct_counters)
         HIP_TRY(hipMemcpyAsync(idx->h_counters, idx->d_counters, (size_t)Q * 8 * sizeof(int32_t), hipMemcpyDeviceToHost, stream));
     int* scal = idx->h_scalars;
@@ -954,7 +1095,7 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
     // there, the next launches get a table twice the size.  (The bucket form turns away only the ids that find their
     // three buckets full, a handful per query at a load where linear probing freezes the table: it takes the larger
     // table only when more than a fiftieth of all first visits went to the bitmap.)
-    const bool lds_table = !(policy == CORAL_POLICY_BEST_FIRST && (idx->bf_ready || idx->bf_shared)) && !plan.big;
+    const bool lds_table = !use_levels && !(policy == CORAL_POLICY_BEST_FIRST && (idx->bf_ready || idx->bf_shared)) && !plan.big;
     bool grow = lds_table && idx->tuning.visited_slots_log2 == 0 && (int64_t)scal[1] * 20 > Q && plan.slots_log2 < 16;
     if (grow && plan.choices != 0 && sum.visited_requests / 2 * 50 <= sum.dist_evals) {
         // few ids left LDS: the larger table is worth taking only if it costs the CU no workgroup
@@ -1082,6 +1223,11 @@ int coral_search_plan_info(const coral_index* idx, coral_plan_info* out) {
         out->kernel = 0;  // (a workgroup per query)
         out->threads = 256, out->workgroups = out->query_slots = idx->bf_slots, out->lds_bytes = idx->bf_shared_lds;
         out->screening = idx->bf_screen, out->visited_form = 1;
+    } else if (idx->prepared_policy == CORAL_POLICY_ROUNDS && idx->level_plan.levels) {
+        const coral_search_plan& lp = idx->level_plan;
+        out->kernel = 0;
+        out->threads = lp.threads, out->workgroups = out->query_slots = std::min(lp.workgroups, idx->Q), out->lds_bytes = (int32_t)lp.lds_bytes;
+        out->screening = 3, out->visited_form = 6, out->todo_cap = lp.tcap, out->cand_cap = lp.ccap;
     } else {
         out->kernel = 0;
         out->threads = p.threads, out->workgroups = p.workgroups, out->lds_bytes = (int32_t)p.lds_bytes;

@@ -32,6 +32,7 @@ struct coral_search_plan {
     size_t lds_bytes = 0;
     size_t spill_words = 0;   // words of one workgroup's overflow bitmap in global memory (0: never used)
     size_t beam_stride = 0;   // 64-bit words of one workgroup's beam block in global memory (0 unless big)
+    int levels = 0;  // the launch takes levels (bruteforce.h); table_words hold them
 };
 
 struct coral_index {
@@ -95,6 +96,12 @@ struct coral_index {
     uint32_t* d_bf_epochs = nullptr;
     size_t bf_stride = 0, bf_alloc_bytes = 0;
     int bf_slots = 0, bf_alloc_slots = 0, bf_rows_in_flight = 8, bf_packed = 0, bf_bitmap_words = 0, bf_shared_lds = 0, bf_bloom_log2 = 0;
+    // rounds policy: the launch for batches whose distances are bounded by levels from the matrix cores (levels = 0: none
+    // planned), and its scratch: the levels of level_rows queries and what makes them
+    coral_search_plan level_plan{};
+    void* d_level_block = nullptr;
+    size_t level_block_bytes = 0;
+    int level_rows = 0;
     bool bf_shared = false;  // best-first: four wavefronts share a query's steps
     int bf_table_log2 = 0, bf_table_rem_bits = 0;
     // ... or, for long beams, with an insert buffer in LDS and the long sorted run of every slot in global memory
@@ -133,5 +140,6 @@ struct coral_index {
 namespace coral {
 void free_build_state(coral_index* idx);
 int ensure_base_norms(coral_index* idx, hipStream_t stream);  // d_bnorm, d_bnorm_max (bruteforce_api.cpp)
+int ensure_base_loss(coral_index* idx, hipStream_t stream);   // d_bnorm_max[1]
 }
 

@@ -233,12 +233,16 @@ typedef struct {
     int32_t threads;         /* per workgroup */
     int32_t workgroups;      /* persistent workgroups (the wavefront kernels: query slots / 4) */
     int32_t lds_bytes;       /* per workgroup */
-    int32_t screening;       /* 0 none, 1 half precision, 2 eight-bit codes */
+    int32_t screening;       /* 0 none, 1 half precision, 2 eight-bit codes, 3 levels: four bits per query and node that bound
+                                the distance, made for the whole batch on the matrix cores (rounds policy, 512 queries and
+                                more, where the launch is left to the library and they pay); rows they settle are read
+                                by no search and counted in no class of coral_search_row_counters */
     int32_t screen_row_bytes;/* bytes of one row of the smaller copy (0 without screening) */
     int32_t visited_form;    /* 0 table of 16-bit cells in LDS + bitmap in global memory, 1 bitmap of all ids in LDS,
                                 2 bytes per node and slot in global memory, 3 packed words in global memory,
                                 4 table of 16-bit cells in LDS in front of form 2 or 3, 5 form 0 with the table in
-                                its bucket form (three candidate buckets of four cells per id) */
+                                its bucket form (three candidate buckets of four cells per id), 6 four bits per id in
+                                LDS: its level, or visited */
     int32_t visited_slots_log2; /* cells of the LDS table (forms 0 and 4), else 0 */
     int32_t beam_in_hbm;     /* the beam (or the long run) lives in global memory */
     int32_t todo_cap, cand_cap; /* LDS list capacities of the workgroup kernel */

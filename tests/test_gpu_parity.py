@@ -963,3 +963,77 @@ def test_small_calls_with_host_buffers_take_one_block_of_pinned_memory(Q, k, dim
         only, none, _ = idx.search(q, k, L, policy=policy, want_dists=False)
         assert np.array_equal(only, ids) and none is None
     idx.close()
+
+
+@pytest.mark.parametrize("law,metric,n,dim,L,M,Q,deleted", [
+    ("gauss", "l2", 20001, 264, 256, 16, 1600, False),   # two workgroups per CU; the base's last tile is nearly empty
+    ("gauss", "ip", 20096, 132, 101, 5, 2400, True),
+    ("gauss", "l2", 30000, 1028, 64, 40, 1024, False),
+    ("gauss", "ip", 9000, 520, 200, 130, 1300, False),
+    ("gauss", "l2", 130000, 260, 400, 16, 17000, False),  # one workgroup per CU, levels made in two pieces
+    ("lattice", "l2", 20000, 264, 256, 16, 1600, False),  # ties at the threshold, exact in halves
+    ("magnitudes", "l2", 20000, 264, 256, 16, 1600, False),
+    ("magnitudes", "ip", 20000, 264, 256, 16, 1600, False),
+    ("offset", "l2", 20000, 264, 256, 16, 1600, False),   # the products' loss is wider than a level
+    ("outliers", "l2", 20000, 264, 256, 16, 1600, False), # rows of 3e18 and more take no part, some not finite
+    ("outliers", "ip", 20000, 264, 256, 16, 1600, False),
+    ("queries", "l2", 20000, 264, 256, 16, 1600, False),  # zero, tiny, huge and not finite queries
+    ("clusters", "l2", 20000, 264, 256, 16, 1600, False),
+])
+def test_levels_from_the_matrix_cores_change_nothing(orc, law, metric, n, dim, L, M, Q, deleted):
+    """Large batches whose rows are settled on four bits per query and node: ids, distance bits and counters are those
+    of a launch without, and the oracle's on the first queries."""
+    m = capi.IP if metric == "ip" else capi.L2
+    rng = np.random.RandomState(n % 1000 + dim)
+    base = synth.gaussian_matrix(77, n, dim)
+    if metric == "ip":
+        base = synth.normalize_rows(base)
+    q = make_queries(Q, dim, 78, metric)
+    if law == "lattice":
+        base = rng.randint(-2, 3, (n, dim)).astype(np.float32)
+        q = rng.randint(-2, 3, (Q, dim)).astype(np.float32)
+    if law == "magnitudes":
+        base *= (10.0 ** rng.randint(-2, 3, (n, 1))).astype(np.float32)
+    if law == "offset":
+        base += np.float32(40.0)
+        q += np.float32(40.0)
+    if law == "clusters":
+        base = (rng.randn(40, dim).astype(np.float32) * 3)[rng.randint(0, 40, n)] + np.float32(0.1) * base
+        q = base[rng.choice(n, Q, replace=False)] + np.float32(0.05) * q
+    nbrs = ragged(gpu_graph(base, 32, metric), 7)
+    if law == "outliers":
+        base[::50] *= np.float32(1e18)
+        base[7::501] *= np.float32(1e25)
+        base[11, 3], base[12, 0] = np.inf, np.nan
+    if law == "queries":
+        q[0], q[1:200:3] = 0.0, q[1:200:3] * np.float32(1e-25)
+        q[2:200:3] *= np.float32(1e15)
+        q[5, 1], q[6, 2] = np.inf, np.nan
+    starts = rng.choice(n, M, replace=False).astype(np.int32)
+    idx = capi.Index(base, nbrs, starts, m)
+    mask = synth.tombstone_mask(n, 3, modulo=4) if deleted else None
+    if deleted:
+        idx.set_deleted(mask)
+    k = min(L, 50)
+    print("levels", law, metric, n, dim, L, M, Q, flush=True)
+    idx.prepare(Q, L, threads=512, screening=-1)
+    want, want_d, _ = idx.search(q, k, L, have_delete=deleted)
+    want_c = idx.query_counters(Q)
+    idx.prepare(Q, L)
+    assert idx.plan_info().visited_form == 6 and idx.plan_info().screening == 3
+    for rep in range(2):
+        ids, dists, st = idx.search(q, k, L, have_delete=deleted)
+        assert np.array_equal(ids, want) and dists.tobytes() == want_d.tobytes()
+        assert np.array_equal(idx.query_counters(Q), want_c) and st.spills == 0
+        assert (idx.row_counters(Q)[:, 1] <= want_c[:, 2]).all()
+    if law == "gauss" and n > 10000:  # most rows are settled without a look at them
+        assert st.exact_rows < 0.7 * st.dist_evals
+    few, few_d, _ = idx.search(q[:100], k, L, have_delete=deleted)  # too few to pay: the launch without
+    assert np.array_equal(few, want[:100]) and few_d.tobytes() == np.ascontiguousarray(want_d[:100]).tobytes()
+    idx.close()
+    if law not in ("outliers", "queries"):
+        s = 40
+        oi, od, os_, _ = orc.search_B(orc.Problem(base, nbrs, starts, mask), q[:s], k, L, metric=m, start_order=WAVE64,
+                                      nbr_order=WAVE64)
+        assert np.array_equal(want[:s], oi) and np.ascontiguousarray(want_d[:s]).tobytes() == od.tobytes()
+        assert np.array_equal(want_c[:s], os_)
