@@ -218,10 +218,17 @@ struct WgState {
     uint64_t live;    // key of the worst entry of a full beam, else kKeyMax
 };
 
-// LEVELS: the launch comes with four bits per (query, node) that bound the distance (bruteforce.h), made on the matrix
-// cores for the whole batch.  They are the visited set as well, and nothing is read of most rows a search visits.
-template <int G, int CPL, bool BIG, bool LEVELS>
+// FORM: 0 takes any launch.  The others leave out what their launches never do, whose arguments the compiler otherwise keeps
+// in scalar registers that it does not have (64 x 1: 174 of them spilled to lanes of vector registers, 103 in form 2; 1M x 200,
+// L = 512, 10 000 queries 16.5 -> 15.8 ms; 250 000 x 200, L = 4096 4.67 -> 4.39; 64 queries on 200 000 x 200, L = 128 78 -> 72 us):
+// rounds policy on a bitmap of all ids, with (2) and without (3) the screening on codes; on the table of cells in its bucket
+// form, with (4) and without (5).
+// 1: the launch comes with four bits per (query, node) that bound the distance (bruteforce.h), made on the matrix cores
+// for the whole batch.  They are the visited set as well, and nothing is read of most rows a search visits.
+template <int G, int CPL, bool BIG, int FORM>
 __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
+    constexpr bool LEVELS = FORM == 1, BITMAP = FORM == 2 || FORM == 3, BUCKETS = FORM == 4 || FORM == 5;
+    constexpr bool CODED = FORM == 2 || FORM == 4, PLAIN = FORM == 3 || FORM == 5;
     static_assert(!(BIG && LEVELS), "the levels of all nodes leave LDS no room for what a long beam keeps there");
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, NT = blockDim.x;
@@ -268,9 +275,9 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
     vs.smask = (uint32_t)slots - 1u, vs.bmask = a.id_bits >= 32 ? 0xffffffffu : (1u << a.id_bits) - 1u;
     vs.rb = a.rem_bits, vs.rmask = (1u << a.rem_bits) - 1u;
     vs.xs = a.id_bits > 1 ? a.id_bits / 2 : 1, vs.dmax = a.dmax, vs.ocap = a.ocap;
-    vs.direct = a.direct_bitmap != 0;
-    vs.buckets = a.bucket_choices != 0, vs.bkmask = ((uint32_t)slots >> 2) - 1u, vs.dupflag = &s_dup;
-    vs.skew = a.bucket_choices == 4 ? wave : -1;
+    vs.direct = BITMAP || (!BUCKETS && a.direct_bitmap != 0);
+    vs.buckets = BUCKETS || (!BITMAP && a.bucket_choices != 0), vs.bkmask = ((uint32_t)slots >> 2) - 1u, vs.dupflag = &s_dup;
+    vs.skew = !BUCKETS && a.bucket_choices == 4 ? wave : -1;
     (void)slots;
 
     constexpr int GPW = 64 / G;                    // row groups per wave
@@ -318,7 +325,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
         // first read after the barriers of the seeds' merge.
         signed char* qh8 = reinterpret_cast<signed char*>(qs + ((dim + 3) & ~3));
         signed char* ql8 = qh8 + ((dim + 15) & ~15);
-        if (!LEVELS && a.vec8 != nullptr && wave == 0) {
+        if ((CODED || (!LEVELS && !PLAIN && a.vec8 != nullptr)) && wave == 0) {
             float qq, sq, eq;
             code_query(qs, dim, lane, qh8, ql8, qq, sq, eq);
             if (lane == 0) s_qq = qq, s_qscale = sq, s_qerr = eq;
@@ -777,8 +784,8 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
 
         // ---- the rows the screening left open, todo2[0..s_ntodo2): exact distances (entered by every thread after a
         // barrier; the candidates they add must fit the buffer)
-        const bool screening = !LEVELS && (a.vec16 != nullptr || a.vec8 != nullptr) && a.policy == 0;
-        const int policy = LEVELS ? 0 : a.policy;
+        const bool screening = CODED || (!LEVELS && !PLAIN && (a.vec16 != nullptr || a.vec8 != nullptr) && a.policy == 0);
+        const int policy = FORM != 0 ? 0 : a.policy;
         auto flush_exact = [&]() {
             const int n2 = ntodo2_u;
             if (n2 == 0) return;
@@ -803,7 +810,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                     flush_exact();
                     n = min(T - off, a.tcap2);
                 }
-                if (a.vec8 != nullptr)
+                if (CODED || a.vec8 != nullptr)
                     screening_phase8(todo + off, n);
                 else
                     screening_phase(todo + off, n);
@@ -918,7 +925,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
             // whole passes of the workgroup, the rest waiting in the list for the next ids, gains nothing: measured.)
             int tprev = 0;  // ids in the todo list from the chunks before, not yet screened
             for (int e0 = 0; e0 < nexp; e0 += ech) {
-                if (!spill && nvis > a.vis_limit) spill = true;
+                if (FORM == 0 && !spill && nvis > a.vis_limit) spill = true;
                 if (tid == 0 && tprev == 0) s_ntodo = 0;
                 __syncthreads();
                 const int total = min(ech, nexp - e0) * R;
@@ -1106,12 +1113,12 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                 {
                     int32_t* rc = a.counters + ((size_t)a.Q + qid) * 4;
                     // (ids sent to the bitmap in global memory: one atomic each; the clean-up writes them once more)
-                    rc[0] = s_rows_screened, rc[1] = s_rows_exact, rc[2] = s_beam_words, rc[3] = LEVELS ? 0 : 2 * s_nover;
+                    rc[0] = s_rows_screened, rc[1] = s_rows_exact, rc[2] = s_beam_words, rc[3] = LEVELS || BITMAP ? 0 : 2 * s_nover;
                 }
-                if (!LEVELS && s_nover > 0) atomicAdd(a.spill_count, 1);
+                if (!LEVELS && !BITMAP && s_nover > 0) atomicAdd(a.spill_count, 1);
             }
             // leave the global bitmap clean: word by word from the list, or all of it
-            const int nover = LEVELS ? 0 : s_nover;
+            const int nover = LEVELS || BITMAP ? 0 : s_nover;
             if (nover > a.ocap) {
                 for (size_t i = tid; i < a.spill_words; i += NT) vs.bitmap[i] = 0u;
             } else {
@@ -1166,21 +1173,35 @@ __global__ __launch_bounds__(256) void begin_search_kernel(uint32_t* scalars, co
 
 typedef void (*kernel_fn)(const SearchArgs);
 
-template <bool BIG, bool LEVELS>
+template <bool BIG, int FORM>
 static kernel_fn pick_kernel_form(int chunks) {
-    if (chunks <= 16) return beam_search_kernel<16, 1, BIG, LEVELS>;
-    if (chunks <= 32) return beam_search_kernel<32, 1, BIG, LEVELS>;
-    if (chunks <= 64) return beam_search_kernel<64, 1, BIG, LEVELS>;
-    if (chunks <= 128) return beam_search_kernel<64, 2, BIG, LEVELS>;
-    if (chunks <= 256) return beam_search_kernel<64, 4, BIG, LEVELS>;
-    if (chunks <= 512) return beam_search_kernel<64, 8, BIG, LEVELS>;
+    constexpr int NARROW = FORM == 2 || FORM == 4 ? 0 : FORM;  // rows of up to 64 floats have no codes
+    if (chunks <= 16) return beam_search_kernel<16, 1, BIG, NARROW>;
+    if (chunks <= 32) return beam_search_kernel<32, 1, BIG, FORM>;
+    if (chunks <= 64) return beam_search_kernel<64, 1, BIG, FORM>;
+    if (chunks <= 128) return beam_search_kernel<64, 2, BIG, FORM>;
+    if (chunks <= 256) return beam_search_kernel<64, 4, BIG, FORM>;
+    if (chunks <= 512) return beam_search_kernel<64, 8, BIG, FORM>;
     return nullptr;
 }
 
-static kernel_fn pick_kernel(int dim, bool big, bool levels) {
-    return levels ? (big ? nullptr : pick_kernel_form<false, true>(dim / 4))
-           : big  ? pick_kernel_form<true, false>(dim / 4)
-                  : pick_kernel_form<false, false>(dim / 4);
+static kernel_fn pick_kernel(int dim, bool big, int form) {
+    switch (form) {
+        case 0: return big ? pick_kernel_form<true, 0>(dim / 4) : pick_kernel_form<false, 0>(dim / 4);
+        case 1: return big ? nullptr : pick_kernel_form<false, 1>(dim / 4);
+        case 2: return big ? pick_kernel_form<true, 2>(dim / 4) : pick_kernel_form<false, 2>(dim / 4);
+        case 3: return big ? pick_kernel_form<true, 3>(dim / 4) : pick_kernel_form<false, 3>(dim / 4);
+        case 4: return big ? nullptr : pick_kernel_form<false, 4>(dim / 4);
+        case 5: return big ? nullptr : pick_kernel_form<false, 5>(dim / 4);
+    }
+    return nullptr;
+}
+
+int search_kernel_form(int policy, bool big, bool direct, int choices, int screen) {
+    if (policy != 0 || screen == 1) return 0;
+    if (direct) return screen == 2 ? 2 : 3;
+    if (choices == 3 && !big) return screen == 2 ? 4 : 5;
+    return 0;
 }
 
 size_t search_lds_bytes(int L, int dim, int table_words, int tcap, int ccap, int ocap, bool big, bool screening) {
@@ -1197,8 +1218,8 @@ size_t search_beam_stride(int L) {
     return (2 * Lp + Lp / 2 + 15) & ~(size_t)15;  // [2][Lp] keys + Lp 32-bit ids, a multiple of 128 bytes
 }
 
-hipError_t search_kernel_prepare(int dim, bool big, bool levels, size_t lds_bytes, int threads, int* max_wg_per_cu) {
-    kernel_fn fn = pick_kernel(dim, big, levels);
+hipError_t search_kernel_prepare(int dim, bool big, int form, size_t lds_bytes, int threads, int* max_wg_per_cu) {
+    kernel_fn fn = pick_kernel(dim, big, form);
     if (!fn) return hipErrorInvalidValue;
     // The limit on a kernel's dynamic LDS is only ever raised: a launch planned earlier (the entry point that
     // allocates nothing keeps its plan) must stay valid after a later plan for a shorter beam.
@@ -1227,7 +1248,11 @@ hipError_t search_kernel_prepare(int dim, bool big, bool levels, size_t lds_byte
 
 hipError_t launch_search(const SearchArgs& a, bool big, int workgroups, int threads, size_t lds_bytes,
                          hipStream_t stream) {
-    kernel_fn fn = pick_kernel(a.dim, big, a.levels != nullptr);
+    const int form = a.levels != nullptr
+                         ? 1
+                         : search_kernel_form(a.policy, big, a.direct_bitmap != 0, a.bucket_choices,
+                                              a.vec8 != nullptr ? 2 : a.vec16 != nullptr ? 1 : 0);
+    kernel_fn fn = pick_kernel(a.dim, big, form);
     if (!fn) return hipErrorInvalidValue;
     if (a.levels && (a.policy != 0 || !a.ranges || a.level_pitch % 16 != 0 || (int64_t)a.level_pitch * 2 < a.n ||
                      (size_t)a.table_words * 4 != a.level_pitch || a.tcap < 2 * a.R))

@@ -487,15 +487,21 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     if (threads != 128 && threads != 256 && threads != 512 && threads != 1024)
         return fail(CORAL_ERR_ARG, "threads must be 128, 256, 512 or 1024");
     p.lds_bytes = coral::search_lds_bytes(L, idx->dim, p.table_words, tcap, ccap, ocap, p.big, screen);
+    // (the kernel that launch_search picks for such a plan; without the memory for the codes the plan is made again)
+    const int form = coral::search_kernel_form(t.policy, p.big, p.direct != 0, p.choices, p.screen);
+    if (form != 0) {  // a call with the other policy runs on the plan through the form for any launch
+        int any = 0;
+        HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, 0, p.lds_bytes, threads, &any));
+    }
     int wg_per_cu = 0;
-    HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, false, p.lds_bytes, threads, &wg_per_cu));
+    HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, form, p.lds_bytes, threads, &wg_per_cu));
     if (wg_per_cu <= 0) return fail(CORAL_ERR_DEVICE, "kernel does not fit the device");
     // A small batch that the chip cannot take at once in workgroups of 512 threads, but can in workgroups of 256 (twice
     // as many per CU where LDS allows), runs in one go instead of two: 1000 queries on a 100 000-node graph at L = 64
     // take 276 us instead of 312.
     if (t.threads == 0 && threads == 512 && !best_first && Q > (int64_t)wg_per_cu * idx->num_cu) {
         int wg256 = 0;
-        if (coral::search_kernel_prepare(idx->dim, p.big, false, p.lds_bytes, 256, &wg256) == hipSuccess && wg256 > wg_per_cu &&
+        if (coral::search_kernel_prepare(idx->dim, p.big, form, p.lds_bytes, 256, &wg256) == hipSuccess && wg256 > wg_per_cu &&
             Q <= (int64_t)wg256 * idx->num_cu)
             threads = 256, wg_per_cu = wg256;
     }
@@ -589,7 +595,7 @@ static int plan_levels(coral_index* idx, int32_t Q, int32_t L, const coral_searc
     p.tcap = p.ccap = cap, p.threads = two ? 512 : 1024;
     p.lds_bytes = lds_for(cap) - kStaticLds;
     int wg_per_cu = 0;
-    HIP_TRY(coral::search_kernel_prepare(idx->dim, false, true, p.lds_bytes, p.threads, &wg_per_cu));
+    HIP_TRY(coral::search_kernel_prepare(idx->dim, false, 1, p.lds_bytes, p.threads, &wg_per_cu));
     if (wg_per_cu <= 0) return CORAL_OK;
     p.workgroups = wg_per_cu * idx->num_cu;
     p.prefetch = wg_per_cu == 1;
