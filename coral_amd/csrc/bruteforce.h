@@ -15,17 +15,22 @@ hipError_t launch_row_select(const float* D, int64_t ldD, int nq, int64_t n, int
 hipError_t launch_merge_segments(const unsigned long long* part, int nq, int nseg, int k, int metric,
                                  int32_t* ids, float* dists, hipStream_t stream);
 // --- the screening pass on the matrix cores (bruteforce_mfma.hip) ---
-// out[r] (optional) = |x_r|^2; *max_bits (optional, zero before) = bit pattern of the largest of them; res[r], *res_max (optional):
+// out[r] (optional) = |x_r|^2; *max_bits (optional, zero before) = bit pattern of the largest of them; *res_max (optional):
 // the same for a bound on |x_r - hi(x_r)|, what one half per component leaves out
-hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, float* res, uint32_t* res_max,
+hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, uint32_t* res_max,
                             hipStream_t stream);
-// the queries in the form the two launches below take them (split into halves, tile by tile); out: that many bytes.
+// the queries in the form the two launches below take them (split into halves, tile by tile) into out (that many bytes),
+// qn[q] = |q|^2, and, where given, res[q] = that bound, cnt[q * kCntStride] = 0, zero[0] = zero[1] = 0.
 // products: 3 (hi.hi + hi.lo + lo.hi, about fp32 accuracy) or 1 (hi.hi alone), the same in all launches of a call
 size_t split_queries_bytes(int nq, int dim, int products);
-hipError_t launch_split_queries(const float* queries, int nq, int dim, int products, const float* qn, void* out,
-                                hipStream_t stream);
+size_t split_queries_offset(int64_t row, int dim, int products);  // of a row that is a multiple of kQueryTile
+constexpr int kQueryTile = 256;
+// ints of an index's pinned memory for what a call reads back: the flags of 1024 queries and one more (4 KB over the bus)
+constexpr int kKnnFlags = 1025;
+hipError_t launch_prepare_queries(const float* queries, int nq, int dim, int products, float* qn, float* res, void* out,
+                                  unsigned int* cnt, int* zero, hipStream_t stream);
 // as launch_distance_tile, with D[q][b] = |q|^2 + |b|^2 - 2 q.b (L2) or -q.b (IP) from inner products on the matrix
-// cores; queries: what launch_split_queries wrote.
+// cores; queries: what launch_prepare_queries wrote.
 // sample_tiles > 0: only that many tiles of 128 base points, every tile_stride-th of the base, side by side in D
 hipError_t launch_approx_tile(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, int products,
                               const float* qn, const float* bn, const uint32_t* deleted, int64_t base_id0, float* D,
@@ -39,7 +44,7 @@ hipError_t launch_approx_filter(const void* queries, const float* base, int nq, 
                                 unsigned long long* lists, int64_t cap, unsigned int* cnt, int tile_step,
                                 hipStream_t stream);
 // the k (<= 1024) smallest keys of every list, sorted, as ids [nq][k] (-1: none) and values; *overflow (zero before)
-// counts the lists that could not be done
+// counts the lists that could not be done; their ids are -1
 hipError_t launch_list_select(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, int32_t* ids,
                               float* dists, int* overflow, hipStream_t stream);
 // the same selection in place, between two launches that append: the list shrinks to its k smallest keys, tau[q]
@@ -47,11 +52,12 @@ hipError_t launch_list_select(unsigned long long* lists, int64_t cap, unsigned i
 hipError_t launch_list_shrink(unsigned long long* lists, int64_t cap, unsigned int* cnt, int nq, int k, float* tau,
                               int* overflow, hipStream_t stream);
 // cand_ids / cand_d [nq][kc] (ascending approximate signed distance, -1 = none) -> the exact k best per query in the
-// reference's summation order; redo[q] = 1 where the candidates cannot vouch for the result
+// reference's summation order; redo[q] = 1 where the candidates cannot vouch for the result,
+// redo[nq] = *lost (null: 0)
 hipError_t launch_rerank(const float* queries, const float* base, int nq, int dim, int metric, const int32_t* cand_ids,
                          const float* cand_d, int kc, int k, const float* qn, const uint32_t* bn_max_bits, const float* qres,
-                         const uint32_t* bres_max_bits, int32_t* ids, float* dists, int* redo, hipStream_t stream);
-// (qres, *bres_max_bits: what launch_row_norms gave, for candidates chosen on one product; else null)
+                         const uint32_t* bres_max_bits, int32_t* ids, float* dists, int* redo, const int* lost, hipStream_t stream);
+// (qres, *bres_max_bits: what launch_prepare_queries and launch_row_norms gave, for candidates chosen on one product; else null)
 // *extra += the entries of D's rows, beyond kc, that one product cannot tell from those up to tau
 hipError_t launch_count_close(const float* D, int64_t ldD, int nq, int64_t n, int kc, int metric, const float* qn,
                               const uint32_t* bn_max_bits, const float* qres, const uint32_t* bres_max_bits, const float* tau,

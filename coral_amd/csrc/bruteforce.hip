@@ -273,7 +273,8 @@ __global__ __launch_bounds__(T) void row_select_kernel(const float* __restrict__
 // One workgroup per query: the k smallest of the cnt[q] keys in lists[q * cap ...] (distinct: every key carries its
 // id), sorted, into out.  The scheme of row_select_kernel on keys: the k-th smallest of the per-thread minima bounds
 // the k-th smallest key from above, a second pass collects what lies up to it, a sort finishes.  *overflow is raised
-// when a list lost entries (cnt[q] > cap) or the collection outgrows LDS; the caller then takes another path.
+// when a list lost entries (cnt[q] > cap) or the collection outgrows LDS; the query has no ids then, and the caller takes
+// another path.
 // The result goes out as ids (-1: none) and values; SHRINK: it replaces the list and its count, and tau[q] becomes the
 // value of the k-th key -- or stays, where the list has fewer: the bound that let them through holds for the whole row
 // whether its k smallest lie in the tiles seen so far or not.  (Without it every entry of the tiles to come would pass;
@@ -288,10 +289,12 @@ __global__ __launch_bounds__(T) void list_select_kernel(unsigned long long* __re
     __shared__ unsigned int s_count;
     const int tid = threadIdx.x;
     const unsigned int have = cnt[(size_t)blockIdx.x * kCntStride];
-    if (have > (unsigned)cap) {
+    auto give_up = [&]() {
         if (tid == 0) atomicAdd(overflow, 1);
-        return;
-    }
+        if constexpr (!SHRINK)
+            for (int i = tid; i < k; i += T) ids[(size_t)blockIdx.x * k + i] = -1;
+    };
+    if (have > (unsigned)cap) return give_up();
     const int n = (int)have;
     unsigned long long* list = lists + (size_t)blockIdx.x * cap;
     const int kk = min(k, n);
@@ -320,10 +323,7 @@ __global__ __launch_bounds__(T) void list_select_kernel(unsigned long long* __re
     }
     __syncthreads();
     const unsigned count = s_count;
-    if (count > (unsigned)kSelCap) {
-        if (tid == 0) atomicAdd(overflow, 1);
-        return;
-    }
+    if (count > (unsigned)kSelCap) return give_up();
     int P = 2;
     while (P < (int)count) P <<= 1;
     for (int i = (int)count + tid; i < P; i += T) skeys[i] = ~0ull;

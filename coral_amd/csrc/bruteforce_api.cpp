@@ -22,7 +22,7 @@ constexpr int64_t kBufferFloats = (int64_t)1 << 29;  // 2 GiB distance buffer
 // of D, and at the end the k best of the per-segment winners.  screen: approximate distances from the matrix cores
 // (qn, bn: squared norms) instead of the reference-order ones.
 int knn_passes(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, int32_t have_delete, bool screen,
-               const float* d_qn, int metric_out, int32_t* d_ids, float* d_dists, hipStream_t stream) {
+               float* d_qn, int metric_out, int32_t* d_ids, float* d_dists, hipStream_t stream) {
     const int64_t n = idx->n;
     int64_t seg = std::min(n, kSegment);
     int64_t nseg = (n + seg - 1) / seg;
@@ -59,7 +59,8 @@ int knn_passes(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, i
     for (int64_t q0 = 0; q0 < Q; q0 += qc) {
         const int nq = (int)std::min<int64_t>(qc, Q - q0);
         if (screen)
-            HIP_TRY_R(coral::launch_split_queries(d_queries + (size_t)q0 * idx->dim, nq, idx->dim, 3, d_qn + q0, d_split, stream));
+            HIP_TRY_R(coral::launch_prepare_queries(d_queries + (size_t)q0 * idx->dim, nq, idx->dim, 3, d_qn + q0, nullptr, d_split,
+                                                    nullptr, nullptr, stream));
         for (int64_t s = 0; s < nseg; ++s) {
             const int64_t b0 = s * seg, nb = std::min(seg, n - b0);
             const float* qp = d_queries + (size_t)q0 * idx->dim;
@@ -91,7 +92,7 @@ int ensure_base_norms(coral_index* idx, hipStream_t stream) {
     float* norms = nullptr;
     HIP_TRY(hipMalloc(&norms, (size_t)idx->n * sizeof(float)));
     hipError_t e = launch_fill_u32(idx->d_bnorm_max, 2, 0u, stream);
-    if (e == hipSuccess) e = launch_row_norms(idx->d_vec, idx->n, idx->dim, norms, idx->d_bnorm_max, nullptr, nullptr, stream);
+    if (e == hipSuccess) e = launch_row_norms(idx->d_vec, idx->n, idx->dim, norms, idx->d_bnorm_max, nullptr, stream);
     if (e != hipSuccess) {
         (void)hipFree(norms);
         HIP_TRY(e);
@@ -104,7 +105,7 @@ int ensure_base_norms(coral_index* idx, hipStream_t stream) {
 // ensure_base_norms
 int ensure_base_loss(coral_index* idx, hipStream_t stream) {
     if (idx->bloss_ready) return CORAL_OK;
-    HIP_TRY(launch_row_norms(idx->d_vec, idx->n, idx->dim, nullptr, nullptr, nullptr, idx->d_bnorm_max + 1, stream));
+    HIP_TRY(launch_row_norms(idx->d_vec, idx->n, idx->dim, nullptr, nullptr, idx->d_bnorm_max + 1, stream));
     HIP_TRY(hipStreamSynchronize(stream));
     idx->bloss_ready = true;
     return CORAL_OK;
@@ -153,6 +154,8 @@ public:
         for (auto& p : parts_) *p.first = static_cast<char*>(base_) + p.second;
         return hipSuccess;
     }
+    // pinned room for the flags of Q queries and one more, or null: for the holder of the kept block
+    int* flags(int32_t Q) const { return kept_ && Q < coral::kKnnFlags ? idx_->h_knn_flags : nullptr; }
 
 private:
     coral_index* idx_;
@@ -203,7 +206,7 @@ struct FusedScreen {
         // hundreds of tiles per compute unit; the sample's matrix is made and read for 2048 at a time
         const int64_t rows = ((int64_t)Q + 127) & ~(int64_t)127;
         qc = std::min<int64_t>(4096, rows);
-        qs = std::min<int64_t>(2048, std::min(qc, std::max<int64_t>(128, (kBufferFloats / ns) & ~(int64_t)127)));
+        qs = std::min<int64_t>(2048, std::min(qc, std::max<int64_t>(256, (kBufferFloats / ns) & ~(int64_t)255)));
     }
     void reserve(const coral_index* idx, KnnScratch& mem) {
         if (!suits) return;
@@ -212,14 +215,14 @@ struct FusedScreen {
         mem.reserve(&redo, (size_t)qs), mem.reserve(&overflow, 2);
         mem.reserve(&split, coral::split_queries_bytes((int)qc, idx->dim, 3));  // (the larger form: one product may give way to three)
     }
-    // *used = false when a list overflowed (sample unlike the base, rows of equal values, too few live points in the
-    // sample): the caller then goes through the matrix; and with one product when the sample says that too many entries
-    // lie where it cannot tell them apart (d_qres: what it loses per query)
-    int run(coral_index* idx, const float* d_queries, int32_t Q, int32_t have_delete, const float* d_qn, const float* d_qres,
+    // *used = false, with one product, when the sample says that too many entries lie where it cannot tell them apart
+    // (d_qres: what it loses per query).  *overflow != 0 in the end where a list did (sample unlike the base, rows of equal
+    // values, too few live points in the sample): its query has no candidates, and the caller goes through the matrix.
+    // d_qn, d_qres: written here.
+    int run(coral_index* idx, const float* d_queries, int32_t Q, int32_t have_delete, float* d_qn, float* d_qres,
             int32_t* d_cid, float* d_cd, hipStream_t stream, bool* used) {
         *used = false;
         const int64_t n = idx->n;
-        HIP_TRY(coral::launch_fill_u32(reinterpret_cast<uint32_t*>(overflow), 2, 0u, stream));
         const uint32_t* del = have_delete ? idx->d_deleted : nullptr;
         if (products == 1) {
             // The kc kept are meant to hold the k best whatever one product lost: kScreenSlack entries may lie too close.
@@ -228,7 +231,7 @@ struct FusedScreen {
             // Gaussian).  (Costs 60 us whatever the answer.)
             const int probe = std::min(Q, 64);
             int extra = 0;
-            HIP_TRY(coral::launch_split_queries(d_queries, probe, idx->dim, 1, d_qn, split, stream));
+            HIP_TRY(coral::launch_prepare_queries(d_queries, probe, idx->dim, 1, d_qn, d_qres, split, nullptr, overflow, stream));
             HIP_TRY(coral::launch_approx_tile(split, idx->d_vec, probe, n, idx->dim, idx->metric, 1, d_qn, idx->d_bnorm, del, 0, D,
                                               ns, stream, tiles, (int)stride));
             HIP_TRY(coral::launch_row_select(D, ns, probe, ns, kc, 0, nullptr, 0, redo, stream, tau));
@@ -242,16 +245,16 @@ struct FusedScreen {
         for (int64_t q0 = 0; q0 < Q; q0 += qc) {
             const int nq = (int)std::min<int64_t>(qc, Q - q0);
             const float* qp = d_queries + (size_t)q0 * idx->dim;
-            const float* qn = d_qn + q0;
+            float* qn = d_qn + q0;
+            HIP_TRY(coral::launch_prepare_queries(qp, nq, idx->dim, products, qn, d_qres ? d_qres + q0 : nullptr, split, cnt,
+                                                  q0 == 0 ? overflow : nullptr, stream));
             for (int64_t s0 = 0; s0 < nq; s0 += qs) {
                 const int ms = (int)std::min<int64_t>(qs, nq - s0);
-                HIP_TRY(coral::launch_split_queries(qp + (size_t)s0 * idx->dim, ms, idx->dim, products, qn + s0, split, stream));
-                HIP_TRY(coral::launch_approx_tile(split, idx->d_vec, ms, n, idx->dim, idx->metric, products, qn + s0, idx->d_bnorm, del,
-                                                  0, D, ns, stream, tiles, (int)stride));
+                HIP_TRY(coral::launch_approx_tile(split + coral::split_queries_offset(s0, idx->dim, products), idx->d_vec, ms, n,
+                                                  idx->dim, idx->metric, products, qn + s0, idx->d_bnorm, del, 0, D, ns, stream,
+                                                  tiles, (int)stride));
                 HIP_TRY(coral::launch_row_select(D, ns, ms, ns, kc, 0, nullptr, 0, redo, stream, tau + s0));
             }
-            if (nq > qs) HIP_TRY(coral::launch_split_queries(qp, nq, idx->dim, products, qn, split, stream));
-            HIP_TRY(coral::launch_fill_u32(cnt, (size_t)nq * coral::kCntStride, 0u, stream));
             HIP_TRY(coral::launch_approx_filter(split, idx->d_vec, nq, n, idx->dim, idx->metric, products, qn, idx->d_bnorm, del, tau,
                                                 lists, cap, cnt, step, stream));
             if (step > 1) {
@@ -262,10 +265,7 @@ struct FusedScreen {
             HIP_TRY(coral::launch_list_select(lists, cap, cnt, nq, kc, d_cid + (size_t)q0 * kc, d_cd + (size_t)q0 * kc,
                                               overflow, stream));
         }
-        int lost = 0;
-        HIP_TRY(hipMemcpyAsync(&lost, overflow, sizeof(int), hipMemcpyDeviceToHost, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
-        *used = lost == 0;
+        *used = true;
         return CORAL_OK;
     }
 };
@@ -310,43 +310,59 @@ struct Screening {
     int32_t* d_cid = nullptr;
     int* d_redo = nullptr;
     FusedScreen fused_screen;
+    bool waited = false;  // the call's last work was what run() has waited for and `done` stands behind
 
     void reserve(const coral_index* idx, int32_t Q, int32_t k, int products_, KnnScratch& mem) {
         products = products_, kc = k + kScreenSlack;
         mem.reserve(&d_qn, (size_t)Q), mem.reserve(&d_qres, (size_t)Q), mem.reserve(&d_cid, (size_t)Q * kc);
-        mem.reserve(&d_cd, (size_t)Q * kc), mem.reserve(&d_redo, (size_t)Q);
+        mem.reserve(&d_cd, (size_t)Q * kc), mem.reserve(&d_redo, (size_t)Q + 1);
         if (idx->knn_mode == 0) fused_screen.plan(idx, Q, kc, products);
         fused_screen.reserve(idx, mem);
     }
 
+    // flags: pinned room for Q + 1 of them, or null; done (or null): recorded behind the re-rank
     int run(coral_index* idx, const float* d_queries, int32_t Q, int32_t k, int32_t have_delete, int32_t* d_ids, float* d_dists,
-            hipStream_t stream) {
+            hipStream_t stream, int* flags, hipEvent_t done) {
         if (int rc = coral::ensure_base_norms(idx, stream)) return rc;
         if (products == 1)
             if (int rc = coral::ensure_base_loss(idx, stream)) return rc;
-        const float* qres = products == 1 ? d_qres : nullptr;
-        HIP_TRY(coral::launch_row_norms(d_queries, Q, idx->dim, d_qn, nullptr, products == 1 ? d_qres : nullptr, nullptr, stream));
-        bool fused = false;
-        while (fused_screen.suits && !fused) {
-            if (int rc = fused_screen.run(idx, d_queries, Q, have_delete, d_qn, qres, d_cid, d_cd, stream, &fused)) return rc;
-            if (fused || products == 3) break;
-            products = fused_screen.products = 3, qres = nullptr;  // in the same scratch, from the start
+        std::vector<int> copied;
+        if (!flags) copied.resize((size_t)Q + 1);
+        const int* redo = flags ? flags : copied.data();
+        // One wait per attempt, behind the re-rank of its candidates: whether the lists were whole comes back with the
+        // flags.  (Waits of their own for that and for the clock, two copies and three launches more were 50 of the 173 us of
+        // a call with 100 queries.)
+        for (bool matrix = !fused_screen.suits;; matrix = products == 3, products = fused_screen.products = 3) {
+            const float* qres = products == 1 ? d_qres : nullptr;
+            if (matrix) {
+                products = 3, qres = nullptr;
+                if (int rc = knn_passes(idx, d_queries, Q, kc, have_delete, true, d_qn, /*signed distances*/ 0, d_cid, d_cd, stream))
+                    return rc;
+            } else {
+                bool used = false;
+                if (int rc = fused_screen.run(idx, d_queries, Q, have_delete, d_qn, products == 1 ? d_qres : nullptr, d_cid, d_cd,
+                                              stream, &used))
+                    return rc;
+                if (!used) continue;
+            }
+            idx->knn_last_fused = !matrix;
+            HIP_TRY(coral::launch_rerank(d_queries, idx->d_vec, Q, idx->dim, idx->metric, d_cid, d_cd, kc, k, d_qn, idx->d_bnorm_max,
+                                         qres, idx->d_bnorm_max + 1, d_ids, d_dists, flags ? flags : d_redo,
+                                         matrix ? nullptr : fused_screen.overflow, stream));
+            if (done) HIP_TRY(hipEventRecord(done, stream));
+            if (!flags)
+                HIP_TRY(hipMemcpyAsync(copied.data(), d_redo, copied.size() * sizeof(int), hipMemcpyDeviceToHost, stream));
+            HIP_TRY(hipStreamSynchronize(stream));
+            if (redo[Q] == 0) break;  // (the matrix path loses none)
         }
-        if (!fused) products = 3, qres = nullptr;
-        idx->knn_last_fused = fused;
-        if (!fused)
-            if (int rc = knn_passes(idx, d_queries, Q, kc, have_delete, true, d_qn, /*signed distances*/ 0, d_cid, d_cd, stream))
-                return rc;
-        std::vector<int> redo((size_t)Q);
-        HIP_TRY(coral::launch_rerank(d_queries, idx->d_vec, Q, idx->dim, idx->metric, d_cid, d_cd, kc, k, d_qn, idx->d_bnorm_max,
-                                     qres, idx->d_bnorm_max + 1, d_ids, d_dists, d_redo, stream));
-        HIP_TRY(hipMemcpyAsync(redo.data(), d_redo, (size_t)Q * sizeof(int), hipMemcpyDeviceToHost, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
         std::vector<int32_t> rows;
         for (int32_t q = 0; q < Q; ++q)
             if (redo[(size_t)q]) rows.push_back(q);
         if (products == 3) idx->knn_last_redone = (int64_t)rows.size();
-        if (rows.empty()) return CORAL_OK;
+        if (rows.empty()) {
+            waited = done != nullptr;
+            return CORAL_OK;
+        }
         const int m = (int)rows.size();
         float *d_rq = nullptr, *d_rd = nullptr;
         int32_t *d_rows = nullptr, *d_rid = nullptr;
@@ -362,9 +378,9 @@ struct Screening {
                                : knn_passes(idx, d_rq, m, k, have_delete, false, nullptr, idx->metric, d_rid, d_rd, stream);
             if (rc == CORAL_OK) e = coral::launch_scatter_results(d_rows, m, k, d_rid, d_rd, d_ids, d_dists, stream);
         }
-        const hipError_t done = hipStreamSynchronize(stream);  // before the scratch and `rows` go
+        const hipError_t ended = hipStreamSynchronize(stream);  // before the scratch and `rows` go
         if (rc == CORAL_OK) HIP_TRY(e);
-        if (rc == CORAL_OK) HIP_TRY(done);
+        if (rc == CORAL_OK) HIP_TRY(ended);
         return rc;
     }
 
@@ -374,7 +390,7 @@ struct Screening {
         KnnScratch mem(idx);
         next.reserve(idx, Q, k, 3, mem);
         HIP_TRY(mem.allocate());
-        const int rc = next.run(idx, d_queries, Q, k, have_delete, d_ids, d_dists, stream);
+        const int rc = next.run(idx, d_queries, Q, k, have_delete, d_ids, d_dists, stream, mem.flags(Q), nullptr);
         if (rc != CORAL_OK) (void)hipStreamSynchronize(stream);  // nothing is in flight when the scratch goes back
         return rc;
     }
@@ -418,10 +434,10 @@ static int knn_call(coral_index* idx, const float* d_queries, const float* h_que
     if (!screen)
         rc = knn_passes(idx, d_queries, Q, k, have_delete, false, nullptr, idx->metric, d_ids, d_dists, stream);
     else
-        rc = screening.run(idx, d_queries, Q, k, have_delete, d_ids, d_dists, stream);
+        rc = screening.run(idx, d_queries, Q, k, have_delete, d_ids, d_dists, stream, mem.flags(Q), ev1);
     if (rc == CORAL_OK) {
         float ms = 0.f;
-        if (ok(hipEventRecord(ev1, stream), "event") && ok(hipEventSynchronize(ev1), "synchronize") &&
+        if ((screening.waited || (ok(hipEventRecord(ev1, stream), "event") && ok(hipEventSynchronize(ev1), "synchronize"))) &&
             ok(hipEventElapsedTime(&ms, ev0, ev1), "event") && time_s)
             *time_s = ms / 1000.0;
     }

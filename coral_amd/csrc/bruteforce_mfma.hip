@@ -61,83 +61,104 @@ __device__ __forceinline__ float mf_unord32(uint32_t o) {
     return __uint_as_float(u);
 }
 
-// |x|^2 per row, and the largest of them (as the bit pattern of a non-negative float); with res or res_max also a bound on
-// what the row loses when each component of it, scaled as the tile kernel scales it, becomes one half: |x - half(x)|.
-// (Halves below the format's normal range count as lost whole, so the bound holds whether or not the matrix cores
-// take them for zero.  A row of infinite or NaN norm gives an infinite or NaN bound, which no comparison passes.)
-// One wavefront per row, lane by lane side by side.  (A thread per row read 16 bytes of a line at a time: the norms of 1M x
-// 200 took 724 us, of a batch of 2000 x 512 as long as 45.)
+// |x|^2 of a row, lane by lane side by side; in every lane
+__device__ __forceinline__ float row_norm(const float4* __restrict__ p, int chunks, int lane) {
+    float s = 0.0f;
+    for (int c = lane; c < chunks; c += 64) {
+        const float4 v = p[c];
+        s = __fmaf_rn(v.x, v.x, s), s = __fmaf_rn(v.y, v.y, s), s = __fmaf_rn(v.z, v.z, s), s = __fmaf_rn(v.w, v.w, s);
+    }
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    return s;
+}
+
+// a bound on what a row of squared norm s loses when each component of it, scaled as the tile kernel scales it, becomes one
+// half: |x - half(x)|.  (Halves below the format's normal range count as lost whole, so the bound holds whether or not the
+// matrix cores take them for zero.  A row of infinite or NaN norm gives an infinite or NaN bound, which no comparison passes.)
+__device__ __forceinline__ float row_loss(const float4* __restrict__ p, int chunks, int lane, float s) {
+    const int e = mf_scale_exp(s);
+    const float up = mf_pow2(e);
+    float l2 = 0.0f;
+    for (int c = lane; c < chunks; c += 64) {
+        const float4 v = p[c];
+        const float w[4] = {v.x * up, v.y * up, v.z * up, v.w * up};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float h = (float)(_Float16)w[j];
+            const float d = fabsf(h) < 6.2e-5f ? w[j] : w[j] - h;
+            l2 = __fmaf_rn(d, d, l2);
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) l2 += __shfl_xor(l2, off, 64);
+    // (2^-51 <= 2^e <= 2^60; the sum of squares is within dim 2^-24 of itself; the last term for squares that leave the
+    // normal range)
+    const float lost = (sqrtf(l2) * (1.0f + 2.0e-4f) + 1.0e-17f) * mf_pow2(-e);
+    return s <= 3.0e38f ? lost : __int_as_float(0x7f800000);
+}
+
+// |x|^2 per row, the largest of them (as the bit pattern of a non-negative float), and the largest loss.
+// One wavefront per row.  (A thread per row read 16 bytes of a line at a time: the norms of 1M x 200 took 724 us, of a
+// batch of 2000 x 512 as long as 45.  An atomic per wavefront of 8192 workgroups, all on one word, made 50 000 x 100 take 374.)
 __global__ __launch_bounds__(256) void row_norms_kernel(const float* __restrict__ x, int64_t n, int dim,
                                                        float* __restrict__ out, uint32_t* __restrict__ max_bits,
-                                                       float* __restrict__ res, uint32_t* __restrict__ res_max) {
+                                                       uint32_t* __restrict__ res_max) {
     const int lane = threadIdx.x & 63, chunks = dim >> 2;
     const int64_t waves = (int64_t)gridDim.x * 4;
     float most = 0.0f, most_lost = 0.0f;
     for (int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); r < n; r += waves) {
         const float4* p = reinterpret_cast<const float4*>(x + (size_t)r * dim);
-        float s = 0.0f;
-        for (int c = lane; c < chunks; c += 64) {
-            const float4 v = p[c];
-            s = __fmaf_rn(v.x, v.x, s), s = __fmaf_rn(v.y, v.y, s), s = __fmaf_rn(v.z, v.z, s), s = __fmaf_rn(v.w, v.w, s);
-        }
-        for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+        const float s = row_norm(p, chunks, lane);
         if (out && lane == 0) out[r] = s;
         most = s > most ? s : (s != s ? s : most);  // (a NaN stays)
-        if (res || res_max) {
-            const int e = mf_scale_exp(s);
-            const float up = mf_pow2(e);
-            float l2 = 0.0f;
-            for (int c = lane; c < chunks; c += 64) {
-                const float4 v = p[c];
-                const float w[4] = {v.x * up, v.y * up, v.z * up, v.w * up};
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float h = (float)(_Float16)w[j];
-                    const float d = fabsf(h) < 6.2e-5f ? w[j] : w[j] - h;
-                    l2 = __fmaf_rn(d, d, l2);
-                }
-            }
-            for (int off = 32; off > 0; off >>= 1) l2 += __shfl_xor(l2, off, 64);
-            // (2^-51 <= 2^e <= 2^60; the sum of squares is within dim 2^-24 of itself; the last term for squares that
-            // leave the normal range)
-            float lost = (sqrtf(l2) * (1.0f + 2.0e-4f) + 1.0e-17f) * mf_pow2(-e);
-            if (!(s <= 3.0e38f)) lost = __int_as_float(0x7f800000);
-            if (res && lane == 0) res[r] = lost;
-            most_lost = fmaxf(most_lost, lost);
-        }
+        if (res_max) most_lost = fmaxf(most_lost, row_loss(p, chunks, lane, s));
     }
-    if (lane == 0) {
-        if (max_bits) atomicMax(max_bits, __float_as_uint(most));
-        if (res_max) atomicMax(res_max, __float_as_uint(most_lost));
+    __shared__ uint32_t wave_most[4][2];
+    if (lane == 0) wave_most[threadIdx.x >> 6][0] = __float_as_uint(most), wave_most[threadIdx.x >> 6][1] = __float_as_uint(most_lost);
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        uint32_t* to = threadIdx.x == 0 ? max_bits : res_max;
+        const uint32_t m = max(max(wave_most[0][threadIdx.x], wave_most[1][threadIdx.x]),
+                               max(wave_most[2][threadIdx.x], wave_most[3][threadIdx.x]));
+        if (to && __hip_atomic_load(to, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < m) atomicMax(to, m);
     }
 }
 
 // The queries as the tile kernel reads them: per tile of 256 queries and stage, two planes of [256 rows][16 halves] --
 // a stage of a tile is 16 KB in the order in which it lies in LDS.  NP = 3: the hi and the lo plane of 16 dimensions;
-// NP = 1: the hi planes of 32.  Rows beyond the batch and dimensions beyond dim are zero.
+// NP = 1: the hi planes of 32.  Rows beyond the batch and dimensions beyond dim are zero.  On the way |q|^2 (and with res
+// the bound on what one half per component leaves out), the query's counter and the two words of `zero` are set: what
+// would be three launches more, each longer on its way to the chip than on it for a small batch.
+// One wavefront per row, as row_norms_kernel reads it.
 template <int NP>
-__global__ __launch_bounds__(256) void split_queries_kernel(const float* __restrict__ queries, int nq, int dim, int stages,
-                                                           const float* __restrict__ qn, _Float16* __restrict__ out) {
-    const int st = blockIdx.x, row = threadIdx.x;
-    const int64_t q = (int64_t)blockIdx.y * MT + row;
-    _Float16* dst = out + ((size_t)blockIdx.y * stages + st) * kStageA + row * BK;
-    const float s = q < nq ? mf_pow2(mf_scale_exp(qn[q])) : 0.0f;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        float4 v[2];
-#pragma unroll
-        for (int plane = 0; plane < (NP == 1 ? 2 : 1); ++plane) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int k = st * kStageDims<NP> + plane * BK + 8 * h + 4 * u;
-                v[u] = make_float4(0, 0, 0, 0);
-                if (q < nq && k < dim) v[u] = *reinterpret_cast<const float4*>(queries + (size_t)q * dim + k);
-            }
-            v8h hi, lo;
-            mf_split8(v[0], v[1], s, hi, lo);
-            *reinterpret_cast<v8h*>(dst + plane * MT * BK + 8 * h) = hi;
-            if (NP == 3) *reinterpret_cast<v8h*>(dst + MT * BK + 8 * h) = lo;
+__global__ __launch_bounds__(256) void prepare_queries_kernel(const float* __restrict__ queries, int nq, int dim, int stages,
+                                                             float* __restrict__ qn, float* __restrict__ res,
+                                                             _Float16* __restrict__ out, unsigned int* __restrict__ cnt,
+                                                             int* __restrict__ zero) {
+    const int lane = threadIdx.x & 63, chunks = dim >> 2;
+    const int64_t q = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const float4* p = reinterpret_cast<const float4*>(queries + (size_t)q * dim);
+    float s = 0.0f;
+    if (q < nq) {
+        s = row_norm(p, chunks, lane);
+        const float lost = res ? row_loss(p, chunks, lane, s) : 0.0f;
+        if (lane == 0) {
+            qn[q] = s;
+            if (res) res[q] = lost;
+            if (cnt) cnt[(size_t)q * kCntStride] = 0u;
         }
+    }
+    if (zero && q == 0 && lane < 2) zero[lane] = 0;
+    const float up = mf_pow2(mf_scale_exp(s));
+    _Float16* tile = out + (size_t)(q / MT) * stages * kStageA + (q % MT) * BK;
+    for (int c = lane; c < stages * (kStageDims<NP> / 4); c += 64) {
+        const int k = 4 * c;
+        float4 v = make_float4(0, 0, 0, 0);
+        if (q < nq && k < dim) v = p[c];
+        v4h hi, lo;
+        mf_split4(v, up, hi, lo);
+        _Float16* dst = tile + (size_t)(k / kStageDims<NP>) * kStageA + (k % kStageDims<NP>) / BK * (MT * BK) + k % BK;
+        *reinterpret_cast<v4h*>(dst) = hi;
+        if (NP == 3) *reinterpret_cast<v4h*>(dst + MT * BK) = lo;
     }
 }
 
@@ -160,7 +181,7 @@ __global__ __launch_bounds__(256) void split_queries_kernel(const float* __restr
 // pair-dimensions at the card's dense rate), in practice by LDS: a wavefront reads 12 KB per 24 multiplications
 // (768 cycles of its matrix core; the reads of a CU's four wavefronts take 384 cycles of its LDS, parking the next
 // stage 192), which is why a wavefront has a 128 x 64 tile and not the 64 x 64 that the fp32 form had.  The queries
-// come split (split_queries_kernel: every query tile is read by thousands of workgroups); the base is split here, on
+// come split (prepare_queries_kernel: every query tile is read by thousands of workgroups); the base is split here, on
 // its way to LDS, eight components per thread and stage under the other wavefronts' multiplications: a split copy of
 // the base would double the index or cost a pass over it per call, which small batches would feel.
 template <int MODE, bool L2, int NP>
@@ -504,17 +525,31 @@ __global__ __launch_bounds__(256) void count_close_kernel(const float* __restric
     if (threadIdx.x == 0) atomicAdd(extra, max(0, s_count - kc));
 }
 
+__device__ __forceinline__ float rerank_add(const float4 a, const float4 b, float s, int metric) {
+    if (metric == 0) {
+        float t;
+        t = a.x - b.x, s = __fmaf_rn(t, t, s);
+        t = a.y - b.y, s = __fmaf_rn(t, t, s);
+        t = a.z - b.z, s = __fmaf_rn(t, t, s);
+        t = a.w - b.w, s = __fmaf_rn(t, t, s);
+    } else {
+        s = __fmaf_rn(a.x, b.x, s), s = __fmaf_rn(a.y, b.y, s), s = __fmaf_rn(a.z, b.z, s), s = __fmaf_rn(a.w, b.w, s);
+    }
+    return s;
+}
+
 // One workgroup per query: the kc candidates (ids, -1 = none; approximate signed distances, ascending) are measured
 // in the reference's order (one thread walks the dimensions of one candidate with one fused multiply-add each,
 // include/utils.cuh:254-275, 307-323: the arithmetic of distance_tile_kernel), sorted by (distance, id), and the k
-// best written.  redo[q] = 1 when the result cannot be vouched for (see the head of this file).
+// best written.  redo[q] = 1 when the result cannot be vouched for (see the head of this file); redo[number of queries] =
+// *lost: the call reads both after one wait.
 __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ queries, const float* __restrict__ base,
                                                     int dim, int metric, const int32_t* __restrict__ cand_ids,
                                                     const float* __restrict__ cand_d, int kc, int k,
                                                     const float* __restrict__ qn, const uint32_t* __restrict__ bn_max_bits,
                                                     const float* __restrict__ qres, const uint32_t* __restrict__ bres_max_bits,
                                                     int32_t* __restrict__ ids, float* __restrict__ dists,
-                                                    int* __restrict__ redo) {
+                                                    int* __restrict__ redo, const int* __restrict__ lost) {
     extern __shared__ unsigned long long rkeys[];
     const int q = blockIdx.x, tid = threadIdx.x;
     int P = 2;
@@ -527,22 +562,17 @@ __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ q
             const float4* b4 = reinterpret_cast<const float4*>(base + (size_t)id * dim);
             const float4* q4 = reinterpret_cast<const float4*>(qv);
             float s = 0.0f;
-            if (metric == 0) {
-                for (int c = 0; c < dim / 4; ++c) {
-                    const float4 a = q4[c], b = b4[c];
-                    float t;
-                    t = a.x - b.x, s = __fmaf_rn(t, t, s);
-                    t = a.y - b.y, s = __fmaf_rn(t, t, s);
-                    t = a.z - b.z, s = __fmaf_rn(t, t, s);
-                    t = a.w - b.w, s = __fmaf_rn(t, t, s);
-                }
-            } else {
-                for (int c = 0; c < dim / 4; ++c) {
-                    const float4 a = q4[c], b = b4[c];
-                    s = __fmaf_rn(a.x, b.x, s), s = __fmaf_rn(a.y, b.y, s), s = __fmaf_rn(a.z, b.z, s), s = __fmaf_rn(a.w, b.w, s);
-                }
-                s = 0.0f - s;
+            // eight loads of the row on their way at a time: few threads have a row, and each waits for its own
+            int c = 0;
+            for (; c + 8 <= dim / 4; c += 8) {
+                float4 b[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) b[u] = b4[c + u];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) s = rerank_add(q4[c + u], b[u], s, metric);
             }
+            for (; c < dim / 4; ++c) s = rerank_add(q4[c], b4[c], s, metric);
+            if (metric != 0) s = 0.0f - s;
             key = ((unsigned long long)mf_ord32(s) << 32) | (uint32_t)id;
         }
         rkeys[i] = key;
@@ -587,6 +617,7 @@ __global__ __launch_bounds__(256) void rerank_kernel(const float* __restrict__ q
             if (kth == ~0ull || !(sk < worst - delta)) bad = 1;
         }
         redo[q] = bad;
+        if (q == 0) redo[gridDim.x] = lost ? *lost : 0;
     }
 }
 
@@ -604,11 +635,11 @@ __global__ void scatter_results_kernel(const int32_t* __restrict__ rows, int cou
 
 }  // namespace
 
-hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, float* res, uint32_t* res_max,
+hipError_t launch_row_norms(const float* x, int64_t n, int dim, float* out, uint32_t* max_bits, uint32_t* res_max,
                             hipStream_t stream) {
     if (n <= 0) return hipErrorInvalidValue;
-    const int64_t blocks = std::min<int64_t>((n + 3) / 4, 8192);
-    hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, dim, out, max_bits, res, res_max);
+    const int64_t blocks = std::min<int64_t>((n + 3) / 4, 2048);  // 32 wavefronts per compute unit
+    hipLaunchKernelGGL(row_norms_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, x, n, dim, out, max_bits, res_max);
     return hipGetLastError();
 }
 
@@ -620,13 +651,17 @@ size_t split_queries_bytes(int nq, int dim, int products) {
     return (size_t)((nq + MT - 1) / MT) * stages_of(dim, products) * kStageA * sizeof(_Float16);
 }
 
-hipError_t launch_split_queries(const float* queries, int nq, int dim, int products, const float* qn, void* out,
-                                hipStream_t stream) {
-    const int stages = stages_of(dim, products), tiles = (nq + MT - 1) / MT;
-    if (nq <= 0 || tiles > 65535) return hipErrorInvalidValue;
-    auto kernel = products == 1 ? split_queries_kernel<1> : split_queries_kernel<3>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)stages, (unsigned)tiles), dim3(MT), 0, stream, queries, nq, dim,
-                       stages, qn, static_cast<_Float16*>(out));
+size_t split_queries_offset(int64_t row, int dim, int products) {
+    return (size_t)(row / MT) * stages_of(dim, products) * kStageA * sizeof(_Float16);
+}
+
+hipError_t launch_prepare_queries(const float* queries, int nq, int dim, int products, float* qn, float* res, void* out,
+                                  unsigned int* cnt, int* zero, hipStream_t stream) {
+    const int tiles = (nq + MT - 1) / MT;
+    if (nq <= 0) return hipErrorInvalidValue;
+    auto kernel = products == 1 ? prepare_queries_kernel<1> : prepare_queries_kernel<3>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)tiles * (MT / 4)), dim3(256), 0, stream, queries, nq, dim, stages_of(dim, products),
+                       qn, res, static_cast<_Float16*>(out), cnt, zero);
     return hipGetLastError();
 }
 
@@ -706,11 +741,12 @@ hipError_t launch_levels(const void* queries, const float* base, int nq, int64_t
 
 hipError_t launch_rerank(const float* queries, const float* base, int nq, int dim, int metric, const int32_t* cand_ids,
                          const float* cand_d, int kc, int k, const float* qn, const uint32_t* bn_max_bits, const float* qres,
-                         const uint32_t* bres_max_bits, int32_t* ids, float* dists, int* redo, hipStream_t stream) {
+                         const uint32_t* bres_max_bits, int32_t* ids, float* dists, int* redo, const int* lost,
+                         hipStream_t stream) {
     int P = 2;
     while (P < kc) P <<= 1;
     hipLaunchKernelGGL(rerank_kernel, dim3(nq), dim3(256), (size_t)P * 8, stream, queries, base, dim, metric, cand_ids,
-                       cand_d, kc, k, qn, bn_max_bits, qres, bres_max_bits, ids, dists, redo);
+                       cand_d, kc, k, qn, bn_max_bits, qres, bres_max_bits, ids, dists, redo, lost);
     return hipGetLastError();
 }
 

@@ -178,6 +178,8 @@ int coral_index_create(const coral_index_desc* d, coral_index** out) {
         HIP_TRY_C(hipMalloc(&idx->d_start, (size_t)d->n_start * sizeof(int32_t)));
     }
     HIP_TRY_C(hipMalloc(&idx->d_scalars, 4 * sizeof(int)));
+    HIP_TRY_C(hipHostMalloc(&idx->h_scalars, (16 + coral::kKnnFlags) * sizeof(int)));
+    idx->h_knn_flags = idx->h_scalars + 16;
     HIP_TRY_C(hipMalloc(&idx->d_hit, sizeof(unsigned long long)));
     HIP_TRY_C(hipMemcpy(idx->d_vec, d->base, vec_bytes, hipMemcpyHostToDevice));
     if (!vectors_only) {
@@ -739,7 +741,6 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         HIP_TRY(hipMalloc(&idx->d_beam, need_beam * sizeof(uint64_t)));
         idx->beam_alloc_words = need_beam;
     }
-    if (!idx->h_scalars) HIP_TRY(hipHostMalloc(&idx->h_scalars, 4 * sizeof(int)));
     // per query: the four traversal counters, then (behind those of the whole batch) the four counts of what it read
     const size_t need_counters = (size_t)Q * 8;
     if (need_counters > idx->counters_alloc) {
@@ -1040,8 +1041,7 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
             const int m = std::min(idx->level_rows, Q - q0);
             const float* q = d_queries + (size_t)q0 * idx->dim;
             if (q0) HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_scalars, 1, 0u, stream));
-            HIP_TRY(coral::launch_row_norms(q, m, idx->dim, w.qn, nullptr, w.qres, nullptr, stream));
-            HIP_TRY(coral::launch_split_queries(q, m, idx->dim, 1, w.qn, w.split, stream));
+            HIP_TRY(coral::launch_prepare_queries(q, m, idx->dim, 1, w.qn, w.qres, w.split, nullptr, nullptr, stream));
             HIP_TRY(coral::launch_approx_tile(w.split, idx->d_vec, m, idx->n, idx->dim, idx->metric, 1, w.qn, idx->d_bnorm, nullptr, 0,
                                               w.D, kLevelSampleTiles * 128, stream, tiles, (int)std::max<int64_t>(1, idx->n / 128 / tiles)));
             HIP_TRY(coral::launch_level_ranges(w.D, kLevelSampleTiles * 128, m, (int)sampled, idx->dim, idx->metric, w.qn, idx->d_bnorm_max,

@@ -62,7 +62,7 @@ struct coral_index {
     unsigned long long* d_hit = nullptr;
     unsigned long long* d_phase = nullptr;  // debug builds only
     int32_t* h_counters = nullptr;  // pinned, counters_alloc entries
-    int* h_scalars = nullptr;       // pinned, what d_scalars held after a launch
+    int* h_scalars = nullptr;       // pinned (from the start: an allocation takes 300 us), what d_scalars held after a launch
     void* h_io = nullptr;           // pinned: queries and results of small calls with host buffers
     int last_Q = 0;
     // the entry point that allocates nothing: its last plan (kernel attributes and occupancy are looked up once per
@@ -87,6 +87,7 @@ struct coral_index {
     // scratch of the exact kNN, kept between calls up to kKnnKeepBytes (bruteforce_api.cpp); one call has it at a time
     void* knn_block = nullptr;
     size_t knn_block_bytes = 0;
+    int* h_knn_flags = nullptr;  // pinned, behind h_scalars: what a call of up to kKnnFlags - 1 queries reads back
     std::atomic<bool> knn_block_taken{false};
     int64_t knn_last_redone = 0;  // queries of the last call that went through the exact passes after screening
 

@@ -15,6 +15,7 @@
 namespace coral {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 // e with |x| 2^e in [2^13, 2^14) for a row of squared norm n2; at most 60, which rows of norm 0 and of norms whose square
@@ -28,6 +29,16 @@ __device__ __forceinline__ int mf_scale_exp(float n2) {
     return max(kLeast, min(60, 13 - (E >> 1)));
 }
 __device__ __forceinline__ float mf_pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// four scaled components as two planes of halves
+__device__ __forceinline__ void mf_split4(const float4 a, float s, v4h& hi, v4h& lo) {
+    const float x[4] = {a.x * s, a.y * s, a.z * s, a.w * s};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        hi[j] = (_Float16)x[j];
+        lo[j] = (_Float16)(x[j] - (float)hi[j]);
+    }
+}
 
 // eight scaled components as two planes of halves
 __device__ __forceinline__ void mf_split8(const float4 a, const float4 b, float s, v8h& hi, v8h& lo) {

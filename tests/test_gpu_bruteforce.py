@@ -443,3 +443,30 @@ def test_screening_on_one_product_answers_what_the_plain_passes_answer(law, metr
     idx.close()
     assert np.array_equal(ids, want_ids) and dists.tobytes() == want_d.tobytes()
     assert np.array_equal(ids3, want_ids) and dists3.tobytes() == want_d.tobytes()
+
+
+@pytest.mark.parametrize("Q", [1, 3, 255, 257, 1024, 1025, 4500])
+@pytest.mark.parametrize("metric,dim,k", [("l2", 4, 1), ("ip", 12, 10), ("l2", 100, 10), ("ip", 260, 33), ("l2", 516, 5)])
+def test_prepared_queries_at_the_edges_of_tiles_and_flags(Q, metric, dim, k):
+    """Batches about the query tile of 256, the 1024 queries whose flags go to pinned memory and the 2048 and 4096 of a block
+    of the screening; dimensions short of a stage of 16 and beyond the 64 lanes that read a row.  Twice on one index (the
+    counters start at zero again), and with every second base row equal, where lists overflow or leave ties open: ids and
+    distance bits are those of the search that measures every pair."""
+    rng = np.random.RandomState(Q + dim)
+    base = synth.gaussian_matrix(9, 12000, dim)
+    q = synth.shifted_queries(Q, dim, 6, 7, 8)
+    for twins in (False, True):
+        if twins:
+            base[1::2] = base[:1]
+            q[::3] = base[rng.choice(12000, len(q[::3]))]
+        idx = capi.Index(base, None, None, metric=capi.IP if metric == "ip" else capi.L2)
+        print("prepared", Q, metric, dim, k, twins, flush=True)
+        first = idx.bruteforce(q, k)
+        again = idx.bruteforce(q, k)
+        fused = idx.bruteforce_last_fused()
+        idx.bruteforce_exact_only(True)
+        want_ids, want_d, _ = idx.bruteforce(q, k)
+        idx.close()
+        assert fused or twins
+        for ids, dists, _ in (first, again):
+            assert np.array_equal(ids, want_ids) and dists.tobytes() == want_d.tobytes()
