@@ -31,6 +31,7 @@ L_STEP = 512
 # files whose text decides what the search kernels do; profiles/search_kernels_traffic.txt names their digest
 # (the kernels, and the host code that plans their launches: workgroup size, list capacities, visited form, screening form)
 KERNEL_SOURCES = ("coral_amd/csrc/beam_search.hip", "coral_amd/csrc/beam_search.h", "coral_amd/csrc/best_first.hip",
+                  "coral_amd/csrc/best_first_shared.hip", "coral_amd/csrc/best_first_device.h",
                   "coral_amd/csrc/best_first_long.hip", "coral_amd/csrc/search_device.h",
                   "coral_amd/csrc/coral_search.cpp", "coral_amd/csrc/index_internal.h")
 T0 = time.time()

@@ -6,8 +6,9 @@
 // (src/search_gpu.cu:347-580, tombstone variant :582-833) and, with
 // policy == CORAL_POLICY_BEST_FIRST, of its CPU path (src/search_in_cpu.cpp:63-108).
 // How it computes it is specific to this GPU:
-//   * per query the sorted beam (64-bit keys), the exact visited set (open
-//     addressing, 32-bit ids), the candidate buffer and the query live in LDS;
+//   * per query the sorted beam (64-bit keys), the exact visited set (a bitmap of all
+//     ids, a table of 16-bit cells, or four bits per id that hold its distance's level
+//     until it is visited), the candidate buffer and the query live in LDS;
 //     the reference keeps beam scratch and an N-bit visited bitmap per block in
 //     global memory and clears the bitmap for every query (:388);
 //   * a graph row is 32 int32 = one 128-byte line, read by half a wavefront;

@@ -140,8 +140,8 @@ typedef struct {
                                    copy (512 bytes per row at dim 200): L2 only, rows of more than 128 floats;
                                    -1 = off; 0 = the library's choice where the memory for the copy is there: rows of
                                    more than 128 floats on codes (L2 rows of more than 1024 floats in half precision)
-                                   under the rounds policy; under best-first rows of 132 .. 512 floats on codes for
-                                   beams of 410 entries and more. */
+                                   under the rounds policy; under best-first rows of 132 .. 512 floats on codes in
+                                   graphs of at least 80 nodes per beam entry. */
     int32_t visited_choices;    /* form of the table of 16-bit cells: 1 = open addressing with linear probing (a cell
                                    carries its displacement), 3 = buckets of four cells, three candidate buckets per
                                    id (a cell carries which of the three: 14 bits of the id per cell whatever the
@@ -221,7 +221,8 @@ CORAL_API int coral_search_query_counters(coral_index* idx, int32_t* host_out, i
 /* What the last coral_search_gpu call read per query, by class, int32 [Q][4] on the host: rows measured on the
  * smaller copy of the vectors, fp32 vector rows read, 32-bit words of beam state moved in global memory, visited-state
  * requests to global memory.  Every distance evaluation reads one row of one or both kinds: screened_rows +
- * exact_rows >= dist_evals >= exact_rows.  No counterpart in the reference (which reads the fp32 row for every
+ * exact_rows >= dist_evals >= exact_rows -- but where levels bound the distances (coral_plan_info.screening = 3) a row
+ * that they settle is read by no search and is in neither count.  No counterpart in the reference (which reads the fp32 row for every
  * evaluation, include/utils.cuh:254-275); these counts price the launch's memory traffic. */
 CORAL_API int coral_search_row_counters(coral_index* idx, int32_t* host_out, int32_t Q);
 
@@ -281,7 +282,8 @@ CORAL_API int coral_bruteforce_knn(coral_index* idx, const float* h_queries, int
  * query, measures those in the reference's summation order and sends the rare query whose candidates cannot vouch
  * for the result through the plain passes: same ids and distance bits either way.  The candidates are selected
  * inside the matrix-core kernel (entries up to a per-query bound, taken from a sample of the base, go to a short
- * list per query; no distance matrix is written); where that does not apply -- k + 32 > 1024, a base of fewer than
+ * list per query; no distance matrix is written; from 1e11 pair dimensions on with one product of halves per pair
+ * instead of three, unless a sample says that it leaves too much open); where that does not apply -- k + 32 > 1024, a base of fewer than
  * 64 sample tiles, a list that overflows -- the screening goes through the distance matrix instead.  on = 1 skips
  * the screening (every pair in the reference's order on the vector units); on = 2 keeps the screening and always
  * goes through the distance matrix; on = 0 restores the default.  No counterpart in the reference (faiss does this
