@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kWavesPerWg * 64, WGS) void best_first_long_kernel(
             }
             wave_sync();
             if (nc == 0) return;
-            // ---- the new keys into buf, in place (the merge of best_first.hip; buf has room for them)
+            // ---- the new keys into buf, in place: by rank, from the top (buf has room for them)
             uint64_t ck = 0;
             int p = 0x7fffffff, rank = 0;
             if (lane < nc) {

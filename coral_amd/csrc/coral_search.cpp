@@ -660,8 +660,8 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     const int id_bits = plan.id_bits;
     const int workgroups = plan.workgroups;
 
-    // Best-first on one wavefront per query: with the beam in LDS (best_first.hip; four wavefronts of a workgroup must
-    // fit) or, for longer beams, with a sorted insert buffer in LDS in front of a long run in global memory
+    // Best-first on one wavefront per query: with the beam in registers (best_first.hip; four wavefronts of a workgroup
+    // must fit) or, for longer beams, with a sorted insert buffer in LDS in front of a long run in global memory
     // (best_first_long.hip).  best_first_in_lds = 1 keeps the policy on the workgroup-per-query kernel.
     if (t.best_first_buffer != 0 && (t.best_first_buffer < 64 || t.best_first_buffer > 4096 || t.best_first_buffer % 64))
         return fail(CORAL_ERR_ARG, "best_first_buffer must be a multiple of 64 in 64..4096");
