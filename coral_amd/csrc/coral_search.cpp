@@ -489,11 +489,13 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     if (threads != 128 && threads != 256 && threads != 512 && threads != 1024)
         return fail(CORAL_ERR_ARG, "threads must be 128, 256, 512 or 1024");
     p.lds_bytes = coral::search_lds_bytes(L, idx->dim, p.table_words, tcap, ccap, ocap, p.big, screen);
-    // (the kernel that launch_search picks for such a plan; without the memory for the codes the plan is made again)
+    // The kernel that launch_search picks for such a plan; without the memory for the codes the plan is made again.  A call
+    // with the other policy runs on the plan too, and through another form: whichever of the two policies the plan is for,
+    // both forms are made ready for its LDS.
     const int form = coral::search_kernel_form(t.policy, p.big, p.direct != 0, p.choices, p.screen);
-    if (form != 0) {  // a call with the other policy runs on the plan through the form for any launch
+    for (int other : {0, coral::search_kernel_form(CORAL_POLICY_ROUNDS, p.big, p.direct != 0, p.choices, p.screen)}) {
         int any = 0;
-        HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, 0, p.lds_bytes, threads, &any));
+        if (other != form) HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, other, p.lds_bytes, threads, &any));
     }
     int wg_per_cu = 0;
     HIP_TRY(coral::search_kernel_prepare(idx->dim, p.big, form, p.lds_bytes, threads, &wg_per_cu));

@@ -1037,3 +1037,33 @@ def test_levels_from_the_matrix_cores_change_nothing(orc, law, metric, n, dim, L
                                       nbr_order=WAVE64)
         assert np.array_equal(want[:s], oi) and np.ascontiguousarray(want_d[:s]).tobytes() == od.tobytes()
         assert np.array_equal(want_c[:s], os_)
+
+
+@pytest.mark.parametrize("n,dim,L,kw", [
+    (600000, 64, 64, dict(visited_slots_log2=-1)),                        # a bitmap of all ids: 75 KB of LDS
+    (40000, 200, 600, dict(visited_choices=3, visited_slots_log2=16)),    # the table of cells in its bucket form: 128 KB
+    (20000, 200, 2000, dict(visited_slots_log2=15)),
+])
+def test_a_call_may_take_the_other_policy_than_the_plan(n, dim, L, kw):
+    """A plan made for one policy, a call with the other, both ways round: the results of a plan for the call's policy."""
+    rng = np.random.RandomState(n % 997)
+    base = synth.gaussian_matrix(31, n, dim)
+    nbrs = rng.randint(0, n, (n, 32)).astype(np.int32)
+    starts = rng.choice(n, 16, replace=False).astype(np.int32)
+    q = make_queries(300, dim, 32)
+    import torch
+    dq = torch.from_numpy(q).cuda()
+    ids, dists = torch.empty((300, 10), dtype=torch.int32, device="cuda"), torch.empty((300, 10), device="cuda")
+    print("other policy", n, dim, L, kw, flush=True)
+
+    def call(plan_policy, policy):
+        idx = capi.Index(base, nbrs, starts)
+        idx.prepare(300, L, policy=plan_policy, best_first_in_lds=True, **kw)
+        idx.search_device(dq.data_ptr(), ids.data_ptr(), dists.data_ptr(), 300, 10, policy=policy)
+        out = ids.cpu().numpy(), dists.cpu().numpy().tobytes(), idx.query_counters(300)
+        idx.close()
+        return out
+
+    for policy in (0, 1):
+        own, other = call(policy, policy), call(1 - policy, policy)
+        assert np.array_equal(own[0], other[0]) and own[1] == other[1] and np.array_equal(own[2], other[2])

@@ -1,0 +1,78 @@
+"""How the library plans, allocates and launches, without a GPU: the shared library itself with a HIP runtime in front of
+it that hands out host memory, runs no kernel and records what it is asked for (tests/fake_hip.cpp).  Every case runs in
+a process of its own, so that the stand-in meets nothing else that uses the runtime."""
+import ctypes as C
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+CASES = {}
+
+
+def case(fn):
+    CASES[fn.__name__] = fn
+    return fn
+
+
+def make(capi, n, dim, metric=0, M=4):
+    """An index whose rows and vectors are never looked at."""
+    nbrs = np.full((n, 32), -1, np.int32)
+    nbrs[:, 0] = (np.arange(n) + 1) % n
+    return capi.Index(np.ones((n, dim), np.float32), nbrs, np.arange(M, dtype=np.int32), metric)
+
+
+def call(idx, Q, k, policy):
+    q = np.zeros((Q, idx.dim), np.float32)
+    ids, dists = np.empty((Q, k), np.int32), np.empty((Q, k), np.float32)
+    return idx.search_device(q.ctypes.data, ids.ctypes.data, dists.ctypes.data, Q, k, policy=policy)
+
+
+@case
+def either_policy_may_be_called_on_a_plan_of_the_other(capi, fake):
+    # (visited set, beam) beyond the 64 KB that a kernel takes without being asked: a bitmap of all ids, a table of cells
+    # in its bucket form, a long beam
+    for n, dim, L, kw in ((600000, 64, 64, dict(visited_slots_log2=-1)), (300000, 200, 600, dict(visited_choices=3, visited_slots_log2=16)),
+                          (600000, 200, 64, dict(visited_slots_log2=-1)), (600000, 72, 4096, dict(visited_slots_log2=-1)),
+                          (20000, 200, 2000, dict(visited_slots_log2=15))):
+        for policy in (1, 0):
+            idx = make(capi, n, dim)
+            idx.prepare(700, L, policy=policy, best_first_in_lds=True, **kw)
+            fake.fake_forget()
+            for p in (policy, 1 - policy):
+                call(idx, 700, 10, p)
+            assert max(fake.fake_launch_lds(i) for i in range(fake.fake_launches())) > 65536, (n, L, policy)
+            assert fake.fake_launches_beyond_limit() == 0, (n, L, policy)
+            idx.close()
+
+
+@pytest.fixture(scope="module")
+def fake_runtime(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    r = subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__",
+                        "-I/opt/rocm/include", os.path.join(HERE, "fake_hip.cpp"), "-o", out], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    return out
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_host_side(fake_runtime, name):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), fake_runtime, name], capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
+    runtime = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+    for name in ("fake_live_bytes", "fake_live_of_size", "fake_launches", "fake_launch_lds", "fake_launches_beyond_limit"):
+        getattr(runtime, name).restype = C.c_size_t
+    runtime.fake_live_of_size.argtypes = [C.c_size_t]
+    runtime.fake_refuse.argtypes = [C.c_size_t, C.c_size_t]
+    runtime.fake_launch_lds.argtypes = runtime.fake_launch_threads.argtypes = [C.c_size_t]
+    from coral_amd import capi as binding
+    CASES[sys.argv[2]](binding, runtime)
