@@ -172,6 +172,9 @@ constexpr int kMaxByteRowDimRounds = 2048;  // ... in the workgroup-per-query ke
 hipError_t launch_half_rows(const float* vec, int64_t n, int dim, unsigned char* out, hipStream_t stream);
 // 64-bit words of global scratch one workgroup of a BIG launch needs for a beam of capacity L
 size_t search_beam_stride(int L);
+// The limit on a kernel's dynamic LDS on the current device is only ever raised: a launch planned earlier -- the entry
+// point that allocates nothing keeps its plan, another index has its own -- must stay valid after a later plan with less.
+hipError_t raise_lds_limit(const void* kernel, size_t lds_bytes);
 // form: 1 with levels, else what search_kernel_form says of the launch; 0 takes any
 hipError_t search_kernel_prepare(int dim, bool big, int form, size_t lds_bytes, int threads, int* max_wg_per_cu);
 int search_kernel_form(int policy, bool big, bool direct, int choices, int screen);

@@ -1219,26 +1219,25 @@ size_t search_beam_stride(int L) {
     return (2 * Lp + Lp / 2 + 15) & ~(size_t)15;  // [2][Lp] keys + Lp 32-bit ids, a multiple of 128 bytes
 }
 
-hipError_t search_kernel_prepare(int dim, bool big, int form, size_t lds_bytes, int threads, int* max_wg_per_cu) {
-    kernel_fn fn = pick_kernel(dim, big, form);
-    if (!fn) return hipErrorInvalidValue;
-    // The limit on a kernel's dynamic LDS is only ever raised: a launch planned earlier (the entry point that
-    // allocates nothing keeps its plan) must stay valid after a later plan for a shorter beam.
+hipError_t raise_lds_limit(const void* kernel, size_t lds_bytes) {
     static std::mutex mu;
     static std::map<std::pair<const void*, int>, size_t> limit;
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
-    {
-        std::lock_guard<std::mutex> lock(mu);
-        size_t& have = limit[{reinterpret_cast<const void*>(fn), device}];
-        if (lds_bytes > have) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds_bytes);
-            if (e != hipSuccess) return e;
-            have = lds_bytes;
-        }
-    }
+    std::lock_guard<std::mutex> lock(mu);
+    size_t& have = limit[{kernel, device}];
+    if (lds_bytes <= have) return hipSuccess;
+    e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
+    if (e == hipSuccess) have = lds_bytes;
+    return e;
+}
+
+hipError_t search_kernel_prepare(int dim, bool big, int form, size_t lds_bytes, int threads, int* max_wg_per_cu) {
+    kernel_fn fn = pick_kernel(dim, big, form);
+    if (!fn) return hipErrorInvalidValue;
+    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(fn), lds_bytes);
+    if (e != hipSuccess) return e;
     int nb = 0;
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(fn), threads,
                                                      lds_bytes);

@@ -121,8 +121,7 @@ hipError_t best_first_prepare(int dim, int L, int rows_in_flight, int screen, si
     const size_t lds = wave_lds * kWavesPerWg;
     bf_kernel_fn fn = pick_bf_kernel(dim, rows_in_flight, screen, L);
     if (!fn) return hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds);
+    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(fn), lds);
     if (e != hipSuccess) return e;
     int nb = 0;
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(fn), kWavesPerWg * 64, lds);

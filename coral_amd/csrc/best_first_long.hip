@@ -545,8 +545,7 @@ hipError_t best_first_long_prepare(int dim, bool packed, bool screen, int bcap, 
     const size_t lds = best_first_long_lds_bytes(bcap, scap, screen ? best_first_long_coded_bytes(dim) : 0) * kWavesPerWg;
     bfl_kernel_fn fn = pick(dim, packed, screen, wgs_class(lds));
     if (!fn) return hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds);
+    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(fn), lds);
     if (e != hipSuccess) return e;
     int nb = 0;
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(fn), kWavesPerWg * 64, lds);

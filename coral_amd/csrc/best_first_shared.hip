@@ -38,7 +38,7 @@ hipError_t best_first_shared_prepare(int dim, int L, int screen, size_t lds, int
     if (screen == 1 || (screen == 2 && dim > kMaxByteRowDim)) return hipErrorInvalidValue;
     bf_kernel_fn fn = screen == 2 ? pick_shared<2>(dim, L) : pick_shared<0>(dim, L);
     if (!fn) return hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    hipError_t e = raise_lds_limit(reinterpret_cast<const void*>(fn), lds);
     if (e != hipSuccess) return e;
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(max_wg_per_cu, reinterpret_cast<const void*>(fn), kWavesPerWg * 64, lds);
 }

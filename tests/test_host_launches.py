@@ -50,6 +50,26 @@ def either_policy_may_be_called_on_a_plan_of_the_other(capi, fake):
             idx.close()
 
 
+@case
+def a_plan_of_one_index_stays_valid_after_a_smaller_one_of_another(capi, fake):
+    # the same kernel, with more LDS on the larger index: wavefronts with a bitmap of all ids, four wavefronts per query,
+    # the long beam with a larger insert buffer, a workgroup per query
+    for nodes, dim, L, Q, policy, kw in (((250000, 20000), 200, 64, 1000, 1, {}), ((600000, 200000), 200, 64, 100, 1, {}),
+                                         ((9000, 9000), 96, 2000, 20, 1, dict(best_first_buffer=(1024, 768))),
+                                         ((600000, 200000), 200, 64, 100, 0, {})):
+        pair = []
+        for i, n in enumerate(nodes):
+            pair.append(make(capi, n, dim))
+            pair[-1].prepare(Q, L, policy=policy, **{k: v[i] for k, v in kw.items()})
+        fake.fake_forget()
+        for idx in pair:
+            call(idx, Q, 10, policy)
+        lds = [fake.fake_launch_lds(i) for i in range(fake.fake_launches())]
+        assert max(lds) > 65536 and fake.fake_launches_beyond_limit() == 0, (nodes, L, policy, lds)
+        for idx in pair:
+            idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
