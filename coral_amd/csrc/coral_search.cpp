@@ -852,8 +852,14 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         const int rif = eight && L <= 1024 && idx->bf_screen != 1 ? 32 : idx->bf_screen != 0 ? 8 : 16;
         idx->bf_rows_in_flight = rif;
         HIP_TRY(coral::best_first_prepare(idx->dim, L, rif, idx->bf_screen, wave_lds, &bf_wg_per_cu));
-        auto reprepare = [&](int*) -> hipError_t { return hipSuccess; };  // (one kernel for both forms)
-        if (int rc = visited_slots(bf_wg_per_cu, reprepare, 0)) return rc;
+        if (bitmap_words != 0) {
+            // (nothing of the visited state lies in HBM: a slot costs no memory)
+            idx->bf_slots = (int)std::min<int64_t>((int64_t)bf_wg_per_cu * idx->num_cu * 4, Q);
+            idx->bf_ready = idx->bf_slots > 0;
+        } else {
+            auto reprepare = [&](int*) -> hipError_t { return hipSuccess; };  // (one kernel for both forms)
+            if (int rc = visited_slots(bf_wg_per_cu, reprepare, 0)) return rc;
+        }
     } else if (long_form) {
         // the insert buffer: 512 keys unless the caller names a size; a sample of at most 128 keys of the long run
         const int bcap = t.best_first_buffer ? t.best_first_buffer : 512;

@@ -70,6 +70,26 @@ def a_plan_of_one_index_stays_valid_after_a_smaller_one_of_another(capi, fake):
             idx.close()
 
 
+@case
+def a_best_first_launch_on_the_bitmap_takes_no_visited_state_in_global_memory(capi, fake):
+    n, dim, Q, L = 250000, 200, 1000, 64
+    state = n * Q  # a byte per node and query slot (n is a multiple of 16)
+    idx = make(capi, n, dim)
+    for refused in (False, True):  # nor does a refusal of it send the policy to the workgroup-per-query kernel
+        fake.fake_refuse(state, state + 1 if refused else state)
+        idx.prepare(Q, L, policy=1)
+        plan = idx.plan_info()
+        assert plan.kernel == 1 and plan.visited_form == 1 and plan.query_slots == Q
+        assert fake.fake_live_of_size(state) == 0
+    call(idx, Q, 10, 1)
+    idx.prepare(Q, L, policy=1, best_first_table_log2=-1)  # without the bitmap the state is there
+    assert idx.plan_info().kernel == 0  # (refused: the other kernel)
+    fake.fake_refuse(0, 0)
+    idx.prepare(Q, L, policy=1, best_first_table_log2=-1)
+    assert idx.plan_info().kernel == 1 and fake.fake_live_of_size(state) == 1
+    idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
