@@ -917,9 +917,14 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
                 }
             }
             if (lp.levels) {
-                if (int rc = coral::ensure_base_norms(idx, idx->stream)) return rc;
-                if (int rc = coral::ensure_base_loss(idx, idx->stream)) return rc;
-                idx->level_plan = lp, idx->level_rows = rows;
+                int rc = coral::ensure_base_norms(idx, idx->stream);
+                if (rc == CORAL_OK) rc = coral::ensure_base_loss(idx, idx->stream);
+                if (rc == CORAL_OK)
+                    idx->level_plan = lp, idx->level_rows = rows;
+                else if (rc == CORAL_ERR_MEMORY)
+                    (void)hipGetLastError();  // no room for the norms: the search runs without, too
+                else
+                    return rc;
             }
         }
     }

@@ -90,6 +90,26 @@ def a_best_first_launch_on_the_bitmap_takes_no_visited_state_in_global_memory(ca
     idx.close()
 
 
+@case
+def without_memory_for_what_levels_need_the_search_runs_without_them(capi, fake):
+    n, dim, Q, L = 60000, 512, 2000, 256
+    pitch = (n + 127) // 128 * 64  # bytes of one query's levels
+    for at_least, below in ((n * 4, n * 4 + 1), (pitch * Q, 1 << 40), (8, 9)):  # norms; the block of levels; the norms' largest
+        idx = make(capi, n, dim)
+        fake.fake_refuse(at_least, below)
+        if at_least == 8:  # (as large as the word for the hits of a verification, which is there by now)
+            assert fake.fake_live_of_size(8) == 1
+        idx.prepare(Q, L)
+        plan = idx.plan_info()
+        assert plan.visited_form != 6 and plan.screening == 2
+        call(idx, Q, 10, 0)
+        fake.fake_refuse(0, 0)
+        idx.prepare(Q, L)
+        assert idx.plan_info().visited_form == 6
+        call(idx, Q, 10, 0)
+        idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
