@@ -89,6 +89,13 @@ static hipError_t quiesce(coral_index* idx) {
     return e;
 }
 
+// (every search that reads it has been waited for)
+void coral::free_levels(coral_index* idx) {
+    (void)hipFree(idx->d_level_block);
+    idx->d_level_block = nullptr, idx->level_block_bytes = 0, idx->level_rows = 0;
+    idx->level_plan = coral_search_plan{};
+}
+
 extern "C" {
 
 const char* coral_last_error(void) { return g_err.c_str(); }
@@ -214,7 +221,7 @@ void coral_index_destroy(coral_index* idx) {
     (void)hipFree(idx->d_bnorm);
     (void)hipFree(idx->d_bnorm_max);
     (void)hipFree(idx->knn_block);
-    (void)hipFree(idx->d_level_block);
+    coral::free_levels(idx);
     (void)hipFree(idx->d_io_q);
     (void)hipFree(idx->d_io_ids);
     (void)hipFree(idx->d_io_dists);
@@ -893,7 +900,8 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         idx->bf_long = idx->bf_ready;
         idx->bf_bcap = bcap, idx->bf_scap = scap, idx->bf_sshift = sshift, idx->bf_beam_stride = beam_stride;
     }
-    // levels for the whole batch, where the caller leaves the launch to the library
+    // levels for the whole batch, where the caller leaves the launch to the library; their scratch goes back with a plan
+    // that has none
     idx->level_plan = coral_search_plan{};
     if (!best_first && !t.visited_slots_log2 && !t.workgroups && !t.threads && !t.beam_in_hbm && !t.prefetch_rows && !t.cand_cap &&
         !t.screening && !t.visited_choices) {
@@ -928,6 +936,7 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
             }
         }
     }
+    if (!idx->level_plan.levels) coral::free_levels(idx);
     HIP_TRY(hipStreamSynchronize(idx->stream));
     idx->Q = Q, idx->L = L, idx->plan = plan;
     idx->prepared_policy = t.policy;

@@ -189,6 +189,7 @@ int coral_build_end(coral_index* idx) {
     HIP_TRY(hipSetDevice(idx->device));
     HIP_TRY(hipStreamSynchronize(idx->stream));
     coral::free_build_state(idx);
+    coral::free_levels(idx);  // (a search on the plan that the construction left runs without)
     return CORAL_OK;
 }
 

@@ -140,6 +140,7 @@ struct coral_index {
 
 namespace coral {
 void free_build_state(coral_index* idx);
+void free_levels(coral_index* idx);  // the scratch of the levels and the plan that takes it (coral_search.cpp)
 int ensure_base_norms(coral_index* idx, hipStream_t stream);  // d_bnorm, d_bnorm_max (bruteforce_api.cpp)
 int ensure_base_loss(coral_index* idx, hipStream_t stream);   // d_bnorm_max[1]
 }

@@ -188,7 +188,9 @@ CORAL_API int coral_index_info(const coral_index* idx, int64_t* n, int32_t* dim,
 #define CORAL_MAX_BEAM 65536
 
 /* GPUFuncs::search_prepare(Q, L) (src/search.cu:400-408): fixes the beam
- * capacity (1..CORAL_MAX_BEAM) and (re)allocates per-workgroup scratch. */
+ * capacity (1..CORAL_MAX_BEAM) and (re)allocates per-workgroup scratch.  A plan with levels (coral_plan_info.screening
+ * = 3) holds n / 2 bytes per query for up to 1 GiB of them at a time, and 2 KB and 2 dim bytes per query to make them,
+ * until a plan without, coral_build_end or coral_index_destroy; where that finds no memory the plan is one without. */
 CORAL_API int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tuning* tuning);
 
 /* GPUFuncs::search_gpu (src/search_gpu.cu:835-886): device pointers in and out,
@@ -368,7 +370,8 @@ CORAL_API int coral_build_params_default(coral_build_params* p);
 
 /* Graph ctor in construction mode: every row empty.  On a vectors-only index this creates the rows. */
 CORAL_API int coral_build_begin(coral_index* idx, int32_t R);
-/* frees the per-neighbour distances and the staging; the rows and start ids stay */
+/* frees the per-neighbour distances, the staging and the levels' scratch of the construction's searches; the rows and
+ * start ids stay */
 CORAL_API int coral_build_end(coral_index* idx);
 
 /* Graph ctor in Mode::CE (include/graph.cuh:252-256, DS.load_batch_slots of every node): construction state from

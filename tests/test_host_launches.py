@@ -110,6 +110,36 @@ def without_memory_for_what_levels_need_the_search_runs_without_them(capi, fake)
         idx.close()
 
 
+@case
+def the_scratch_of_the_levels_goes_back(capi, fake):
+    n, dim, Q, L = 60000, 512, 2000, 256
+    least = (n + 127) // 128 * 64 * Q
+    idx = make(capi, n, dim)
+    idx.prepare(Q, L, threads=512)  # (named: no levels; the copy in codes and the counters are there from here on)
+    assert idx.plan_info().visited_form != 6
+
+    def hold_levels():
+        idx.prepare(Q, L)
+        assert idx.plan_info().visited_form == 6
+        return fake.fake_live_bytes()
+
+    for q, again in ((Q, dict(threads=512)), (Q, dict(policy=1, best_first_in_lds=True)), (100, {})):  # plans without
+        held = hold_levels()
+        idx.prepare(q, L, **again)
+        assert fake.fake_live_bytes() < held - least, again
+    held = hold_levels()
+    fake.fake_forget()
+    call(idx, Q, 10, 0)
+    levels = fake.fake_launch_fn(fake.fake_launches() - 1)
+    assert capi.lib().coral_build_end(idx._h) == 0  # the end of a construction, whose searches plan them too
+    assert fake.fake_live_bytes() < held - least and idx.plan_info().visited_form != 6
+    call(idx, Q, 10, 0)  # the plan that is left is one without
+    assert fake.fake_launch_fn(fake.fake_launches() - 1) != levels and fake.fake_launches_beyond_limit() == 0
+    hold_levels()
+    idx.close()
+    assert fake.fake_live_bytes() == 0
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
@@ -134,5 +164,6 @@ if __name__ == "__main__":
     runtime.fake_live_of_size.argtypes = [C.c_size_t]
     runtime.fake_refuse.argtypes = [C.c_size_t, C.c_size_t]
     runtime.fake_launch_lds.argtypes = runtime.fake_launch_threads.argtypes = [C.c_size_t]
+    runtime.fake_launch_fn.restype, runtime.fake_launch_fn.argtypes = C.c_void_p, [C.c_size_t]
     from coral_amd import capi as binding
     CASES[sys.argv[2]](binding, runtime)
