@@ -48,9 +48,9 @@ class PlanInfo(C.Structure):
                 ("cand_cap", C.c_int32), ("query_slots", C.c_int32), ("reserved", C.c_int32 * 4)]
 
     KERNELS = ("beam_search_kernel", "best_first_wave_kernel", "best_first_long_kernel")
-    SCREENING = ("none", "fp16", "int8")
+    SCREENING = ("none", "fp16", "int8", "levels")
     VISITED = ("lds_table16+hbm_bitmap", "lds_bitmap", "hbm_bytes", "hbm_packed_words", "lds_table16+hbm_state",
-               "lds_buckets16x3+hbm_bitmap")
+               "lds_buckets16x3+hbm_bitmap", "lds_levels")
 
     def as_dict(self):
         d = {f: getattr(self, f) for f, _ in self._fields_ if f != "reserved"}

@@ -140,6 +140,18 @@ def the_scratch_of_the_levels_goes_back(capi, fake):
     assert fake.fake_live_bytes() == 0
 
 
+@case
+def every_plan_has_its_names(capi, fake):
+    idx = make(capi, 60000, 512)
+    for Q, L, kw, screening, visited in ((2000, 256, {}, "levels", "lds_levels"), (2000, 256, dict(threads=512), "int8", None),
+                                         (100, 64, dict(screening=-1), "none", "lds_bitmap"), (100, 64, dict(screening=1), "fp16", None)):
+        idx.prepare(Q, L, **kw)
+        plan = idx.plan_info().as_dict()
+        assert plan["kernel"] == "beam_search_kernel" and plan["screening"] == screening
+        assert visited is None or plan["visited_form"] == visited
+    idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
