@@ -50,11 +50,12 @@ def algorithmic_bytes(expansions, dist_evals, Q, dim, k, R=32):
 def scheme_bytes(st, plan, Q, dim, k, R=32):
     """What this library's kernels must read for the traversal, from the kernels' own counts of the rows they
     requested: a graph row per expansion, a row of the smaller copy (eight-bit codes or half precision) per screened
-    evaluation, an fp32 row per evaluation the screening left open (all of them without screening), the queries,
-    the ids and the per-query counters written.  No credit for scratch (beam passes, visited state): those are
+    evaluation, an fp32 row per evaluation the screening left open (all of them without screening), a query's levels
+    written and read where the launch has them (not the matrix-core kernel's reads of the base), the queries, the ids
+    and the per-query counters written.  No credit for scratch (beam passes, visited state): those are
     `scratch_bytes`."""
     return (st.expansions * R * 4 + st.screened_rows * plan.screen_row_bytes + st.exact_rows * dim * 4 +
-            Q * (dim * 4 + k * 4 + 32))
+            Q * (dim * 4 + k * 4 + 32 + 2 * plan.level_bytes))
 
 
 def scratch_bytes(st):

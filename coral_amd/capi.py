@@ -45,7 +45,8 @@ class PlanInfo(C.Structure):
     _fields_ = [("kernel", C.c_int32), ("threads", C.c_int32), ("workgroups", C.c_int32), ("lds_bytes", C.c_int32),
                 ("screening", C.c_int32), ("screen_row_bytes", C.c_int32), ("visited_form", C.c_int32),
                 ("visited_slots_log2", C.c_int32), ("beam_in_hbm", C.c_int32), ("todo_cap", C.c_int32),
-                ("cand_cap", C.c_int32), ("query_slots", C.c_int32), ("reserved", C.c_int32 * 4)]
+                ("cand_cap", C.c_int32), ("query_slots", C.c_int32), ("level_bytes", C.c_int32),
+                ("reserved", C.c_int32 * 3)]
 
     KERNELS = ("beam_search_kernel", "best_first_wave_kernel", "best_first_long_kernel")
     SCREENING = ("none", "fp16", "int8", "levels")

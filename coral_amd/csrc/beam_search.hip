@@ -1114,7 +1114,7 @@ __global__ __launch_bounds__(1024) void beam_search_kernel(const SearchArgs a) {
                 {
                     int32_t* rc = a.counters + ((size_t)a.Q + qid) * 4;
                     // (ids sent to the bitmap in global memory: one atomic each; the clean-up writes them once more)
-                    rc[0] = s_rows_screened, rc[1] = s_rows_exact, rc[2] = s_beam_words, rc[3] = LEVELS || BITMAP ? 0 : 2 * s_nover;
+                    rc[0] = LEVELS ? s_new : s_rows_screened, rc[1] = s_rows_exact, rc[2] = s_beam_words, rc[3] = LEVELS || BITMAP ? 0 : 2 * s_nover;
                 }
                 if (!LEVELS && !BITMAP && s_nover > 0) atomicAdd(a.spill_count, 1);
             }

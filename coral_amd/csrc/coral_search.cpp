@@ -1255,7 +1255,7 @@ int coral_search_plan_info(const coral_index* idx, coral_plan_info* out) {
         const coral_search_plan& lp = idx->level_plan;
         out->kernel = 0;
         out->threads = lp.threads, out->workgroups = out->query_slots = std::min(lp.workgroups, idx->Q), out->lds_bytes = (int32_t)lp.lds_bytes;
-        out->screening = 3, out->visited_form = 6, out->todo_cap = lp.tcap, out->cand_cap = lp.ccap;
+        out->screening = 3, out->visited_form = 6, out->level_bytes = (int32_t)coral::level_pitch(idx->n), out->todo_cap = lp.tcap, out->cand_cap = lp.ccap;
     } else {
         out->kernel = 0;
         out->threads = p.threads, out->workgroups = p.workgroups, out->lds_bytes = (int32_t)p.lds_bytes;

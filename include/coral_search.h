@@ -223,9 +223,10 @@ CORAL_API int coral_search_query_counters(coral_index* idx, int32_t* host_out, i
 /* What the last coral_search_gpu call read per query, by class, int32 [Q][4] on the host: rows measured on the
  * smaller copy of the vectors, fp32 vector rows read, 32-bit words of beam state moved in global memory, visited-state
  * requests to global memory.  Every distance evaluation reads one row of one or both kinds: screened_rows +
- * exact_rows >= dist_evals >= exact_rows -- but where levels bound the distances (coral_plan_info.screening = 3) a row
- * that they settle is read by no search and is in neither count.  No counterpart in the reference (which reads the fp32 row for every
- * evaluation, include/utils.cuh:254-275); these counts price the launch's memory traffic. */
+ * exact_rows >= dist_evals >= exact_rows.  Where levels bound the distances (coral_plan_info.screening = 3) screened_rows
+ * counts the rows whose level was looked at, in LDS: what such a launch moves beside exact_rows is level_bytes per query,
+ * written and read, and the base, once per block of queries.  No counterpart in the reference (which reads the fp32 row
+ * for every evaluation, include/utils.cuh:254-275); these counts price the launch's memory traffic. */
 CORAL_API int coral_search_row_counters(coral_index* idx, int32_t* host_out, int32_t Q);
 
 /* The launch geometry the last coral_search_prepare chose (what a search call on this index runs with). */
@@ -239,7 +240,7 @@ typedef struct {
     int32_t screening;       /* 0 none, 1 half precision, 2 eight-bit codes, 3 levels: four bits per query and node that bound
                                 the distance, made for the whole batch on the matrix cores (rounds policy, 512 queries and
                                 more, where the launch is left to the library and they pay); rows they settle are read
-                                by no search and counted in no class of coral_search_row_counters */
+                                by no search */
     int32_t screen_row_bytes;/* bytes of one row of the smaller copy (0 without screening) */
     int32_t visited_form;    /* 0 table of 16-bit cells in LDS + bitmap in global memory, 1 bitmap of all ids in LDS,
                                 2 bytes per node and slot in global memory, 3 packed words in global memory,
@@ -250,7 +251,8 @@ typedef struct {
     int32_t beam_in_hbm;     /* the beam (or the long run) lives in global memory */
     int32_t todo_cap, cand_cap; /* LDS list capacities of the workgroup kernel */
     int32_t query_slots;     /* queries in flight */
-    int32_t reserved[4];
+    int32_t level_bytes;     /* levels: bytes of one query's (0 without) */
+    int32_t reserved[3];
 } coral_plan_info;
 CORAL_API int coral_search_plan_info(const coral_index* idx, coral_plan_info* out);
 

@@ -1067,3 +1067,23 @@ def test_a_call_may_take_the_other_policy_than_the_plan(n, dim, L, kw):
     for policy in (0, 1):
         own, other = call(policy, policy), call(1 - policy, policy)
         assert np.array_equal(own[0], other[0]) and own[1] == other[1] and np.array_equal(own[2], other[2])
+
+
+def test_row_counters_of_a_launch_with_levels():
+    """Every evaluation is counted as looked at on its level, in fp32, or both, as with every other screening; the start
+    ids alone are measured without."""
+    n, dim, L, M, Q = 20000, 264, 256, 16, 1600
+    base, nbrs, starts = problem(n, dim, 32, 77, "l2", M)
+    q = make_queries(Q, dim, 78)
+    idx = capi.Index(base, nbrs, starts)
+    idx.prepare(Q, L)
+    plan = idx.plan_info()
+    assert plan.screening == 3 and plan.level_bytes == (n + 127) // 128 * 64
+    print("levels' counters", flush=True)
+    _, _, st = idx.search(q, 50, L)
+    cnt, rows = idx.query_counters(Q), idx.row_counters(Q)
+    assert np.array_equal(rows[:, 0], cnt[:, 2] - M) and (rows[:, 1] >= M).all() and (rows[:, 1] <= cnt[:, 2]).all()
+    assert (st.screened_rows, st.exact_rows, st.beam_words, st.visited_requests) == tuple(int(x) for x in rows.sum(0))
+    idx.prepare(Q, L, threads=512)
+    assert idx.plan_info().level_bytes == 0
+    idx.close()
