@@ -46,7 +46,7 @@ class PlanInfo(C.Structure):
                 ("screening", C.c_int32), ("screen_row_bytes", C.c_int32), ("visited_form", C.c_int32),
                 ("visited_slots_log2", C.c_int32), ("beam_in_hbm", C.c_int32), ("todo_cap", C.c_int32),
                 ("cand_cap", C.c_int32), ("query_slots", C.c_int32), ("level_bytes", C.c_int32),
-                ("reserved", C.c_int32 * 3)]
+                ("levels_unfit", C.c_int32), ("reserved", C.c_int32 * 2)]
 
     KERNELS = ("beam_search_kernel", "best_first_wave_kernel", "best_first_long_kernel")
     SCREENING = ("none", "fp16", "int8", "levels")

@@ -67,10 +67,11 @@ hipError_t launch_count_close(const float* D, int64_t ldD, int nq, int64_t n, in
 // the lower end void for l = 0 and the upper one for l = 0 and l = 14; ranges[q] = origin, 1 / step, step, E (1 / step = 0: all
 // levels are 0).  Point i of query q: bits 4 (i & 1) of byte levels[q * level_pitch(n) + i / 2].
 size_t level_pitch(int64_t n);
-// D: [nq][n] approximate distances to a sample of the base, made on one product
+// D: [nq][n] approximate distances to a sample of the base, made on one product; unfit: null, or a word that grows by the
+// queries whose levels would settle little
 hipError_t launch_level_ranges(const float* D, int64_t ldD, int nq, int n, int dim, int metric, const float* qn,
                                const uint32_t* bn_max_bits, const float* qres, const uint32_t* bres_max_bits, float4* ranges,
-                               hipStream_t stream);
+                               int* unfit, hipStream_t stream);
 // queries: split for one product
 hipError_t launch_levels(const void* queries, const float* base, int nq, int64_t nb, int dim, int metric, const float* qn,
                          const float* bn, const float4* ranges, unsigned char* levels, hipStream_t stream);

@@ -17,6 +17,7 @@
 #include "beam_search.h"
 #include "bruteforce.h"
 #include "error.h"
+#include "graph_build.h"
 #include "index_internal.h"
 
 namespace {
@@ -558,6 +559,49 @@ static size_t level_block(const coral_index* idx, int rows, void* block, LevelSc
     return at;
 }
 
+// The scratch's qn, qres, split and ranges of m queries, from the distances to a sample of the base: what launch_levels
+// takes.  unfit: as in launch_level_ranges.
+static hipError_t launch_level_scratch(const coral_index* idx, const float* d_queries, int m, const LevelScratch& w, int* unfit,
+                                       hipStream_t stream) {
+    const int64_t tiles = std::min<int64_t>(kLevelSampleTiles, std::max<int64_t>(1, idx->n / 128));
+    const int64_t sampled = std::min<int64_t>(tiles * 128, idx->n);
+    hipError_t e = coral::launch_prepare_queries(d_queries, m, idx->dim, 1, w.qn, w.qres, w.split, nullptr, nullptr, stream);
+    if (e == hipSuccess)
+        e = coral::launch_approx_tile(w.split, idx->d_vec, m, idx->n, idx->dim, idx->metric, 1, w.qn, idx->d_bnorm, nullptr, 0, w.D,
+                                      kLevelSampleTiles * 128, stream, tiles, (int)std::max<int64_t>(1, idx->n / 128 / tiles));
+    if (e == hipSuccess)
+        e = coral::launch_level_ranges(w.D, kLevelSampleTiles * 128, m, (int)sampled, idx->dim, idx->metric, w.qn, idx->d_bnorm_max,
+                                       w.qres, idx->d_bnorm_max + 1, w.ranges, unfit, stream);
+    return e;
+}
+
+// Once per index: do levels settle rows of this base?  The bound that widens them grows with the largest row of the base
+// and the origin with what all rows have in common, so an offset or a single huge row can leave every row open, at up to
+// 2.2 times the time without.  Asked of the base's own rows: 256 of them as queries (a batch of other queries than that is
+// looked at afterwards, see search_launch).
+static int probe_levels(coral_index* idx) {
+    LevelScratch w;
+    (void)level_block(idx, idx->level_rows, idx->d_level_block, &w);
+    const int m = (int)std::min<int64_t>(256, idx->n);
+    const size_t row_bytes = (size_t)m * idx->dim * sizeof(float);
+    // (the queries and their ids lie where the levels will: hundreds of rows of n / 2 bytes)
+    if (row_bytes + (size_t)m * sizeof(int32_t) > (size_t)idx->level_rows * coral::level_pitch(idx->n)) return CORAL_OK;
+    float* d_rows = reinterpret_cast<float*>(w.levels);
+    int32_t* d_ids = reinterpret_cast<int32_t*>(w.levels + row_bytes);
+    std::vector<int32_t> ids((size_t)m);
+    for (int i = 0; i < m; ++i) ids[(size_t)i] = (int32_t)((int64_t)i * idx->n / m);
+    int* d_unfit = idx->d_scalars + 3;
+    int unfit = 0;
+    HIP_TRY(hipMemcpyAsync(d_ids, ids.data(), (size_t)m * sizeof(int32_t), hipMemcpyHostToDevice, idx->stream));
+    HIP_TRY(coral::launch_fill_u32((uint32_t*)d_unfit, 1, 0u, idx->stream));
+    HIP_TRY(coral::launch_gather_rows(idx->d_vec, idx->dim, d_ids, m, d_rows, idx->stream));
+    HIP_TRY(launch_level_scratch(idx, d_rows, m, w, d_unfit, idx->stream));
+    HIP_TRY(hipMemcpyAsync(&unfit, d_unfit, sizeof unfit, hipMemcpyDeviceToHost, idx->stream));
+    HIP_TRY(hipStreamSynchronize(idx->stream));
+    idx->levels_fit = 2 * unfit <= m;
+    return CORAL_OK;
+}
+
 // Do levels pay?  Per query they cost what the matrix cores and their way into LDS take of every node, about 0.65 + 0.002
 // dim picoseconds, and spare the rows (bytes each, on codes or in fp32) that a search reads without need, four in five, at
 // 7 TB/s: of x = 45 first visits per beam entry under L2, 1.7 times as many under the inner product, x / (1 + x / c n) as
@@ -612,6 +656,40 @@ static int plan_levels(coral_index* idx, int32_t Q, int32_t L, const coral_searc
     p.prefetch = wg_per_cu == 1;
     p.levels = 1;
     *out = p;
+    return CORAL_OK;
+}
+
+// The index's plan with levels and its scratch.  Where that finds no memory there is none; where the base has been found
+// unfit there is the plan, for coral_search_plan_info, but no scratch.
+static int take_levels(coral_index* idx, int32_t Q, const coral_search_plan& lp) {
+    if (idx->levels_fit != 0) {
+        const int64_t fit = std::max<int64_t>(1, (int64_t)(kLevelBytes / coral::level_pitch(idx->n)) / 256);
+        const int rows = (int)(std::min<int64_t>(fit, ((int64_t)Q + 255) / 256) * 256);
+        const size_t need = level_block(idx, rows, nullptr, nullptr);
+        int rc = CORAL_OK;
+        if (need > idx->level_block_bytes) {
+            coral::free_levels(idx);
+            const hipError_t e = hipMalloc(&idx->d_level_block, need);
+            if (e == hipSuccess)
+                idx->level_block_bytes = need;
+            else if (e == hipErrorOutOfMemory)
+                rc = CORAL_ERR_MEMORY;
+            else
+                HIP_TRY(e);
+        }
+        if (rc == CORAL_OK) rc = coral::ensure_base_norms(idx, idx->stream);
+        if (rc == CORAL_OK) rc = coral::ensure_base_loss(idx, idx->stream);
+        if (rc == CORAL_ERR_MEMORY) {
+            (void)hipGetLastError();
+            return CORAL_OK;
+        }
+        if (rc != CORAL_OK) return rc;
+        idx->level_rows = rows;
+        if (idx->levels_fit < 0)
+            if (int bad = probe_levels(idx)) return bad;
+    }
+    if (idx->levels_fit == 0) coral::free_levels(idx);
+    idx->level_plan = lp;
     return CORAL_OK;
 }
 
@@ -902,39 +980,13 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     }
     // levels for the whole batch, where the caller leaves the launch to the library; their scratch goes back with a plan
     // that has none
-    idx->level_plan = coral_search_plan{};
+    idx->level_plan = coral_search_plan{}, idx->levels_failed = false;
     if (!best_first && !t.visited_slots_log2 && !t.workgroups && !t.threads && !t.beam_in_hbm && !t.prefetch_rows && !t.cand_cap &&
         !t.screening && !t.visited_choices) {
         coral_search_plan lp;
         if (int rc = plan_levels(idx, Q, L, plan, &lp)) return rc;
-        if (lp.levels) {
-            const size_t pitch = coral::level_pitch(idx->n);
-            const int64_t fit = std::max<int64_t>(1, (int64_t)(kLevelBytes / pitch) / 256);
-            const int rows = (int)(std::min<int64_t>(fit, ((int64_t)Q + 255) / 256) * 256);
-            const size_t need = level_block(idx, rows, nullptr, nullptr);
-            if (need > idx->level_block_bytes) {
-                (void)hipFree(idx->d_level_block);
-                idx->d_level_block = nullptr, idx->level_block_bytes = 0;
-                const hipError_t e = hipMalloc(&idx->d_level_block, need);
-                if (e == hipSuccess) {
-                    idx->level_block_bytes = need;
-                } else {
-                    HIP_TRY(e == hipErrorOutOfMemory ? hipSuccess : e);
-                    (void)hipGetLastError();
-                    lp.levels = 0;  // the search runs without
-                }
-            }
-            if (lp.levels) {
-                int rc = coral::ensure_base_norms(idx, idx->stream);
-                if (rc == CORAL_OK) rc = coral::ensure_base_loss(idx, idx->stream);
-                if (rc == CORAL_OK)
-                    idx->level_plan = lp, idx->level_rows = rows;
-                else if (rc == CORAL_ERR_MEMORY)
-                    (void)hipGetLastError();  // no room for the norms: the search runs without, too
-                else
-                    return rc;
-            }
-        }
+        if (lp.levels)
+            if (int rc = take_levels(idx, Q, lp)) return rc;
     }
     if (!idx->level_plan.levels) coral::free_levels(idx);
     HIP_TRY(hipStreamSynchronize(idx->stream));
@@ -987,7 +1039,8 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
     hipStream_t stream = stream_ ? (hipStream_t)stream_ : idx->stream;
 
     const coral_search_plan& plan = idx->plan;
-    const bool use_levels = policy == CORAL_POLICY_ROUNDS && idx->level_plan.levels && levels_pay(idx, plan, Q, idx->L);
+    const bool use_levels = policy == CORAL_POLICY_ROUNDS && idx->level_plan.levels && idx->levels_fit != 0 &&
+                            !idx->levels_failed && levels_pay(idx, plan, Q, idx->L);
     coral::SearchArgs a = search_args(idx, use_levels ? idx->level_plan : plan, d_queries, d_ids, d_dists, Q, k, policy, have_delete);
     // The counters of a small batch go straight to pinned memory (32 bytes a query): the copy and its wait would take as
     // long as many such searches.
@@ -1056,18 +1109,12 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
         const coral_search_plan& lp = idx->level_plan;
         LevelScratch w;
         (void)level_block(idx, idx->level_rows, idx->d_level_block, &w);
-        const int64_t tiles = std::min<int64_t>(kLevelSampleTiles, std::max<int64_t>(1, idx->n / 128));
-        const int64_t sampled = std::min<int64_t>(tiles * 128, idx->n);
         a.levels = w.levels, a.ranges = w.ranges, a.level_pitch = coral::level_pitch(idx->n);
         for (int q0 = 0; q0 < Q; q0 += idx->level_rows) {
             const int m = std::min(idx->level_rows, Q - q0);
             const float* q = d_queries + (size_t)q0 * idx->dim;
             if (q0) HIP_TRY(coral::launch_fill_u32((uint32_t*)idx->d_scalars, 1, 0u, stream));
-            HIP_TRY(coral::launch_prepare_queries(q, m, idx->dim, 1, w.qn, w.qres, w.split, nullptr, nullptr, stream));
-            HIP_TRY(coral::launch_approx_tile(w.split, idx->d_vec, m, idx->n, idx->dim, idx->metric, 1, w.qn, idx->d_bnorm, nullptr, 0,
-                                              w.D, kLevelSampleTiles * 128, stream, tiles, (int)std::max<int64_t>(1, idx->n / 128 / tiles)));
-            HIP_TRY(coral::launch_level_ranges(w.D, kLevelSampleTiles * 128, m, (int)sampled, idx->dim, idx->metric, w.qn, idx->d_bnorm_max,
-                                               w.qres, idx->d_bnorm_max + 1, w.ranges, stream));
+            HIP_TRY(launch_level_scratch(idx, q, m, w, nullptr, stream));
             HIP_TRY(coral::launch_levels(w.split, idx->d_vec, m, idx->n, idx->dim, idx->metric, w.qn, idx->d_bnorm, w.ranges, w.levels,
                                          stream));
             a.q_begin = q0, a.q_end = q0 + m;
@@ -1118,6 +1165,9 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
         sum.screened_rows += r[0], sum.exact_rows += r[1], sum.beam_words += r[2], sum.visited_requests += r[3];
     }
     sum.spills = scal[1], sum.visited_dedupes = scal[2];
+    // Queries that the base's own rows do not stand for (probe_levels): a batch that found four rows in five open ran
+    // slower than it would have without the levels, and the next ones on this plan run without.
+    if (use_levels && sum.exact_rows * 5 > sum.dist_evals * 4) idx->levels_failed = true;
     // The table size the library picks assumes about 75 first visits per beam entry.  Data on which a query visits
     // more sends queries to the global bitmap (same results, slower): when more than a twentieth of a batch went
     // there, the next launches get a table twice the size.  (The bucket form turns away only the ids that find their
@@ -1137,7 +1187,10 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
         idx->bump_log2 = idx->bump_L == idx->L ? idx->bump_log2 + 1 : 1;
         idx->bump_L = idx->L;
         coral_tuning t = idx->tuning;
-        if (coral_search_prepare(idx, idx->Q, idx->L, &t) != CORAL_OK || idx->plan.slots_log2 == had) {
+        const bool failed = idx->levels_failed;
+        const int rc = coral_search_prepare(idx, idx->Q, idx->L, &t);
+        idx->levels_failed = failed;
+        if (rc != CORAL_OK || idx->plan.slots_log2 == had) {
             idx->bump_log2 -= 1;  // no room in LDS for more: stay
             if (!idx->prepared) return fail(CORAL_ERR_DEVICE, "could not restore the search scratch");
         }
@@ -1255,7 +1308,9 @@ int coral_search_plan_info(const coral_index* idx, coral_plan_info* out) {
         const coral_search_plan& lp = idx->level_plan;
         out->kernel = 0;
         out->threads = lp.threads, out->workgroups = out->query_slots = std::min(lp.workgroups, idx->Q), out->lds_bytes = (int32_t)lp.lds_bytes;
-        out->screening = 3, out->visited_form = 6, out->level_bytes = (int32_t)coral::level_pitch(idx->n), out->todo_cap = lp.tcap, out->cand_cap = lp.ccap;
+        out->screening = 3, out->visited_form = 6, out->level_bytes = (int32_t)coral::level_pitch(idx->n);
+        out->levels_unfit = idx->levels_fit == 0 || idx->levels_failed;
+        out->todo_cap = lp.tcap, out->cand_cap = lp.ccap;
     } else {
         out->kernel = 0;
         out->threads = p.threads, out->workgroups = p.workgroups, out->lds_bytes = (int32_t)p.lds_bytes;

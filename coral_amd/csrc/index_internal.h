@@ -103,6 +103,8 @@ struct coral_index {
     void* d_level_block = nullptr;
     size_t level_block_bytes = 0;
     int level_rows = 0;
+    int levels_fit = -1;  // 0: the base's rows lie so that levels settle little (probe_levels; -1: not looked at yet)
+    bool levels_failed = false;  // the last batch on this plan found most rows open
     bool bf_shared = false;  // best-first: four wavefronts share a query's steps
     int bf_table_log2 = 0, bf_table_rem_bits = 0;
     // ... or, for long beams, with an insert buffer in LDS and the long sorted run of every slot in global memory

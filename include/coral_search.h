@@ -252,7 +252,10 @@ typedef struct {
     int32_t todo_cap, cand_cap; /* LDS list capacities of the workgroup kernel */
     int32_t query_slots;     /* queries in flight */
     int32_t level_bytes;     /* levels: bytes of one query's (0 without) */
-    int32_t reserved[3];
+    int32_t levels_unfit;    /* 1 = planned, but the base's rows lie so that levels settle little of them (an offset common
+                                to all beside which they hardly differ, a few huge rows), or the last batch found most
+                                rows open: searches run as this plan does without levels */
+    int32_t reserved[2];
 } coral_plan_info;
 CORAL_API int coral_search_plan_info(const coral_index* idx, coral_plan_info* out);
 

@@ -41,7 +41,7 @@ LAYOUT_PROBE = r"""
 int main(void) {
     S(coral_stats); F(coral_stats, hops); F(coral_stats, screened_rows); F(coral_stats, visited_dedupes);
     S(coral_tuning); F(coral_tuning, visited_choices);
-    S(coral_plan_info); F(coral_plan_info, query_slots); F(coral_plan_info, level_bytes);
+    S(coral_plan_info); F(coral_plan_info, query_slots); F(coral_plan_info, level_bytes); F(coral_plan_info, levels_unfit);
     S(coral_build_params); F(coral_build_params, top_hit_num); F(coral_build_params, test_search_frequency);
     F(coral_build_params, monitor);
     S(coral_build_monitor); F(coral_build_monitor, L); F(coral_build_monitor, report); F(coral_build_monitor, user);

@@ -1087,3 +1087,48 @@ def test_row_counters_of_a_launch_with_levels():
     idx.prepare(Q, L, threads=512)
     assert idx.plan_info().level_bytes == 0
     idx.close()
+
+
+@pytest.mark.parametrize("law,metric,unfit", [
+    ("offset 6", "l2", 0), ("offset 40", "l2", 1),      # what all rows have in common: 0.9 and 40 steps' width lost
+    ("row 7777 x 10", "l2", 0), ("row 7777 x 100", "l2", 1), ("row 7777 x 10", "ip", 0), ("row 7777 x 100", "ip", 1),
+    ("row 5 x 3", "l2", 0), ("row 5 x 10", "l2", 1),    # a row of the sample that sets the steps
+    ("row 9 x inf", "l2", 1), ("row 9 x nan", "ip", 1),
+    ("queries", "l2", 0),                               # of a law that the base does not tell of: found out by the batch
+])
+def test_levels_are_left_out_where_they_settle_little(law, metric, unfit):
+    """Bases on which the products' loss is as wide as the levels, or one row decides the range of all: the plan says so
+    and the launch without levels answers; short of that the levels do, and leave rows unread.  Ids, distance bits and
+    counters are the same either way."""
+    n, dim, L, M, Q = 20000, 264, 256, 16, 1600
+    m = capi.IP if metric == "ip" else capi.L2
+    base, nbrs, starts = problem(n, dim, 32, 77, metric, M)
+    q = make_queries(Q, dim, 78, metric)
+    what = law.split()
+    if what[0] == "offset":
+        base, q = base + np.float32(what[1]), q + np.float32(what[1])
+    if what[0] == "row":
+        base[int(what[1])] *= np.float32(what[3])
+    if what[0] == "queries":  # far outside the space of the base's rows
+        base[:, 200:] = 0.0
+        q[:, 200:] = 300.0
+    idx = capi.Index(base, nbrs, starts, m)
+    print("levels left out", law, metric, flush=True)
+    idx.prepare(Q, L, threads=512, screening=-1)
+    want, want_d, _ = idx.search(q, 50, L)
+    want_c = idx.query_counters(Q)
+    for again in range(2):  # (a later plan of the same index knows)
+        idx.prepare(Q, L)
+        plan = idx.plan_info()
+        assert plan.screening == 3 and plan.levels_unfit == unfit
+        for rep in range(2):
+            ids, dists, st = idx.search(q, 50, L)
+            assert np.array_equal(ids, want) and dists.tobytes() == want_d.tobytes()
+            assert np.array_equal(idx.query_counters(Q), want_c)
+            if what[0] != "queries":
+                assert idx.plan_info().levels_unfit == unfit
+                assert unfit or st.exact_rows < 0.8 * st.dist_evals
+            else:
+                assert idx.plan_info().levels_unfit == 1  # after the first batch; until the next plan
+                assert rep == 1 or st.exact_rows > 0.8 * st.dist_evals
+    idx.close()
