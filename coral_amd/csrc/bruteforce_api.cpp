@@ -120,8 +120,9 @@ constexpr size_t kKnnKeepBytes = (size_t)384 << 20;
 
 // Scratch of one call, carved from one block.  A block of up to kKnnKeepBytes stays with the index until it is
 // destroyed: a dozen allocations and releases were 150 of the 274 us of a call with 100 queries.  Every call waits for
-// its stream before it returns, so a call on another stream finds the block idle; a call that finds it taken by another
-// thread, or needs more, has a block of its own.
+// its stream before it returns, so a call on another stream finds the block idle.  What needs more, and what finds the
+// block taken -- by the call it is part of, which sends some of its queries through another screening -- has a block of
+// its own.
 class KnnScratch {
 public:
     explicit KnnScratch(coral_index* idx) : idx_(idx) {}
@@ -202,11 +203,13 @@ struct FusedScreen {
         const int64_t expect = kc * (step > 1 ? (stride + step - 1) / step + step : stride) + kc;
         cap = 2048;
         while (cap < 3 * expect && cap < kListCap) cap <<= 1;
-        // queries per block: what 4096 lists take is kept between calls, and a pass over the base for so many is
-        // hundreds of tiles per compute unit; the sample's matrix is made and read for 2048 at a time
+        // Queries per block: a pass over the base for 4096 is hundreds of tiles per compute unit, and their lists of up to
+        // 8192 entries, beside the sample's matrix for 1024 queries at a time, stay within what is kept between calls (10 000
+        // queries of a million points, k = 100: 349 MB; with 2048 at a time 413, allocated and released by each call).
+        // Lists of 16 384, for k in the hundreds, do not.
         const int64_t rows = ((int64_t)Q + 127) & ~(int64_t)127;
         qc = std::min<int64_t>(4096, rows);
-        qs = std::min<int64_t>(2048, std::min(qc, std::max<int64_t>(256, (kBufferFloats / ns) & ~(int64_t)255)));
+        qs = std::min<int64_t>(1024, std::min(qc, std::max<int64_t>(256, (kBufferFloats / ns) & ~(int64_t)255)));
     }
     void reserve(const coral_index* idx, KnnScratch& mem) {
         if (!suits) return;

@@ -152,6 +152,20 @@ def every_plan_has_its_names(capi, fake):
     idx.close()
 
 
+@case
+def exact_neighbours_of_a_large_batch_keep_their_scratch(capi, fake):
+    # a million points, 10 000 queries, k = 100: lists of 8192 entries, and the matrix of the sample
+    idx = capi.Index(np.ones((1000000, 8), np.float32), None, None)
+    q = np.zeros((10000, 8), np.float32)
+    idx.bruteforce(q, 100)
+    kept = fake.fake_live_bytes()
+    assert kept > 1000000 * 8 * 4 + (256 << 20)
+    fake.fake_refuse(1 << 20, 1 << 40)  # the next call allocates nothing of note
+    idx.bruteforce(q, 100)
+    assert fake.fake_live_bytes() == kept
+    idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
