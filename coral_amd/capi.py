@@ -177,6 +177,7 @@ SIGNATURES = {
     "coral_start_ids_fps": (C.c_int, [C.c_void_p, C.c_int32, C.c_int32, C.c_void_p]),
     "coral_bruteforce_set_exact_only": (C.c_int, [C.c_void_p, C.c_int32]),
     "coral_bruteforce_last_redone": (C.c_int64, [C.c_void_p]),
+    "coral_bruteforce_last_handed_on": (C.c_int64, [C.c_void_p]),
     "coral_bruteforce_last_fused": (C.c_int32, [C.c_void_p]),
     "coral_membench": (C.c_int, [C.c_int32, C.c_size_t, C.c_int32, C.c_int32, C.POINTER(C.c_double),
                                  C.POINTER(C.c_double)]),
@@ -340,6 +341,9 @@ class Index:
 
     def bruteforce_last_fused(self):
         return int(lib().coral_bruteforce_last_fused(self._h))
+
+    def bruteforce_last_handed_on(self):
+        return int(lib().coral_bruteforce_last_handed_on(self._h))
 
     def bruteforce_last_redone(self):
         return int(lib().coral_bruteforce_last_redone(self._h))

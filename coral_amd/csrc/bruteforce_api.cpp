@@ -286,6 +286,8 @@ int coral_bruteforce_set_exact_only(coral_index* idx, int32_t on) {
 
 int64_t coral_bruteforce_last_redone(coral_index* idx) { return idx ? idx->knn_last_redone : -1; }
 
+int64_t coral_bruteforce_last_handed_on(coral_index* idx) { return idx ? idx->knn_last_handed_on : -1; }
+
 int32_t coral_bruteforce_last_fused(coral_index* idx) { return idx ? (int32_t)idx->knn_last_fused : -1; }
 
 static int check_knn(const coral_index* idx, int32_t Q, int32_t k, int32_t have_delete) {
@@ -361,6 +363,7 @@ struct Screening {
         std::vector<int32_t> rows;
         for (int32_t q = 0; q < Q; ++q)
             if (redo[(size_t)q]) rows.push_back(q);
+        if (products == 1) idx->knn_last_handed_on = (int64_t)rows.size();
         if (products == 3) idx->knn_last_redone = (int64_t)rows.size();
         if (rows.empty()) {
             waited = done != nullptr;
@@ -432,7 +435,7 @@ static int knn_call(coral_index* idx, const float* d_queries, const float* h_que
     HIP_TRY(hipEventCreate(&ev0));
     HIP_TRY(hipEventCreate(&ev1));
     HIP_TRY(hipEventRecord(ev0, stream));
-    idx->knn_last_redone = 0;
+    idx->knn_last_redone = 0, idx->knn_last_handed_on = -1;
     idx->knn_last_fused = false;
     if (!screen)
         rc = knn_passes(idx, d_queries, Q, k, have_delete, false, nullptr, idx->metric, d_ids, d_dists, stream);

@@ -89,6 +89,7 @@ struct coral_index {
     size_t knn_block_bytes = 0;
     int* h_knn_flags = nullptr;  // pinned, behind h_scalars: what a call of up to kKnnFlags - 1 queries reads back
     std::atomic<bool> knn_block_taken{false};
+    int64_t knn_last_handed_on = -1;  // queries of the last call that went from one product to three (-1: not on one)
     int64_t knn_last_redone = 0;  // queries of the last call that went through the exact passes after screening
 
     // best-first on one wavefront per query: per-slot visited epochs in global memory

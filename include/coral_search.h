@@ -298,6 +298,9 @@ CORAL_API int coral_bruteforce_knn(coral_index* idx, const float* h_queries, int
 CORAL_API int coral_bruteforce_set_exact_only(coral_index* idx, int32_t on);
 /* 1 if the candidates of the last coral_bruteforce_knn* call were selected inside the matrix-core kernel */
 CORAL_API int32_t coral_bruteforce_last_fused(coral_index* idx);
+/* queries of the last coral_bruteforce_knn* call that the screening on one product handed on to the one on three; -1 if
+ * its candidates were not chosen on one product (a small batch, or a sample that left too much open) */
+CORAL_API int64_t coral_bruteforce_last_handed_on(coral_index* idx);
 /* queries of the last coral_bruteforce_knn* call that went through the plain passes after the screening */
 CORAL_API int64_t coral_bruteforce_last_redone(coral_index* idx);
 

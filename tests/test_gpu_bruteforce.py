@@ -403,6 +403,7 @@ def test_bruteforce_ground_truth_at_full_size(orc):
     ("lattice", "l2", 100, 10, False),   # exact in halves, thousands of equal distances
     ("scales", "l2", 100, 20, False),    # rows of norms 1e-3 .. 1e3: a few decide the bound for all
     ("tiny", "ip", 100, 20, False),      # components below what scaled halves hold
+    ("crowd", "l2", 100, 10, False),     # a few queries among rows that one product, or three, cannot tell apart
 ])
 def test_screening_on_one_product_answers_what_the_plain_passes_answer(law, metric, dim, k, dele):
     """Batches large enough to be screened on one product of halves per pair (1e11 pair dimensions; their last stage of
@@ -429,12 +430,23 @@ def test_screening_on_one_product_answers_what_the_plain_passes_answer(law, metr
         base *= (10.0 ** rng.randint(-3, 4, (n, 1))).astype(np.float32)
     if law == "tiny":
         base[:, 1:] *= np.float32(1e-7)
+    if law == "crowd":
+        for at, width in ((1000, 5e-3), (2000, 1e-4)):
+            base[at:at + 500] = base[at] + np.float32(width) * base[at:at + 500]
+            q[at:at + 40] = base[at] + np.float32(0.5) * q[at:at + 40]
     idx = capi.Index(base, None, None, metric=capi.IP if metric == "ip" else capi.L2)
     if dele:
         idx.mark_deleted(rng.choice(n, n // 5, replace=False).astype(np.int32))
     print("one product", law, metric, dim, k, dele, flush=True)
     ids, dists, _ = idx.bruteforce(q, k, have_delete=dele)
-    redone = idx.bruteforce_last_redone()
+    redone, handed_on = idx.bruteforce_last_redone(), idx.bruteforce_last_handed_on()
+    # which way it went: on one product, on to three by the sample's word, or on to three query by query
+    if law in ("offset", "scales", "tiny"):
+        assert handed_on == -1
+    elif law == "crowd":
+        assert 40 <= redone < handed_on <= 80
+    else:
+        assert handed_on >= 0
     idx.bruteforce_exact_only(2)
     ids3, dists3, _ = idx.bruteforce(q, k, have_delete=dele)
     assert idx.bruteforce_last_redone() == redone  # what one product leaves open three decide as they did
@@ -448,8 +460,8 @@ def test_screening_on_one_product_answers_what_the_plain_passes_answer(law, metr
 @pytest.mark.parametrize("Q", [1, 3, 255, 257, 1024, 1025, 4500])
 @pytest.mark.parametrize("metric,dim,k", [("l2", 4, 1), ("ip", 12, 10), ("l2", 100, 10), ("ip", 260, 33), ("l2", 516, 5)])
 def test_prepared_queries_at_the_edges_of_tiles_and_flags(Q, metric, dim, k):
-    """Batches about the query tile of 256, the 1024 queries whose flags go to pinned memory and whose sample is looked at at a time, and the 4096 of a block
-    of the screening; dimensions short of a stage of 16 and beyond the 64 lanes that read a row.  Twice on one index (the
+    """Batches about the query tile of 256, the 1024 queries whose flags go to pinned memory and sample
+    is looked at at a time, and the 4096 of a block of the screening; dimensions short of a stage of 16 and beyond the 64 lanes that read a row.  Twice on one index (the
     counters start at zero again), and with every second base row equal, where lists overflow or leave ties open: ids and
     distance bits are those of the search that measures every pair."""
     rng = np.random.RandomState(Q + dim)
