@@ -55,18 +55,24 @@ __global__ __launch_bounds__(256) void find_repeated_ids_kernel(const int32_t* _
 using bf_kernel_fn = void (*)(const SearchArgs, const BestFirstArgs);
 
 // The form for a row width: G lanes per row, CPL chunks per lane.  Rows of more than 512 floats have no copy in
-// eight-bit codes; rows of up to 128 have no other, rows of up to 64 none.
+// eight-bit codes, rows of up to 128 no other, rows of up to 64 none: what no launch asks for is not built.
 template <int RIF, int KPL, int SCREEN, int WGS>
 bf_kernel_fn pick_bf_width(int chunks) {
-    constexpr int WIDE = SCREEN == 2 ? 0 : SCREEN;
     // (what fits the registers beside the beam without spilling two dozen of them)
     constexpr int RIF4 = WGS > 2 && KPL >= 8 ? 8 : RIF, RIF8 = WGS > 2 ? 8 : RIF;
-    if (chunks <= 16) return best_first_wave_kernel<16, 1, (RIF > 16 ? 16 : RIF), KPL, 0, WGS, 1>;
-    if (chunks <= 32) return best_first_wave_kernel<32, 1, (RIF > 16 ? 16 : RIF), KPL, (SCREEN == 2 ? 2 : 0), WGS, 1>;
+    if constexpr (SCREEN == 0) {
+        if (chunks <= 16) return best_first_wave_kernel<16, 1, (RIF > 16 ? 16 : RIF), KPL, 0, WGS, 1>;
+    }
+    if constexpr (SCREEN != 1) {
+        if (chunks <= 32) return chunks > 16 ? best_first_wave_kernel<32, 1, (RIF > 16 ? 16 : RIF), KPL, SCREEN, WGS, 1> : nullptr;
+    }
+    if (chunks <= 32) return nullptr;
     if (chunks <= 64) return best_first_wave_kernel<64, 1, RIF, KPL, SCREEN, WGS, 1>;
     if (chunks <= 128) return best_first_wave_kernel<64, 2, RIF, KPL, SCREEN, WGS, 1>;
-    if (chunks <= 256) return best_first_wave_kernel<64, 4, RIF4, KPL, WIDE, WGS, 1>;
-    if (chunks <= 512) return best_first_wave_kernel<64, 8, RIF8, KPL, WIDE, WGS, 1>;
+    if constexpr (SCREEN != 2) {
+        if (chunks <= 256) return best_first_wave_kernel<64, 4, RIF4, KPL, SCREEN, WGS, 1>;
+        if (chunks <= 512) return best_first_wave_kernel<64, 8, RIF8, KPL, SCREEN, WGS, 1>;
+    }
     return nullptr;
 }
 
@@ -90,13 +96,13 @@ bf_kernel_fn pick_bf_length(int dim, int rif, int L) {
         if (L <= 1280) return pick_bf_width<16, 20, 0, 3>(chunks);
         if (L <= kMaxWaveBeam) return pick_bf_width<16, 32, 0, 2>(chunks);
     } else {
-        if (SCREEN == 2 && rif >= 32) {
-            if (L <= 128) return pick_bf_width<32, 2, SCREEN, 2>(chunks);
-            if (L <= 256) return pick_bf_width<32, 4, SCREEN, 2>(chunks);
-            if (L <= 512) return pick_bf_width<32, 8, SCREEN, 2>(chunks);
-            if (L <= 1024) return pick_bf_width<32, 16, SCREEN, 2>(chunks);
-        }
-        if (SCREEN == 2) {
+        if constexpr (SCREEN == 2) {
+            if (rif >= 32) {
+                if (L <= 128) return pick_bf_width<32, 2, SCREEN, 2>(chunks);
+                if (L <= 256) return pick_bf_width<32, 4, SCREEN, 2>(chunks);
+                if (L <= 512) return pick_bf_width<32, 8, SCREEN, 2>(chunks);
+                if (L <= 1024) return pick_bf_width<32, 16, SCREEN, 2>(chunks);
+            }
             if (L <= 128) return pick_bf_width<8, 2, SCREEN, 4>(chunks);
             if (L <= 256) return pick_bf_width<8, 4, SCREEN, 4>(chunks);
         }

@@ -10,11 +10,12 @@ using bf_kernel_fn = void (*)(const SearchArgs, const BestFirstArgs);
 
 template <int KPL, int SCREEN>
 bf_kernel_fn pick_shared_width(int chunks) {
-    constexpr int WIDE = 0;  // rows of more than 512 floats have no copy in eight-bit codes
     if (chunks <= 64) return best_first_wave_kernel<64, 1, 8, KPL, SCREEN, 2, 4>;
     if (chunks <= 128) return best_first_wave_kernel<64, 2, 16, KPL, SCREEN, 2, 4>;
-    if (chunks <= 256) return best_first_wave_kernel<64, 4, 32, KPL, WIDE, 2, 4>;
-    if (chunks <= 512) return best_first_wave_kernel<64, 8, 32, KPL, WIDE, 2, 4>;
+    if constexpr (SCREEN == 0) {  // (rows of more than 512 floats have no copy in eight-bit codes)
+        if (chunks <= 256) return best_first_wave_kernel<64, 4, 32, KPL, SCREEN, 2, 4>;
+        if (chunks <= 512) return best_first_wave_kernel<64, 8, 32, KPL, SCREEN, 2, 4>;
+    }
     return nullptr;
 }
 

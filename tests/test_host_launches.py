@@ -166,6 +166,30 @@ def exact_neighbours_of_a_large_batch_keep_their_scratch(capi, fake):
     idx.close()
 
 
+@case
+def every_best_first_launch_that_is_accepted_has_its_kernel(capi, fake):
+    for dim in (4, 64, 68, 128, 132, 256, 260, 512, 516, 1024, 1028, 2048):
+        for metric in (0, 1):
+            idx = make(capi, 3000, dim, metric)
+            for screening in (-1, 0, 1, 2):
+                taken = (screening < 1 or (screening == 1 and dim > 128 and metric == 0) or
+                         (screening == 2 and 64 < dim <= 512))
+                for L in (4, 128, 129, 256, 257, 512, 513, 1024, 1025, 1280, 1281, 2048):
+                    for Q in (1, 5000):
+                        try:
+                            idx.prepare(Q, L, policy=1, screening=screening, best_first_long=-1)
+                        except capi.CoralError as e:
+                            assert e.code == capi.ERR_ARG and not taken, (dim, metric, screening, L, Q)
+                            continue
+                        assert taken, (dim, metric, screening, L, Q)
+                        fake.fake_forget()
+                        call(idx, Q, min(L, 10), 1)
+                        assert idx.plan_info().kernel == 1 and fake.fake_launches_beyond_limit() == 0
+                        if screening > 0:
+                            assert idx.plan_info().screening == screening
+            idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
