@@ -25,7 +25,7 @@ bf_kernel_fn pick_shared(int dim, int L) {
     if (L <= 256) return pick_shared_width<4, SCREEN>(dim / 4);
     if (L <= 512) return pick_shared_width<8, SCREEN>(dim / 4);
     if (L <= 1024) return pick_shared_width<16, SCREEN>(dim / 4);
-    if (L <= kMaxWaveBeam) return pick_shared_width<32, SCREEN>(dim / 4);
+    if (L <= 1280) return pick_shared_width<20, SCREEN>(dim / 4);
     return nullptr;
 }
 

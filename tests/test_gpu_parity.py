@@ -909,7 +909,7 @@ def test_randomised_shapes(orc):
     (9000, 200, "l2", 300, 16, 100, dict(best_first_table_log2=-1)), (9000, 200, "l2", 300, 16, 100, dict(best_first_packed=True)),
     # four wavefronts per query: beams of every number of keys per lane, one query and several per workgroup
     (33000, 132, "ip", 48, 40, 3, {}), (33000, 132, "ip", 200, 5, 300, {}), (33000, 516, "ip", 300, 5, 40, {}),
-    (33000, 260, "ip", 600, 70, 20, {}), (33000, 132, "ip", 1280, 5, 12, {}), (33000, 1028, "ip", 100, 5, 40, {}),
+    (33000, 260, "ip", 600, 70, 20, {}), (33000, 132, "ip", 1025, 5, 12, {}), (33000, 132, "ip", 1280, 5, 12, {}), (33000, 1028, "ip", 100, 5, 40, {}),
     (33000, 260, "ip", 412, 3, 40, {}), (33000, 260, "ip", 413, 3, 40, {}),  # 80 nodes per entry: screened, and not
 ])
 def test_best_first_with_the_beam_in_registers_at_the_edges_of_its_sizes(orc, n, dim, metric, L, M, Q, kw):
