@@ -785,11 +785,20 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         // beam length (sixteen wavefronts per CU or one; 200 000 x 200, L = 64 / 512, one query: 226 / 1600 without, 147 /
         // 1321 us with; 5000 queries: 774 / 6469, 551 / 4549) -- except on graphs so small for the beam that most
         // neighbours have been visited and a step has few rows to read (one query, 40 000 x 300: L = 400 941 / 963, L =
-        // 512 1147 / 1230; 30 000 x 512, L = 1000 2241 / 2697; 100 000 x 512 under the inner product, L = 1000, still
-        // 4407 / 4349, and 5000 queries 35 100 / 19 600).
+        // 512 1147 / 1230; 30 000 x 512, L = 1000 2241 / 2697).
+        // There the wait is worth its while only where the rows of all queries in flight are what memory cannot deliver.
+        // Time with over time without, n / L of 25 .. 79, on exact 32-NN graphs and graphs built from queries: inner product,
+        // 2000 / 5000 queries of 512 floats 0.49 .. 0.60 and 0.60 .. 0.88, of 264 0.55 .. 0.92 and 0.86 .. 1.07; 1000 of 512 0.54 .. 0.85
+        // and 0.90 .. 1.05, of 200 0.84 .. 0.96 and 1.00 .. 1.09.  L2, 5000 of 512 floats 0.62 .. 0.88 and 0.94 .. 1.16, of 384 0.65 .. 1.08
+        // and 1.05 .. 1.15, of 264 0.78 .. 1.07 and 1.05 .. 1.14; 1000 of 512 0.87 .. 1.10 and 1.05 .. 1.17.  The lines lie where
+        // going without was slower than the kernel with the beam in LDS had been, which screened such batches: up to 1.7
+        // times under the inner product, 1.3 under L2 (40 000 x 512 near a 16-dimensional subspace).
+        const int64_t floats_in_flight = (int64_t)std::min<int64_t>(Q, 16 * idx->num_cu) * idx->dim;
+        const bool heavy = idx->metric == CORAL_IP ? floats_in_flight >= (int64_t)1920 * idx->num_cu
+                                                   : floats_in_flight >= (int64_t)3600 * idx->num_cu && idx->dim > 320 && idx->n >= (int64_t)32 * L;
         const int form = t.screening == 1 || idx->dim > coral::kMaxByteRowDim ? 1 : 2;
         const bool can = (idx->dim / 4 > 32 || narrow_codes) && (form == 2 || idx->metric == CORAL_L2);
-        if (can && (t.screening > 0 || (t.screening == 0 && form == 2 && idx->n >= (int64_t)80 * L))) bf_form = form;
+        if (can && (t.screening > 0 || (t.screening == 0 && form == 2 && (heavy || idx->n >= (int64_t)80 * L)))) bf_form = form;
         const int coded = bf_form == 2 ? coral::coded_query_bytes(idx->dim) : 0;
         // The visited set: a bitmap of all ids in LDS where every wavefront that the batch gives a CU finds room for one
         // (one atomic per id, nothing to hash or probe; 200 000 x 200, L = 128, one query: 244 us, the table 314, the

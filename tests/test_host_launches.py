@@ -190,6 +190,22 @@ def every_best_first_launch_that_is_accepted_has_its_kernel(capi, fake):
             idx.close()
 
 
+@case
+def best_first_screens_heavy_batches_on_small_graphs_too(capi, fake):
+    # fewer than 80 nodes per beam entry: only what memory could not deliver in fp32
+    for n, dim, metric, L, cases in ((30000, 512, 1, 759, {1: 0, 900: 0, 960: 2, 5000: 2}),
+                                     (30000, 200, 1, 500, {2400: 0, 2500: 2}),
+                                     (30000, 512, 0, 500, {1: 0, 1700: 0, 1900: 2, 5000: 2}),
+                                     (30000, 512, 0, 1000, {5000: 0}),  # ... and enough of a graph to find new rows in
+                                     (30000, 264, 0, 500, {5000: 0}),
+                                     (30000, 264, 0, 300, {1: 2, 5000: 2})):
+        idx = make(capi, n, dim, metric)
+        for Q, screening in cases.items():
+            idx.prepare(Q, L, policy=1)
+            assert idx.plan_info().screening == screening, (n, dim, metric, L, Q)
+        idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
