@@ -76,6 +76,7 @@ struct BestFirstArgs {
     int32_t slots;      // wavefronts = queries in flight
     int32_t rows_in_flight;  // 8, 16 or 32: float4 registers of vector data a lane requests before it adds them up
     int32_t rows_unique;     // no graph row lists an id twice (checked by launch_find_repeated_ids)
+    int32_t waves_per_wg;    // 1 .. 4 wavefronts, each with a query of its own
     int32_t packed;          // visited is [slots][stride] of 32-bit words, 8 bits of epoch over 24 node flags each
     int32_t bitmap_words;    // the visited set is a bitmap of all ids in LDS (32-bit words per wavefront, a multiple of 4);
                              // 0: it is not, and what follows and the state above hold it

@@ -139,13 +139,13 @@ hipError_t best_first_prepare(int dim, int L, int rows_in_flight, int screen, si
 hipError_t launch_best_first(const SearchArgs& a, const BestFirstArgs& b, hipStream_t stream) {
     const int screen = b.vec8 != nullptr ? 2 : b.vec16 != nullptr ? 1 : 0;
     if (screen == 2 && (a.dim > kMaxByteRowDim || b.coded_bytes != coded_query_bytes(a.dim))) return hipErrorInvalidValue;
-    if (a.R > kBatch || a.M <= 0) return hipErrorInvalidValue;
+    if (a.R > kBatch || a.M <= 0 || b.waves_per_wg < 1 || b.waves_per_wg > kWavesPerWg) return hipErrorInvalidValue;
     if (b.bitmap_words != 0 && ((b.bitmap_words & 3) != 0 || (int64_t)b.bitmap_words * 32 < a.n)) return hipErrorInvalidValue;
-    const size_t lds = best_first_wave_lds_bytes(b.bloom_log2, b.table_log2, b.coded_bytes, b.bitmap_words) * kWavesPerWg;
+    const size_t lds = best_first_wave_lds_bytes(b.bloom_log2, b.table_log2, b.coded_bytes, b.bitmap_words) * b.waves_per_wg;
     bf_kernel_fn fn = pick_bf_kernel(a.dim, b.rows_in_flight, screen, a.L);
     if (!fn) return hipErrorInvalidValue;
-    const int wgs = (b.slots + kWavesPerWg - 1) / kWavesPerWg;
-    hipLaunchKernelGGL(fn, dim3(wgs), dim3(kWavesPerWg * 64), lds, stream, a, b);
+    const int wgs = (b.slots + b.waves_per_wg - 1) / b.waves_per_wg;
+    hipLaunchKernelGGL(fn, dim3(wgs), dim3(b.waves_per_wg * 64), lds, stream, a, b);
     return hipGetLastError();
 }
 

@@ -945,6 +945,12 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         const bool eight = wave_lds * 12 > (size_t)kMaxLdsBytes || Q <= 8 * idx->num_cu;
         const int rif = eight && L <= 1024 && idx->bf_screen != 1 ? 32 : idx->bf_screen != 0 ? 8 : 16;
         idx->bf_rows_in_flight = rif;
+        // Wavefronts come to the CUs by workgroups.  On rows of more than 512 floats four of them keep a CU's path to its
+        // caches busy, and a CU that gets a second workgroup where others have one takes nearly twice as long: there each
+        // wavefront is a workgroup of its own (1000 / 1100 / 1300 queries, four to a workgroup and one: 200 000 x 1024, L = 256: 3.19 /
+        // 4.36 / 4.54 and 3.15 / 3.76 / 4.53 ms; 70 000 x 2048: 5.67 / 7.61 / 7.84 and 5.53 / 6.60 / 7.77; 40 000 x 2048, inner
+        // product, L = 1000: 27.5 / 37.8 / 38.4 and 26.4 / 31.6 / 37.2; narrower rows: the same within 3 %).
+        idx->bf_waves_per_wg = idx->dim > 512 && t.workgroups == 0 ? 1 : 4;
         HIP_TRY(coral::best_first_prepare(idx->dim, L, rif, idx->bf_screen, wave_lds, &bf_wg_per_cu));
         if (bitmap_words != 0) {
             // (nothing of the visited state lies in HBM: a slot costs no memory)
@@ -1094,6 +1100,7 @@ static int search_launch(coral_index* idx, const float* d_queries, const float* 
     } else if (wave_kernel) {
         coral::BestFirstArgs b;
         b.rows_unique = idx->rows_unique == 1;
+        b.waves_per_wg = idx->bf_waves_per_wg;
         b.packed = idx->bf_packed;
         b.bitmap_words = idx->bf_bitmap_words;
         b.bloom_log2 = idx->bf_bloom_log2;
@@ -1294,9 +1301,10 @@ int coral_search_plan_info(const coral_index* idx, coral_plan_info* out) {
     const bool wave = idx->prepared_policy == CORAL_POLICY_BEST_FIRST && idx->bf_ready;
     if (wave) {
         out->kernel = idx->bf_long ? 2 : 1;
-        out->threads = 256;
+        const int waves = idx->bf_long ? 4 : idx->bf_waves_per_wg;
+        out->threads = 64 * waves;
         out->query_slots = std::min(idx->bf_slots, idx->Q);
-        out->workgroups = (out->query_slots + 3) / 4;
+        out->workgroups = (out->query_slots + waves - 1) / waves;
         const size_t per_wave =
             idx->bf_long
                 ? coral::best_first_long_lds_bytes(idx->bf_bcap, idx->bf_scap,
@@ -1304,7 +1312,7 @@ int coral_search_plan_info(const coral_index* idx, coral_plan_info* out) {
                 : coral::best_first_wave_lds_bytes(idx->bf_bloom_log2, idx->bf_table_log2,
                                                    idx->bf_screen == 2 ? coral::coded_query_bytes(idx->dim) : 0,
                                                    idx->bf_bitmap_words);
-        out->lds_bytes = (int32_t)(per_wave * 4);
+        out->lds_bytes = (int32_t)(per_wave * waves);
         out->screening = idx->bf_screen;
         out->visited_form = !idx->bf_long && idx->bf_bitmap_words ? 1 : !idx->bf_long && idx->bf_table_log2 ? 4 : idx->bf_packed ? 3 : 2;
         out->visited_slots_log2 = idx->bf_long ? 0 : idx->bf_table_log2;

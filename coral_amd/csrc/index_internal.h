@@ -97,7 +97,7 @@ struct coral_index {
     uint8_t* d_bf_visited = nullptr;
     uint32_t* d_bf_epochs = nullptr;
     size_t bf_stride = 0, bf_alloc_bytes = 0;
-    int bf_slots = 0, bf_alloc_slots = 0, bf_rows_in_flight = 8, bf_packed = 0, bf_bitmap_words = 0, bf_shared_lds = 0, bf_bloom_log2 = 0;
+    int bf_slots = 0, bf_alloc_slots = 0, bf_rows_in_flight = 8, bf_waves_per_wg = 4, bf_packed = 0, bf_bitmap_words = 0, bf_shared_lds = 0, bf_bloom_log2 = 0;
     // rounds policy: the launch for batches whose distances are bounded by levels from the matrix cores (levels = 0: none
     // planned), and its scratch: the levels of level_rows queries and what makes them
     coral_search_plan level_plan{};

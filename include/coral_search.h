@@ -235,7 +235,7 @@ typedef struct {
                                 best_first_wave_kernel, four to a query), 1 best_first_wave_kernel, a wavefront per
                                 query, 2 best_first_long_kernel */
     int32_t threads;         /* per workgroup */
-    int32_t workgroups;      /* persistent workgroups (the wavefront kernels: query slots / 4) */
+    int32_t workgroups;      /* persistent workgroups (the wavefront kernels: query slots by threads / 64) */
     int32_t lds_bytes;       /* per workgroup */
     int32_t screening;       /* 0 none, 1 half precision, 2 eight-bit codes, 3 levels: four bits per query and node that bound
                                 the distance, made for the whole batch on the matrix cores (rounds policy, 512 queries and

@@ -35,6 +35,7 @@ void fake_refuse(size_t at_least, size_t below) { refuse_at_least = at_least, re
 void fake_forget() { launches.clear(); }
 size_t fake_launches() { return launches.size(); }
 size_t fake_launch_lds(size_t i) { return launches[i].lds; }
+unsigned fake_launch_blocks(size_t i) { return launches[i].blocks; }
 unsigned fake_launch_threads(size_t i) { return launches[i].threads; }
 const void* fake_launch_fn(size_t i) { return launches[i].fn; }
 // launches that asked for more LDS than their kernel's limit was raised to (64 KB before it is)

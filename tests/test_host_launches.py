@@ -206,6 +206,22 @@ def best_first_screens_heavy_batches_on_small_graphs_too(capi, fake):
         idx.close()
 
 
+@case
+def wavefronts_on_wide_rows_are_workgroups_of_their_own(capi, fake):
+    for dim, waves, kw in ((512, 4, {}), (516, 1, {}), (2048, 1, {}), (2048, 4, dict(workgroups=300))):
+        idx = make(capi, 9000, dim)
+        idx.prepare(1100, 64, policy=1, **kw)
+        plan = idx.plan_info()
+        assert plan.kernel == 1 and plan.query_slots == 1100
+        assert plan.threads == 64 * waves and plan.workgroups == 1100 // waves
+        fake.fake_forget()
+        call(idx, 1100, 10, 1)
+        last = fake.fake_launches() - 1
+        assert fake.fake_launch_threads(last) == 64 * waves and fake.fake_launch_blocks(last) == 1100 // waves
+        assert fake.fake_launch_lds(last) == plan.lds_bytes
+        idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
@@ -229,7 +245,7 @@ if __name__ == "__main__":
         getattr(runtime, name).restype = C.c_size_t
     runtime.fake_live_of_size.argtypes = [C.c_size_t]
     runtime.fake_refuse.argtypes = [C.c_size_t, C.c_size_t]
-    runtime.fake_launch_lds.argtypes = runtime.fake_launch_threads.argtypes = [C.c_size_t]
+    runtime.fake_launch_lds.argtypes = runtime.fake_launch_threads.argtypes = runtime.fake_launch_blocks.argtypes = [C.c_size_t]
     runtime.fake_launch_fn.restype, runtime.fake_launch_fn.argtypes = C.c_void_p, [C.c_size_t]
     from coral_amd import capi as binding
     CASES[sys.argv[2]](binding, runtime)
