@@ -943,7 +943,13 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
         // wavefronts may as well use 256 registers per lane: all 32 rows of a step.  Where a screening leaves few rows
         // to read in fp32, 8.
         const bool eight = wave_lds * 12 > (size_t)kMaxLdsBytes || Q <= 8 * idx->num_cu;
-        const int rif = eight && L <= 1024 && idx->bf_screen != 1 ? 32 : idx->bf_screen != 0 ? 8 : 16;
+        // On rows of more than 512 floats that ends where the batch has more under way than the caches keep, a row's floats
+        // times the queries in flight.  Time of the smaller form over that of the larger: 200 000 x 1024, 1100 .. 2000 queries 0.86
+        // .. 1.00; 70 000 x 768, 2000 queries 0.97 .. 1.02, 1000 and 1100 0.99 .. 1.33; 70 000 x 2048, 1000 .. 2000 queries 0.81 .. 1.02; 70 000 x
+        // 1028, 2000 queries 0.92 .. 0.98, 1000 .. 1500 1.10 .. 1.55.
+        const int64_t under_way = (int64_t)std::min<int64_t>(Q, 16 * idx->num_cu) * idx->dim;
+        const bool too_much = idx->dim > 512 && under_way >= (int64_t)(idx->dim > 1024 ? 6800 : 4300) * idx->num_cu;
+        const int rif = eight && !too_much && L <= 1024 && idx->bf_screen != 1 ? 32 : idx->bf_screen != 0 ? 8 : 16;
         idx->bf_rows_in_flight = rif;
         // Wavefronts come to the CUs by workgroups.  On rows of more than 512 floats four of them keep a CU's path to its
         // caches busy, and a CU that gets a second workgroup where others have one takes nearly twice as long: there each

@@ -222,6 +222,21 @@ def wavefronts_on_wide_rows_are_workgroups_of_their_own(capi, fake):
         idx.close()
 
 
+@case
+def batches_of_wide_rows_that_fill_the_caches_take_fewer_at_a_time(capi, fake):
+    def kernel(idx, Q):
+        idx.prepare(Q, 64, policy=1)
+        fake.fake_forget()
+        call(idx, Q, 10, 1)
+        return fake.fake_launch_fn(fake.fake_launches() - 1)
+
+    for dim, few, many, same in ((2048, 800, 900, False), (1028, 1600, 1700, False), (1024, 1000, 1100, False),
+                                 (516, 1800, 2040, True), (512, 1000, 2040, True)):
+        idx = make(capi, 9000, dim)
+        assert (kernel(idx, few) == kernel(idx, many)) == same, dim
+        idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
