@@ -611,9 +611,12 @@ static int probe_levels(coral_index* idx) {
 // time without: spared / cost 1.5 1.13 (100 000 x 128, L = 32); 2.5 0.97 (L = 100); 5.1 0.69 (L = 256); inner product, 1.7 0.84 (200 000 x 512, L = 100);
 // 3.1 0.58 (60 000 x 512, L = 64); 11 0.46 (L = 256); 80 000 x 1028, L = 256, 0.22.  From 3 on, 2 under the inner product.
 // A batch costs another 60 us for its norms, its sample and the launches: 512 queries and more, which spare three times
-// that.  With one workgroup per CU (more than about 140 000 nodes) the waits of a round stand where the rows of up to 256
-// floats were (200 000 x 200, L = 256 / 800: 1.15 / 1.05; under the inner product 512 floats 0.57 / 0.55, 120 000 x 256, L =
-// 800, 0.61).
+// that.  With one workgroup per CU (more than about 140 000 nodes) the waits of a round stand where narrow rows were, so
+// rows of up to 256 floats go without (252 under the inner product).  150 000 .. 260 000 nodes, 1000 and 5000 queries, L = 256 / 500 /
+// 800: L2, rows of 132 .. 240 floats 1.09 .. 1.41 / 1.06 .. 1.14 / 1.00 .. 1.07 of the time, of 252 and 256 1.01 .. 1.18 / 0.88 .. 0.95 / 0.82 .. 0.89,
+// of 260 .. 320 1.01 .. 1.17 / 0.95 .. 0.99 / 0.90 .. 0.94, of 400 0.76 .. 0.92; inner product, 132 .. 232 floats 0.78 .. 0.91 / 0.80 .. 0.88 / 0.73
+// .. 0.80, 256 .. 400 0.53 .. 0.78.  (Below the lines the inner product, and long beams under L2 on more than 240 floats, would
+// gain as well.)
 static bool levels_pay(const coral_index* idx, const coral_search_plan& base, int32_t Q, int32_t L) {
     const bool ip = idx->metric == CORAL_IP;
     const double row = base.screen == 2   ? (double)coral::byte_row_stride(idx->dim)
@@ -812,10 +815,13 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
             coral::best_first_wave_lds_bytes(0, 0, coded, bits) * 4 * wgs_wanted <= (size_t)kMaxLdsBytes) {
             bitmap_words = bits;
         } else {
-            // (a full chip of narrow rows wants its sixteen wavefronts per CU more than a table that leaves eight:
-            // 200 000 x 200, 5000 queries, L = 256 / 330 / 400: 2456 / 3361 / 4164 us with it, 2400 / 3030 / 3632 without;
-            // rows of 256 floats: 3601 / 4880 / 5824, 4024 / 5160 / 6076; 2048 queries gain by it everywhere)
-            const int fewest_waves = idx->dim <= 208 && L > 256 && Q > 8 * idx->num_cu ? 12 : 8;
+            // A full chip of narrow rows wants its sixteen wavefronts per CU more than a table that leaves eight.  Time with
+            // the table over time without, 200 000 nodes, L = 260 .. 400: rows of 132 .. 240 floats (whose codes are 256 bytes, 384
+            // from there on) 1.08 .. 1.34 with 2100 .. 8192 queries, 0.99 .. 1.16 with 5000 of them, a little over one pass of sixteen
+            // wavefronts; of 248 and 256 floats 0.93 .. 1.03 with 5000, 0.97 .. 1.16 with 3500 .. 8192; of 320 0.89 .. 1.12; of 512 0.85 ..
+            // 1.02.  (On those, 2100 and 3000 queries, one pass without the table and two with it, lose up to 1.32.)  2048
+            // queries gain by it everywhere.
+            const int fewest_waves = idx->dim <= 240 && L > 256 && Q > 8 * idx->num_cu ? 12 : 8;
             if (int rc = choose_bf_table(L, id_bits, narrow_codes ? -1 : t.best_first_table_log2, coded, fewest_waves, &table_log2))
                 return rc;
         }

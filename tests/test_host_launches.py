@@ -237,6 +237,17 @@ def batches_of_wide_rows_that_fill_the_caches_take_fewer_at_a_time(capi, fake):
         idx.close()
 
 
+@case
+def full_batches_of_narrow_rows_go_without_the_table(capi, fake):
+    for dim, table in ((200, 0), (240, 0), (244, 13)):
+        idx = make(capi, 200000, dim)
+        idx.prepare(5000, 330, policy=1)
+        assert idx.plan_info().visited_slots_log2 == table, dim
+        idx.prepare(2048, 330, policy=1)
+        assert idx.plan_info().visited_slots_log2 == 13, dim
+        idx.close()
+
+
 @pytest.fixture(scope="module")
 def fake_runtime(tmp_path_factory):
     out = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
