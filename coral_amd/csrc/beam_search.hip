@@ -220,8 +220,9 @@ struct WgState {
 };
 
 // FORM: 0 takes any launch.  The others leave out what their launches never do, whose arguments the compiler otherwise keeps
-// in scalar registers that it does not have (64 x 1: 174 of them spilled to lanes of vector registers, 103 in form 2; 1M x 200,
-// L = 512, 10 000 queries 16.5 -> 15.8 ms; 250 000 x 200, L = 4096 4.67 -> 4.39; 64 queries on 200 000 x 200, L = 128 78 -> 72 us):
+// in scalar registers that it does not have (64 x 1: 174 of them spilled to lanes of vector registers, 103 in form 2; with beams
+// in global memory 197 and 134; 1M x 200, L = 512, 10 000 queries 16.5 -> 15.8 ms; 250 000 x 200, L = 4096 4.67 -> 4.39; 64 queries
+// on 200 000 x 200, L = 128 78 -> 72 us):
 // rounds policy on a bitmap of all ids, with (2) and without (3) the screening on codes; on the table of cells in its bucket
 // form, with (4) and without (5).
 // 1: the launch comes with four bits per (query, node) that bound the distance (bruteforce.h), made on the matrix cores

@@ -328,7 +328,7 @@ static int plan_search(const coral_index* idx, int32_t Q, int32_t L, const coral
     const size_t lds_max = (size_t)kMaxLdsBytes;
     // ---- screening on a smaller copy of the vectors (rounds policy, L2, rows of 132 .. 2048 floats): eight-bit codes
     // (tuning 2; the library's choice up to 512 floats) or half precision (tuning 1); see beam_search.hip
-    // (best-first: the wavefront-per-query kernel with the beam in LDS screens too, see coral_search_prepare)
+    // (best-first: the wavefront kernels screen by a rule of their own, see coral_search_prepare)
     // (the inner product is screened on codes only)
     const bool codes_possible = idx->dim <= (best_first ? coral::kMaxByteRowDim : coral::kMaxByteRowDimRounds);
     // (the rounds kernel takes codes for rows of more than 64 floats; half precision, and the best-first kernels,
@@ -606,7 +606,7 @@ static int probe_levels(coral_index* idx) {
 // dim picoseconds, and spare the rows (bytes each, on codes or in fp32) that a search reads without need, four in five, at
 // 7 TB/s: of x = 45 first visits per beam entry under L2, 1.7 times as many under the inner product, x / (1 + x / c n) as
 // the graph runs out of new nodes (c = 1 / 4 and 3 / 5).  The kernels for rows of more than 512 and 1024 floats spill
-// registers where this form does not: two and three times the bytes stand for that.
+// 34 .. 45 and 91 .. 171 vector registers where this form spills none and 4: two and three times the bytes stand for that.
 // Measured over 144 launches (30 000 .. 280 000 nodes of 64 .. 1028 floats, L = 32 .. 800, 512 .. 5000 queries), the time with over the
 // time without: spared / cost 1.5 1.13 (100 000 x 128, L = 32); 2.5 0.97 (L = 100); 5.1 0.69 (L = 256); inner product, 1.7 0.84 (200 000 x 512, L = 100);
 // 3.1 0.58 (60 000 x 512, L = 64); 11 0.46 (L = 256); 80 000 x 1028, L = 256, 0.22.  From 3 on, 2 under the inner product.
@@ -857,10 +857,6 @@ int coral_search_prepare(coral_index* idx, int32_t Q, int32_t L, const coral_tun
     // form), up to a third of what is free and 64 GiB.  wg_per_cu: what the chosen kernel's occupancy allows;
     // reprepare(packed): sets that kernel up in the packed form and returns its occupancy.
     idx->bf_ready = false, idx->bf_long = false, idx->bf_shared = false, idx->bf_screen = 0;
-    // Best-first with the beam in LDS screens rows in half precision too, where a CU holds sixteen wavefronts (beams
-    // without the LDS table: L > 409): +12 % at L = 512 and 1024.  With the table (eight wavefronts per CU) the extra
-    // wait per step costs more than the bytes it spares (L = 256 / 320: -27 %), so those launches go without unless
-    // the caller asks for it by name.
     if (long_form && (idx->dim / 4 > 32 || narrow_codes) && idx->dim <= coral::kMaxByteRowDim &&
         (t.screening == 2 || t.screening == 0)) {
         // the kernel of long beams screens on eight-bit codes only.  (The longer the queue, the larger the share of
@@ -1398,8 +1394,6 @@ int coral_search(coral_index* idx, const float* h_queries, int32_t Q, int32_t k,
         if (h_dists) std::memcpy(h_dists, hd, dbytes);
         return CORAL_OK;
     }
-    HIP_TRY(grow((void**)&idx->d_io_ids, &idx->io_ids_bytes, ibytes));
-    if (h_dists) HIP_TRY(grow((void**)&idx->d_io_dists, &idx->io_dists_bytes, dbytes));
     HIP_TRY(grow((void**)&idx->d_io_ids, &idx->io_ids_bytes, ibytes));
     if (h_dists) HIP_TRY(grow((void**)&idx->d_io_dists, &idx->io_dists_bytes, dbytes));
     HIP_TRY(hipMemcpy(idx->d_io_q, h_queries, qbytes, hipMemcpyHostToDevice));

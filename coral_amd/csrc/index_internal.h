@@ -109,7 +109,7 @@ struct coral_index {
     bool bf_shared = false;  // best-first: four wavefronts share a query's steps
     int bf_table_log2 = 0, bf_table_rem_bits = 0;
     // ... or, for long beams, with an insert buffer in LDS and the long sorted run of every slot in global memory
-    int bf_screen = 0;  // the kernel with the beam in LDS screens rows: 1 in half precision (d_vec16), 2 in eight-bit codes (d_vec8)
+    int bf_screen = 0;  // the wavefront kernels screen rows: 1 in half precision (d_vec16), 2 in eight-bit codes (d_vec8)
     bool bf_long = false;
     uint64_t* d_bf_beams = nullptr;
     size_t bf_beam_alloc_words = 0, bf_beam_stride = 0;
