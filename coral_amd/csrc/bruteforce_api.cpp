@@ -155,6 +155,7 @@ public:
         for (auto& p : parts_) *p.first = static_cast<char*>(base_) + p.second;
         return hipSuccess;
     }
+    size_t total() const { return total_; }
     // pinned room for the flags of Q queries and one more, or null: for the holder of the kept block
     int* flags(int32_t Q) const { return kept_ && Q < coral::kKnnFlags ? idx_->h_knn_flags : nullptr; }
 
@@ -203,16 +204,22 @@ struct FusedScreen {
         const int64_t expect = kc * (step > 1 ? (stride + step - 1) / step + step : stride) + kc;
         cap = 2048;
         while (cap < 3 * expect && cap < kListCap) cap <<= 1;
-        // Queries per block: a pass over the base for 4096 is hundreds of tiles per compute unit, and their lists of up to
-        // 8192 entries, beside the sample's matrix for 1024 queries at a time, stay within what is kept between calls (10 000
-        // queries of a million points, k = 100: 349 MB; with 2048 at a time 413, allocated and released by each call).
-        // Lists of 16 384, for k in the hundreds, do not.
+        // queries per block: a pass over the base for 4096 is hundreds of tiles per compute unit; the sample's matrix is
+        // made and read for 2048 at a time
         const int64_t rows = ((int64_t)Q + 127) & ~(int64_t)127;
         qc = std::min<int64_t>(4096, rows);
-        qs = std::min<int64_t>(1024, std::min(qc, std::max<int64_t>(256, (kBufferFloats / ns) & ~(int64_t)255)));
+        qs = std::min<int64_t>(2048, std::min(qc, std::max<int64_t>(256, (kBufferFloats / ns) & ~(int64_t)255)));
     }
     void reserve(const coral_index* idx, KnnScratch& mem) {
         if (!suits) return;
+        // What is kept between calls holds 4096 lists of up to 8192 entries beside the sample's matrix for 1024 queries, but not
+        // for 2048: 10 000 queries of a million points, k = 100, 349 MB and 413, which each call would allocate and release (11.0 and
+        // 11.4 ms).  Elsewhere half the queries at a time cost up to 8 % of a call.  (Lists of 16 384, for k in the hundreds, are not
+        // kept.)
+        const size_t lists_bytes = (size_t)qc * cap * sizeof(unsigned long long) + (size_t)qc * coral::kCntStride * sizeof(unsigned int) +
+                                   coral::split_queries_bytes((int)qc, idx->dim, 3) + 4096 * 8;  // (and the small parts, each rounded up)
+        const auto fits = [&](int64_t rows) { return mem.total() + lists_bytes + (size_t)rows * ns * sizeof(float) <= kKnnKeepBytes; };
+        if (!fits(qs) && qs > 1024 && fits(1024)) qs = 1024;
         mem.reserve(&D, (size_t)qs * ns), mem.reserve(&tau, (size_t)qc);
         mem.reserve(&lists, (size_t)qc * cap), mem.reserve(&cnt, (size_t)qc * coral::kCntStride);
         mem.reserve(&redo, (size_t)qs), mem.reserve(&overflow, 2);

@@ -460,8 +460,8 @@ def test_screening_on_one_product_answers_what_the_plain_passes_answer(law, metr
 @pytest.mark.parametrize("Q", [1, 3, 255, 257, 1024, 1025, 4500])
 @pytest.mark.parametrize("metric,dim,k", [("l2", 4, 1), ("ip", 12, 10), ("l2", 100, 10), ("ip", 260, 33), ("l2", 516, 5)])
 def test_prepared_queries_at_the_edges_of_tiles_and_flags(Q, metric, dim, k):
-    """Batches about the query tile of 256, the 1024 queries whose flags go to pinned memory and sample
-    is looked at at a time, and the 4096 of a block of the screening; dimensions short of a stage of 16 and beyond the 64 lanes that read a row.  Twice on one index (the
+    """Batches about the query tile of 256, the 1024 queries whose flags go to pinned memory and the 2048 and 4096 of a block
+    of the screening; dimensions short of a stage of 16 and beyond the 64 lanes that read a row.  Twice on one index (the
     counters start at zero again), and with every second base row equal, where lists overflow or leave ties open: ids and
     distance bits are those of the search that measures every pair."""
     rng = np.random.RandomState(Q + dim)
