@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kWavesPerWg * 64, WGS) void best_first_wave_kernel(
     constexpr int kMine = kBatch / WPQ;  // rows of a step per wavefront
     extern __shared__ __align__(16) unsigned char smem[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int slot = WPQ > 1 ? (int)blockIdx.x : (int)(blockIdx.x * (blockDim.x >> 6)) + wave;
+    const int slot = WPQ > 1 ? (int)blockIdx.x : (int)blockIdx.x * b.waves_per_wg + wave;
     const int part = WPQ > 1 ? wave : 0;  // the wavefront's place among those of its query
     if (slot >= b.slots) return;  // the whole wavefront, and where a workgroup has barriers the whole workgroup
     const int L = a.L, R = a.R, dim = a.dim, chunks = dim >> 2, M = a.M;
